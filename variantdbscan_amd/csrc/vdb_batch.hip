@@ -1,5 +1,4 @@
-// Batched variants from one fine grid and one truncated, distance-sorted
-// neighbour table.
+// Batched variants from one fine grid and one truncated neighbour table.
 //
 // Levels k = 0..K-1 are the distinct eps values in ascending order (T_k their
 // thresholds), j = 0..J-1 the distinct minpts values, L = max minpts.
@@ -8,9 +7,10 @@
 //     clique at eps_0 (its point bbox diagonal passes the exact predicate),
 //     so all core points of a cell are mutually connected at every level.
 //  2. Truncated table: for each point of a cell holding fewer than L points,
-//     the L nearest neighbours within eps_{K-1}, sorted by (s, id). A smaller
-//     eps is a prefix cut of that list and a larger minpts a filter on its
-//     length; points of cells holding >= L points have >= L neighbours within
+//     its neighbours with their levels, at all levels below the first with L
+//     neighbours (from there on the point is core for every minpts value).
+//     A smaller eps is a filter on the levels and a larger minpts one on the
+//     counts; points of cells holding >= L points have >= L neighbours within
 //     eps_0 and are core in every variant.
 //  3. Core level kc_j(p) = first k with count_k(p) >= m_j.
 //  4. Cell pairs within eps_{K-1} (bbox distance), with the first level at
@@ -64,8 +64,10 @@ constexpr unsigned kMaxPersistent = 1024; // largest maxb of kBatchShapes
 struct FG {
     const double *xs, *ys, *box;
     const uint32_t *cell_start, *cell_of_pos, *row_lo, *row_hi;
-    const uint32_t *cell_key, *cell_ds, *sncy;
-    int W;
+    const uint32_t *cell_key;
+    const uint2 *row_pts, *row_in;
+    int W, m, RSin; // window rows (2 RS + 1), strip width, inner rows each way
+    double wlow;    // points |k| columns apart differ by at least (|k| - 1) wlow in x
 };
 
 // Truncated lists are stored in blocks of 64 lists, entry-major inside a
@@ -81,7 +83,10 @@ __host__ __device__ __forceinline__ size_t lst_at(uint32_t i, uint32_t e, int L)
 FG fview(const Grid &G)
 {
     return FG{G.xs,     G.ys,       G.cell_box, G.cell_start, G.cell_of_pos, G.row_lo,
-              G.row_hi, G.cell_key, G.cell_ds,  G.sncy,       2 * G.R + 1};
+              G.row_hi, G.cell_key, G.row_pts,  G.row_in,     2 * G.RS + 1,  G.m,
+              G.RSin,
+              // computed cell coordinates are within 2^-31 of exact
+              G.w * (1.0 - std::ldexp(1.0, -20))};
 }
 
 __device__ __forceinline__ uint32_t ld_u32(const uint32_t *p)
@@ -156,17 +161,35 @@ __device__ __forceinline__ void cf_hook(uint32_t *parent, uint32_t x, uint32_t m
 }
 
 // ------------------------------------------------------------- cliques
-__global__ void k_clique_check(const double *box, uint32_t ncell, double T0, uint32_t *bad)
+// bad[0] counts the cells that are not cliques at eps_0, bad[1] the points of
+// cells with < L points (those that get a neighbour list)
+__global__ void __launch_bounds__(kBlock)
+    k_clique_check(const double *box, const uint32_t *cell_start, uint32_t ncell, double T0,
+                   uint32_t L, uint32_t *bad)
 {
     uint32_t c = blockIdx.x * kBlock + threadIdx.x;
-    if (c >= ncell) return;
-    const double *b = box + 4 * (size_t)c;
-    double dx = __dsub_rn(b[1], b[0]), dy = __dsub_rn(b[3], b[2]);
-    double s = __dadd_rn(__dmul_rn(dx, dx), __dmul_rn(dy, dy));
-    if (!(s <= T0)) atomicAdd(bad, 1u);
+    uint32_t listed = 0;
+    if (c < ncell) {
+        const double *b = box + 4 * (size_t)c;
+        double dx = __dsub_rn(b[1], b[0]), dy = __dsub_rn(b[3], b[2]);
+        double s = __dadd_rn(__dmul_rn(dx, dx), __dmul_rn(dy, dy));
+        if (!(s <= T0)) atomicAdd(bad, 1u);
+        uint32_t pop = cell_start[c + 1] - cell_start[c];
+        listed = pop < L ? pop : 0u;
+    }
+    for (int o = kWave / 2; o > 0; o >>= 1) listed += __shfl_xor(listed, o);
+    __shared__ uint32_t sm[kWPB];
+    if (lane_id() == 0) sm[wave_id_in_block()] = listed;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < kWPB; w++) listed += sm[w];
+        if (listed) atomicAdd(bad + 1, listed);
+    }
 }
 
 // ------------------------------------------------------ list membership
+// Lists are kept at their point's position unless that takes too much memory;
+// then the listed points (those of cells with < L points) are numbered.
 __global__ void k_list_flags(const uint32_t *cell_start, const uint32_t *cell_of_pos,
                              uint32_t n, uint32_t L, uint32_t *flag)
 {
@@ -176,409 +199,558 @@ __global__ void k_list_flags(const uint32_t *cell_start, const uint32_t *cell_of
     flag[p] = (cell_start[c + 1] - cell_start[c] < L) ? 1u : 0u;
 }
 
-// A listed point's list index, and the point itself (coordinates and cell)
-// stored at that index: the list kernel's first loads then need nothing else.
-__global__ void k_list_index(const uint32_t *flag, const uint32_t *excl, const double *xs,
-                             const double *ys, const uint32_t *cell_of_pos, uint32_t n,
-                             double2 *list_xy, uint32_t *list_cell, uint32_t *lst_idx)
-{
-    uint32_t p = blockIdx.x * kBlock + threadIdx.x;
-    if (p >= n) return;
-    if (flag[p]) {
-        uint32_t i = excl[p];
-        list_xy[i] = make_double2(xs[p], ys[p]);
-        list_cell[i] = cell_of_pos[p];
-        lst_idx[p] = i;
-    } else {
-        lst_idx[p] = kNone;
-    }
-}
-
-
 // ------------------------------------------------------ truncated table
-// One wave per listed point. Lane e < L holds entry e of the sorted list.
-__device__ __forceinline__ bool before(double s1, uint32_t i1, double s2, uint32_t i2)
+// Neighbour search of every listed point. A point's list holds its neighbours
+// at levels below its cutoff: the first level at which it has L neighbours
+// (K when it never has). Whatever lies at the cutoff or above is never asked
+// for: the point is core there for every minpts value. So the search keeps
+// only counts per level (8 bits each, packed in registers) and appends
+// (position, level) to the point's list in the order met; nothing is sorted,
+// and the radius shrinks to the last level below the cutoff whenever the
+// cutoff falls.
+//
+// Windows are walked row by row (a row is a strip of columns), centre out, as
+// far as the radius reaches. Where a window is dense, the cells that can hold
+// level-0 neighbours go first, so that a point with L neighbours at level 0
+// sees little more than those.
+//
+// The kernel of a point follows its window's population, because the cost is
+// the serial walk of a lane (about 1 us per step of a latency-bound wave) on
+// one side and the instructions of group and wave bookkeeping on the other:
+//   <= kNearMid       a thread per point, kNearUnroll candidates per step;
+//                     a point whose list fills up goes on to the next kernel
+//   <= kNearCrowded   kNearGroup lanes per point
+//   more              a wave per point, cells pruned by their box
+// Times of the three kernels together against the wave per point for all
+// (which kept the L nearest sorted), MI355X: 256 sets of 17.8M points x 4 eps
+// 11.3 ms against 26.9; 8M skewed points, 1 eps: 1.2 ms against 3.3; 2M points
+// x 8 eps 1.4 ms against 2.1. One thread for windows up to 512 points took
+// 1.5 ms instead of 0.4 on the last (waves wait for their longest walk), 16
+// lanes for windows up to 1024 points 1.1 ms more on the first.
+constexpr uint32_t kNearMid = 128;
+constexpr uint32_t kNearCrowded = 512;
+constexpr int kNearGroup = 16;
+constexpr int kNearUnroll = 4;
+// windows above about this many points take the inner cells first
+constexpr uint32_t kNearDense = 256;
+
+// squared lower bound of the distance of row t's points from the points of
+// the cell with column offset o in its strip
+__device__ __forceinline__ double row_gap2(const FG &g, int t, int o)
 {
-    return s1 < s2 || (s1 == s2 && i1 < i2);
+    int k = t > 0 ? t * g.m - o - 1 : (t < 0 ? o - (t + 1) * g.m : 0); // whole columns between
+    double gap = (double)k * g.wlow;
+    return gap * gap;
 }
 
-// Insert the candidates of one 64-lane block that pass `hit` into the sorted
-// lane-resident list (entry e in lane e < L), keeping the L smallest (s, id).
-__device__ __forceinline__ void knn_block(double s, uint32_t q, bool hit, int L, double Tmax,
-                                          double &es, uint32_t &eid, int &cnt, double &kth,
-                                          uint32_t &kid, double &thr)
+template <int G> __device__ __forceinline__ uint32_t group_or(uint32_t v)
 {
-    int lane = lane_id();
-    uint64_t hm = ballot(hit);
-    while (hm) {
-        int hb = __builtin_ctzll(hm);
-        hm &= hm - 1;
-        double cs = __shfl(s, hb);
-        uint32_t cq = __shfl(q, hb);
-        if (cnt == L && !before(cs, cq, kth, kid)) continue;
-        bool lt = lane < L && before(es, eid, cs, cq);
-        int pos = popc64(ballot(lt));
-        double ps = lane_up1_f64(es);
-        uint32_t pid = lane_up1(eid);
-        if (lane == pos) {
-            es = cs;
-            eid = cq;
-        } else if (lane > pos && lane < L) {
-            es = ps;
-            eid = pid;
-        }
-        if (cnt < L) cnt++;
-        if (cnt == L) {
-            kth = __shfl(es, L - 1);
-            kid = __shfl(eid, L - 1);
-            thr = kth < Tmax ? kth : Tmax;
-        }
+    if constexpr (G > 1) v |= lane_xor<1>(v);
+    if constexpr (G > 2) v |= lane_xor<2>(v);
+    if constexpr (G > 4) v |= lane_xor<4>(v);
+    if constexpr (G > 8) v |= lane_xor<8>(v);
+    return v;
+}
+// sum over the group of values packed in bytes or wider fields without carries
+template <int J> __device__ __forceinline__ uint64_t lane_xor_u64(uint64_t v)
+{
+    return ((uint64_t)lane_xor<J>((uint32_t)(v >> 32)) << 32) | lane_xor<J>((uint32_t)v);
+}
+template <int G> __device__ __forceinline__ uint64_t group_sum(uint64_t v)
+{
+    if constexpr (G > 1) v += lane_xor_u64<1>(v);
+    if constexpr (G > 2) v += lane_xor_u64<2>(v);
+    if constexpr (G > 4) v += lane_xor_u64<4>(v);
+    if constexpr (G > 8) v += lane_xor_u64<8>(v);
+    return v;
+}
+
+// v, the same in every lane, in scalar registers
+__device__ __forceinline__ double uniform_f64(double v)
+{
+    uint64_t u = (uint64_t)__double_as_longlong(v);
+    uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)u);
+    uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(u >> 32));
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+
+// lanes of the group that pass, bit 0 its first lane
+template <int G> __device__ __forceinline__ uint32_t group_ballot(bool pass)
+{
+    if constexpr (G == 1) return pass ? 1u : 0u;
+    return (uint32_t)(ballot(pass) >> (lane_id() & ~(G - 1))) & ((1u << G) - 1u);
+}
+// how many of them before this lane
+template <int G> __device__ __forceinline__ uint32_t group_rank(uint32_t m)
+{
+    if constexpr (G == 1) return 0u;
+    return (uint32_t)__popc(m & ((1u << (lane_id() & (G - 1))) - 1u));
+}
+
+// What the search of a point writes.
+struct NearOut {
+    const uint32_t *lst_idx; // list of a position (null: its own number)
+    uint32_t *lst_id;
+    uint8_t *lst_lev;
+    uint32_t *lst_n;
+    uint8_t *kc;
+    uint32_t *kc4;
+    int L, K, J;
+    const uint32_t *mj;
+};
+
+// Core levels of point p from its counts per level (each lane of the group
+// holds its own part): the first level with m_j neighbours, L at the cutoff;
+// lane gl of the group takes minpts values gl, gl + G, ...
+template <int KL, int G>
+__device__ __forceinline__ void near_levels(const NearOut &O, uint32_t p, const uint64_t *hist,
+                                            int cut)
+{
+    constexpr int KW = (KL + 7) / 8;
+    const int gl = lane_id() & (G - 1);
+    uint64_t tot[KW];
+#pragma unroll
+    for (int w = 0; w < KW; w++) tot[w] = group_sum<G>(hist[w]);
+    uint32_t packed = 0;
+    for (int j = gl; j < O.J; j += G) {
+        uint32_t need = O.mj[j];
+        int lev = 0;
+        uint32_t run = 0;
+#pragma unroll
+        for (int w = 0; w < KW; w++)
+#pragma unroll
+            for (int b = 0; b < 8; b++) {
+                if (8 * w + b >= KL) continue;
+                run += (uint32_t)(tot[w] >> (8 * b)) & 0xffu;
+                lev += (8 * w + b < cut && run < need) ? 1 : 0;
+            }
+        if (need > 0x7fffffffu) lev = O.K;
+        O.kc[(size_t)p * O.J + j] = (uint8_t)lev;
+        packed |= (uint32_t)(lev & 15) << (4 * (j & 7));
+    }
+    // with J <= 8 and K <= 15 also packed, 4 bits per minpts value, for the
+    // label pass that takes all variants of a call at once
+    if (O.kc4) {
+        packed = group_or<G>(packed);
+        if (gl == 0) O.kc4[p] = packed;
     }
 }
 
+// The search of point p of cell c, whose window holds `window` points. KL:
+// at least K; sT (LDS) holds the level thresholds, INF beyond K.
+// False: the list filled up with entries some of which lie above the cutoff,
+// and a single thread (whose 63 neighbours would wait) does not sort them out.
+template <int KL, int G, int U>
+__device__ __forceinline__ bool near_point(const FG &g, const NearOut &O, const double *sT,
+                                           uint32_t p, uint32_t c, uint32_t window)
+{
+    constexpr int KW = (KL + 7) / 8;
+    const int gl = lane_id() & (G - 1);
+    const int L = O.L, K = O.K;
+    uint64_t hist[KW]; // neighbours per level seen by this lane, a byte each
+#pragma unroll
+    for (int w = 0; w < KW; w++) hist[w] = 0;
+    int cut = K; // first level with L neighbours
+    {
+        const int R = g.W / 2, Win = 2 * g.RSin + 1;
+        const uint2 *rows = g.row_pts + (size_t)c * g.W + R; // row d at rows[d]
+        const uint2 *inner = g.row_in ? g.row_in + (size_t)c * Win + g.RSin : nullptr;
+        const int o = (int)(g.cell_key[c] % (uint32_t)g.m);
+        const size_t li = O.lst_idx ? O.lst_idx[p] : p;
+        uint32_t *ids = O.lst_id + lst_at((uint32_t)li, 0, L);
+        uint8_t *levs = O.lst_lev + lst_at((uint32_t)li, 0, L);
+        uint32_t kept = 0; // neighbours found at levels below cut (< L)
+        uint32_t len = 0;  // entries stored, those of levels >= cut among them
+        bool full = false; // a thread's list has no room left
+        const double px = g.xs[p], py = g.ys[p];
+        double thr = sT[K - 1];
+        // thresholds in scalar registers while they fit
+        double T[KL <= 8 ? KL : 1];
+        if constexpr (KL <= 8)
+#pragma unroll
+            for (int k = 0; k < KL; k++) T[k] = uniform_f64(sT[k]);
+        auto take = [&](double s, uint32_t t) {
+            bool hit = s <= thr;
+            uint32_t hm = group_ballot<G>(hit);
+            if (!hm) return;
+            int lev = 0;
+#pragma unroll
+            for (int k = 0; k < KL - 1; k++) lev += s > (KL <= 8 ? T[k] : sT[k]) ? 1 : 0;
+#pragma unroll
+            for (int w = 0; w < KW; w++)
+                if (hit && (KW == 1 || (lev >> 3) == w)) hist[w] += 1ull << (8 * (lev & 7));
+            kept += (uint32_t)__popc(hm);
+            if (kept >= (uint32_t)L) {
+                // the cutoff falls to the first level with L neighbours
+                uint32_t run = 0, before = 0;
+                int k = 0;
+                bool there = false;
+#pragma unroll
+                for (int w = 0; w < KW; w++) {
+                    uint64_t h = group_sum<G>(hist[w]);
+#pragma unroll
+                    for (int b = 0; b < 8; b++)
+                        if (8 * w + b < KL && !there) {
+                            before = run;
+                            run += (uint32_t)(h >> (8 * b)) & 0xffu;
+                            there = run >= (uint32_t)L;
+                            k = 8 * w + b;
+                        }
+                }
+                cut = k;
+                kept = before;
+                thr = cut ? sT[cut - 1] : -1.0;
+                hit = hit && lev < cut;
+                hm = group_ballot<G>(hit);
+            }
+            uint32_t h = (uint32_t)__popc(hm);
+            if (len + h > (uint32_t)L) {
+                if constexpr (G == 1) {
+                    full = true; // left to the group kernel
+                    return;
+                }
+                // drop the entries at or above the cutoff, two reads of a
+                // lane in flight together
+                constexpr int C = 2;
+                uint32_t to = 0;
+                for (uint32_t e0 = 0; e0 < len; e0 += C * G) {
+                    uint8_t v[C];
+                    uint32_t id[C];
+#pragma unroll
+                    for (int x = 0; x < C; x++) {
+                        uint32_t i = e0 + (uint32_t)(x * G + gl);
+                        uint32_t ic = i < len ? i : len - 1;
+                        v[x] = levs[(size_t)ic * 64u];
+                        id[x] = ids[(size_t)ic * 64u];
+                        if (i >= len) v[x] = 0xff;
+                    }
+#pragma unroll
+                    for (int x = 0; x < C; x++) {
+                        bool stay = (int)v[x] < cut;
+                        uint32_t sm = group_ballot<G>(stay);
+                        if (stay) {
+                            uint32_t at = to + group_rank<G>(sm);
+                            ids[(size_t)at * 64u] = id[x];
+                            levs[(size_t)at * 64u] = v[x];
+                        }
+                        to += (uint32_t)__popc(sm);
+                    }
+                }
+                len = to;
+            }
+            if (hit) {
+                uint32_t at = len + group_rank<G>(hm);
+                ids[(size_t)at * 64u] = t;
+                levs[(size_t)at * 64u] = (uint8_t)lev;
+            }
+            len += h;
+        };
+        uint32_t q = 0, e = 0, q2 = 0, e2 = 0; // the span walked, one waiting
+        int u = 0;                             // rows started
+        bool first = inner && window > kNearDense;
+        const bool split = first;
+        while (true) {
+            if (q >= e) {
+                if (q2 < e2) {
+                    q = q2;
+                    e = e2;
+                    q2 = e2;
+                } else if (first) {
+                    if (u == Win) {
+                        // level 0 is complete; with the cutoff at level 1 or
+                        // below nothing beyond it matters
+                        if (cut <= 1) break;
+                        first = false;
+                        u = 0;
+                        continue;
+                    }
+                    int d = (u & 1) ? -((u + 1) >> 1) : (u >> 1);
+                    uint2 r = inner[d];
+                    q = r.x;
+                    e = r.x + r.y;
+                    u++;
+                } else {
+                    if (u == g.W) break;
+                    int ad = (u + 1) >> 1;
+                    int d = (u & 1) ? -ad : ad;
+                    u++;
+                    if (row_gap2(g, d, o) > thr) continue;
+                    uint2 r = rows[d];
+                    q = r.x;
+                    e = r.x + r.y;
+                    if (split && ad <= g.RSin) {
+                        uint2 in = inner[d]; // seen already: the parts beside it
+                        if (in.y) {
+                            q2 = in.x + in.y;
+                            e2 = e;
+                            e = in.x;
+                        }
+                    }
+                }
+            }
+            if (q < e) {
+                // U candidates a lane, their loads issued together
+                double s[U];
+                uint32_t t[U];
+#pragma unroll
+                for (int i = 0; i < U; i++) {
+                    t[i] = q + (uint32_t)(i * G + gl);
+                    uint32_t tc = t[i] < e ? t[i] : e - 1;
+                    s[i] = dist2_exact(px, py, g.xs[tc], g.ys[tc]);
+                    if (t[i] >= e) s[i] = INFINITY;
+                }
+#pragma unroll
+                for (int i = 0; i < U; i++) take(s[i], t[i]);
+                q += U * G;
+                if (cut == 0 || full) break;
+            }
+        }
+        if (full && cut) return false;
+        if (gl == 0) O.lst_n[li] = cut ? len : 0u;
+    }
+    near_levels<KL, G>(O, p, hist, cut);
+    return true;
+}
+
+// append v to list for every lane with take set, one atomic per wave
+__device__ __forceinline__ void list_append(bool take, uint32_t v, uint32_t *list, uint32_t *count)
+{
+    uint64_t m = ballot(take);
+    if (!m) return;
+    int leader = __builtin_ctzll(m);
+    uint32_t base = 0;
+    if (lane_id() == leader) base = atomicAdd(count, (uint32_t)popc64(m));
+    base = __shfl(base, leader);
+    if (take) list[base + mask_rank(m)] = v;
+}
+
+// Every point: core levels of the points of cells with >= L points at once,
+// the search of points with small windows by a thread each, the others to the
+// lists of k_knn_group and k_knn_crowded. few[0] and few[1] count the lists.
+template <int KL>
+__global__ void __launch_bounds__(kBlock)
+    k_knn(FG g, NearOut O, const double *__restrict__ Tk, uint32_t n, uint32_t mid_from,
+          uint32_t crowd_from, uint32_t *__restrict__ mid, uint32_t *__restrict__ crowd,
+          uint32_t *__restrict__ few)
+{
+    __shared__ double sT[KL];
+    if (threadIdx.x < KL) sT[threadIdx.x] = Tk[threadIdx.x];
+    __syncthreads();
+    const uint32_t p = blockIdx.x * kBlock + threadIdx.x;
+    uint32_t c = 0, window = 0;
+    bool listed = false;
+    if (p < n) {
+        c = g.cell_of_pos[p];
+        listed = g.cell_start[c + 1] - g.cell_start[c] < (uint32_t)O.L;
+        if (listed) {
+            const uint2 *rows = g.row_pts + (size_t)c * g.W;
+            for (int d = 0; d < g.W; d++) window += rows[d].y;
+        } else {
+            const uint64_t none[(KL + 7) / 8] = {};
+            near_levels<KL, 1>(O, p, none, 0); // a clique of L points
+        }
+    }
+    bool later = window > mid_from && window <= crowd_from;
+    list_append(window > crowd_from, p, crowd, few + 1);
+    if (listed && window <= mid_from)
+        later = !near_point<KL, 1, kNearUnroll>(g, O, sT, p, c, window);
+    list_append(later, p, mid, few);
+}
+
+// The points of middling windows, a group of kNearGroup lanes each.
+constexpr unsigned kListBlocks = 8192; // grids of the list kernels, at most
+template <int KL>
+__global__ void __launch_bounds__(kBlock)
+    k_knn_group(FG g, NearOut O, const double *__restrict__ Tk, const uint32_t *__restrict__ mid,
+                const uint32_t *__restrict__ nmid)
+{
+    constexpr int G = kNearGroup;
+    const uint32_t nm = *nmid;
+    if (blockIdx.x * (kBlock / G) >= nm) return;
+    __shared__ double sT[KL];
+    if (threadIdx.x < KL) sT[threadIdx.x] = Tk[threadIdx.x];
+    __syncthreads();
+    for (uint32_t i = blockIdx.x * (kBlock / G) + threadIdx.x / G; i < nm;
+         i += gridDim.x * (kBlock / G)) {
+        const uint32_t p = mid[i], c = g.cell_of_pos[p];
+        uint32_t window = 0;
+        const uint2 *rows = g.row_pts + (size_t)c * g.W;
+        for (int d = 0; d < g.W; d++) window += rows[d].y;
+        near_point<KL, kNearGroup, 1>(g, O, sT, p, c, window);
+    }
+}
+
+// The same search for the points of crowded windows: a wave per point, 64
+// candidates per step. Up to 64 entries are held in the lanes. The inner rows
+// go first; then, row by row from the centre, the cells outside them, pruned
+// by their exact box bound against the radius.
 // spans of a row holding at most this many points are swept whole, without
 // per-cell pruning
 constexpr uint32_t kKnnRowSweep = 512;
-// windows holding at most this many points are swept as one flat list
-constexpr uint32_t kKnnFlat = 512;
-
-// one compare-exchange stage of a bitonic network: partner lane ^ J, groups
-// of k sorted ascending when (lane & k) == 0
-template <int J>
-__device__ __forceinline__ void bitonic_stage(double &es, uint32_t &eid, int k, int lane)
+__global__ void __launch_bounds__(kBlock)
+    k_knn_crowded(FG g, NearOut O, const double *__restrict__ Tk,
+                  const uint32_t *__restrict__ crowd, const uint32_t *__restrict__ ncrowd)
 {
-    double ps = lane_xor_f64<J>(es);
-    uint32_t pid = lane_xor<J>(eid);
-    bool low = (lane & J) == 0, asc = (lane & k) == 0;
-    // the lower lane of an ascending pair keeps the smaller entry
-    bool take = (low == asc) ? before(ps, pid, es, eid) : before(es, eid, ps, pid);
-    if (take) {
-        es = ps;
-        eid = pid;
-    }
-}
-
-// sort the lane-resident entries (lane e holds entry e) by (s, id), ascending.
-// Only lanes below cnt hold entries (the rest hold (INF, NONE)), so the
-// bitonic network stops at the first power of two >= cnt: its stages sort
-// every aligned group of that size, the first one ascending. The partner
-// exchanges are DPP moves and row swaps, not LDS permutes.
-__device__ __forceinline__ void wave_sort(double &es, uint32_t &eid, int cnt)
-{
-    int lane = lane_id();
-    if (cnt > 1) {
-        bitonic_stage<1>(es, eid, 2, lane);
-    }
-    if (cnt > 2) {
-        bitonic_stage<2>(es, eid, 4, lane);
-        bitonic_stage<1>(es, eid, 4, lane);
-    }
-    if (cnt > 4) {
-        bitonic_stage<4>(es, eid, 8, lane);
-        bitonic_stage<2>(es, eid, 8, lane);
-        bitonic_stage<1>(es, eid, 8, lane);
-    }
-    if (cnt > 8) {
-        bitonic_stage<8>(es, eid, 16, lane);
-        bitonic_stage<4>(es, eid, 16, lane);
-        bitonic_stage<2>(es, eid, 16, lane);
-        bitonic_stage<1>(es, eid, 16, lane);
-    }
-    if (cnt > 16) {
-        bitonic_stage<16>(es, eid, 32, lane);
-        bitonic_stage<8>(es, eid, 32, lane);
-        bitonic_stage<4>(es, eid, 32, lane);
-        bitonic_stage<2>(es, eid, 32, lane);
-        bitonic_stage<1>(es, eid, 32, lane);
-    }
-    if (cnt > 32) {
-        bitonic_stage<32>(es, eid, 64, lane);
-        bitonic_stage<16>(es, eid, 64, lane);
-        bitonic_stage<8>(es, eid, 64, lane);
-        bitonic_stage<4>(es, eid, 64, lane);
-        bitonic_stage<2>(es, eid, 64, lane);
-        bitonic_stage<1>(es, eid, 64, lane);
-    }
-}
-
-// 8 waves per SIMD: the search is latency-bound, so occupancy pays more
-// than the scalar registers it costs (their spills go to vector lanes)
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8, 8)))
-    k_knn(FG g, const double2 *__restrict__ list_xy, const uint32_t *__restrict__ list_cell,
-          const uint2 *__restrict__ row_pts, const uint32_t *__restrict__ nlist_dev,
-          int L, const double *__restrict__ Tk, int K, double *__restrict__ lst_s,
-          uint32_t *__restrict__ lst_id, uint32_t *__restrict__ lst_n)
-{
-    // the grid is sized for every point, the list count known on the device
-    // only: blocks wholly beyond it leave before anything else
-    const uint32_t nlist = *nlist_dev;
-    if (blockIdx.x * kWPB >= nlist) return;
-    // the level thresholds, for the level order of the entries
-    __shared__ double sTk[kMaxLevels];
-    for (int k = threadIdx.x; k < K; k += kBlock) sTk[k] = Tk[k];
-    __syncthreads();
-    const double Tmax = sTk[K - 1], T0 = sTk[0];
-    // Two modes. While at most 64 candidates within eps_max have been seen,
-    // they are appended unsorted (compacted through LDS) and put in level
-    // order once at the end: a sparse point costs one counting pass instead
-    // of one insertion per candidate. A block that would overflow 64 entries
-    // sorts by (s, id), keeps the L smallest and switches to sorted
-    // insertion with a shrinking threshold (an order by s is also one by
-    // level).
+    const int L = O.L, K = O.K, J = O.J;
+    const uint32_t nc = *ncrowd;
+    if (blockIdx.x * kWPB >= nc) return;
+    __shared__ double sT[kMaxLevels];
     __shared__ double abuf_s[kWPB][kWave];
     __shared__ uint32_t abuf_id[kWPB][kWave];
-    uint32_t i = blockIdx.x * kWPB + wave_id_in_block();
-    if (i >= nlist) return;
+    for (int k = threadIdx.x; k < K; k += kBlock) sT[k] = Tk[k];
+    __syncthreads();
     double *bs = abuf_s[wave_id_in_block()];
     uint32_t *bid = abuf_id[wave_id_in_block()];
-    int lane = lane_id();
-    double2 pxy = list_xy[i];
-    double px = pxy.x, py = pxy.y;
-    uint32_t c = list_cell[i];
-    double es = INFINITY;  // entry s of this lane
-    uint32_t eid = kNone;  // entry id
-    int cnt = 0;           // entries held (uniform)
-    double kth = INFINITY; // L-th smallest s once the list is full (uniform)
-    uint32_t kid = kNone;
-    double thr = Tmax;     // candidates must have s <= thr
-    bool done = false;
-    bool appending = true;
-    // The list's consumers need its entries in order of level (the first k
-    // with s <= T_k), not of s: the core levels are the levels of entries
-    // m_j - 1, and a label walk stops at the first entry beyond its largest
-    // eps. Appended entries that end the search in append mode are only put
-    // in level order (a stable counting pass over the <= 64 lane-resident
-    // entries), and truncated to L: the entries cut are all of the level at
-    // which the point holds L neighbours, where it is core for every minpts
-    // value, so no walk reads them.
-    auto settle_levels = [&]() {
-        int lvl = K;
-        if (lane < cnt) {
-            lvl = 0;
-            while (lvl < K - 1 && es > sTk[lvl]) lvl++;
+    const int lane = lane_id();
+    const int R = g.W / 2, Win = 2 * g.RSin + 1;
+    const uint32_t need = lane < J ? O.mj[lane] : 0u;
+    for (uint32_t i = blockIdx.x * kWPB + wave_id_in_block(); i < nc; i += gridDim.x * kWPB) {
+        const uint32_t p = __builtin_amdgcn_readfirstlane(crowd[i]);
+        const uint32_t c = __builtin_amdgcn_readfirstlane(g.cell_of_pos[p]);
+        const double px = g.xs[p], py = g.ys[p];
+        // lane u holds the u-th row centre-out: its cells, and the points of
+        // its inner part
+        uint32_t rlo = 0, rhi = 0, ia = 0, in = 0;
+        if (lane < g.W) {
+            int d = (lane & 1) ? -((lane + 1) >> 1) : (lane >> 1);
+            size_t t = (size_t)c * g.W + (d + R);
+            rlo = g.row_lo[t];
+            rhi = g.row_hi[t];
+            if (g.row_in && lane < Win) {
+                uint2 r = g.row_in[(size_t)c * Win + (d + g.RSin)];
+                ia = r.x;
+                in = r.y;
+            }
         }
-        const uint64_t valid = cnt >= kWave ? ~0ull : ((1ull << cnt) - 1ull);
-        // lanes of a smaller level (less) and of the same level (eq)
-        uint64_t less = 0, eq = valid;
-#pragma unroll
-        for (int b = 5; b >= 0; b--) {
-            bool bit = (lvl >> b) & 1;
-            uint64_t bal = ballot(bit) & valid;
-            if (bit) less |= eq & ~bal;
-            eq &= bit ? bal : (valid & ~bal);
-        }
-        if (lane < cnt) {
-            int at = popc64(less) + mask_rank(eq);
-            bs[at] = es;
-            bid[at] = eid;
-        }
-        __builtin_amdgcn_wave_barrier();
-        if (lane < cnt && lane < L) {
-            es = bs[lane];
-            eid = bid[lane];
-        } else {
-            es = INFINITY;
-            eid = kNone;
-        }
-        __builtin_amdgcn_wave_barrier();
-        cnt = cnt < L ? cnt : L;
-        appending = false;
-    };
-    // sort the appended entries, keep the L smallest, enter insertion mode
-    auto settle = [&]() {
-        wave_sort(es, eid, cnt);
-        if (lane >= L) {
-            es = INFINITY;
-            eid = kNone;
-        }
-        cnt = cnt < L ? cnt : L;
-        if (cnt == L) {
-            kth = __shfl(es, L - 1);
-            kid = __shfl(eid, L - 1);
-            thr = kth < Tmax ? kth : Tmax;
-        }
-        appending = false;
-    };
-    // one block of candidates: lane's candidate q at squared distance s
-    // (INF: no candidate)
-    auto block = [&](double s, uint32_t q) {
-        if (appending) {
-            bool hit = s <= Tmax;
-            uint64_t hm = ballot(hit);
-            int h = popc64(hm);
-            if (cnt + h <= kWave) {
+        const int o = (int)(g.cell_key[c] % (uint32_t)g.m);
+        double es = INFINITY; // entry of this lane
+        uint32_t eid = 0;
+        uint32_t cnt = 0; // entries held (uniform), all at levels < cut
+        int cut = K;
+        double thr = sT[K - 1];
+        // candidates [a, e), 64 per step, until L are found at level 0
+        auto sweep = [&](uint32_t a, uint32_t e) {
+            for (uint32_t q0 = a; q0 < e && cut; q0 += kWave) {
+                uint32_t q = q0 + (uint32_t)lane;
+                uint32_t qc = q < e ? q : e - 1;
+                double s = dist2_exact(px, py, g.xs[qc], g.ys[qc]);
+                if (q >= e) s = INFINITY;
+                bool hit = s <= thr;
+                uint64_t hm = ballot(hit);
+                if (!hm) continue;
+                uint32_t h = (uint32_t)popc64(hm);
+                if (cnt + h >= (uint32_t)L) {
+                    // the cutoff falls to the first level with L neighbours;
+                    // entries at or above it go
+                    int k = 0;
+                    while (k < cut - 1 &&
+                           (uint32_t)(popc64(ballot(es <= sT[k])) + popc64(ballot(s <= sT[k]))) <
+                               (uint32_t)L)
+                        k++;
+                    cut = k;
+                    if (cut == 0) return;
+                    thr = sT[cut - 1];
+                    bool keep = es <= thr;
+                    uint64_t km = ballot(keep);
+                    hit = s <= thr;
+                    hm = ballot(hit);
+                    if (keep) {
+                        bs[mask_rank(km)] = es;
+                        bid[mask_rank(km)] = eid;
+                    }
+                    cnt = (uint32_t)popc64(km);
+                    h = (uint32_t)popc64(hm);
+                } else if ((uint32_t)lane < cnt) {
+                    bs[lane] = es;
+                    bid[lane] = eid;
+                }
                 if (hit) {
-                    int at = cnt + mask_rank(hm);
-                    bs[at] = s;
-                    bid[at] = q;
+                    bs[cnt + mask_rank(hm)] = s;
+                    bid[cnt + mask_rank(hm)] = q;
                 }
-                __builtin_amdgcn_wave_barrier();
-                if (lane >= cnt && lane < cnt + h) {
-                    es = bs[lane];
-                    eid = bid[lane];
-                }
-                __builtin_amdgcn_wave_barrier();
                 cnt += h;
-                // L entries within eps_0: core in every variant, list unused
-                // (put in level order at the end)
-                if (cnt >= L && popc64(ballot(es <= T0)) >= L) done = true;
-                return;
+                __builtin_amdgcn_wave_barrier();
+                es = (uint32_t)lane < cnt ? bs[lane] : INFINITY;
+                eid = bid[lane];
+                __builtin_amdgcn_wave_barrier();
             }
-            settle();
-        }
-        bool hit = s <= thr && (cnt < L ? true : before(s, q, kth, kid));
-        knn_block(s, q, hit, L, Tmax, es, eid, cnt, kth, kid, thr);
-        // L neighbours within eps_0: core in every variant, list unused
-        if (cnt == L && kth <= T0) done = true;
-    };
-    int R = g.W / 2;
-    // All window rows' point ranges in one round of loads, lane l holding
-    // the l-th row centre-out (0, -1, +1, -2, ...). A window holding few
-    // points is swept as one flat list of candidates in that row order, 64
-    // per step, instead of row by row.
-    uint32_t ra = 0, rn = 0, rlo = 0, rhi = 0;
-    if (lane < g.W) {
-        int dl = (lane & 1) ? -((lane + 1) >> 1) : (lane >> 1);
-        size_t t = (size_t)c * g.W + (dl + g.W / 2);
-        rlo = g.row_lo[t];
-        rhi = g.row_hi[t];
-        uint2 rp = row_pts[t];
-        ra = rp.x;
-        rn = rp.y;
-    }
-    uint32_t pre = rn; // inclusive prefix over rows
-    for (int o = 1; o < kWave; o <<= 1) {
-        uint32_t t = __shfl_up(pre, o);
-        if (lane >= o) pre += t;
-    }
-    uint32_t total = __shfl(pre, kWave - 1);
-    pre -= rn; // exclusive
-    if (total <= kKnnFlat) {
-        for (uint32_t f0 = 0; f0 < total && !done; f0 += kWave) {
-            uint32_t f = f0 + lane;
-            // row of flat index f: the last row whose prefix is <= f
-            int row = 0;
-            for (int r = 1; r < g.W; r++)
-                row += (uint32_t)__builtin_amdgcn_readlane((int)pre, r) <= f ? 1 : 0;
-            uint32_t q = __shfl(ra, row) + (f - __shfl(pre, row));
-            double s = INFINITY;
-            if (f < total) s = dist2_exact(px, py, g.xs[q], g.ys[q]);
-            block(s, f < total ? q : kNone);
-        }
-        done = true;
-    }
-    // Rows path. The 3 x 3 cells around the point's own cell go first, so
-    // that the threshold is tight before the rest of the window is pruned
-    // against it; the rows then follow centre-out, skipping those cells.
-    // Keys are column-major (key = kbase + cx*ncy + cy) and a window row is
-    // one column cx+d, so the centre cells of row d are the cells of its
-    // range with keys within 1 of k0 + d*ncy. Steps 0..2 visit the centre
-    // cells of rows 0, -1, +1; steps 3.. the window rows 0, -1, +1, -2, ...
-    uint32_t k0 = g.cell_key[c], ncy = g.sncy[g.cell_ds[c]];
-    for (int t = 0; t < g.W + 3 && !done; t++) {
-        bool centre_pass = t < 3;
-        int u = centre_pass ? t : t - 3;
-        int d = (u & 1) ? -((u + 1) >> 1) : (u >> 1); // 0, -1, +1, -2, +2, ...
-        if (centre_pass && (d < -R || d > R)) continue;
-        // the row's cell range, held by lane u since the first loads
-        uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)rlo, u);
-        uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)rhi, u);
-        if (lo >= hi) continue;
-        uint32_t kc = k0 + (uint32_t)d * ncy;
-        // a row spans at most 2R+1 <= 64 cells
-        uint32_t C = lo + lane;
-        double S = INFINITY;
-        bool centre = false;
-        if (C < hi) {
-            const double *b = g.box + 4 * (size_t)C;
-            S = box_dist2_min(px, py, b[0], b[1], b[2], b[3]);
-            if (d >= -1 && d <= 1) {
-                uint32_t kC = g.cell_key[C];
-                centre = kC + 1u >= kc && kC <= kc + 1u;
+        };
+        if (g.row_in)
+            for (int u = 0; u < Win && cut; u++) {
+                uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)ia, u);
+                sweep(a, a + (uint32_t)__builtin_amdgcn_readlane((int)in, u));
             }
-        }
-        uint64_t mcen = ballot(centre);
-        // the cells to visit: the centre ones, or the others that can hold a
-        // candidate (exact box bound); the centre cells split the others
-        // into a part below and a part above them
-        uint64_t m = centre_pass ? mcen : ballot(S <= thr && !centre);
-        if (!m) continue;
-        uint64_t below = mcen && !centre_pass ? (1ull << __builtin_ctzll(mcen)) - 1ull : ~0ull;
-        uint64_t parts[2] = {m & below, m & ~below};
+        // (level 0 is complete after the inner rows: a cutoff of 1 ends there)
+        for (int u = 0; u < g.W && cut > (g.row_in ? 1 : 0); u++) {
+            int d = (u & 1) ? -((u + 1) >> 1) : (u >> 1); // 0, -1, +1, -2, +2, ...
+            uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)rlo, u);
+            uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)rhi, u);
+            if (lo >= hi || row_gap2(g, d, o) > thr) continue;
+            uint32_t sa = 0, se = 0; // the row's inner part, seen already
+            if (u < Win) {
+                sa = (uint32_t)__builtin_amdgcn_readlane((int)ia, u);
+                se = sa + (uint32_t)__builtin_amdgcn_readlane((int)in, u);
+            }
+            // a row spans at most 64 cells
+            uint32_t C = lo + (uint32_t)lane, ca = 0;
+            double S = INFINITY;
+            if (C < hi) {
+                ca = g.cell_start[C];
+                const double *b = g.box + 4 * (size_t)C;
+                if (ca < sa || ca >= se) S = box_dist2_min(px, py, b[0], b[1], b[2], b[3]);
+            }
+            uint64_t m = ballot(S <= thr);
+            if (!m) continue;
+            // the inner cells split the others into those below and above
+            uint64_t below = ballot(C < hi && ca < sa);
+            if (sa == se) below = ~0ull;
+            uint64_t parts[2] = {m & below, m & ~below};
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-            uint64_t mm = parts[h];
-            if (!mm || done) continue;
-            // a part's points are one contiguous span (cells of a row are
-            // consecutive): swept whole when short, else cell by cell
-            uint32_t cf = lo + __builtin_ctzll(mm), cl = lo + 63 - __builtin_clzll(mm);
-            bool whole = centre_pass ||
-                         g.cell_start[cl + 1] - g.cell_start[cf] <= kKnnRowSweep;
-            while (mm && !done) {
-                uint32_t a, e;
-                if (whole) {
-                    a = g.cell_start[cf];
-                    e = g.cell_start[cl + 1];
-                    mm = 0;
-                } else {
-                    int bit = __builtin_ctzll(mm);
-                    mm &= mm - 1;
-                    if (__shfl(S, bit) > thr) continue;
-                    a = g.cell_start[lo + bit];
-                    e = g.cell_start[lo + bit + 1];
-                }
-                for (uint32_t q0 = a; q0 < e && !done; q0 += kWave) {
-                    uint32_t q = q0 + lane;
-                    double s = INFINITY;
-                    if (q < e) s = dist2_exact(px, py, g.xs[q], g.ys[q]);
-                    block(s, q);
+            for (int h = 0; h < 2; h++) {
+                uint64_t mm = parts[h];
+                if (!mm || !cut) continue;
+                // a part's points are one contiguous span: swept whole when
+                // short, else cell by cell
+                uint32_t a = g.cell_start[lo + __builtin_ctzll(mm)];
+                uint32_t e = g.cell_start[lo + 64 - __builtin_clzll(mm)];
+                bool whole = e - a <= kKnnRowSweep;
+                while (mm && cut) {
+                    if (whole) {
+                        mm = 0;
+                    } else {
+                        int bit = __builtin_ctzll(mm);
+                        mm &= mm - 1;
+                        if (__shfl(S, bit) > thr) continue;
+                        a = g.cell_start[lo + bit];
+                        e = g.cell_start[lo + bit + 1];
+                    }
+                    sweep(a, e);
                 }
             }
         }
-    }
-    if (appending) settle_levels();
-    if (lane < L) {
-        lst_s[lst_at(i, lane, L)] = es;
-        lst_id[lst_at(i, lane, L)] = eid;
-    }
-    if (lane == 0) lst_n[i] = (uint32_t)cnt;
-}
-
-// kc[p*J+j] = first level k with count_k(p) >= m_j (K = never). A listed
-// point's list holds exact binary64 s in ascending order, so count_k >= m
-// exactly when entry m-1 exists and has s <= T_k; an unlisted point has L
-// (>= every m_j) entries within eps_0.
-// With J <= 8 and K <= 15 every point's levels also go out packed, 4 bits
-// per minpts value (kc4[p] bits 4j..4j+3 = kc_j(p)), for the label pass that
-// takes all variants of a call at once.
-__global__ void k_core_levels(const uint32_t *lst_idx, const double *lst_s,
-                              const uint32_t *lst_n, int L, const double *Tk, int K,
-                              const uint32_t *mj, int J, uint32_t n, uint8_t *kc, uint32_t *kc4)
-{
-    uint32_t p = blockIdx.x * kBlock + threadIdx.x;
-    if (p >= n) return;
-    uint32_t i = lst_idx[p];
-    uint32_t m = i != kNone ? lst_n[i] : 0;
-    uint32_t il = i != kNone ? i : 0;
-    uint32_t packed = 0;
-    for (int j = 0; j < J; j++) {
-        uint32_t need = mj[j];
-        int lev = K;
-        if (need <= 0x7fffffffu) {
-            if (i == kNone) {
-                lev = need <= (uint32_t)L ? 0 : K;
-            } else if (need == 0) {
-                lev = 0;
-            } else if (need <= m) {
-                double sv = lst_s[lst_at(il, need - 1, L)];
-                lev = 0;
-                while (lev < K && sv > Tk[lev]) lev++;
-            }
+        // levels of the entries, and the core levels: lane j counts the
+        // levels below the cutoff with fewer than m_j neighbours
+        int lev = 0, lj = 0;
+        for (int k = 0; k < cut; k++) {
+            uint64_t at = ballot(es <= sT[k]);
+            lev += es > sT[k] ? 1 : 0;
+            lj += (uint32_t)popc64(at) < need ? 1 : 0;
         }
-        kc[(size_t)p * J + j] = (uint8_t)lev;
-        packed |= (uint32_t)(lev & 15) << (4 * (j & 7));
+        if (need > 0x7fffffffu) lj = K;
+        if (lane < J) O.kc[(size_t)p * J + lane] = (uint8_t)lj;
+        if (O.kc4) {
+            uint32_t w = lane < J ? (uint32_t)(lj & 15) << (4 * (lane & 7)) : 0u;
+            w = group_or<8>(w);
+            if (lane == 0) O.kc4[p] = w;
+        }
+        const size_t li = O.lst_idx ? O.lst_idx[p] : p;
+        if (cut && (uint32_t)lane < cnt) {
+            size_t at = lst_at((uint32_t)li, (uint32_t)lane, L);
+            O.lst_id[at] = eid;
+            O.lst_lev[at] = (uint8_t)lev;
+        }
+        if (lane == 0) O.lst_n[li] = cut ? cnt : 0u;
     }
-    if (kc4) kc4[p] = packed;
 }
 
 // per cell, per j, per k: smallest rank of a point with kc_j <= k (cells list
@@ -615,84 +787,89 @@ __global__ void k_cell_core(const uint32_t *cell_start, uint32_t ncell, const ui
 
 // The same tables keyed by caller index (standard border rule). Caller order
 // is not sorted inside a cell, so the smallest key per level takes the whole
-// cell. A thread per cell of at most kCoreSerial points, held in registers;
-// larger cells are then taken by the whole wave one after another, each lane
-// keeping in its own LDS column the smallest key of its points at each exact
-// level, and a running minimum over the levels, reduced across the wave,
-// giving "kc_j <= k". Dynamic LDS: kWPB * K * kWave words.
+// cell: a thread per cell of at most kCoreSerial points, held in registers;
+// larger cells go to a list that k_cell_core_std_big takes, a wave per cell
+// over the whole GPU (neighbouring dense cells taken one after another by the
+// wave of their threads: 0.5 to 1.2 ms at 500,000 points x 16 variants, with
+// the list 0.03).
 constexpr uint32_t kCoreSerial = 16;
 __global__ void __launch_bounds__(kBlock)
     k_cell_core_std(const uint32_t *cell_start, uint32_t ncell, const uint8_t *kc, int J, int K,
-                    const uint32_t *key, uint32_t *cmr, uint8_t *cellkc, uint8_t *cellkc_cm)
+                    const uint32_t *key, uint32_t *cmr, uint8_t *cellkc, uint8_t *cellkc_cm,
+                    uint32_t *big, uint32_t *nbig)
 {
-    extern __shared__ uint32_t lmin[]; // [wave][level][lane]
     uint32_t c = blockIdx.x * kBlock + threadIdx.x;
     uint32_t a = 0, e = 0;
     if (c < ncell) {
         a = cell_start[c];
         e = cell_start[c + 1];
     }
-    bool big = e - a > kCoreSerial;
-    if (c < ncell && !big) {
-        uint32_t np = e - a;
-        uint32_t kq[kCoreSerial];
+    list_append(e - a > kCoreSerial, c, big, nbig);
+    if (c >= ncell || e - a > kCoreSerial) return;
+    uint32_t np = e - a;
+    uint32_t kq[kCoreSerial];
 #pragma unroll
-        for (int i = 0; i < (int)kCoreSerial; i++) kq[i] = (uint32_t)i < np ? key[a + i] : kNone;
-        for (int j = 0; j < J; j++) {
-            int lv[kCoreSerial];
-            int mn = K;
+    for (int i = 0; i < (int)kCoreSerial; i++) kq[i] = (uint32_t)i < np ? key[a + i] : kNone;
+    for (int j = 0; j < J; j++) {
+        int lv[kCoreSerial];
+        int mn = K;
 #pragma unroll
-            for (int i = 0; i < (int)kCoreSerial; i++) {
-                lv[i] = (uint32_t)i < np ? (int)kc[(size_t)(a + i) * J + j] : K;
-                mn = lv[i] < mn ? lv[i] : mn;
-            }
-            uint32_t *row = cmr + (size_t)j * K * ncell + c;
-            for (int k = 0; k < K; k++) {
-                uint32_t m = kNone;
-#pragma unroll
-                for (int i = 0; i < (int)kCoreSerial; i++)
-                    if (lv[i] <= k && kq[i] < m) m = kq[i];
-                row[(size_t)k * ncell] = m;
-            }
-            cellkc[(size_t)j * ncell + c] = (uint8_t)mn;
-            cellkc_cm[(size_t)c * J + j] = (uint8_t)mn;
+        for (int i = 0; i < (int)kCoreSerial; i++) {
+            lv[i] = (uint32_t)i < np ? (int)kc[(size_t)(a + i) * J + j] : K;
+            mn = lv[i] < mn ? lv[i] : mn;
         }
+        uint32_t *row = cmr + (size_t)j * K * ncell + c;
+        for (int k = 0; k < K; k++) {
+            uint32_t m = kNone;
+#pragma unroll
+            for (int i = 0; i < (int)kCoreSerial; i++)
+                if (lv[i] <= k && kq[i] < m) m = kq[i];
+            row[(size_t)k * ncell] = m;
+        }
+        cellkc[(size_t)j * ncell + c] = (uint8_t)mn;
+        cellkc_cm[(size_t)c * J + j] = (uint8_t)mn;
     }
-    uint64_t mb = ballot(big);
-    int lane = lane_id();
-    uint32_t *col = lmin + (size_t)wave_id_in_block() * K * kWave + lane;
-    while (mb) {
-        int bit = __builtin_ctzll(mb);
-        mb &= mb - 1;
-        uint32_t cc = c - (uint32_t)lane + (uint32_t)bit;
-        uint32_t ca = __shfl(a, bit), ce = __shfl(e, bit);
+}
+
+__device__ __forceinline__ uint32_t wave_min(uint32_t m)
+{
+    for (int o = kWave / 2; o > 0; o >>= 1) {
+        uint32_t t = __shfl_xor(m, o);
+        m = t < m ? t : m;
+    }
+    return m;
+}
+
+// A wave per listed cell. In a cell of >= L points every point has the same
+// levels (0, or K for a minpts value nothing reaches); smaller cells (< L <=
+// 64) hold a point per lane.
+__global__ void __launch_bounds__(kBlock)
+    k_cell_core_std_big(const uint32_t *cell_start, uint32_t ncell, const uint8_t *kc, int J,
+                        int K, uint32_t L, const uint32_t *key, uint32_t *cmr, uint8_t *cellkc,
+                        uint8_t *cellkc_cm, const uint32_t *big, const uint32_t *nbig)
+{
+    const uint32_t nb = *nbig;
+    const int lane = lane_id();
+    for (uint32_t i = blockIdx.x * kWPB + wave_id_in_block(); i < nb; i += gridDim.x * kWPB) {
+        const uint32_t c = big[i], a = cell_start[c], e = cell_start[c + 1];
+        const bool clique = e - a >= L;
+        uint32_t kv = kNone;
+        for (uint32_t q = a + lane; q < e; q += kWave) kv = key[q] < kv ? key[q] : kv;
+        const uint32_t all = wave_min(kv);
         for (int j = 0; j < J; j++) {
-            for (int k = 0; k < K; k++) col[k * kWave] = kNone;
-            for (uint32_t q = ca + lane; q < ce; q += kWave) {
-                int lv = kc[(size_t)q * J + j];
-                if (lv < K) {
-                    uint32_t kv = key[q];
-                    uint32_t cur = col[lv * kWave];
-                    col[lv * kWave] = kv < cur ? kv : cur;
-                }
-            }
-            uint32_t *row = cmr + (size_t)j * K * ncell + cc;
-            uint32_t run = kNone;
+            uint32_t *row = cmr + (size_t)j * K * ncell + c;
+            int lv = K;
+            if (clique) lv = kc[(size_t)a * J + j];
+            else if (a + lane < e) lv = kc[(size_t)(a + lane) * J + j];
             int mn = K;
             for (int k = 0; k < K; k++) {
-                uint32_t v = col[k * kWave];
-                run = v < run ? v : run;
-                uint32_t m = run;
-                for (int o = kWave / 2; o > 0; o >>= 1) {
-                    uint32_t t = __shfl_xor(m, o);
-                    m = t < m ? t : m;
-                }
+                uint32_t m = clique ? (lv <= k ? all : kNone) : wave_min(lv <= k ? kv : kNone);
                 if (m != kNone && mn == K) mn = k;
                 if (lane == 0) row[(size_t)k * ncell] = m;
             }
             if (lane == 0) {
-                cellkc[(size_t)j * ncell + cc] = (uint8_t)mn;
-                cellkc_cm[(size_t)cc * J + j] = (uint8_t)mn;
+                cellkc[(size_t)j * ncell + c] = (uint8_t)mn;
+                cellkc_cm[(size_t)c * J + j] = (uint8_t)mn;
             }
         }
     }
@@ -847,6 +1024,7 @@ struct LevelArgs {
     const double *xs, *ys, *box;
     const uint32_t *cell_start, *cell_key;
     const uint32_t *cell_ds, *skbase, *sncy; // dataset of a cell, its key base and ncy
+    uint32_t m;                              // strip width of the keys
     const uint8_t *kc;
     const uint32_t *pa, *pb;
     const uint16_t *pk;
@@ -1345,8 +1523,10 @@ __global__ void __launch_bounds__(kBlock) k_sweep(LevelArgs a, LevelLists L)
                     // both cells belong to one dataset
                     uint32_t ds = a.cell_ds[A], ncy = a.sncy[ds], k0 = a.skbase[ds];
                     uint32_t ka = a.cell_key[A] - k0, kb = a.cell_key[B] - k0;
-                    int64_t dx = (int64_t)(ka / ncy) - (int64_t)(kb / ncy);
-                    int64_t dy = (int64_t)(ka % ncy) - (int64_t)(kb % ncy);
+                    uint32_t qa = ka / a.m, qb = kb / a.m;
+                    int64_t dx = (int64_t)(qa / ncy * a.m + ka % a.m) -
+                                 (int64_t)(qb / ncy * a.m + kb % a.m);
+                    int64_t dy = (int64_t)(qa % ncy) - (int64_t)(qb % ncy);
                     bool adj = dx >= -1 && dx <= 1 && dy >= -1 && dy <= 1;
                     tnear = adj;
                     tfar = !adj;
@@ -1698,7 +1878,6 @@ static_assert(kLabelSlots == 8, "staged labels move as two 16-byte vectors per p
 struct LabelSlots {
     int n;
     int k[kLabelSlots];
-    double T[kLabelSlots];
     const uint32_t *rootrank[kLabelSlots]; // per cell
     const uint32_t *cbits[kLabelSlots];    // root ranks as a bitset over ranks
     const uint32_t *cpre[kLabelSlots];     // per 32-rank word: roots before it
@@ -1741,15 +1920,21 @@ __global__ void k_cell_labels(SnapArgs S, const uint32_t *cell_ds, const uint32_
                                    roots_below(bits, pre, seg[cell_ds[c]]) + base;
 }
 
+// does a point of cell C have a neighbour list?
+__device__ __forceinline__ bool has_list(const uint32_t *cell_start, uint32_t C, int L)
+{
+    return cell_start[C + 1] - cell_start[C] < (uint32_t)L;
+}
+
 // Thread per cell-order position: the point's data are read in sequence, the
 // labels are scattered to caller order. STD: snapshots are keyed by caller
 // index, a non-core point with a core neighbour always joins the smallest
 // such root, clusters count from 0 and noise is NONE.
 template <bool STD>
 __global__ void __launch_bounds__(kBlock)
-    k_labels_j(LabelSlots S, const uint32_t *cell_of_pos,
+    k_labels_j(LabelSlots S, const uint32_t *cell_start, const uint32_t *cell_of_pos,
                const uint32_t *cell_ds, const uint32_t *pos_rank, const uint8_t *kc, int J, int j,
-               const uint32_t *lst_idx, const double *lst_s, const uint32_t *lst_id,
+               const uint32_t *lst_idx, const uint8_t *lst_lev, const uint32_t *lst_id,
                const uint32_t *lst_n, int L, uint32_t n)
 {
     uint32_t p = blockIdx.x * kBlock + threadIdx.x;
@@ -1759,40 +1944,41 @@ __global__ void __launch_bounds__(kBlock)
     int kcp = kc[(size_t)p * J + j];
     uint32_t best[kLabelSlots];
     bool any_border = false;
-    double Tmax = -1.0;
+    int kmax = -1; // largest level of a border slot
 #pragma unroll
     for (int t = 0; t < kLabelSlots; t++) {
         best[t] = kNone;
         if (t < S.n && kcp > S.k[t]) {
             any_border = true;
-            Tmax = S.T[t] > Tmax ? S.T[t] : Tmax;
+            kmax = S.k[t] > kmax ? S.k[t] : kmax;
         }
     }
-    if (any_border) {
+    if (any_border && kcp > 0) {
         // non-core at level k: count_k(p) < m_j <= L, so its list holds every
-        // eps_k neighbour as the prefix with s <= T_k
-        uint32_t li = lst_idx[p];
-        if (li != kNone) {
+        // eps_k neighbour (the entries of levels <= k). A point without a
+        // list (core at level 0 whatever minpts below INT_MAX) is non-core
+        // only for a minpts value that no point reaches.
+        uint32_t li = lst_idx ? lst_idx[p] : p;
+        if (has_list(cell_start, C, L)) {
             uint32_t m = lst_n[li];
-            const double *sv = lst_s + lst_at(li, 0, L); // entry e at sv[64 e]
+            const uint8_t *sv = lst_lev + lst_at(li, 0, L); // entry e at sv[64 e]
             const uint32_t *iv = lst_id + lst_at(li, 0, L);
-            // four entries per step, their loads issued together (the list
-            // is sorted, so the walk ends at the first entry beyond Tmax)
+            // four entries per step, their loads issued together
             constexpr int kU = 4;
             for (uint32_t e0 = 0; e0 < m; e0 += kU) {
-                double se[kU];
+                int se[kU];
                 uint32_t q[kU];
 #pragma unroll
                 for (int u = 0; u < kU; u++) {
                     bool ok = e0 + u < m;
-                    se[u] = ok ? sv[(size_t)(e0 + u) * 64u] : INFINITY;
+                    se[u] = ok ? (int)sv[(size_t)(e0 + u) * 64u] : kMaxLevels;
                     q[u] = ok ? iv[(size_t)(e0 + u) * 64u] : 0u;
                 }
                 int kq[kU];
                 uint32_t cq[kU];
 #pragma unroll
                 for (int u = 0; u < kU; u++) {
-                    bool ok = se[u] <= Tmax;
+                    bool ok = se[u] <= kmax;
                     kq[u] = ok ? (int)kc[(size_t)q[u] * J + j] : kMaxLevels;
                     cq[u] = ok ? cell_of_pos[q[u]] : 0u;
                 }
@@ -1800,13 +1986,12 @@ __global__ void __launch_bounds__(kBlock)
                 for (int u = 0; u < kU; u++) {
 #pragma unroll
                     for (int t = 0; t < kLabelSlots; t++) {
-                        if (t < S.n && kcp > S.k[t] && se[u] <= S.T[t] && kq[u] <= S.k[t]) {
+                        if (t < S.n && kcp > S.k[t] && se[u] <= S.k[t] && kq[u] <= S.k[t]) {
                             uint32_t rr = S.rootrank[t][cq[u]];
                             best[t] = rr < best[t] ? rr : best[t];
                         }
                     }
                 }
-                if (!(se[kU - 1] <= Tmax)) break;
             }
         }
     }
@@ -1876,7 +2061,6 @@ struct AllSlots {
     uint32_t stride;              // staged words per position
     int8_t slot[kAllJ][16];       // (j, k) -> snapshot; -1: not requested
     uint16_t jreq[kAllJ];         // bit k: (j, k) requested
-    double T[16];                 // level thresholds (s <= T_k: within eps_k)
     const uint32_t *root, *lab, *bits, *pre; // snapshot t at + t*ncell (root, lab), + t*nw
     uint32_t ncell, nw;
     const uint32_t *seg;
@@ -1886,17 +2070,15 @@ struct AllSlots {
 template <bool STD, int KB, int JG>
 __global__ void __launch_bounds__(kBlock)
     k_labels_all(AllSlots S, const uint32_t *cell_of_pos, const uint32_t *cell_ds,
-                 const uint32_t *pos_rank, const uint32_t *kc4, const uint32_t *lst_idx,
-                 const double *lst_s, const uint32_t *lst_id, const uint32_t *lst_n, int L,
-                 uint32_t n)
+                 const uint32_t *pos_rank, const uint32_t *kc4, const uint32_t *cell_start,
+                 const uint32_t *lst_idx, const uint8_t *lst_lev, const uint32_t *lst_id,
+                 const uint32_t *lst_n, int L, uint32_t n)
 {
     static_assert((JG * KB) % 4 == 0 && KB <= 16 && JG <= kAllJ, "whole 16-byte groups");
-    // the call's thresholds, slot table and requests in LDS: the walk reads
-    // them at run-time indices without scalar memory round trips
-    __shared__ double sT[16];
+    // the call's slot table and requests in LDS: the walk reads them at
+    // run-time indices without scalar memory round trips
     __shared__ int8_t sslot[kAllJ][16];
     __shared__ uint16_t sjreq[kAllJ];
-    if (threadIdx.x < 16) sT[threadIdx.x] = S.T[threadIdx.x];
     if (threadIdx.x < kAllJ * 16) (&sslot[0][0])[threadIdx.x] = (&S.slot[0][0])[threadIdx.x];
     if (threadIdx.x < kAllJ) sjreq[threadIdx.x] = S.jreq[threadIdx.x];
     __syncthreads();
@@ -1905,22 +2087,23 @@ __global__ void __launch_bounds__(kBlock)
     const uint32_t r = pos_rank[p];
     const uint32_t C = cell_of_pos[p];
     const uint32_t kp4 = kc4[p];
-    const uint32_t li = lst_idx[p];
+    const uint32_t li = lst_idx ? lst_idx[p] : p;
+    const bool listed = has_list(cell_start, C, L);
     const uint32_t s0 = S.seg[cell_ds[C]];
     const int K = S.K;
     for (int j0 = 0; j0 < S.J; j0 += JG) {
         // per minpts value of the group: p's core level, and the walk bound
-        // (largest threshold of a requested level at which p is not core)
+        // (one past the largest requested level at which p is not core)
         int kp[JG];
-        double Tmax = -1.0;
+        int kend = 0;
 #pragma unroll
         for (int jj = 0; jj < JG; jj++) {
             int j = j0 + jj;
             kp[jj] = j < S.J ? (int)((kp4 >> (4 * j)) & 15u) : 0;
             uint32_t below = sjreq[j < S.J ? j : 0] & ((1u << kp[jj]) - 1u);
             if (j < S.J && below) {
-                double t = sT[31 - __builtin_clz(below)];
-                Tmax = t > Tmax ? t : Tmax;
+                int t = 32 - __builtin_clz(below);
+                kend = t > kend ? t : kend;
             }
         }
         uint32_t best[JG][KB];
@@ -1928,34 +2111,33 @@ __global__ void __launch_bounds__(kBlock)
         for (int jj = 0; jj < JG; jj++)
 #pragma unroll
             for (int k = 0; k < KB; k++) best[jj][k] = kNone;
-        if (Tmax >= 0.0 && li != kNone) {
+        if (kend > 0 && listed) {
             // non-core at level k: count_k(p) < m_j <= L, so its list holds
-            // every eps_k neighbour as the prefix with s <= T_k
+            // every eps_k neighbour (the entries of levels <= k)
             uint32_t m = lst_n[li];
-            const double *sv = lst_s + lst_at(li, 0, L); // entry e at sv[64 e]
+            const uint8_t *sv = lst_lev + lst_at(li, 0, L); // entry e at sv[64 e]
             const uint32_t *iv = lst_id + lst_at(li, 0, L);
-            int ke = 0; // level of the current entry (entries ascend in s)
             constexpr int kU = 2;
             for (uint32_t e0 = 0; e0 < m; e0 += kU) {
-                double se[kU];
+                int se[kU];
                 uint32_t q[kU];
 #pragma unroll
                 for (int u = 0; u < kU; u++) {
                     bool ok = e0 + u < m;
-                    se[u] = ok ? sv[(size_t)(e0 + u) * 64u] : INFINITY;
+                    se[u] = ok ? (int)sv[(size_t)(e0 + u) * 64u] : kMaxLevels;
                     q[u] = ok ? iv[(size_t)(e0 + u) * 64u] : 0u;
                 }
                 uint32_t kq[kU], cq[kU];
 #pragma unroll
                 for (int u = 0; u < kU; u++) {
-                    bool ok = se[u] <= Tmax;
+                    bool ok = se[u] < kend;
                     kq[u] = ok ? kc4[q[u]] : 0xffffffffu;
                     cq[u] = ok ? cell_of_pos[q[u]] : 0u;
                 }
 #pragma unroll
                 for (int u = 0; u < kU; u++) {
-                    if (!(se[u] <= Tmax)) break;
-                    while (ke < K && se[u] > sT[ke]) ke++;
+                    const int ke = se[u];
+                    if (ke >= kend) continue;
                     uint32_t v[JG][KB];
 #pragma unroll
                     for (int jj = 0; jj < JG; jj++) {
@@ -1977,7 +2159,6 @@ __global__ void __launch_bounds__(kBlock)
                         for (int k = 0; k < KB; k++)
                             best[jj][k] = v[jj][k] < best[jj][k] ? v[jj][k] : best[jj][k];
                 }
-                if (!(se[kU - 1] <= Tmax)) break;
             }
         }
         uint32_t lbl[JG * KB];
@@ -2216,30 +2397,43 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
     Ev tprep(c.stream(), st != nullptr);
     double d = lev[0] / std::sqrt(2.0) * (1.0 - std::ldexp(1.0, -20));
     int R = (int)std::ceil(lev[K - 1] * (1.0 + std::ldexp(1.0, -30)) / d);
-    // a window row per lane in k_knn (eps ratio 16 gives R = 23)
+    // a window row, at most 2R + 1 cells of each of its columns, is a lane's
+    // cell each in k_knn_crowded (eps ratio 16 gives R = 23)
     if (2 * R + 1 > kWave) {
         set_error("eps range too wide for one fine grid");
         return kErrUnsupported;
     }
     Grid G;
-    G.want_row_pts = true; // the truncated-list kernel reads the rows' point ranges
+    // strips of about R/2 columns: 5 window rows (3 for R = 2) of long runs
+    // instead of 2R + 1 short ones, for up to 1.2 times the cells
+    G.m = std::max(1, std::min(std::max((R + 1) / 2, 2), kWave / (2 * R + 1)));
+    // the truncated-list kernel reads the rows' point ranges, and those of the
+    // cells that can hold neighbours at the smallest eps
+    G.want_row_pts = true;
+    G.Rin = std::min(R, (int)std::ceil(lev[0] * (1.0 + std::ldexp(1.0, -30)) / d));
     bool enlarged = false;
     VDB_TRY(build_grid(c, P, d, R, "gb", G, &enlarged));
     if (enlarged) {
         set_error("fine grid would exceed 32-bit cell keys");
         return kErrUnsupported;
     }
+    // failed clique checks, listed points, the list kernels' counts
     uint32_t *bad;
-    VDB_TRY(c.get("b.bad", 1, &bad));
-    VDB_HIP(hipMemsetAsync(bad, 0, sizeof(uint32_t), c.stream()));
-    k_clique_check<<<ceil_div(G.ncell, kBlock), kBlock, 0, c.stream()>>>(G.cell_box, G.ncell,
-                                                                         Th[0], bad);
+    VDB_TRY(c.get("b.bad", 5, &bad));
+    VDB_HIP(hipMemsetAsync(bad, 0, 5 * sizeof(uint32_t), c.stream()));
+    k_clique_check<<<ceil_div(G.ncell, kBlock), kBlock, 0, c.stream()>>>(
+        G.cell_box, G.cell_start, G.ncell, Th[0], L, bad);
     VDB_HIP(hipGetLastError());
     double *dTk;
     uint32_t *dmj;
-    VDB_TRY(c.get("b.Tk", K, &dTk));
+    const std::vector<double> Tpad = [&] { // INF beyond K: k_knn takes rounded-up counts
+        std::vector<double> t(Th);
+        t.resize(kMaxLevels, INFINITY);
+        return t;
+    }();
+    VDB_TRY(c.get("b.Tk", kMaxLevels, &dTk));
     VDB_TRY(c.get("b.mj", J, &dmj));
-    VDB_HIP(hipMemcpyAsync(dTk, Th.data(), sizeof(double) * K, hipMemcpyHostToDevice,
+    VDB_HIP(hipMemcpyAsync(dTk, Tpad.data(), sizeof(double) * kMaxLevels, hipMemcpyHostToDevice,
                            c.stream()));
     VDB_HIP(hipMemcpyAsync(dmj, mps.data(), sizeof(uint32_t) * J, hipMemcpyHostToDevice,
                            c.stream()));
@@ -2251,35 +2445,21 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
     char *hs = nullptr;
     VDB_TRY(c.host_scratch(32 + 4 * (4 + ncnt_all + (size_t)J * (K + 1) + 1), (void **)&hs));
 
-    // ---- truncated distance-sorted table: the listed points first, so
-    // that the list kernel does not wait behind the pair count
+    // ---- truncated neighbour table: a list per position, so that nothing
+    // counts or numbers the listed points, unless that takes more than 8 GB:
+    // then they are numbered first.
     Ev tknn(c.stream(), st != nullptr);
-    uint32_t *flag, *excl, *list_cell, *lst_idx, *nlist_dev;
-    double2 *list_xy;
-    VDB_TRY(c.get("b.flag", n, &flag));
-    VDB_TRY(c.get("b.excl", n, &excl));
-    VDB_TRY(c.get("b.lst_idx", n, &lst_idx));
-    VDB_TRY(c.get("b.nlist", 1, &nlist_dev));
     unsigned gn = ceil_div(n, kBlock);
-    k_list_flags<<<gn, kBlock, 0, c.stream()>>>(G.cell_start, G.cell_of_pos, n, L, flag);
-    VDB_HIP(hipGetLastError());
-    VDB_TRY(scan_exclusive_u32(c, flag, excl, n, nlist_dev));
-    // Lists are sized for every point, so that nothing waits for their count
-    // (the truncated-list kernel reads it on the device), unless that takes
-    // more than 8 GB: then the count is read first.
-    const bool exact_lists = (size_t)n * L * 12 > ((size_t)8 << 30);
+    uint32_t *lst_idx = nullptr;
     uint32_t nlist_cap = n;
-    if (exact_lists) {
-        VDB_HIP(hipMemcpyAsync(hs + 16, nlist_dev, 4, hipMemcpyDeviceToHost, c.stream()));
-        VDB_HIP(hipStreamSynchronize(c.stream()));
-        memcpy(&nlist_cap, hs + 16, 4);
+    if ((size_t)n * L * 5 > ((size_t)8 << 30)) {
+        uint32_t *flag;
+        VDB_TRY(c.get("b.flag", n, &flag));
+        VDB_TRY(c.get("b.lst_idx", n, &lst_idx));
+        k_list_flags<<<gn, kBlock, 0, c.stream()>>>(G.cell_start, G.cell_of_pos, n, L, flag);
+        VDB_HIP(hipGetLastError());
+        VDB_TRY(compact_count(c, flag, lst_idx, n, &nlist_cap));
     }
-    VDB_TRY(c.get("b.list_xy", nlist_cap ? nlist_cap : 1, &list_xy));
-    VDB_TRY(c.get("b.list_cell", nlist_cap ? nlist_cap : 1, &list_cell));
-    k_list_index<<<gn, kBlock, 0, c.stream()>>>(flag, excl, G.xs, G.ys, G.cell_of_pos, n, list_xy,
-                                                list_cell, lst_idx);
-    VDB_HIP(hipGetLastError());
-    const uint2 *row_pts = G.row_pts; // the window rows' point ranges
     // ---- cell pairs within eps_max: counted on the library's second
     // stream beside the truncated lists (both read only the grid); the pair
     // total and the clique check come back in one read
@@ -2298,7 +2478,7 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
     VDB_TRY(c.get("b.poff", (size_t)G.ncell + 1, &poff));
     unsigned gc = ceil_div(G.ncell, kBlock);
     unsigned gcw = ceil_div(G.ncell, kWPB); // a wave per cell
-    int W = 2 * R + 1;
+    int W = 2 * G.RS + 1;
     {
         StreamScope on(c, ps);
         VDB_TRY(c.kt_begin("k_pair_count"));
@@ -2312,27 +2492,43 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
         VDB_HIP(hipEventRecord(c.aux_event(1), ps));
     }
 
-    double *lst_s;
+    uint8_t *lst_lev;
     uint32_t *lst_id, *lst_n;
     size_t lsz = (size_t)(nlist_cap ? (nlist_cap + 63) / 64 * 64 : 64) * L; // blocks of 64 lists
-    VDB_TRY(c.get("b.lst_s", lsz, &lst_s));
+    VDB_TRY(c.get("b.lst_lev", lsz, &lst_lev));
     VDB_TRY(c.get("b.lst_id", lsz, &lst_id));
     VDB_TRY(c.get("b.lst_n", nlist_cap ? nlist_cap : 1, &lst_n));
-    if (nlist_cap) {
-        VDB_TRY(c.kt_begin("k_knn"));
-        k_knn<<<ceil_div(nlist_cap, kWPB), kBlock, 0, c.stream()>>>(
-            fview(G), list_xy, list_cell, row_pts, nlist_dev, (int)L, dTk, K, lst_s, lst_id, lst_n);
-        VDB_TRY(c.kt_end("k_knn"));
-    }
-    VDB_HIP(hipGetLastError());
     uint8_t *kc, *cellkc;
     uint32_t *cmr;
     VDB_TRY(c.get("b.kc", (size_t)n * J, &kc));
     // packed levels for the one-sweep label pass (J <= kAllJ, K <= kAllK)
     uint32_t *kc4 = nullptr;
     if (J <= kAllJ && K <= kAllK) VDB_TRY(c.get("b.kc4", n, &kc4));
-    k_core_levels<<<gn, kBlock, 0, c.stream()>>>(lst_idx, lst_s, lst_n, (int)L, dTk, K, dmj, J,
-                                                 n, kc, kc4);
+    uint32_t *mid, *crowd;
+    VDB_TRY(c.get("b.mid", n, &mid));
+    VDB_TRY(c.get("b.crowd", n, &crowd));
+    const NearOut no{lst_idx, lst_id, lst_lev, lst_n, kc, kc4, (int)L, K, J, dmj};
+    const FG fg = fview(G);
+    const unsigned gl = std::min(ceil_div(n, kWPB), kListBlocks);
+    VDB_TRY(c.kt_begin("k_knn"));
+    // beyond 16 levels every listed point takes the wave kernel (more packed
+    // counts than that would spill)
+    const uint32_t mid_from = K > 16 ? 0u : kNearMid, crowd_from = K > 16 ? 0u : kNearCrowded;
+#define VDB_KNN(KL)                                                                             \
+    do {                                                                                        \
+        k_knn<KL><<<gn, kBlock, 0, c.stream()>>>(fg, no, dTk, n, mid_from, crowd_from, mid,     \
+                                                 crowd, bad + 2);                               \
+        VDB_HIP(hipGetLastError());                                                             \
+        k_knn_group<KL><<<gl, kBlock, 0, c.stream()>>>(fg, no, dTk, mid, bad + 2);              \
+    } while (0)
+    if (K == 1) VDB_KNN(1);
+    else if (K <= 4) VDB_KNN(4);
+    else if (K <= 8) VDB_KNN(8);
+    else VDB_KNN(16);
+#undef VDB_KNN
+    VDB_HIP(hipGetLastError());
+    k_knn_crowded<<<gl, kBlock, 0, c.stream()>>>(fg, no, dTk, crowd, bad + 3);
+    VDB_TRY(c.kt_end("k_knn"));
     VDB_HIP(hipGetLastError());
     VDB_TRY(c.get("b.cmr", (size_t)G.ncell * J * K, &cmr));
     VDB_TRY(c.get("b.cellkc", (size_t)G.ncell * J, &cellkc));
@@ -2345,13 +2541,19 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
     VDB_TRY(c.get("b.cop", n, &caller_of_pos));
     k_caller_of_pos<<<gn, kBlock, 0, c.stream()>>>(G.pos_rank, P.mapping, n, caller_of_pos);
     VDB_HIP(hipGetLastError());
-    if (std_rule)
-        k_cell_core_std<<<gc0, kBlock, sizeof(uint32_t) * kWPB * (size_t)K * kWave,
-                          c.stream()>>>(
-            G.cell_start, G.ncell, kc, J, K, caller_of_pos, cmr, cellkc, cellkc_cm);
-    else
+    if (std_rule) {
+        uint32_t *big;
+        VDB_TRY(c.get("b.bigcore", G.ncell, &big));
+        k_cell_core_std<<<gc0, kBlock, 0, c.stream()>>>(G.cell_start, G.ncell, kc, J, K,
+                                                        caller_of_pos, cmr, cellkc, cellkc_cm, big,
+                                                        bad + 4);
+        VDB_HIP(hipGetLastError());
+        k_cell_core_std_big<<<std::min(ceil_div(G.ncell, kWPB), 2048u), kBlock, 0, c.stream()>>>(
+            G.cell_start, G.ncell, kc, J, K, L, caller_of_pos, cmr, cellkc, cellkc_cm, big, bad + 4);
+    } else {
         k_cell_core<<<gc0, kBlock, 0, c.stream()>>>(G.cell_start, G.ncell, kc, J, K, G.pos_rank,
                                                     cmr, cellkc, cellkc_cm);
+    }
     VDB_HIP(hipGetLastError());
     tknn.stop();
 
@@ -2485,7 +2687,6 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
         memset(A.slot, -1, sizeof A.slot);
         A.J = J;
         A.K = K;
-        for (int k = 0; k < K; k++) A.T[k] = Th[k];
         // snapshot of (k, j): level-major over the requested pairs, as the
         // level passes number them
         int nsnap = 0;
@@ -2619,7 +2820,7 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
             PairRec *lin = la, *lout = lb;
             for (int k = 0; k <= kmax; k++) {
                 LevelArgs a{G.xs, G.ys, G.cell_box, G.cell_start, G.cell_key, G.cell_ds, G.skbase,
-                            G.sncy, kc, pa, pb, pk, J, j0, k, Th[k]};
+                            G.sncy, (uint32_t)G.m, kc, pa, pb, pk, J, j0, k, Th[k]};
                 LevelLists LL{parent, lin, lout, tests, tests2, cnts, frec, bstart,
                               psz, G.ncell, tcap, (uint32_t)K, tovf, shape.ppb, shape.minb,
                               shape.tpb};
@@ -2692,8 +2893,9 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
                 VDB_TRY(c.kt_begin("k_labels_all"));
 #define VDB_LABELS_ALL(STD, KB, JG)                                                              \
     k_labels_all<STD, KB, JG><<<gn, kBlock, 0, c.stream()>>>(A, G.cell_of_pos, G.cell_ds,        \
-                                                             G.pos_rank, kc4, lst_idx, lst_s,     \
-                                                             lst_id, lst_n, (int)L, n)
+                                                             G.pos_rank, kc4, G.cell_start,       \
+                                                             lst_idx, lst_lev, lst_id, lst_n,     \
+                                                             (int)L, n)
                 if (all_kb == 8) {
                     if (std_rule) VDB_LABELS_ALL(true, 8, 4);
                     else VDB_LABELS_ALL(false, 8, 4);
@@ -2738,7 +2940,6 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
                         size_t sl = sbase[k] + (uint32_t)__builtin_popcountll(
                                                    jmask[k] & ((1ull << jr) - 1ull));
                         S.k[t] = k;
-                        S.T[t] = Th[k];
                         S.rootrank[t] = snap_root + sl * G.ncell;
                         S.cbits[t] = snap_bits + sl * nw;
                         S.cpre[t] = snap_pre + sl * nw;
@@ -2752,14 +2953,14 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
                     if (std_rule) {
                         VDB_TRY(c.kt_begin("k_labels_j"));
                         k_labels_j<true><<<gn, kBlock, 0, c.stream()>>>(
-                            S, G.cell_of_pos, G.cell_ds, G.pos_rank, kc, J, j, lst_idx, lst_s, lst_id,
-                            lst_n, (int)L, n);
+                            S, G.cell_start, G.cell_of_pos, G.cell_ds, G.pos_rank, kc, J, j, lst_idx,
+                            lst_lev, lst_id, lst_n, (int)L, n);
                         VDB_TRY(c.kt_end("k_labels_j"));
                     } else {
                         VDB_TRY(c.kt_begin("k_labels_j"));
                         k_labels_j<false><<<gn, kBlock, 0, c.stream()>>>(
-                            S, G.cell_of_pos, G.cell_ds, G.pos_rank, kc, J, j, lst_idx, lst_s, lst_id,
-                            lst_n, (int)L, n);
+                            S, G.cell_start, G.cell_of_pos, G.cell_ds, G.pos_rank, kc, J, j, lst_idx,
+                            lst_lev, lst_id, lst_n, (int)L, n);
                         VDB_TRY(c.kt_end("k_labels_j"));
                     }
                     VDB_HIP(hipGetLastError());
@@ -2835,7 +3036,7 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
     uint32_t *hc = (uint32_t *)(hs + 32 + 8);
     uint32_t *hb = hc + ncnt_all;
     VDB_HIP(hipMemcpyAsync(hs + 32, tovf, 4, hipMemcpyDeviceToHost, c.stream()));
-    VDB_HIP(hipMemcpyAsync(hs + 36, nlist_dev, 4, hipMemcpyDeviceToHost, c.stream()));
+    VDB_HIP(hipMemcpyAsync(hs + 36, bad + 1, 4, hipMemcpyDeviceToHost, c.stream()));
     if (counters) {
         VDB_HIP(hipMemcpyAsync(hc, cnts, sizeof(uint32_t) * ncnt_all, hipMemcpyDeviceToHost,
                                c.stream()));

@@ -35,7 +35,7 @@ struct GridView {
 GridView view(const Grid &G, uint32_t n)
 {
     return GridView{G.xs,     G.ys,     G.cell_start,   G.row_lo, G.row_hi,
-                    G.row_f0, G.row_f1, 2 * G.R + 1,    n};
+                    G.row_f0, G.row_f1, 2 * G.RS + 1,   n};
 }
 
 // Row r of cell c's window as cell-sorted positions: candidates to test in

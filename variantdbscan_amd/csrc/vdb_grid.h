@@ -43,9 +43,14 @@ void single_segment(Points &P);
 
 struct Grid {
     double w = 0, gx0 = 0, gy0 = 0;
-    uint32_t ncx = 0, ncy = 0; // key = cx*ncy + cy
+    uint32_t ncx = 0, ncy = 0;
+    // Columns are keyed in strips of m (set before build_grid): key =
+    // ((cx/m)*ncy + cy)*m + cx%m, column-major for m = 1. A window of radius R
+    // is then 2*RS + 1 rows, one per strip, each a contiguous run of keys.
+    int m = 1;
     uint32_t ncell = 0;        // non-empty cells
     int R = 1;                 // window radius in cells
+    int RS = 1;                // in strips: ceil(R/m)
     double *xs = nullptr, *ys = nullptr;
     uint32_t *pos_rank = nullptr;   // [n]
     uint32_t *rank_pos = nullptr;   // [n] inverse of pos_rank
@@ -53,12 +58,16 @@ struct Grid {
     uint32_t *cell_key = nullptr;   // [ncell]
     uint32_t *cell_start = nullptr; // [ncell+1]
     double *cell_box = nullptr;     // [ncell*4] x0,x1,y0,y1 of the cell's points
-    uint32_t *row_lo = nullptr;     // [ncell*(2R+1)] first cell of window row
-    uint32_t *row_hi = nullptr;     // [ncell*(2R+1)] one past the last
+    uint32_t *row_lo = nullptr;     // [ncell*(2RS+1)] first cell of window row
+    uint32_t *row_hi = nullptr;     // [ncell*(2RS+1)] one past the last
     // with want_row_pts set before build_grid: (first point, point count)
     // of every window row, beside row_lo/row_hi
+    // and, when Rin < R, those of the rows' parts within Rin cells of the
+    // centre cell on both axes
     bool want_row_pts = false;
-    uint2 *row_pts = nullptr;       // [ncell*(2R+1)]
+    int Rin = 0, RSin = 0;          // RSin = ceil(Rin/m)
+    uint2 *row_pts = nullptr;       // [ncell*(2RS+1)]
+    uint2 *row_in = nullptr;        // [ncell*(2RSin+1)]; null when Rin == R
     // after classify_rows (per-variant grids): inside every window row,
     // cells [row_f0, row_f1) are within eps of the whole centre cell (every
     // pair accepted without a test); row_lo/row_hi are then trimmed to cells
@@ -67,7 +76,7 @@ struct Grid {
     uint32_t *row_f1 = nullptr;
     uint32_t npts = 0;              // points in the grid
     // per dataset: grid origin, dimensions and first key (keys of dataset d
-    // are kbase[d] + cx*ncy[d] + cy)
+    // are kbase[d] + key; kbase[d] is a multiple of m)
     uint32_t nsets = 1;
     double *sgx0 = nullptr, *sgy0 = nullptr;
     uint32_t *sncx = nullptr, *sncy = nullptr;

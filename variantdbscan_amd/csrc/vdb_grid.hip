@@ -202,7 +202,7 @@ __global__ void k_gather_xy(const double *x, const double *y, const uint32_t *id
 __global__ void k_cell_keys(const double *x, const double *y, uint32_t n, const uint32_t *seg,
                             uint32_t nsets, const double *sgx0, const double *sgy0, double w,
                             const uint32_t *sncx, const uint32_t *sncy, const uint32_t *skbase,
-                            uint32_t *keys, uint32_t *vals)
+                            uint32_t m, uint32_t *keys, uint32_t *vals)
 {
     uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
@@ -212,7 +212,8 @@ __global__ void k_cell_keys(const double *x, const double *y, uint32_t n, const 
     double fy = floor(__ddiv_rn(__dsub_rn(y[i], sgy0[d]), w));
     fx = fx < 0.0 ? 0.0 : (fx > (double)(ncx - 1) ? (double)(ncx - 1) : fx);
     fy = fy < 0.0 ? 0.0 : (fy > (double)(ncy - 1) ? (double)(ncy - 1) : fy);
-    keys[i] = skbase[d] + (uint32_t)fx * ncy + (uint32_t)fy;
+    uint32_t cx = (uint32_t)fx, st = cx / m;
+    keys[i] = skbase[d] + (st * ncy + (uint32_t)fy) * m + (cx - st * m);
     vals[i] = i;
 }
 
@@ -420,107 +421,165 @@ __device__ __forceinline__ uint32_t lower_bound_near(const uint32_t *a, uint32_t
     return lo;
 }
 
-// window rows: for cell c and row offset d in [-R, R], the cells of grid row
-// cx+d whose cy lies in [cy-R, cy+R] form one contiguous run of the sorted keys
-// rows stay inside the cell's own dataset grid. A thread takes one row offset
-// for kRowRun consecutive cells: each search starts from the previous cell's
-// answer, a few positions away, instead of galloping across up to R columns.
+// A cell's place in its dataset's grid, from its key.
+struct CellPlace {
+    int64_t cx, cy, strip; // column, row, cx/m
+    uint32_t ds;
+};
+struct GridDims {
+    const uint32_t *sncx, *sncy, *skbase;
+    uint32_t nsets, m;
+};
+
+__device__ __forceinline__ CellPlace cell_place(const GridDims &D, uint32_t key)
+{
+    CellPlace c;
+    c.ds = seg_of(D.skbase, D.nsets, key);
+    uint32_t ncy = D.sncy[c.ds], local = key - D.skbase[c.ds];
+    uint32_t q = local / D.m, st = q / ncy;
+    c.strip = st;
+    c.cy = q - st * ncy;
+    c.cx = (int64_t)st * D.m + (local - q * D.m);
+    return c;
+}
+
+// Keys [*k0, *k1] of the cells of strip c.strip + t with rows within r of
+// c.cy, clipped to the dataset's grid; false when the strip has no column
+// within r of c.cx. (Columns of the strip beyond r are included.)
+__device__ __forceinline__ bool row_keys(const GridDims &D, const CellPlace &c, int t, int r,
+                                         uint64_t *k0, uint64_t *k1)
+{
+    const int64_t m = D.m, st = c.strip + t;
+    const int64_t nst = ((int64_t)D.sncx[c.ds] + m - 1) / m, ncy = D.sncy[c.ds];
+    if (st < 0 || st >= nst || st * m > c.cx + r || st * m + m - 1 < c.cx - r) return false;
+    int64_t y0 = c.cy - r < 0 ? 0 : c.cy - r;
+    int64_t y1 = c.cy + r > ncy - 1 ? ncy - 1 : c.cy + r;
+    const uint64_t kb = D.skbase[c.ds];
+    *k0 = kb + (uint64_t)((st * ncy + y0) * m);
+    *k1 = kb + (uint64_t)((st * ncy + y1) * m + m - 1);
+    return true;
+}
+
+// window rows: for cell c and row t in [-RS, RS], the cells of strip t off
+// c's whose row lies in [cy-R, cy+R] form one contiguous run of the sorted
+// keys; rows stay inside the cell's own dataset grid. A thread takes one row
+// offset for kRowRun consecutive cells: each search starts from the previous
+// cell's answer, a few positions away, instead of galloping across up to R
+// columns.
 constexpr uint32_t kRowRun = 4;
-__global__ void k_row_ranges(const uint32_t *cell_key, uint32_t ncell, const uint32_t *sncx,
-                             const uint32_t *sncy, const uint32_t *skbase, uint32_t nsets, int R,
+__global__ void k_row_ranges(const uint32_t *cell_key, uint32_t ncell, GridDims D, int R, int RS,
                              uint32_t *row_lo, uint32_t *row_hi, uint32_t *cell_ds)
 {
     // 64-bit thread index: runs x window rows exceeds 2^32 on large grids
     uint64_t t = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
-    uint32_t W = 2 * R + 1;
+    uint32_t W = 2 * RS + 1;
     uint32_t nrun = (ncell + kRowRun - 1) / kRowRun;
     if (t >= (uint64_t)nrun * W) return;
     uint32_t run = (uint32_t)(t / W);
-    int dr = (int)(t % W) - R;
+    int dr = (int)(t % W) - RS;
     uint32_t c0 = run * kRowRun;
     uint32_t c1 = c0 + kRowRun < ncell ? c0 + kRowRun : ncell;
     uint32_t hint = c0;
     for (uint32_t c = c0; c < c1; c++) {
-        uint32_t key = cell_key[c];
-        uint32_t ds = seg_of(skbase, nsets, key);
-        if (dr == 0) cell_ds[c] = ds;
-        uint32_t ncx = sncx[ds], ncy = sncy[ds], kb = skbase[ds];
-        uint32_t local = key - kb;
-        int64_t cx = local / ncy, cy = local % ncy;
-        int64_t rx = cx + dr;
+        CellPlace pl = cell_place(D, cell_key[c]);
+        if (dr == 0) cell_ds[c] = pl.ds;
         uint32_t lo = 0, hi = 0;
-        if (rx >= 0 && rx < (int64_t)ncx) {
-            int64_t y0 = cy - R < 0 ? 0 : cy - R;
-            int64_t y1 = cy + R > (int64_t)ncy - 1 ? (int64_t)ncy - 1 : cy + R;
-            uint64_t k0 = kb + (uint64_t)(rx * ncy + y0);
-            uint64_t k1 = kb + (uint64_t)(rx * ncy + y1);
+        uint64_t k0, k1;
+        if (row_keys(D, pl, dr, R, &k0, &k1)) {
             lo = lower_bound_near(cell_key, ncell, (uint32_t)k0, hint);
             hi = k1 >= 0xffffffffull ? ncell
                                      : lower_bound_near(cell_key, ncell, (uint32_t)(k1 + 1), lo);
             hint = lo;
         }
-        row_lo[(size_t)c * W + (dr + R)] = lo;
-        row_hi[(size_t)c * W + (dr + R)] = hi;
+        row_lo[(size_t)c * W + (dr + RS)] = lo;
+        row_hi[(size_t)c * W + (dr + RS)] = hi;
     }
+}
+
+// points (start, count) of the cells [lo, hi)
+__device__ __forceinline__ uint2 cells_points(const uint32_t *cell_start, uint32_t lo, uint32_t hi)
+{
+    uint2 r = make_uint2(0u, 0u);
+    if (lo < hi) {
+        r.x = cell_start[lo];
+        r.y = cell_start[hi] - r.x;
+    }
+    return r;
 }
 
 // The same row ranges from a dense table over the key space: krank[k] = the
 // number of non-empty cells whose key is below k (an exclusive scan of the
 // occupied keys, which k_cells marks), so a row's run is [krank[k0],
 // krank[k1 + 1]). A thread per (cell, row), no search: for key spaces that
-// are a small multiple of the cell count. With row_pts, the run's points too.
-__global__ void k_row_ranges_dense(const uint32_t *cell_key, uint32_t ncell, const uint32_t *sncx,
-                                   const uint32_t *sncy, const uint32_t *skbase, uint32_t nsets,
-                                   int R, const uint32_t *krank, const uint32_t *cell_start,
+// are a small multiple of the cell count. With row_pts, the run's points too
+// (and those of its part within Rin cells of the centre cell, with row_in).
+__global__ void k_row_ranges_dense(const uint32_t *cell_key, uint32_t ncell, GridDims D, int R,
+                                   int RS, const uint32_t *krank, const uint32_t *cell_start,
                                    uint32_t *row_lo, uint32_t *row_hi, uint32_t *cell_ds,
-                                   uint2 *row_pts)
+                                   uint2 *row_pts, int Rin, int RSin, uint2 *row_in)
 {
     uint64_t t = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
-    uint32_t W = 2 * R + 1;
+    uint32_t W = 2 * RS + 1;
     if (t >= (uint64_t)ncell * W) return;
     uint32_t c = (uint32_t)(t / W);
-    int dr = (int)(t - (uint64_t)c * W) - R;
-    uint32_t key = cell_key[c];
-    uint32_t ds = seg_of(skbase, nsets, key);
-    if (dr == 0) cell_ds[c] = ds;
-    uint32_t ncx = sncx[ds], ncy = sncy[ds], kb = skbase[ds];
-    uint32_t local = key - kb;
-    int64_t cx = local / ncy, cy = local % ncy;
-    int64_t rx = cx + dr;
+    int dr = (int)(t - (uint64_t)c * W) - RS;
+    CellPlace pl = cell_place(D, cell_key[c]);
+    if (dr == 0) cell_ds[c] = pl.ds;
     uint32_t lo = 0, hi = 0;
-    if (rx >= 0 && rx < (int64_t)ncx) {
-        int64_t y0 = cy - R < 0 ? 0 : cy - R;
-        int64_t y1 = cy + R > (int64_t)ncy - 1 ? (int64_t)ncy - 1 : cy + R;
-        uint64_t k0 = kb + (uint64_t)(rx * ncy + y0);
-        uint64_t k1 = kb + (uint64_t)(rx * ncy + y1);
+    uint64_t k0, k1;
+    if (row_keys(D, pl, dr, R, &k0, &k1)) {
         lo = krank[k0];
         hi = krank[k1 + 1];
     }
     row_lo[t] = lo;
     row_hi[t] = hi;
-    if (row_pts) {
-        uint2 r = make_uint2(0u, 0u);
-        if (lo < hi) {
-            r.x = cell_start[lo];
-            r.y = cell_start[hi] - r.x;
+    if (row_pts) row_pts[t] = cells_points(cell_start, lo, hi);
+    if (row_in && dr >= -RSin && dr <= RSin) {
+        lo = hi = 0;
+        if (row_keys(D, pl, dr, Rin, &k0, &k1)) {
+            lo = krank[k0];
+            hi = krank[k1 + 1];
         }
-        row_pts[t] = r;
+        row_in[(size_t)c * (2 * RSin + 1) + (dr + RSin)] = cells_points(cell_start, lo, hi);
     }
 }
 
-// Point range (start, count) of every window row, from the row's cells
+// The same point ranges from the rows' cells (rows found by search), the part
+// within Rin cells of the centre cell by bisection over the row's few cells.
 __global__ void k_row_points(const uint32_t *row_lo, const uint32_t *row_hi,
-                             const uint32_t *cell_start, size_t nrows, uint2 *row_pts)
+                             const uint32_t *cell_start, const uint32_t *cell_key, GridDims D,
+                             size_t nrows, int RS, uint2 *row_pts, int Rin, int RSin,
+                             uint2 *row_in)
 {
     size_t t = (size_t)blockIdx.x * kBlock + threadIdx.x;
     if (t >= nrows) return;
     uint32_t lo = row_lo[t], hi = row_hi[t];
-    uint2 r = make_uint2(0u, 0u);
-    if (lo < hi) {
-        r.x = cell_start[lo];
-        r.y = cell_start[hi] - r.x;
+    row_pts[t] = cells_points(cell_start, lo, hi);
+    if (!row_in) return;
+    const uint32_t W = 2 * (uint32_t)RS + 1;
+    uint32_t c = (uint32_t)(t / W);
+    int dr = (int)(t - (size_t)c * W) - RS;
+    if (dr < -RSin || dr > RSin) return;
+    uint64_t k0, k1;
+    if (lo < hi && row_keys(D, cell_place(D, cell_key[c]), dr, Rin, &k0, &k1)) {
+        uint32_t a = lo, b = hi; // first cell with key >= k0
+        while (a < b) {
+            uint32_t m = a + ((b - a) >> 1);
+            if (cell_key[m] < k0) a = m + 1;
+            else b = m;
+        }
+        lo = a;
+        b = hi; // first cell with key > k1
+        while (a < b) {
+            uint32_t m = a + ((b - a) >> 1);
+            if (cell_key[m] <= k1) a = m + 1;
+            else b = m;
+        }
+        hi = a;
+    } else {
+        lo = hi = 0;
     }
-    row_pts[t] = r;
+    row_in[(size_t)c * (2 * RSin + 1) + (dr + RSin)] = cells_points(cell_start, lo, hi);
 }
 
 std::string slot(const char *tag, const char *name) { return std::string(tag) + "." + name; }
@@ -665,7 +724,7 @@ __global__ void k_classify_rows(const double *box, uint32_t ncell, int W, double
 
 int classify_rows(Context &c, Grid &G, double T, const char *tag)
 {
-    size_t W = 2 * (size_t)G.R + 1;
+    size_t W = 2 * (size_t)G.RS + 1;
     VDB_TRY(c.get(slot(tag, "row_f0").c_str(), G.ncell * W, &G.row_f0));
     VDB_TRY(c.get(slot(tag, "row_f1").c_str(), G.ncell * W, &G.row_f1));
     if (G.ncell == 0) return kOk;
@@ -698,6 +757,7 @@ int build_grid(Context &c, const Points &P, double w_min, int R, const char *tag
         w = spanmax / 65000.0;
         *enlarged = true;
     }
+    const uint32_t m = (uint32_t)G.m;
     std::vector<double> gx0(ns), gy0(ns);
     std::vector<uint32_t> ncx(ns), ncy(ns), kbase(ns + 1);
     for (int attempt = 0;; attempt++) {
@@ -715,7 +775,7 @@ int build_grid(Context &c, const Points &P, double w_min, int R, const char *tag
             ncx[d] = ok ? (uint32_t)fx : 1;
             ncy[d] = ok ? (uint32_t)fy : 1;
             kbase[d] = (uint32_t)std::min<uint64_t>(total, 0xffffffffull);
-            total += (uint64_t)ncx[d] * ncy[d];
+            total += ((uint64_t)ncx[d] + m - 1) / m * m * ncy[d]; // whole strips
         }
         kbase[ns] = (uint32_t)std::min<uint64_t>(total, 0xffffffffull);
         if (ok && total < 0xffffffffull) break;
@@ -732,6 +792,8 @@ int build_grid(Context &c, const Points &P, double w_min, int R, const char *tag
     G.ncx = ncx[0];
     G.ncy = ncy[0];
     G.R = R;
+    G.RS = (R + G.m - 1) / G.m;
+    G.RSin = (G.Rin + G.m - 1) / G.m;
     G.npts = n;
     G.nsets = ns;
     uint64_t nkeys = (uint64_t)kbase[ns];
@@ -761,7 +823,7 @@ int build_grid(Context &c, const Points &P, double w_min, int R, const char *tag
     VDB_TRY(c.get(slot(tag, "gtv").c_str(), n, &tv));
     unsigned g = ceil_div(n, kBlock);
     k_cell_keys<<<g, kBlock, 0, c.stream()>>>(P.xb, P.yb, n, P.seg, ns, G.sgx0, G.sgy0, w,
-                                              G.sncx, G.sncy, G.skbase, keys, vals);
+                                              G.sncx, G.sncy, G.skbase, m, keys, vals);
     VDB_HIP(hipGetLastError());
     uint32_t *sk, *sv;
     VDB_TRY(radix_sort_pairs(c, keys, vals, tk, tv, n, bits_for(nkeys), &sk, &sv));
@@ -812,29 +874,36 @@ int build_grid(Context &c, const Points &P, double w_min, int R, const char *tag
         VDB_HIP(hipGetLastError());
     }
 
-    size_t W = 2 * (size_t)R + 1;
+    const int RS = G.RS;
+    size_t W = 2 * (size_t)RS + 1;
+    const GridDims dims{G.sncx, G.sncy, G.skbase, ns, m};
     VDB_TRY(c.get(slot(tag, "row_lo").c_str(), ncell * W, &G.row_lo));
     VDB_TRY(c.get(slot(tag, "row_hi").c_str(), ncell * W, &G.row_hi));
     VDB_TRY(c.get(slot(tag, "cell_ds").c_str(), ncell, &G.cell_ds));
     G.row_pts = nullptr;
     if (G.want_row_pts)
         VDB_TRY(c.get(slot(tag, "row_pts").c_str(), std::max<size_t>(ncell * W, 1), &G.row_pts));
+    G.row_in = nullptr;
+    if (G.want_row_pts && G.Rin < R)
+        VDB_TRY(c.get(slot(tag, "row_in").c_str(),
+                      std::max<size_t>(ncell * (2 * (size_t)G.RSin + 1), 1), &G.row_in));
     if (dense) {
         uint32_t *krank;
         VDB_TRY(c.get(slot(tag, "krank").c_str(), nkeys + 1, &krank));
         VDB_TRY(scan_exclusive_u32(c, kflag, krank, nkeys + 1, nullptr));
         k_row_ranges_dense<<<ceil_div((uint64_t)ncell * W, kBlock), kBlock, 0, c.stream()>>>(
-            G.cell_key, ncell, G.sncx, G.sncy, G.skbase, ns, R, krank, G.cell_start, G.row_lo,
-            G.row_hi, G.cell_ds, G.row_pts);
+            G.cell_key, ncell, dims, R, RS, krank, G.cell_start, G.row_lo, G.row_hi, G.cell_ds,
+            G.row_pts, G.Rin, G.RSin, G.row_in);
         VDB_HIP(hipGetLastError());
         return kOk;
     }
     k_row_ranges<<<ceil_div(ceil_div(ncell, kRowRun) * W, kBlock), kBlock, 0, c.stream()>>>(
-        G.cell_key, ncell, G.sncx, G.sncy, G.skbase, ns, R, G.row_lo, G.row_hi, G.cell_ds);
+        G.cell_key, ncell, dims, R, RS, G.row_lo, G.row_hi, G.cell_ds);
     VDB_HIP(hipGetLastError());
     if (G.row_pts && ncell) {
         k_row_points<<<ceil_div(ncell * W, kBlock), kBlock, 0, c.stream()>>>(
-            G.row_lo, G.row_hi, G.cell_start, ncell * W, G.row_pts);
+            G.row_lo, G.row_hi, G.cell_start, G.cell_key, dims, ncell * W, RS, G.row_pts, G.Rin,
+            G.RSin, G.row_in);
         VDB_HIP(hipGetLastError());
     }
     return kOk;

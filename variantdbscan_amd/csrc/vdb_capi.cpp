@@ -99,13 +99,24 @@ int run_per_variant(Context &c, Points &P, const double *eps, const uint32_t *mi
         Grid G;
         Items I;
         Timer t0(c.stream(), st != nullptr);
-        int k = 0;
-        VDB_TRY(tune_cells_per_eps(c, P, e, precision, cells, &k));
+        // the fused engine in binary64 only asks which points reach the
+        // largest minpts of this eps; the table needs every count, and the
+        // float32 screening reports its rechecks over all of them
+        const bool core_only = mode == 0 && precision == VDB_PREC_FP64;
+        int k = cells ? cells : kFusedCellsPerEps;
+        if (!core_only) VDB_TRY(tune_cells_per_eps(c, P, e, precision, cells, &k));
         VDB_TRY(build_eps_grid(c, P, e, k, "g1", G));
-        VDB_TRY(build_items(c, G, "g1", I));
+        if (!core_only) VDB_TRY(build_items(c, G, "g1", I));
         if (st) st->ms_prepare += t0.ms();
         Timer t1(c.stream(), st != nullptr);
-        VDB_TRY(count_neighbors(c, G, I, e, precision, counts, (uint64_t *)rc));
+        if (core_only) {
+            uint32_t need = 0; // minpts above INT_MAX is never reached
+            for (uint32_t v : kv.second)
+                if (minpts[v] <= 0x7fffffffu) need = std::max(need, minpts[v]);
+            VDB_TRY(count_core(c, G, e, need, counts));
+        } else {
+            VDB_TRY(count_neighbors(c, G, I, e, precision, counts, (uint64_t *)rc));
+        }
         if (st) st->ms_count += t1.ms();
         if (verbose) {
             uint32_t largest = 0;

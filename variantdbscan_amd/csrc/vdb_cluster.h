@@ -43,6 +43,10 @@ int build_eps_grid(Context &c, const Points &P, double eps, int k, const char *t
 // Cells per eps for the per-variant kernels: the option's value when set
 // (1..kMaxCellsPerEps), else 0 (let tune_cells_per_eps choose).
 constexpr int kMaxCellsPerEps = 8;
+// The fused engine in binary64 (whose counts stop at minpts and whose
+// components run over cells) gains little from finer cells: 1M points, eps 0.4
+// and 0.6, minpts 100, kernel time 2.05, 2.12, 2.26, 2.47 ms at 2, 3, 4, 5.
+constexpr int kFusedCellsPerEps = 2;
 int cells_per_eps(const vdb_options *opt);
 
 // Autotuner: the first time a workload (point count, eps, extent, precision)
@@ -57,6 +61,9 @@ int tune_cells_per_eps(Context &c, const Points &P, double eps, int precision, i
 int count_neighbors(Context &c, const Grid &G, const Items &I, double eps, int precision,
                     uint32_t *counts, uint64_t *recheck_dev);
 
+// counts[p] is >= need exactly when |N_eps(p)| is, and exact below (binary64).
+int count_core(Context &c, const Grid &G, double eps, uint32_t need, uint32_t *counts);
+
 // Full per-variant clustering; labels written in caller order to out (device).
 // mode 0 = fused (no table), 1 = CSR table (count/scan/fill, union-find over
 // the table), tiled when the table exceeds table_budget bytes. border =
@@ -64,6 +71,7 @@ int count_neighbors(Context &c, const Grid &G, const Items &I, double eps, int p
 // the same clusters 0.. by their smallest core caller index, gives every
 // non-core point with a core neighbour the lowest-numbered adjacent cluster
 // and marks noise 0xffffffff.
+// (I: the items of G in mode 1; unused in mode 0)
 int cluster_variant(Context &c, const Points &P, const Grid &G, const Items &I, double eps,
                     uint32_t minpts, const uint32_t *counts, int mode, int border,
                     size_t table_budget, uint32_t *out, PhaseTimes *pt);
@@ -78,9 +86,9 @@ int cluster_variant(Context &c, const Points &P, const Grid &G, const Items &I, 
 //   border_pairs: for every non-core p with cl_of_pos[p] = C != 0, the
 //     pairs (C, root) for the distinct roots among p's core neighbours, as
 //     uint32 pairs; at most cap stored, *count_dev = all (repeats possible).
-int core_forest(Context &c, const Grid &G, const Items &I, double eps, uint32_t minpts,
+int core_forest(Context &c, const Grid &G, double eps, uint32_t minpts,
                 const uint32_t *counts, uint8_t *core, uint32_t *parent, uint32_t *best);
-int border_min_key(Context &c, const Grid &G, const Items &I, double eps, const uint8_t *core,
+int border_min_key(Context &c, const Grid &G, double eps, const uint8_t *core,
                    const uint32_t *parent, const uint32_t *key, uint32_t *best);
 int border_pairs(Context &c, const Grid &G, const Items &I, double eps, const uint8_t *core,
                  const uint32_t *parent, const uint32_t *cl_of_pos, uint32_t *pairs,

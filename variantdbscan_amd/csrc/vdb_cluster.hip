@@ -24,6 +24,7 @@ constexpr int kBlock = 256;
 constexpr int kWavesPerBlock = kBlock / kWave;
 constexpr uint32_t kNone = 0xffffffffu;
 constexpr int kDefaultCellsPerEps = 2;
+constexpr unsigned kListBlocks = 8192; // grids of the list kernels, at most
 
 struct GridView {
     const double *xs, *ys;
@@ -245,6 +246,137 @@ __global__ void __launch_bounds__(kBlock)
         if (lane_id() == b) mine = cnt[b] + full;
     if (lane_id() < (int)nb) counts[o0 + lane_id()] = mine;
     if (PREC == 1 && nre && lane_id() == 0) atomicAdd(recheck, (unsigned long long)nre);
+}
+
+// ------------------------------------------------------------ core test
+// Counts that only have to tell whether a point has `need` neighbours: they
+// stop there. Windows up to kFewCands points take a thread per point (about
+// 15 vector instructions for 64 candidates of 64 points); the others go, 8
+// origins of a cell at a time, to a wave each, which first adds up the cells
+// accepted whole: where those hold `need` points nothing is tested. At 1M
+// points, eps 0.4, need 100: the exact count (6 to 8 cells per eps) 1.66 ms, this 0.26.
+constexpr uint32_t kFewCands = 192;
+constexpr int kFewUnroll = 4;
+
+// points of cell c's window
+__device__ __forceinline__ uint32_t window_points(const GridView &g, uint32_t c)
+{
+    uint32_t w = 0;
+    for (int r = 0; r < g.W; r++) {
+        size_t t = (size_t)c * g.W + r;
+        uint32_t lo = g.row_lo[t], hi = g.row_hi[t];
+        if (lo < hi) w += g.cell_start[hi] - g.cell_start[lo];
+    }
+    return w;
+}
+
+// append v to list for every lane with take set, one atomic per wave
+__device__ __forceinline__ void list_append(bool take, uint32_t v, uint32_t *list, uint32_t *count)
+{
+    uint64_t m = ballot(take);
+    if (!m) return;
+    int leader = __builtin_ctzll(m);
+    uint32_t base = 0;
+    if (lane_id() == leader) base = atomicAdd(count, (uint32_t)popc64(m));
+    base = __shfl(base, leader);
+    if (take) list[base + mask_rank(m)] = v;
+}
+
+__global__ void __launch_bounds__(kBlock)
+    k_core_near(GridView g, const uint32_t *__restrict__ cell_of_pos, double T, uint32_t need,
+                uint32_t *__restrict__ counts, uint32_t *__restrict__ list,
+                uint32_t *__restrict__ nlist)
+{
+    uint32_t p = blockIdx.x * kBlock + threadIdx.x;
+    bool valid = p < g.n, far = false;
+    uint32_t c = 0;
+    if (valid) {
+        c = cell_of_pos[p];
+        far = window_points(g, c) > kFewCands;
+    }
+    list_append(far && (p - g.cell_start[c]) % kOrigins == 0, p, list, nlist);
+    if (!valid || far) return;
+    const double px = g.xs[p], py = g.ys[p];
+    uint32_t cnt = 0;
+    const int R = g.W / 2;
+    for (int u = 0; u < g.W && cnt < need; u++) {
+        int d = (u & 1) ? -((u + 1) >> 1) : (u >> 1); // centre out
+        size_t t = (size_t)c * g.W + (d + R);
+        uint32_t lo = g.row_lo[t], hi = g.row_hi[t];
+        if (lo >= hi) continue;
+        uint32_t a = g.cell_start[lo], e = g.cell_start[hi];
+        for (; a < e && cnt < need; a += kFewUnroll) {
+#pragma unroll
+            for (int i = 0; i < kFewUnroll; i++) {
+                uint32_t q = a + i < e ? a + i : e - 1;
+                bool in = dist2_exact(px, py, g.xs[q], g.ys[q]) <= T;
+                cnt += in && a + i < e ? 1u : 0u;
+            }
+        }
+    }
+    counts[p] = cnt;
+}
+
+__global__ void __launch_bounds__(kBlock)
+    k_core_far(GridView g, const uint32_t *__restrict__ cell_of_pos, double T, uint32_t need,
+               uint32_t *__restrict__ counts, const uint32_t *__restrict__ list,
+               const uint32_t *__restrict__ nlist)
+{
+    const uint32_t nl = *nlist;
+    const int R = g.W / 2, lane = lane_id();
+    const double qnan = __longlong_as_double(0x7ff8000000000000ll);
+    for (uint32_t i = blockIdx.x * kWavesPerBlock + wave_id_in_block(); i < nl;
+         i += gridDim.x * kWavesPerBlock) {
+        const uint32_t o0 = sgpr_u32(list[i]), c = sgpr_u32(cell_of_pos[o0]);
+        uint32_t nb = sgpr_u32(g.cell_start[c + 1]) - o0;
+        nb = nb < kOrigins ? nb : kOrigins;
+        uint32_t full = 0;
+        for (int r = lane; r < g.W; r += kWave) {
+            RowSeg sg = row_seg(g, c, r);
+            full += sg.f1 - sg.f0;
+        }
+        for (int o = kWave / 2; o > 0; o >>= 1) full += __shfl_xor(full, o);
+        full = sgpr_u32(full);
+        uint32_t cnt[kOrigins];
+#pragma unroll
+        for (int b = 0; b < kOrigins; b++) cnt[b] = full;
+        if (full < need) {
+            double ox[kOrigins], oy[kOrigins];
+#pragma unroll
+            for (int b = 0; b < kOrigins; b++) {
+                uint32_t ob = o0 + (b < (int)nb ? b : 0);
+                ox[b] = b < (int)nb ? sgpr_d(g.xs[ob]) : qnan;
+                oy[b] = sgpr_d(g.ys[ob]);
+            }
+            bool done = false;
+            auto test = [&](uint32_t a, uint32_t e) {
+                for (uint32_t q0 = a; q0 < e && !done; q0 += kWave) {
+                    uint32_t q = q0 + (uint32_t)lane;
+                    uint32_t qc = q < e ? q : e - 1;
+                    double qx = g.xs[qc], qy = g.ys[qc];
+                    if (q >= e) qx = qnan;
+                    done = true;
+#pragma unroll
+                    for (int b = 0; b < kOrigins; b++) {
+                        if (b >= (int)nb) break;
+                        cnt[b] += (uint32_t)popc64(ballot(dist2_exact(ox[b], oy[b], qx, qy) <= T));
+                        done = done && cnt[b] >= need;
+                    }
+                }
+            };
+            for (int u = 0; u < g.W && !done; u++) {
+                int d = (u & 1) ? -((u + 1) >> 1) : (u >> 1); // centre out
+                RowSeg sg = row_seg(g, c, d + R);
+                test(sg.a, sg.f0);
+                test(sg.f1, sg.e);
+            }
+        }
+        uint32_t mine = 0;
+#pragma unroll
+        for (int b = 0; b < kOrigins; b++)
+            if (lane == b) mine = cnt[b];
+        if (lane < (int)nb) counts[o0 + lane] = mine;
+    }
 }
 
 // ----------------------------------------------------------------- table
@@ -604,9 +736,10 @@ __device__ void uf_unite(uint32_t *parent, const uint32_t *rank, uint32_t a, uin
 }
 
 __global__ void k_core_init(const uint32_t *counts, uint32_t n, uint32_t minpts,
-                            uint8_t *core, uint32_t *parent, uint32_t *best)
+                            uint8_t *core, uint32_t *parent, uint32_t *best, uint32_t *nborder)
 {
     uint32_t p = blockIdx.x * kBlock + threadIdx.x;
+    if (p == 0) *nborder = 0; // the border pass's list
     if (p >= n) return;
     // minpts above INT_MAX wraps negative in the reference's int and no point
     // is core (src/structs.h:37, src/DBScan.cpp:552)
@@ -623,65 +756,68 @@ __global__ void k_fill_u32_n(uint32_t *a, uint32_t v, uint32_t n)
 }
 
 __global__ void __launch_bounds__(kBlock)
-    k_uf_fused(GridView g, const uint32_t *__restrict__ item_cell,
-               const uint32_t *__restrict__ item_o0, uint32_t nitems, double T,
+    k_uf_fused(GridView g, const uint32_t *__restrict__ cell_of_pos, double T,
                const uint8_t *__restrict__ core, const uint32_t *__restrict__ rank,
-               uint32_t *parent)
+               uint32_t *parent, const uint32_t *noclique)
 {
-    uint32_t it = blockIdx.x * kWavesPerBlock + wave_id_in_block();
-    if (it >= nitems) return;
-    uint32_t c = item_cell[it], o0 = item_o0[it];
-    uint32_t nb = g.cell_start[c + 1] - o0;
-    nb = nb < kOrigins ? nb : kOrigins;
-    double ox[kOrigins], oy[kOrigins];
-    uint32_t rp[kOrigins];
-    uint32_t any = 0;
-#pragma unroll
-    for (int b = 0; b < kOrigins; b++) {
-        uint32_t ob = o0 + (b < (int)nb ? b : nb - 1);
-        bool isc = b < (int)nb && core[ob];
-        ox[b] = sgpr_d(isc ? g.xs[ob] : __longlong_as_double(0x7ff8000000000000ll));
-        oy[b] = sgpr_d(g.ys[ob]);
-        rp[b] = isc ? uf_find(parent, ob) : kNone;
-        any |= isc;
-    }
-    if (!any) return;
-    uint32_t qmax = o0 + nb;
-    // the half window (rows below the centre, the centre row before the
-    // item's last origin), row segments accepted without a test included
-    auto blockfn = [&](uint32_t q, bool v, double qx, double qy, bool full) {
-        bool qc = v && core[q];
-        if (!ballot(qc)) return;
-        uint32_t pq = qc ? ld_par(parent + q) : 0u;
+    if (!*noclique) return; // k_cf_unite's
+    // 8 positions a wave, run by run of one cell
+    const uint32_t i0 = (blockIdx.x * kWavesPerBlock + wave_id_in_block()) * kOrigins;
+    const uint32_t i1 = i0 + kOrigins < g.n ? i0 + kOrigins : g.n;
+    for (uint32_t o0 = i0, nb; o0 < i1; o0 += nb) {
+        const uint32_t c = cell_of_pos[o0];
+        nb = sgpr_u32(g.cell_start[c + 1]) - o0;
+        nb = o0 + nb < i1 ? nb : i1 - o0;
+        double ox[kOrigins], oy[kOrigins];
+        uint32_t rp[kOrigins];
+        uint32_t any = 0;
 #pragma unroll
         for (int b = 0; b < kOrigins; b++) {
-            if (rp[b] == kNone) continue;
-            bool e = qc && (full || dist2_exact(ox[b], oy[b], qx, qy) <= T) && pq != rp[b];
-            uint64_t m = ballot(e);
-            if (m) {
-                if (e) uf_unite(parent, rank, q, o0 + b);
-                rp[b] = uf_find(parent, o0 + b);
+            uint32_t ob = o0 + (b < (int)nb ? b : nb - 1);
+            bool isc = b < (int)nb && core[ob];
+            ox[b] = sgpr_d(isc ? g.xs[ob] : __longlong_as_double(0x7ff8000000000000ll));
+            oy[b] = sgpr_d(g.ys[ob]);
+            rp[b] = isc ? uf_find(parent, ob) : kNone;
+            any |= isc;
+        }
+        if (!any) continue;
+        uint32_t qmax = o0 + nb;
+        // the half window (rows below the centre, the centre row before the
+        // item's last origin), row segments accepted without a test included
+        auto blockfn = [&](uint32_t q, bool v, double qx, double qy, bool full) {
+            bool qc = v && core[q];
+            if (!ballot(qc)) return;
+            uint32_t pq = qc ? ld_par(parent + q) : 0u;
+#pragma unroll
+            for (int b = 0; b < kOrigins; b++) {
+                if (rp[b] == kNone) continue;
+                bool e = qc && (full || dist2_exact(ox[b], oy[b], qx, qy) <= T) && pq != rp[b];
+                uint64_t m = ballot(e);
+                if (m) {
+                    if (e) uf_unite(parent, rank, q, o0 + b);
+                    rp[b] = uf_find(parent, o0 + b);
+                }
             }
+        };
+        int R = g.W / 2;
+        for (int r = 0; r <= R; r++) {
+            RowSeg sg = row_seg(g, c, r);
+            if (r == R) {
+                sg.e = sg.e < qmax ? sg.e : qmax;
+                sg.f1 = sg.f1 < sg.e ? sg.f1 : sg.e;
+                sg.f0 = sg.f0 < sg.f1 ? sg.f0 : sg.f1;
+            }
+            run_blocks(g, sg.a, sg.f0, [&](uint32_t q, bool v, double qx, double qy) {
+                blockfn(q, v, qx, qy, false);
+            });
+            for (uint32_t q0 = sg.f0; q0 < sg.f1; q0 += kWave) {
+                uint32_t q = q0 + lane_id();
+                blockfn(q, q < sg.f1, 0.0, 0.0, true);
+            }
+            run_blocks(g, sg.f1, sg.e, [&](uint32_t q, bool v, double qx, double qy) {
+                blockfn(q, v, qx, qy, false);
+            });
         }
-    };
-    int R = g.W / 2;
-    for (int r = 0; r <= R; r++) {
-        RowSeg sg = row_seg(g, c, r);
-        if (r == R) {
-            sg.e = sg.e < qmax ? sg.e : qmax;
-            sg.f1 = sg.f1 < sg.e ? sg.f1 : sg.e;
-            sg.f0 = sg.f0 < sg.f1 ? sg.f0 : sg.f1;
-        }
-        run_blocks(g, sg.a, sg.f0, [&](uint32_t q, bool v, double qx, double qy) {
-            blockfn(q, v, qx, qy, false);
-        });
-        for (uint32_t q0 = sg.f0; q0 < sg.f1; q0 += kWave) {
-            uint32_t q = q0 + lane_id();
-            blockfn(q, q < sg.f1, 0.0, 0.0, true);
-        }
-        run_blocks(g, sg.f1, sg.e, [&](uint32_t q, bool v, double qx, double qy) {
-            blockfn(q, v, qx, qy, false);
-        });
     }
 }
 
@@ -699,59 +835,284 @@ __device__ uint32_t uf_root(const uint32_t *parent, uint32_t x)
     return x;
 }
 
-__global__ void k_compress(uint32_t *parent, const uint8_t *core, uint32_t n)
+__global__ void k_compress(uint32_t *parent, const uint8_t *core, uint32_t n,
+                           const uint32_t *noclique)
 {
     uint32_t p = blockIdx.x * kBlock + threadIdx.x;
-    if (p >= n || !core[p]) return;
+    if (p >= n || !core[p] || !*noclique) return;
     st_par(parent + p, uf_root(parent, p));
 }
 
-// border: best[p] = smallest rank[root] among core neighbours of non-core p
-// (rank is the binned rank, or any per-root key the caller orders roots by)
-__global__ void __launch_bounds__(kBlock)
-    k_border_fused(GridView g, const uint32_t *__restrict__ item_cell,
-                   const uint32_t *__restrict__ item_o0, uint32_t nitems, double T,
-                   const uint8_t *__restrict__ core, const uint32_t *__restrict__ rank,
-                   const uint32_t *__restrict__ parent, uint32_t *__restrict__ best)
+// ------------------------------------------- core components over cells
+// When every cell is a clique (classify_rows found no other: cells of eps/2
+// or less) the core points of a cell are connected, and the components are
+// those of the cells holding core points: an edge wherever some core-core
+// pair of two cells is within eps. A cell is represented by its first core
+// position (ranks ascend inside a cell, so also its smallest core rank).
+// Pairs of cells wholly within eps need no test; a partial pair is tested only
+// while its cells are not connected, which after the adjacent cells are
+// united leaves the gaps between clusters. Against uniting point pairs
+// (k_uf_fused, still used where some cell is no clique): 7.35 ms -> 1.12
+// at 2M points, eps 0.3.
+struct CellForest {
+    uint32_t *par;  // parent cell (smaller index), a root points at itself
+    uint32_t *rep;  // first core position of a cell, NONE without one
+    uint32_t *low;  // smallest core rank of a root's component
+    const uint32_t *noclique;
+};
+
+__global__ void k_cf_init(CellForest F, uint32_t ncell)
 {
-    uint32_t it = blockIdx.x * kWavesPerBlock + wave_id_in_block();
-    if (it >= nitems) return;
-    uint32_t c = item_cell[it], o0 = item_o0[it];
-    uint32_t nb = g.cell_start[c + 1] - o0;
-    nb = nb < kOrigins ? nb : kOrigins;
-    double ox[kOrigins], oy[kOrigins];
-    uint32_t bst[kOrigins];
-    uint32_t any = 0;
-#pragma unroll
-    for (int b = 0; b < kOrigins; b++) {
-        uint32_t ob = o0 + (b < (int)nb ? b : nb - 1);
-        bool nc = b < (int)nb && !core[ob];
-        ox[b] = sgpr_d(nc ? g.xs[ob] : __longlong_as_double(0x7ff8000000000000ll));
-        oy[b] = sgpr_d(g.ys[ob]);
-        bst[b] = kNone;
-        any |= nc;
+    uint32_t c = blockIdx.x * kBlock + threadIdx.x;
+    if (c >= ncell || *F.noclique) return;
+    F.par[c] = c;
+    F.rep[c] = kNone;
+    F.low[c] = kNone;
+}
+
+__global__ void k_cf_rep(CellForest F, const uint8_t *core, const uint32_t *cell_of_pos,
+                         const uint32_t *cell_start, uint32_t n)
+{
+    uint32_t p = blockIdx.x * kBlock + threadIdx.x;
+    if (p >= n || *F.noclique || !core[p]) return;
+    uint32_t c = cell_of_pos[p];
+    // runs of core points: only their first competes
+    if (p > cell_start[c] && core[p - 1]) return;
+    atomicMin(F.rep + c, p);
+}
+
+__device__ uint32_t cell_find(uint32_t *par, uint32_t x)
+{
+    while (true) {
+        uint32_t p = ld_par(par + x);
+        if (p == x) return x;
+        uint32_t gp = ld_par(par + p);
+        if (gp == p) return p;
+        st_par(par + x, gp);
+        x = gp;
     }
-    if (!any) return;
-    window_blocks(g, c, false, 0, [&](uint32_t q, bool v, double qx, double qy) {
-        bool qc = v && core[q];
-        if (!ballot(qc)) return;
-        uint32_t rr = qc ? rank[parent[q]] : kNone;
-#pragma unroll
-        for (int b = 0; b < kOrigins; b++) {
-            uint32_t cand = (qc && dist2_exact(ox[b], oy[b], qx, qy) <= T) ? rr : kNone;
-            if (!ballot(cand != kNone)) continue;
-            for (int o = kWave / 2; o > 0; o >>= 1) {
-                uint32_t t = __shfl_xor(cand, o);
-                cand = t < cand ? t : cand;
-            }
-            bst[b] = cand < bst[b] ? cand : bst[b];
+}
+
+__device__ void cell_unite(uint32_t *par, uint32_t a, uint32_t b)
+{
+    while (true) {
+        a = cell_find(par, a);
+        b = cell_find(par, b);
+        if (a == b) return;
+        if (a > b) {
+            uint32_t t = a;
+            a = b;
+            b = t;
         }
-    });
-    uint32_t mine = kNone;
+        if (atomicCAS(par + b, b, a) == b) return;
+    }
+}
+
+// some core-core pair of cells A and B within eps? The smaller cell is
+// screened 64 points at a time against the other's box.
+__device__ bool cells_touch(const GridView &g, const double *box, const uint8_t *core, double T,
+                            uint32_t A, uint32_t B)
+{
+    uint32_t a0 = g.cell_start[A], a1 = g.cell_start[A + 1];
+    uint32_t b0 = g.cell_start[B], b1 = g.cell_start[B + 1];
+    if (a1 - a0 > b1 - b0) { // lanes sweep the larger cell
+        uint32_t t = A;
+        A = B;
+        B = t;
+        t = a0;
+        a0 = b0;
+        b0 = t;
+        t = a1;
+        a1 = b1;
+        b1 = t;
+    }
+    const int lane = lane_id();
+    const double *bb = box + 4 * (size_t)B;
+    const double bx0 = bb[0], bx1 = bb[1], by0 = bb[2], by1 = bb[3];
+    for (uint32_t p0 = a0; p0 < a1; p0 += kWave) {
+        uint32_t p = p0 + (uint32_t)lane, pc = p < a1 ? p : a1 - 1;
+        double px = g.xs[pc], py = g.ys[pc];
+        bool cand = p < a1 && core[pc] && box_dist2_min(px, py, bx0, bx1, by0, by1) <= T;
+        uint64_t m = ballot(cand);
+        while (m) {
+            int bit = __builtin_ctzll(m);
+            m &= m - 1;
+            double cx = __shfl(px, bit), cy = __shfl(py, bit);
+            for (uint32_t q0 = b0; q0 < b1; q0 += kWave) {
+                uint32_t q = q0 + (uint32_t)lane, qc = q < b1 ? q : b1 - 1;
+                bool hit = q < b1 && core[qc] && dist2_exact(cx, cy, g.xs[qc], g.ys[qc]) <= T;
+                if (ballot(hit)) return true;
+            }
+        }
+    }
+    return false;
+}
+
+// A wave per cell A with a core point, lanes over the cells B < A of its
+// window: the adjacent ones (near), or all.
+__global__ void __launch_bounds__(kBlock)
+    k_cf_unite(GridView g, CellForest F, const uint32_t *cell_key, uint32_t ncell, uint32_t ncy,
+               const double *box, const uint8_t *core, double T, bool near)
+{
+    uint32_t A = blockIdx.x * kWavesPerBlock + wave_id_in_block();
+    if (A >= ncell || *F.noclique) return;
+    A = sgpr_u32(A);
+    if (F.rep[A] == kNone) return;
+    const int R = g.W / 2, lane = lane_id();
+    uint32_t ra = sgpr_u32(cell_find(F.par, A));
+    const uint32_t kA = cell_key[A];
+    for (int r = near && R > 0 ? R - 1 : 0; r <= R; r++) {
+        size_t t = (size_t)A * g.W + r;
+        uint32_t lo = g.row_lo[t], hi = g.row_hi[t], f0 = g.row_f0[t], f1 = g.row_f1[t];
+        if (hi > A) hi = A;
+        for (uint32_t B0 = lo; B0 < hi; B0 += kWave) {
+            uint32_t B = B0 + (uint32_t)lane;
+            bool on = B < hi;
+            uint32_t Bc = on ? B : hi - 1;
+            uint32_t pb = ld_par(F.par + Bc);
+            on = on && F.rep[Bc] != kNone;
+            if (near) {
+                uint32_t k = kA + (uint32_t)(r - R) * ncy; // beside A in B's column
+                uint32_t kb = cell_key[Bc];
+                on = on && kb + 1u >= k && kb <= k + 1u;
+            }
+            if (on && pb != ra) on = cell_find(F.par, pb) != ra;
+            else on = false;
+            uint64_t m = ballot(on);
+            if (!m) continue;
+            bool whole = on && B >= f0 && B < f1;
+            if (whole) cell_unite(F.par, A, B);
+            m &= ~ballot(whole);
+            while (m) {
+                int bit = __builtin_ctzll(m);
+                m &= m - 1;
+                uint32_t Bb = B0 + (uint32_t)bit;
+                if (cell_find(F.par, Bb) == cell_find(F.par, A)) continue;
+                if (cells_touch(g, box, core, T, A, Bb)) {
+                    if (lane == 0) cell_unite(F.par, A, Bb);
+                }
+            }
+            ra = sgpr_u32(cell_find(F.par, A));
+        }
+    }
+}
+
+// every cell at its root, and the smallest core rank of each component (one
+// atomic per wave for the lanes sharing the first lane's root)
+__global__ void k_cf_flat(CellForest F, uint32_t ncell, const uint32_t *rank, bool low)
+{
+    uint32_t c = blockIdx.x * kBlock + threadIdx.x;
+    if (*F.noclique) return;
+    bool valid = c < ncell && F.rep[c] != kNone;
+    uint32_t root = kNone, v = kNone;
+    if (valid) {
+        root = uf_root(F.par, c);
+        st_par(F.par + c, root);
+    }
+    if (!low) return;
+    if (valid) v = rank[F.rep[c]];
+    uint64_t todo = ballot(valid);
+    if (todo) {
+        int leader = __builtin_ctzll(todo);
+        uint32_t r = __shfl(root, leader);
+        bool same = valid && root == r;
+        todo &= ~ballot(same);
+        uint32_t m = same ? v : kNone;
+        for (int o = kWave / 2; o > 0; o >>= 1) {
+            uint32_t t = __shfl_xor(m, o);
+            m = t < m ? t : m;
+        }
+        if (lane_id() == leader && m < ld_par(F.low + r)) atomicMin(F.low + r, m);
+    }
+    if (((todo >> lane_id()) & 1ull) && v < ld_par(F.low + root)) atomicMin(F.low + root, v);
+}
+
+// parent[p] = position of the smallest-rank core point of p's component.
+// parent and F.rep may be one array: F.rep is not read here.
+__global__ void k_cf_points(CellForest F, const uint8_t *core, const uint32_t *cell_of_pos,
+                            const uint32_t *rank_pos, uint32_t n, uint32_t *parent)
+{
+    uint32_t p = blockIdx.x * kBlock + threadIdx.x;
+    if (p >= n || *F.noclique) return;
+    parent[p] = core[p] ? rank_pos[F.low[F.par[cell_of_pos[p]]]] : p;
+}
+
+// border: best[p] = smallest rank[root] among core neighbours of non-core p
+// (rank is the binned rank, or any per-root key the caller orders roots by).
+// A thread per point for windows up to kFewCands points, a wave for others;
+// minima stay in the lanes until the end (8 origins a wave with a reduction
+// across lanes per block: 0.57 ms at 1M points, eps 0.4 to 0.6; now 0.25).
+__global__ void __launch_bounds__(kBlock)
+    k_border_near(GridView g, const uint32_t *__restrict__ cell_of_pos, double T,
+                  const uint8_t *__restrict__ core, const uint32_t *__restrict__ rank,
+                  const uint32_t *__restrict__ parent, uint32_t *__restrict__ best,
+                  uint32_t *__restrict__ list, uint32_t *__restrict__ nlist)
+{
+    uint32_t p = blockIdx.x * kBlock + threadIdx.x;
+    bool valid = p < g.n && !core[p], far = false;
+    uint32_t c = 0;
+    if (valid) {
+        c = cell_of_pos[p];
+        far = window_points(g, c) > kFewCands;
+    }
+    list_append(far, p, list, nlist);
+    if (!valid || far) return;
+    const double px = g.xs[p], py = g.ys[p];
+    uint32_t m = kNone;
+    for (int r = 0; r < g.W; r++) {
+        size_t t = (size_t)c * g.W + r;
+        uint32_t lo = g.row_lo[t], hi = g.row_hi[t];
+        if (lo >= hi) continue;
+        uint32_t a = g.cell_start[lo], e = g.cell_start[hi];
+        for (; a < e; a += kFewUnroll) {
+            bool hit[kFewUnroll];
 #pragma unroll
-    for (int b = 0; b < kOrigins; b++)
-        if (lane_id() == b) mine = bst[b];
-    if (lane_id() < (int)nb && !core[o0 + lane_id()]) best[o0 + lane_id()] = mine;
+            for (int i = 0; i < kFewUnroll; i++) {
+                uint32_t q = a + i < e ? a + i : e - 1;
+                hit[i] = core[q] && dist2_exact(px, py, g.xs[q], g.ys[q]) <= T;
+            }
+#pragma unroll
+            for (int i = 0; i < kFewUnroll; i++)
+                if (hit[i]) {
+                    uint32_t v = rank[parent[a + i < e ? a + i : e - 1]];
+                    m = v < m ? v : m;
+                }
+        }
+    }
+    best[p] = m;
+}
+
+__global__ void __launch_bounds__(kBlock)
+    k_border_far(GridView g, const uint32_t *__restrict__ cell_of_pos, double T,
+                 const uint8_t *__restrict__ core, const uint32_t *__restrict__ rank,
+                 const uint32_t *__restrict__ parent, uint32_t *__restrict__ best,
+                 const uint32_t *__restrict__ list, const uint32_t *__restrict__ nlist)
+{
+    const uint32_t nl = *nlist;
+    for (uint32_t i = blockIdx.x * kWavesPerBlock + wave_id_in_block(); i < nl;
+         i += gridDim.x * kWavesPerBlock) {
+        const uint32_t p = sgpr_u32(list[i]), c = sgpr_u32(cell_of_pos[p]);
+        const double px = sgpr_d(g.xs[p]), py = sgpr_d(g.ys[p]);
+        uint32_t m = kNone;
+        for (int r = 0; r < g.W; r++) {
+            RowSeg sg = row_seg(g, c, r);
+            for (uint32_t q0 = sg.a; q0 < sg.e; q0 += kWave) {
+                uint32_t q = q0 + (uint32_t)lane_id();
+                uint32_t qc = q < sg.e ? q : sg.e - 1;
+                bool hit = q < sg.e && core[qc] &&
+                           dist2_exact(px, py, g.xs[qc], g.ys[qc]) <= T;
+                if (hit) {
+                    uint32_t v = rank[parent[qc]];
+                    m = v < m ? v : m;
+                }
+            }
+        }
+        for (int o = kWave / 2; o > 0; o >>= 1) {
+            uint32_t t = __shfl_xor(m, o);
+            m = t < m ? t : m;
+        }
+        if (lane_id() == 0) best[p] = m;
+    }
 }
 
 // (C, root) pairs for the reuse emulation: for every non-core position p with
@@ -1119,6 +1480,78 @@ int count_neighbors(Context &c, const Grid &G, const Items &I, double eps, int p
     return kOk;
 }
 
+int count_core(Context &c, const Grid &G, double eps, uint32_t need, uint32_t *counts)
+{
+    uint32_t n = G.npts;
+    uint32_t *list; // a buffer of the label pass, unused until then
+    VDB_TRY(c.get("lab.flag", n, &list));
+    const double T = threshold_for_eps(eps);
+    VDB_TRY(c.kt_begin("k_count"));
+    k_core_near<<<ceil_div(n, kBlock), kBlock, 0, c.stream()>>>(
+        view(G, n), G.cell_of_pos, T, need, counts, list, G.words + 2);
+    VDB_HIP(hipGetLastError());
+    k_core_far<<<std::min(ceil_div(n, kWavesPerBlock * kOrigins), kListBlocks), kBlock, 0,
+                 c.stream()>>>(view(G, n), G.cell_of_pos, T, need, counts, list, G.words + 2);
+    VDB_TRY(c.kt_end("k_count"));
+    VDB_HIP(hipGetLastError());
+    return kOk;
+}
+
+// The flat core forest: parent[p] = position of the smallest-rank point of
+// core p's component. Over cells when all are cliques, else over points (the
+// device decides: the kernels of the other way return at once).
+static int core_components(Context &c, const Grid &G, double T,
+                           const uint8_t *core, uint32_t *parent)
+{
+    const uint32_t n = G.npts, nc = G.ncell;
+    const unsigned g = ceil_div(n, kBlock);
+    if (n) {
+        VDB_TRY(c.kt_begin("k_uf_fused"));
+        // buffers of the label pass, and parent, which k_cf_points writes last
+        CellForest F{nullptr, parent, nullptr, G.words + 1};
+        VDB_TRY(c.get("lab.flag", n, &F.par));
+        VDB_TRY(c.get("lab.cid", n, &F.low));
+        const unsigned gc = ceil_div(nc, kBlock), gw = ceil_div(nc, kWavesPerBlock);
+        k_cf_init<<<gc, kBlock, 0, c.stream()>>>(F, nc);
+        VDB_HIP(hipGetLastError());
+        k_cf_rep<<<g, kBlock, 0, c.stream()>>>(F, core, G.cell_of_pos, G.cell_start, n);
+        VDB_HIP(hipGetLastError());
+        for (int pass = 0; pass < 2; pass++) {
+            k_cf_unite<<<gw, kBlock, 0, c.stream()>>>(view(G, n), F, G.cell_key, nc, G.ncy,
+                                                     G.cell_box, core, T, pass == 0);
+            VDB_HIP(hipGetLastError());
+            k_cf_flat<<<gc, kBlock, 0, c.stream()>>>(F, nc, G.pos_rank, pass == 1);
+            VDB_HIP(hipGetLastError());
+        }
+        k_cf_points<<<g, kBlock, 0, c.stream()>>>(F, core, G.cell_of_pos, G.rank_pos, n, parent);
+        VDB_HIP(hipGetLastError());
+        k_uf_fused<<<ceil_div(n, kWavesPerBlock * kOrigins), kBlock, 0, c.stream()>>>(
+            view(G, n), G.cell_of_pos, T, core, G.pos_rank, parent, G.words + 1);
+        VDB_HIP(hipGetLastError());
+        VDB_TRY(c.kt_end("k_uf_fused"));
+    }
+    k_compress<<<g, kBlock, 0, c.stream()>>>(parent, core, n, G.words + 1);
+    VDB_HIP(hipGetLastError());
+    return kOk;
+}
+
+static int border_pass(Context &c, const Grid &G, double T, const uint8_t *core,
+                       const uint32_t *key, const uint32_t *parent, uint32_t *best)
+{
+    const uint32_t n = G.npts;
+    uint32_t *list; // a buffer of the label pass
+    VDB_TRY(c.get("lab.flag", n, &list));
+    VDB_TRY(c.kt_begin("k_border_fused"));
+    k_border_near<<<ceil_div(n, kBlock), kBlock, 0, c.stream()>>>(
+        view(G, n), G.cell_of_pos, T, core, key, parent, best, list, G.words + 3);
+    VDB_HIP(hipGetLastError());
+    k_border_far<<<std::min(ceil_div(n, kWavesPerBlock), kListBlocks), kBlock, 0, c.stream()>>>(
+        view(G, n), G.cell_of_pos, T, core, key, parent, best, list, G.words + 3);
+    VDB_TRY(c.kt_end("k_border_fused"));
+    VDB_HIP(hipGetLastError());
+    return kOk;
+}
+
 static int finish_labels(Context &c, const Points &P, const Grid &G, const uint8_t *core,
                          const uint32_t *parent, const uint32_t *best, const uint32_t *key,
                          uint32_t *out)
@@ -1173,29 +1606,14 @@ int cluster_variant(Context &c, const Points &P, const Grid &G, const Items &I, 
     };
     const uint32_t *bkey = key ? key : G.pos_rank;
     EvTimer tm(c.stream());
-    k_core_init<<<g, kBlock, 0, c.stream()>>>(counts, n, minpts, core, parent, best);
+    k_core_init<<<g, kBlock, 0, c.stream()>>>(counts, n, minpts, core, parent, best, G.words + 3);
     VDB_HIP(hipGetLastError());
-    unsigned blocks = ceil_div(I.n, kWavesPerBlock);
     if (mode == 0) {
         if (pt) tm.start();
-        if (I.n) {
-            VDB_TRY(c.kt_begin("k_uf_fused"));
-            k_uf_fused<<<blocks, kBlock, 0, c.stream()>>>(view(G, G.npts), I.cell, I.o0, I.n, T, core,
-                                                          G.pos_rank, parent);
-            VDB_TRY(c.kt_end("k_uf_fused"));
-        }
-        VDB_HIP(hipGetLastError());
-        k_compress<<<g, kBlock, 0, c.stream()>>>(parent, core, n);
-        VDB_HIP(hipGetLastError());
+        VDB_TRY(core_components(c, G, T, core, parent));
         VDB_TRY(root_keys());
         if (pt) pt->uf += tm.stop(), tm.start();
-        if (I.n) {
-            VDB_TRY(c.kt_begin("k_border_fused"));
-            k_border_fused<<<blocks, kBlock, 0, c.stream()>>>(view(G, G.npts), I.cell, I.o0, I.n, T,
-                                                              core, bkey, parent, best);
-            VDB_TRY(c.kt_end("k_border_fused"));
-        }
-        VDB_HIP(hipGetLastError());
+        VDB_TRY(border_pass(c, G, T, core, bkey, parent, best));
         if (pt) pt->border += tm.stop();
     } else {
         // table mode: offsets over positions, then tiles of whole cells
@@ -1230,20 +1648,10 @@ int cluster_variant(Context &c, const Points &P, const Grid &G, const Items &I, 
         VDB_TRY(c.get("cv.ids", want ? want : 1, &ids));
         // tiles never exceed the buffer actually held
         cap = want;
-        // Core components: the fused half-window union-find (distances
-        // recomputed, each unordered pair once) rather than a pass over the
-        // table, which would read every row's ids again (95 GB at 2M points,
-        // eps 0.5) at gather speed.
+        // Core components from the grid rather than from the table, which
+        // would read every row's ids again (95 GB at 2M points, eps 0.5).
         if (pt) tm.start();
-        if (I.n) {
-            VDB_TRY(c.kt_begin("k_uf_fused"));
-            k_uf_fused<<<blocks, kBlock, 0, c.stream()>>>(view(G, G.npts), I.cell, I.o0, I.n, T,
-                                                          core, G.pos_rank, parent);
-            VDB_TRY(c.kt_end("k_uf_fused"));
-        }
-        VDB_HIP(hipGetLastError());
-        k_compress<<<g, kBlock, 0, c.stream()>>>(parent, core, n);
-        VDB_HIP(hipGetLastError());
+        VDB_TRY(core_components(c, G, T, core, parent));
         VDB_TRY(root_keys());
         if (pt) pt->uf += tm.stop();
         // The table, tile by tile (tiles are runs of items: items are ordered
@@ -1305,40 +1713,26 @@ __global__ void k_pos_to_caller(const uint32_t *v, const uint32_t *pos_rank,
 }
 } // namespace
 
-int core_forest(Context &c, const Grid &G, const Items &I, double eps, uint32_t minpts,
+int core_forest(Context &c, const Grid &G, double eps, uint32_t minpts,
                 const uint32_t *counts, uint8_t *core, uint32_t *parent, uint32_t *best)
 {
     uint32_t n = G.npts;
     double T = threshold_for_eps(eps);
     unsigned g = ceil_div(n, kBlock);
-    k_core_init<<<g, kBlock, 0, c.stream()>>>(counts, n, minpts, core, parent, best);
+    k_core_init<<<g, kBlock, 0, c.stream()>>>(counts, n, minpts, core, parent, best, G.words + 3);
     VDB_HIP(hipGetLastError());
-    if (I.n) {
-        VDB_TRY(c.kt_begin("k_uf_fused"));
-        k_uf_fused<<<ceil_div(I.n, kWavesPerBlock), kBlock, 0, c.stream()>>>(
-            view(G, n), I.cell, I.o0, I.n, T, core, G.pos_rank, parent);
-        VDB_TRY(c.kt_end("k_uf_fused"));
-    }
-    VDB_HIP(hipGetLastError());
-    k_compress<<<g, kBlock, 0, c.stream()>>>(parent, core, n);
-    VDB_HIP(hipGetLastError());
-    return kOk;
+    return core_components(c, G, T, core, parent);
 }
 
-int border_min_key(Context &c, const Grid &G, const Items &I, double eps, const uint8_t *core,
+int border_min_key(Context &c, const Grid &G, double eps, const uint8_t *core,
                    const uint32_t *parent, const uint32_t *key, uint32_t *best)
 {
     uint32_t n = G.npts;
     k_fill_u32_n<<<ceil_div(n, kBlock), kBlock, 0, c.stream()>>>(best, kNone, n);
     VDB_HIP(hipGetLastError());
-    if (I.n) {
-        VDB_TRY(c.kt_begin("k_border_fused"));
-        k_border_fused<<<ceil_div(I.n, kWavesPerBlock), kBlock, 0, c.stream()>>>(
-            view(G, n), I.cell, I.o0, I.n, threshold_for_eps(eps), core, key, parent, best);
-        VDB_TRY(c.kt_end("k_border_fused"));
-    }
+    k_fill_u32_n<<<1, kBlock, 0, c.stream()>>>(G.words + 3, 0u, 1);
     VDB_HIP(hipGetLastError());
-    return kOk;
+    return border_pass(c, G, threshold_for_eps(eps), core, key, parent, best);
 }
 
 int border_pairs(Context &c, const Grid &G, const Items &I, double eps, const uint8_t *core,

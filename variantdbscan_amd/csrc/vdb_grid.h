@@ -75,6 +75,10 @@ struct Grid {
     uint32_t *row_f0 = nullptr;
     uint32_t *row_f1 = nullptr;
     uint32_t npts = 0;              // points in the grid
+    // device words, zero after build_grid: [1] set by classify_rows when some
+    // cell is not a clique (two of its points not within eps), [2] and [3] list
+    // counts of the per-variant kernels ([0] is the box pass's)
+    uint32_t *words = nullptr;
     // per dataset: grid origin, dimensions and first key (keys of dataset d
     // are kbase[d] + key; kbase[d] is a multiple of m)
     uint32_t nsets = 1;

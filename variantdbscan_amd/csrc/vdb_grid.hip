@@ -243,12 +243,10 @@ __global__ void k_cells(const uint32_t *keys, const uint32_t *flags, const uint3
     }
 }
 
-__global__ void k_cell_tail(uint32_t *cell_start, uint32_t ncell, uint32_t n, uint32_t *nbig)
+__global__ void k_cell_tail(uint32_t *cell_start, uint32_t ncell, uint32_t n, uint32_t *words)
 {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        cell_start[ncell] = n;
-        *nbig = 0; // the box pass's list of large cells
-    }
+    if (threadIdx.x == 0 && blockIdx.x == 0) cell_start[ncell] = n;
+    if (threadIdx.x < 4) words[threadIdx.x] = 0; // Grid::words
 }
 
 // Bounding box of every cell's points. Thread per cell for the common small
@@ -698,16 +696,18 @@ int build_rank_order(Context &c, Points &P, const char *tag)
 // Thread per (cell, window row). Rows are runs of consecutive cells whose
 // point boxes are ordered along the row, so trimming from both ends removes
 // every cell whose box lies beyond eps of the centre cell's box; the first
-// run of cells wholly within eps becomes the full range.
+// run of cells wholly within eps becomes the full range. *noclique is set
+// when some cell's own box is not within eps of itself.
 __global__ void k_classify_rows(const double *box, uint32_t ncell, int W, double T,
                                 uint32_t *row_lo, uint32_t *row_hi, uint32_t *row_f0,
-                                uint32_t *row_f1)
+                                uint32_t *row_f1, uint32_t *noclique)
 {
     // 64-bit thread index: cells x window rows exceeds 2^32 on large grids
     uint64_t t = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
     if (t >= (uint64_t)ncell * (uint32_t)W) return;
     uint32_t c = (uint32_t)(t / (uint32_t)W);
     const double *A = box + 4 * (size_t)c;
+    if ((int)(t - (uint64_t)c * (uint32_t)W) == W / 2 && !(boxes_dist2_max(A, A) <= T)) *noclique = 1;
     uint32_t lo = row_lo[t], hi = row_hi[t];
     while (lo < hi && boxes_dist2_min(A, box + 4 * (size_t)lo) > T) lo++;
     while (hi > lo && boxes_dist2_min(A, box + 4 * (size_t)(hi - 1)) > T) hi--;
@@ -729,7 +729,7 @@ int classify_rows(Context &c, Grid &G, double T, const char *tag)
     VDB_TRY(c.get(slot(tag, "row_f1").c_str(), G.ncell * W, &G.row_f1));
     if (G.ncell == 0) return kOk;
     k_classify_rows<<<ceil_div(G.ncell * W, kBlock), kBlock, 0, c.stream()>>>(
-        G.cell_box, G.ncell, (int)W, T, G.row_lo, G.row_hi, G.row_f0, G.row_f1);
+        G.cell_box, G.ncell, (int)W, T, G.row_lo, G.row_hi, G.row_f0, G.row_f1, G.words + 1);
     VDB_HIP(hipGetLastError());
     return kOk;
 }
@@ -860,7 +860,8 @@ int build_grid(Context &c, const Points &P, double w_min, int R, const char *tag
     VDB_HIP(hipGetLastError());
     uint32_t *bigc, *nbig;
     VDB_TRY(c.get(slot(tag, "bigcells").c_str(), std::max<uint32_t>(ncell, 1), &bigc));
-    VDB_TRY(c.get(slot(tag, "nbig").c_str(), 1, &nbig));
+    VDB_TRY(c.get(slot(tag, "nbig").c_str(), 4, &nbig));
+    G.words = nbig;
     k_cell_tail<<<1, 64, 0, c.stream()>>>(G.cell_start, ncell, n, nbig);
     VDB_HIP(hipGetLastError());
 

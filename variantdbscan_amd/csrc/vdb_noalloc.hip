@@ -93,8 +93,15 @@ int noalloc_impl(Context &c, const double *x, const double *y, uint32_t n, const
         Grid G;
         Items I;
         VDB_TRY(build_eps_grid(c, P, e, k, "g1", G));
-        VDB_TRY(build_items(c, G, "g1", I));
-        VDB_TRY(count_neighbors(c, G, I, e, precision, counts, (uint64_t *)rc));
+        if (precision == VDB_PREC_FP64) {
+            uint32_t need = 0; // minpts above INT_MAX is never reached
+            for (uint32_t v : kv.second)
+                if (minpts[v] <= 0x7fffffffu) need = minpts[v] > need ? minpts[v] : need;
+            VDB_TRY(count_core(c, G, e, need, counts));
+        } else {
+            VDB_TRY(build_items(c, G, "g1", I));
+            VDB_TRY(count_neighbors(c, G, I, e, precision, counts, (uint64_t *)rc));
+        }
         for (uint32_t v : kv.second)
             VDB_TRY(cluster_variant(c, P, G, I, e, minpts[v], counts, 0, border, 0,
                                     labels + (size_t)v * n, nullptr));

@@ -255,7 +255,7 @@ int reuse_step(Context &c, const Points &P, const Grid &G, const Items &I,
     VDB_TRY(c.get("ru.cl", n, &cl));
     VDB_TRY(c.get("ru.cnt", 1, &cnt));
     VDB_TRY(c.get("ru.nroots", 1, &nroots_dev));
-    VDB_TRY(core_forest(c, G, I, ev, mp, counts, core, parent, best));
+    VDB_TRY(core_forest(c, G, ev, mp, counts, core, parent, best));
     k_fill<<<g, kBlock, 0, c.stream()>>>(claim, kNone, n);
     VDB_HIP(hipGetLastError());
     uint32_t *procL_dev = nullptr;
@@ -320,8 +320,8 @@ int reuse_step(Context &c, const Points &P, const Grid &G, const Items &I,
     k_unclaimed<<<g, kBlock, 0, c.stream()>>>(core, parent, claim, G.pos_rank, n, rankkey, flag);
     VDB_HIP(hipGetLastError());
     VDB_TRY(scan_exclusive_u32(c, flag, fid, n, nroots_dev));
-    VDB_TRY(border_min_key(c, G, I, ev, core, parent, claim, best));
-    VDB_TRY(border_min_key(c, G, I, ev, core, parent, rankkey, best2));
+    VDB_TRY(border_min_key(c, G, ev, core, parent, claim, best));
+    VDB_TRY(border_min_key(c, G, ev, core, parent, rankkey, best2));
     k_reuse_labels<<<g, kBlock, 0, c.stream()>>>(old, procL_dev, core, parent, claim, best, best2,
                                                 fid, G.pos_rank, P.mapping, nvisited, n, lab,
                                                 out);

@@ -161,12 +161,25 @@ __device__ __forceinline__ void cf_hook(uint32_t *parent, uint32_t x, uint32_t m
 }
 
 // ------------------------------------------------------------- cliques
+// The call's level thresholds (INF beyond K) and minpts values: kernel
+// arguments that the first kernel stores for the others.
+struct CallParams {
+    double T[kMaxLevels];
+    uint32_t mj[kMaxMinpts];
+};
+
 // bad[0] counts the cells that are not cliques at eps_0, bad[1] the points of
 // cells with < L points (those that get a neighbour list)
 __global__ void __launch_bounds__(kBlock)
-    k_clique_check(const double *box, const uint32_t *cell_start, uint32_t ncell, double T0,
-                   uint32_t L, uint32_t *bad)
+    k_clique_check(const double *box, const uint32_t *cell_start, uint32_t ncell, uint32_t L,
+                   CallParams P, double *Tk, uint32_t *mj, uint32_t *bad)
 {
+    static_assert(kMaxLevels <= kBlock && kMaxMinpts <= kBlock, "one block stores them");
+    if (blockIdx.x == 0) {
+        if (threadIdx.x < kMaxLevels) Tk[threadIdx.x] = P.T[threadIdx.x];
+        if (threadIdx.x < kMaxMinpts) mj[threadIdx.x] = P.mj[threadIdx.x];
+    }
+    const double T0 = P.T[0];
     uint32_t c = blockIdx.x * kBlock + threadIdx.x;
     uint32_t listed = 0;
     if (c < ncell) {
@@ -2236,19 +2249,35 @@ __global__ void __launch_bounds__(kBlock)
         for (int e = R.first[w]; e < R.first[w + 1]; e++) base[(size_t)R.row[e] * nd] = v[w];
 }
 
-__global__ void k_pos_of_caller(const uint32_t *caller_of_pos, uint32_t n, uint32_t *pos_of_caller)
+__global__ void k_caller_of_pos(const uint32_t *pos_rank, const uint32_t *mapping, uint32_t n,
+                                uint32_t *caller_of_pos, uint32_t *pos_of_caller)
 {
     uint32_t p = blockIdx.x * kBlock + threadIdx.x;
     if (p >= n) return;
-    pos_of_caller[caller_of_pos[p]] = p;
+    uint32_t i = mapping[pos_rank[p]];
+    caller_of_pos[p] = i;
+    pos_of_caller[i] = p;
 }
 
-__global__ void k_caller_of_pos(const uint32_t *pos_rank, const uint32_t *mapping, uint32_t n,
-                                uint32_t *caller_of_pos)
+// What the host waits for, straight to its pinned memory (a copy per value
+// costs a launch each).
+__global__ void k_report_pairs(const uint64_t *npairs, const uint32_t *bad, uint64_t *host)
 {
-    uint32_t p = blockIdx.x * kBlock + threadIdx.x;
-    if (p >= n) return;
-    caller_of_pos[p] = mapping[pos_rank[p]];
+    if (threadIdx.x == 0) {
+        host[0] = *npairs;
+        host[1] = *bad;
+    }
+}
+
+__global__ void k_report_final(const uint32_t *bad, const uint32_t *tovf, const uint32_t *cnts,
+                               uint32_t ncnt, const uint32_t *bstart, uint32_t nb, uint32_t *host)
+{
+    if (threadIdx.x == 0) {
+        host[0] = *tovf;
+        host[1] = bad[1];
+    }
+    for (uint32_t i = threadIdx.x; i < ncnt; i += kBlock) host[2 + i] = cnts[i];
+    for (uint32_t i = threadIdx.x; i < nb; i += kBlock) host[2 + ncnt + i] = bstart[i];
 }
 
 __global__ void k_fill_u32(uint32_t *a, uint32_t v, uint32_t n)
@@ -2417,30 +2446,24 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
         set_error("fine grid would exceed 32-bit cell keys");
         return kErrUnsupported;
     }
-    // failed clique checks, listed points, the list kernels' counts
-    uint32_t *bad;
-    VDB_TRY(c.get("b.bad", 5, &bad));
-    VDB_HIP(hipMemsetAsync(bad, 0, 5 * sizeof(uint32_t), c.stream()));
-    k_clique_check<<<ceil_div(G.ncell, kBlock), kBlock, 0, c.stream()>>>(
-        G.cell_box, G.cell_start, G.ncell, Th[0], L, bad);
-    VDB_HIP(hipGetLastError());
+    // failed clique checks, listed points, the list kernels' counts, test-list
+    // overflow
+    uint32_t *bad = G.words + 4;
+    uint32_t *tovf = G.words + 9;
     double *dTk;
     uint32_t *dmj;
-    const std::vector<double> Tpad = [&] { // INF beyond K: k_knn takes rounded-up counts
-        std::vector<double> t(Th);
-        t.resize(kMaxLevels, INFINITY);
-        return t;
-    }();
     VDB_TRY(c.get("b.Tk", kMaxLevels, &dTk));
-    VDB_TRY(c.get("b.mj", J, &dmj));
-    VDB_HIP(hipMemcpyAsync(dTk, Tpad.data(), sizeof(double) * kMaxLevels, hipMemcpyHostToDevice,
-                           c.stream()));
-    VDB_HIP(hipMemcpyAsync(dmj, mps.data(), sizeof(uint32_t) * J, hipMemcpyHostToDevice,
-                           c.stream()));
+    VDB_TRY(c.get("b.mj", kMaxMinpts, &dmj));
+    CallParams cp;
+    for (int k = 0; k < kMaxLevels; k++) cp.T[k] = k < K ? Th[k] : INFINITY;
+    for (int j = 0; j < kMaxMinpts; j++) cp.mj[j] = j < J ? mps[j] : 0u;
+    k_clique_check<<<ceil_div(G.ncell, kBlock), kBlock, 0, c.stream()>>>(
+        G.cell_box, G.cell_start, G.ncell, L, cp, dTk, dmj, bad);
+    VDB_HIP(hipGetLastError());
     tprep.stop();
-    // pinned read-back area of the call: [0, 8) pair count, [8, 12) clique
-    // check, [16, 20) list count, [32, ...) the final overflow flag, list
-    // count and worklist counters
+    // pinned read-back area of the call, written by k_report_*: [0, 8) pair
+    // count, [8, 16) clique check, [32, ...) the final overflow flag, list count
+    // and worklist counters
     const size_t ncnt_all = (size_t)J * 3 * ((size_t)K + 1);
     char *hs = nullptr;
     VDB_TRY(c.host_scratch(32 + 4 * (4 + ncnt_all + (size_t)J * (K + 1) + 1), (void **)&hs));
@@ -2487,8 +2510,8 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
         VDB_TRY(c.kt_end("k_pair_count"));
         VDB_HIP(hipGetLastError());
         VDB_TRY(scan_exclusive_u32_u64(c, pcnt, poff, G.ncell, poff + G.ncell));
-        VDB_HIP(hipMemcpyAsync(hs, poff + G.ncell, 8, hipMemcpyDeviceToHost, ps));
-        VDB_HIP(hipMemcpyAsync(hs + 8, bad, 4, hipMemcpyDeviceToHost, ps));
+        k_report_pairs<<<1, kWave, 0, ps>>>(poff + G.ncell, bad, (uint64_t *)hs);
+        VDB_HIP(hipGetLastError());
         VDB_HIP(hipEventRecord(c.aux_event(1), ps));
     }
 
@@ -2537,9 +2560,11 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
     unsigned gc0 = ceil_div(G.ncell, kBlock);
     // caller index of every position: the standard rule's key, and the label
     // pass's scatter order
-    uint32_t *caller_of_pos;
+    uint32_t *caller_of_pos, *pos_of_caller;
     VDB_TRY(c.get("b.cop", n, &caller_of_pos));
-    k_caller_of_pos<<<gn, kBlock, 0, c.stream()>>>(G.pos_rank, P.mapping, n, caller_of_pos);
+    VDB_TRY(c.get("b.poc", n, &pos_of_caller));
+    k_caller_of_pos<<<gn, kBlock, 0, c.stream()>>>(G.pos_rank, P.mapping, n, caller_of_pos,
+                                                   pos_of_caller);
     VDB_HIP(hipGetLastError());
     if (std_rule) {
         uint32_t *big;
@@ -2593,8 +2618,6 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
         unsigned long long v = strtoull(ev, nullptr, 10);
         if (v > 0 && v < tcap) tcap = (uint32_t)v;
     }
-    uint32_t *pos_of_caller;
-    VDB_TRY(c.get("b.poc", n, &pos_of_caller));
     // the cell pairs stored on the second stream too, beside the lists; the
     // main stream waits for them before the level passes
     {
@@ -2637,7 +2660,7 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
             if (w.first.second >= j0 && w.first.second < j0 + jc) ns++;
         max_slots = std::max(max_slots, ns);
     }
-    uint32_t *parent, *compmin, *ekey, *eval, *stk, *stv, *bstart, *tovf;
+    uint32_t *parent, *compmin, *ekey, *eval, *stk, *stv, *bstart;
     VDB_TRY(c.get("b.parent", (size_t)jc * G.ncell, &parent));
     VDB_TRY(c.get("b.compmin", (size_t)jc * G.ncell, &compmin));
     VDB_TRY(c.get("b.la", (size_t)jc * psz, &la));
@@ -2667,7 +2690,6 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
     PairRec *frec; // pair records sorted by (minpts value, level)
     VDB_TRY(c.get("b.frec", (size_t)jc * psz, &frec));
     VDB_TRY(c.get("b.bstart", (size_t)jc * (K + 1) + 2, &bstart));
-    VDB_TRY(c.get("b.tovf", 1, &tovf));
     // per-slot snapshots: cell root ranks, cell labels, the root ranks as a
     // bitset over ranks with its per-word prefix counts (cluster ids)
     uint32_t *snap_root, *snap_lab, *snap_bits, *snap_pre;
@@ -2736,10 +2758,6 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
     // pooled buffers: no host read, no allocation. With `events`, the label
     // passes are bracketed by events (not inside a graph).
     auto sequence = [&](bool events, const BatchShape &shape) -> int {
-        k_pos_of_caller<<<gn, kBlock, 0, c.stream()>>>(caller_of_pos, n, pos_of_caller);
-        VDB_HIP(hipGetLastError());
-        k_fill_u32<<<1, kBlock, 0, c.stream()>>>(tovf, 0u, 1);
-        VDB_HIP(hipGetLastError());
         for (int j0 = 0; j0 < J; j0 += jc) {
             const int nj = std::min(jc, J - j0);
             // requested minpts values of the pass at each level, and the slots
@@ -3035,14 +3053,11 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
     const bool counters = jc == J && npairs;
     uint32_t *hc = (uint32_t *)(hs + 32 + 8);
     uint32_t *hb = hc + ncnt_all;
-    VDB_HIP(hipMemcpyAsync(hs + 32, tovf, 4, hipMemcpyDeviceToHost, c.stream()));
-    VDB_HIP(hipMemcpyAsync(hs + 36, bad + 1, 4, hipMemcpyDeviceToHost, c.stream()));
-    if (counters) {
-        VDB_HIP(hipMemcpyAsync(hc, cnts, sizeof(uint32_t) * ncnt_all, hipMemcpyDeviceToHost,
-                               c.stream()));
-        VDB_HIP(hipMemcpyAsync(hb, bstart, sizeof(uint32_t) * ((size_t)J * (K + 1) + 1),
-                               hipMemcpyDeviceToHost, c.stream()));
-    }
+    k_report_final<<<1, kBlock, 0, c.stream()>>>(bad, tovf, cnts,
+                                                 counters ? (uint32_t)ncnt_all : 0u, bstart,
+                                                 counters ? (uint32_t)(J * (K + 1) + 1) : 0u,
+                                                 (uint32_t *)(hs + 32));
+    VDB_HIP(hipGetLastError());
     VDB_TRY(c.wait(c.stream()));
     uint32_t htovf = 0, nlist = 0;
     memcpy(&htovf, hs + 32, 4);

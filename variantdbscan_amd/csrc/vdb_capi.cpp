@@ -45,12 +45,22 @@ struct Timer {
 };
 
 int upload_points(Context &c, const double *x, const double *y, uint32_t n, uint32_t flags,
-                  Points &P)
+                  Points &P, bool one_set = true)
 {
     P.n = n;
     if (flags & VDB_DEVICE_PTRS) {
         P.x = x;
         P.y = y;
+        return kOk;
+    }
+    if (one_set && small_points(n)) {
+        // staged in pinned memory, which the rank-order kernel reads itself
+        double *h = nullptr;
+        VDB_TRY(c.host_stage(16 * (size_t)n, (void **)&h));
+        memcpy(h, x, 8 * (size_t)n);
+        memcpy(h + n, y, 8 * (size_t)n);
+        P.x = h;
+        P.y = h + n;
         return kOk;
     }
     double *dx, *dy;
@@ -60,6 +70,24 @@ int upload_points(Context &c, const double *x, const double *y, uint32_t n, uint
     VDB_HIP(hipMemcpyAsync(dy, y, sizeof(double) * n, hipMemcpyHostToDevice, c.stream()));
     P.x = dx;
     P.y = dy;
+    return kOk;
+}
+
+// Result array to the caller's host memory, and the call's last wait: small
+// ones through pinned memory (a copy to pageable memory waits for the runtime's
+// own staging, about 40 us).
+int download(Context &c, void *dst, const void *src, size_t bytes)
+{
+    if (bytes > Context::kStageBytes) {
+        VDB_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c.stream()));
+        VDB_HIP(hipStreamSynchronize(c.stream()));
+        return kOk;
+    }
+    void *h = nullptr;
+    VDB_TRY(c.host_stage(bytes, &h));
+    VDB_HIP(hipMemcpyAsync(h, src, bytes, hipMemcpyDeviceToHost, c.stream()));
+    VDB_TRY(c.wait(c.stream()));
+    memcpy(dst, h, bytes);
     return kOk;
 }
 
@@ -298,11 +326,10 @@ int cluster_impl(const double *x, const double *y, uint32_t n, const double *eps
         VDB_TRY(cluster_points(c, P, "pts", eps, minpts, nvar, all_variants(nvar), out, opt, st,
                                &used));
     }
-    if (!(flags & VDB_DEVICE_PTRS)) {
-        VDB_HIP(hipMemcpyAsync(labels, out, sizeof(uint32_t) * (size_t)n * nvar,
-                               hipMemcpyDeviceToHost, c.stream()));
-    }
-    VDB_HIP(hipStreamSynchronize(c.stream()));
+    if (!(flags & VDB_DEVICE_PTRS))
+        VDB_TRY(download(c, labels, out, sizeof(uint32_t) * (size_t)n * nvar));
+    else
+        VDB_TRY(c.wait(c.stream()));
     if (st) {
         st->ms_total = total.ms();
         st->path_used = used;
@@ -423,7 +450,7 @@ int vdb_cluster_multi(const double *x, const double *y, const uint64_t *offsets,
     std::lock_guard<std::mutex> lock(c.mu);
     Timer total(c.stream(), st != nullptr);
     Points all;
-    VDB_TRY(upload_points(c, x, y, (uint32_t)ntot, flags, all));
+    VDB_TRY(upload_points(c, x, y, (uint32_t)ntot, flags, all, false));
     uint32_t *out = labels;
     if (!(flags & VDB_DEVICE_PTRS)) VDB_TRY(c.get("out.labels", (size_t)ntot * nvar, &out));
     int used = 0;
@@ -640,13 +667,13 @@ int libVDBSCAN(double *inputx, double *inputy, unsigned int datasetSize, double 
     opt.path = VDB_PATH_AUTO;
     opt.precision = VDB_PREC_FP64;
     opt.verbose = verbose ? 1 : 0;
-    vdb_stats st;
+    vdb_stats st; // only asked for when it is printed: its phase timers cost waits
     // VDBSCAN_REUSE=1 in the environment: the reference's greedy reuse with
     // one search thread (VDB_REUSE_REFERENCE) instead of scratch labels
     const char *ru = getenv("VDBSCAN_REUSE");
     uint32_t flags = (ru && ru[0] == '1') ? VDB_REUSE_REFERENCE : 0u;
     int s = vdb_cluster(inputx, inputy, datasetSize, inputEpsilon, inputMinpts, numVariants,
-                        retArr, flags, &opt, &st);
+                        retArr, flags, &opt, verbose ? &st : nullptr);
     if (verbose) {
         if (s == 0)
             printf("\n[vdbscan] %u points x %u variants, path %d, %.3f ms device time\n",

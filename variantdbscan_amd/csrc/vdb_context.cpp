@@ -37,6 +37,7 @@ Context::~Context()
     release_all(); // also drops the graphs
     for (hipEvent_t e : kt_ev_) hipEventDestroy(e);
     if (host_) hipHostFree(host_);
+    if (stage_) hipHostFree(stage_);
     for (hipEvent_t e : aux_ev_)
         if (e) hipEventDestroy(e);
     if (wait_ev_) hipEventDestroy(wait_ev_);
@@ -171,6 +172,24 @@ int Context::host_scratch(size_t bytes, void **out)
         host_bytes_ = want;
     }
     *out = host_;
+    return kOk;
+}
+
+int Context::host_stage(size_t bytes, void **out)
+{
+    if (stage_bytes_ < bytes) {
+        if (stage_) {
+            VDB_HIP(hipStreamSynchronize(stream_));
+            hipHostFree(stage_);
+            stage_ = nullptr;
+            stage_bytes_ = 0;
+        }
+        size_t want = 4096;
+        while (want < bytes) want *= 2;
+        VDB_HIP(hipHostMalloc(&stage_, want, hipHostMallocDefault));
+        stage_bytes_ = want;
+    }
+    *out = stage_;
     return kOk;
 }
 

@@ -50,6 +50,11 @@ public:
     // Pinned host staging for small device->host reads.
     int host_scratch(size_t bytes, void **out);
 
+    // A second pinned area, for the arrays of small host calls (grow-only, so
+    // at most kStageBytes; device kernels may read and write it).
+    static constexpr size_t kStageBytes = (size_t)1 << 20;
+    int host_stage(size_t bytes, void **out);
+
     // A second stream of the library (default priority, created on first
     // use) for work that may run beside the current stream's, with events
     // (no timing) to order the two: aux_event(i), i < kAuxEvents.
@@ -127,6 +132,8 @@ private:
     std::unordered_map<std::string, Buffer> pool_;
     void *host_ = nullptr;
     size_t host_bytes_ = 0;
+    void *stage_ = nullptr;
+    size_t stage_bytes_ = 0;
     std::unordered_map<std::string, int> tuned_;
     bool tuned_loaded_ = false;
     std::string dev_tag_; // "<arch>:<CUs>:" prefix of tuning keys

@@ -1,7 +1,7 @@
 // Point layout in HBM.
 //
 //   caller order  : x[i], y[i]                      (as handed in)
-//   rank order    : xb[r], yb[r], mapping[r]         r = position in the reference's
+//   rank order    : xyb[r], mapping[r]               r = position in the reference's
 //                                                    binned visit order
 //   cell order    : xs[p], ys[p], pos_rank[p]        p = position after a stable sort by
 //                                                    grid cell; inside a cell, ranks ascend
@@ -25,7 +25,7 @@ double threshold_for_eps(double eps);
 struct Points {
     uint32_t n = 0;
     const double *x = nullptr, *y = nullptr; // caller order (device)
-    double *xb = nullptr, *yb = nullptr;     // rank order
+    double2 *xyb = nullptr;                  // rank order
     uint32_t *mapping = nullptr;             // rank -> caller index
     double ext[4] = {0, 0, 0, 0};            // extent of all points
     uint32_t nsets = 1;
@@ -38,8 +38,13 @@ struct Points {
 // P.hseg must be set (nsets+1 host offsets); fills the rank order of P.
 // Returns kErrUnsupported when a bin is out of range.
 int build_rank_order(Context &c, Points &P, const char *tag);
+// One dataset of at most this many points is put in order by one block, which
+// may read the coordinates from pinned host memory.
+bool small_points(uint32_t n);
 // One dataset covering all points.
 void single_segment(Points &P);
+
+constexpr uint32_t kGridWords = 16;
 
 struct Grid {
     double w = 0, gx0 = 0, gy0 = 0;
@@ -48,6 +53,7 @@ struct Grid {
     // ((cx/m)*ncy + cy)*m + cx%m, column-major for m = 1. A window of radius R
     // is then 2*RS + 1 rows, one per strip, each a contiguous run of keys.
     int m = 1;
+    uint64_t nkeys = 0;        // size of the key space
     uint32_t ncell = 0;        // non-empty cells
     int R = 1;                 // window radius in cells
     int RS = 1;                // in strips: ceil(R/m)
@@ -75,9 +81,10 @@ struct Grid {
     uint32_t *row_f0 = nullptr;
     uint32_t *row_f1 = nullptr;
     uint32_t npts = 0;              // points in the grid
-    // device words, zero after build_grid: [1] set by classify_rows when some
-    // cell is not a clique (two of its points not within eps), [2] and [3] list
-    // counts of the per-variant kernels ([0] is the box pass's)
+    // kGridWords device words, zero after build_grid: [0] the box pass's list
+    // count, [1] set by classify_rows when some cell is not a clique (two of
+    // its points not within eps), [2] and [3] list counts of the per-variant
+    // kernels, [4..] the batched engine's
     uint32_t *words = nullptr;
     // per dataset: grid origin, dimensions and first key (keys of dataset d
     // are kbase[d] + key; kbase[d] is a multiple of m)

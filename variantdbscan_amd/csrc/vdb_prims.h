@@ -1,5 +1,5 @@
 // Device-wide primitives written for wave64: exclusive scans, a stable LSD
-// radix sort of (u32 key, u32 value) pairs and float64 extent reductions.
+// radix sort of (u32 key, u32 value) pairs.
 #pragma once
 
 #include "vdb_context.h"
@@ -20,9 +20,6 @@ int scan_exclusive_u32_u64(Context &c, const uint32_t *in, uint64_t *out, size_t
 int radix_sort_pairs(Context &c, uint32_t *keys, uint32_t *vals, uint32_t *tmp_keys,
                      uint32_t *tmp_vals, size_t n, int key_bits, uint32_t **keys_out,
                      uint32_t **vals_out);
-
-// ext_dev[0..3] = (min x, max x, min y, max y) over n points (n >= 1).
-int extent_f64(Context &c, const double *x, const double *y, size_t n, double *ext_dev);
 
 // Exclusive scan of flags -> out (u32); returns the total on the host.
 int compact_count(Context &c, const uint32_t *flags, uint32_t *out, size_t n,

@@ -1,0 +1,39 @@
+"""Batched engine around its groups of 8 minpts values: one, a full group, one
+beyond it and two groups and one, with values that make every point core (1)
+and none (above the point count), on points whose levels leave pairs open from
+one level to the next. Labels are the oracle's."""
+import numpy as np
+import pytest
+
+import oracle
+
+import variantdbscan_amd as vd
+from variantdbscan_amd import datasets
+
+pytestmark = pytest.mark.gpu
+
+N = 12_000
+MINPTS = [1, 4, 2, 9, 6, 30, 3, 50_000, 5, 12, 7, 16, 8, 60, 25, 40, 100]
+
+
+@pytest.fixture(scope="module")
+def points():
+    # filaments and noise beside a knot far denser than the rest
+    x, y = datasets.aniso(N - 2000, seed=57)
+    r = np.random.default_rng(58)
+    kx, ky = r.normal(x.mean(), 0.15, 2000), r.normal(y.mean(), 0.15, 2000)
+    return np.concatenate([x, kx]), np.concatenate([y, ky])
+
+
+@pytest.mark.parametrize("levels", [1, 4], ids=["one-level", "four-levels"])
+@pytest.mark.parametrize("nmp", [1, 7, 8, 9, 17])
+def test_minpts_groups(points, nmp, levels):
+    x, y = points
+    E = [0.3, 0.37, 0.55, 0.8][:levels]
+    eps = np.repeat(E, nmp)
+    mp = np.tile(np.array(MINPTS[:nmp], dtype=np.uint32), levels)
+    print("12k points, %d minpts values x %d levels" % (nmp, levels), flush=True)
+    got = vd.cluster(x, y, eps, mp, path=vd.PATH_BATCH)
+    want = oracle.libvdbscan(x, y, eps, mp)
+    for v in range(len(eps)):
+        assert (got[v] == want[v]).all(), (eps[v], mp[v])

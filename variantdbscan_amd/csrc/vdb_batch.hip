@@ -53,13 +53,13 @@ struct BatchShape {
     unsigned maxb, minb, ppb, tpb, maxtb;
 };
 constexpr BatchShape kBatchShapes[] = {
-    {1024, 512, 8192, 64, 2048}, // best with one minpts value per launch
-    {512, 256, 8192, 64, 1024},
-    {256, 128, 8192, 32, 1024},
-    {1024, 256, 4096, 32, 2048},
+    {1280, 512, 1024, 32, 2048}, // 2M points x 64 variants, 500K x 16
+    {640, 128, 2048, 32, 1024},  // one minpts value
+    {2560, 512, 512, 16, 4096},  // 256 datasets at once: many tests, one level
+    {320, 128, 4096, 32, 1024},
 };
 constexpr int kNumBatchShapes = sizeof(kBatchShapes) / sizeof(kBatchShapes[0]);
-constexpr unsigned kMaxPersistent = 1024; // largest maxb of kBatchShapes
+constexpr unsigned kMaxPersistent = 4096; // at least any maxb or maxtb of kBatchShapes
 
 struct FG {
     const double *xs, *ys, *box;
@@ -98,44 +98,30 @@ __device__ __forceinline__ void st_u32(uint32_t *p, uint32_t v)
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// union-find over cells: parents point to smaller cell indices
+// Union-find over cells, 8 minpts values (a group) side by side: cell x's
+// parent for value j of the group is parent[8 x + j], so that one 32-byte read
+// gives a cell's parents for all of them. The functions below take the array
+// already offset by j. Parents point to smaller cell indices.
+constexpr int kGroup = 8;
+__device__ __forceinline__ size_t cf_at(uint32_t x) { return (size_t)x * kGroup; }
+
 __device__ uint32_t cf_find(uint32_t *parent, uint32_t x)
 {
     while (true) {
-        uint32_t p = ld_u32(parent + x);
+        uint32_t p = ld_u32(parent + cf_at(x));
         if (p == x) return x;
-        uint32_t gp = ld_u32(parent + p);
+        uint32_t gp = ld_u32(parent + cf_at(p));
         if (gp == p) return p;
-        st_u32(parent + x, gp);
+        st_u32(parent + cf_at(x), gp);
         x = gp;
     }
-}
-
-// same component? Parent pointers stay inside a component, so equal parents
-// settle it after one pair of loads issued together (the common case once a
-// snapshot has flattened the forest); otherwise the roots decide.
-__device__ __forceinline__ bool cf_same(uint32_t *parent, uint32_t a, uint32_t b)
-{
-    uint32_t pa = ld_u32(parent + a), pb = ld_u32(parent + b);
-    return pa == pb || cf_find(parent, pa) == cf_find(parent, pb);
-}
-
-// cf_same that also returns the roots when the components differ
-__device__ __forceinline__ bool cf_roots(uint32_t *parent, uint32_t a, uint32_t b,
-                                         uint32_t &ra, uint32_t &rb)
-{
-    uint32_t pa = ld_u32(parent + a), pb = ld_u32(parent + b);
-    if (pa == pb) return true;
-    ra = cf_find(parent, pa);
-    rb = cf_find(parent, pb);
-    return ra == rb;
 }
 
 __device__ void cf_unite(uint32_t *parent, uint32_t a, uint32_t b)
 {
     while (true) {
         // both parents in one round of loads: equal parents settle it
-        uint32_t pa = ld_u32(parent + a), pb = ld_u32(parent + b);
+        uint32_t pa = ld_u32(parent + cf_at(a)), pb = ld_u32(parent + cf_at(b));
         if (pa == pb) return;
         if (pa != a) a = cf_find(parent, pa);
         if (pb != b) b = cf_find(parent, pb);
@@ -145,7 +131,7 @@ __device__ void cf_unite(uint32_t *parent, uint32_t a, uint32_t b)
             a = b;
             b = t;
         }
-        uint32_t ret = atomicCAS(parent + b, b, a);
+        uint32_t ret = atomicCAS(parent + cf_at(b), b, a);
         // hooked, or another wave hooked b under the same root
         if (ret == b || ret == a) return;
         b = ret; // b was hooked elsewhere: go on from its new parent
@@ -156,8 +142,30 @@ __device__ void cf_unite(uint32_t *parent, uint32_t a, uint32_t b)
 // common loss: another wave hooked x under the same m, then nothing is left)
 __device__ __forceinline__ void cf_hook(uint32_t *parent, uint32_t x, uint32_t m)
 {
-    uint32_t ret = atomicCAS(parent + x, x, m);
+    uint32_t ret = atomicCAS(parent + cf_at(x), x, m);
     if (ret != x && ret != m) cf_unite(parent, ret, m);
+}
+
+// a cell's 8 parents as other waves left them
+__device__ __forceinline__ void cf_load8(const uint32_t *parent, uint32_t x, uint32_t (&p)[kGroup])
+{
+    const uint64_t *q = (const uint64_t *)(parent + cf_at(x));
+#pragma unroll
+    for (int i = 0; i < kGroup / 2; i++) {
+        uint64_t v = __hip_atomic_load(q + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        p[2 * i] = (uint32_t)v;
+        p[2 * i + 1] = (uint32_t)(v >> 32);
+    }
+}
+
+// Core levels of a point or cell for the 8 minpts values of a word, a byte
+// each (levels stay below 64; values past the last have level K): bit j of
+// the result is set when level j <= k.
+__device__ __forceinline__ uint32_t levels_reached(uint64_t w, int k)
+{
+    const uint64_t ones = 0x0101010101010101ull;
+    uint64_t m = ((0x80ull + (uint64_t)k) * ones - w) & (0x80ull * ones);
+    return (uint32_t)(((m >> 7) * 0x0102040810204080ull) >> 56);
 }
 
 // ------------------------------------------------------------- cliques
@@ -308,7 +316,7 @@ struct NearOut {
     uint32_t *lst_n;
     uint8_t *kc;
     uint32_t *kc4;
-    int L, K, J;
+    int L, K, J, JP; // JP: J rounded up to whole words of 8 levels
     const uint32_t *mj;
 };
 
@@ -325,8 +333,8 @@ __device__ __forceinline__ void near_levels(const NearOut &O, uint32_t p, const 
 #pragma unroll
     for (int w = 0; w < KW; w++) tot[w] = group_sum<G>(hist[w]);
     uint32_t packed = 0;
-    for (int j = gl; j < O.J; j += G) {
-        uint32_t need = O.mj[j];
+    for (int j = gl; j < O.JP; j += G) {
+        uint32_t need = j < O.J ? O.mj[j] : kNone; // (never reached)
         int lev = 0;
         uint32_t run = 0;
 #pragma unroll
@@ -338,7 +346,7 @@ __device__ __forceinline__ void near_levels(const NearOut &O, uint32_t p, const 
                 lev += (8 * w + b < cut && run < need) ? 1 : 0;
             }
         if (need > 0x7fffffffu) lev = O.K;
-        O.kc[(size_t)p * O.J + j] = (uint8_t)lev;
+        O.kc[(size_t)p * O.JP + j] = (uint8_t)lev;
         packed |= (uint32_t)(lev & 15) << (4 * (j & 7));
     }
     // with J <= 8 and K <= 15 also packed, 4 bits per minpts value, for the
@@ -604,7 +612,7 @@ __global__ void __launch_bounds__(kBlock)
     k_knn_crowded(FG g, NearOut O, const double *__restrict__ Tk,
                   const uint32_t *__restrict__ crowd, const uint32_t *__restrict__ ncrowd)
 {
-    const int L = O.L, K = O.K, J = O.J;
+    const int L = O.L, K = O.K, J = O.JP;
     const uint32_t nc = *ncrowd;
     if (blockIdx.x * kWPB >= nc) return;
     __shared__ double sT[kMaxLevels];
@@ -616,7 +624,7 @@ __global__ void __launch_bounds__(kBlock)
     uint32_t *bid = abuf_id[wave_id_in_block()];
     const int lane = lane_id();
     const int R = g.W / 2, Win = 2 * g.RSin + 1;
-    const uint32_t need = lane < J ? O.mj[lane] : 0u;
+    const uint32_t need = lane < O.J ? O.mj[lane] : kNone;
     for (uint32_t i = blockIdx.x * kWPB + wave_id_in_block(); i < nc; i += gridDim.x * kWPB) {
         const uint32_t p = __builtin_amdgcn_readfirstlane(crowd[i]);
         const uint32_t c = __builtin_amdgcn_readfirstlane(g.cell_of_pos[p]);
@@ -769,32 +777,47 @@ __global__ void __launch_bounds__(kBlock)
 // per cell, per j, per k: smallest rank of a point with kc_j <= k (cells list
 // their points in ascending rank, so it is the first such point), and the
 // first level at which the cell holds a core point. Thread per cell: one pass
-// over the cell's points keeps the lowest level seen so far, and a point that
-// lowers it is the first for every level it newly covers. Both tables are
-// stored level-major (cmr[(j*K + k)*ncell + c], cellkc[j*ncell + c]) so that
-// the per-level passes over all cells read them contiguously; cellkc also
-// goes out cell-major (cellkc_cm[c*J + j]) for the pass over cell pairs,
-// which reads both cells' levels for several minpts values at once.
+// over the cell's points keeps the lowest levels seen so far, 8 minpts values
+// to a word, and a point that lowers one is the first for every level it
+// newly covers. cmr is stored level-major (cmr[(j*K + k)*ncell + c]) so that
+// the per-level passes over all cells read it contiguously; the levels as a
+// word of 8 minpts values per cell (cellkc[c*JP + j]).
 __global__ void k_cell_core(const uint32_t *cell_start, uint32_t ncell, const uint8_t *kc, int J,
-                            int K, const uint32_t *pos_rank, uint32_t *cmr, uint8_t *cellkc,
-                            uint8_t *cellkc_cm)
+                            int JP, int K, const uint32_t *pos_rank, uint32_t *cmr,
+                            uint8_t *cellkc)
 {
     uint32_t c = blockIdx.x * kBlock + threadIdx.x;
     if (c >= ncell) return;
     uint32_t a = cell_start[c], e = cell_start[c + 1];
-    for (int j = 0; j < J; j++) {
-        uint32_t *row = cmr + (size_t)j * K * ncell + c;
-        int mn = K; // levels [mn, K) have their first point
-        for (uint32_t q = a; q < e && mn > 0; q++) {
-            int lv = kc[(size_t)q * J + j];
-            if (lv >= mn) continue;
+    for (int j0 = 0; j0 < JP; j0 += kGroup) {
+        int mn[kGroup]; // levels [mn, K) have their first point
+#pragma unroll
+        for (int g = 0; g < kGroup; g++) mn[g] = K;
+        for (uint32_t q = a; q < e; q++) {
+            uint64_t w = *(const uint64_t *)(kc + (size_t)q * JP + j0);
             uint32_t r = pos_rank[q];
-            for (int k = lv; k < mn; k++) row[(size_t)k * ncell] = r;
-            mn = lv;
+            int top = 0;
+#pragma unroll
+            for (int g = 0; g < kGroup; g++) {
+                int lv = (int)((w >> (8 * g)) & 0xffu);
+                if (lv < mn[g]) {
+                    for (int k = lv; k < mn[g]; k++)
+                        cmr[((size_t)(j0 + g) * K + k) * ncell + c] = r;
+                    mn[g] = lv;
+                }
+                if (j0 + g < J) top = mn[g] > top ? mn[g] : top;
+            }
+            if (!top) break; // every value has a point at level 0
         }
-        for (int k = 0; k < mn; k++) row[(size_t)k * ncell] = kNone;
-        cellkc[(size_t)j * ncell + c] = (uint8_t)mn;
-        cellkc_cm[(size_t)c * J + j] = (uint8_t)mn; // cell-major copy for pair passes
+        uint64_t w = 0;
+#pragma unroll
+        for (int g = 0; g < kGroup; g++) {
+            if (j0 + g < J)
+                for (int k = 0; k < mn[g]; k++)
+                    cmr[((size_t)(j0 + g) * K + k) * ncell + c] = kNone;
+            w |= (uint64_t)mn[g] << (8 * g);
+        }
+        *(uint64_t *)(cellkc + (size_t)c * JP + j0) = w;
     }
 }
 
@@ -807,9 +830,8 @@ __global__ void k_cell_core(const uint32_t *cell_start, uint32_t ncell, const ui
 // the list 0.03).
 constexpr uint32_t kCoreSerial = 16;
 __global__ void __launch_bounds__(kBlock)
-    k_cell_core_std(const uint32_t *cell_start, uint32_t ncell, const uint8_t *kc, int J, int K,
-                    const uint32_t *key, uint32_t *cmr, uint8_t *cellkc, uint8_t *cellkc_cm,
-                    uint32_t *big, uint32_t *nbig)
+    k_cell_core_std(const uint32_t *cell_start, uint32_t ncell, const uint8_t *kc, int J, int JP,
+                    int K, const uint32_t *key, uint32_t *cmr, uint8_t *cellkc, uint32_t *big, uint32_t *nbig)
 {
     uint32_t c = blockIdx.x * kBlock + threadIdx.x;
     uint32_t a = 0, e = 0;
@@ -828,7 +850,7 @@ __global__ void __launch_bounds__(kBlock)
         int mn = K;
 #pragma unroll
         for (int i = 0; i < (int)kCoreSerial; i++) {
-            lv[i] = (uint32_t)i < np ? (int)kc[(size_t)(a + i) * J + j] : K;
+            lv[i] = (uint32_t)i < np ? (int)kc[(size_t)(a + i) * JP + j] : K;
             mn = lv[i] < mn ? lv[i] : mn;
         }
         uint32_t *row = cmr + (size_t)j * K * ncell + c;
@@ -839,9 +861,9 @@ __global__ void __launch_bounds__(kBlock)
                 if (lv[i] <= k && kq[i] < m) m = kq[i];
             row[(size_t)k * ncell] = m;
         }
-        cellkc[(size_t)j * ncell + c] = (uint8_t)mn;
-        cellkc_cm[(size_t)c * J + j] = (uint8_t)mn;
+        cellkc[(size_t)c * JP + j] = (uint8_t)mn;
     }
+    for (int j = J; j < JP; j++) cellkc[(size_t)c * JP + j] = (uint8_t)K;
 }
 
 __device__ __forceinline__ uint32_t wave_min(uint32_t m)
@@ -858,8 +880,8 @@ __device__ __forceinline__ uint32_t wave_min(uint32_t m)
 // 64) hold a point per lane.
 __global__ void __launch_bounds__(kBlock)
     k_cell_core_std_big(const uint32_t *cell_start, uint32_t ncell, const uint8_t *kc, int J,
-                        int K, uint32_t L, const uint32_t *key, uint32_t *cmr, uint8_t *cellkc,
-                        uint8_t *cellkc_cm, const uint32_t *big, const uint32_t *nbig)
+                        int JP, int K, uint32_t L, const uint32_t *key, uint32_t *cmr,
+                        uint8_t *cellkc, const uint32_t *big, const uint32_t *nbig)
 {
     const uint32_t nb = *nbig;
     const int lane = lane_id();
@@ -872,19 +894,17 @@ __global__ void __launch_bounds__(kBlock)
         for (int j = 0; j < J; j++) {
             uint32_t *row = cmr + (size_t)j * K * ncell + c;
             int lv = K;
-            if (clique) lv = kc[(size_t)a * J + j];
-            else if (a + lane < e) lv = kc[(size_t)(a + lane) * J + j];
+            if (clique) lv = kc[(size_t)a * JP + j];
+            else if (a + lane < e) lv = kc[(size_t)(a + lane) * JP + j];
             int mn = K;
             for (int k = 0; k < K; k++) {
                 uint32_t m = clique ? (lv <= k ? all : kNone) : wave_min(lv <= k ? kv : kNone);
                 if (m != kNone && mn == K) mn = k;
                 if (lane == 0) row[(size_t)k * ncell] = m;
             }
-            if (lane == 0) {
-                cellkc[(size_t)j * ncell + c] = (uint8_t)mn;
-                cellkc_cm[(size_t)c * J + j] = (uint8_t)mn;
-            }
+            if (lane == 0) cellkc[(size_t)c * JP + j] = (uint8_t)mn;
         }
+        if (lane < JP - J) cellkc[(size_t)c * JP + J + lane] = (uint8_t)K;
     }
 }
 
@@ -997,16 +1017,18 @@ __global__ void __launch_bounds__(kBlock)
     }
 }
 
-// For every minpts value j (blockIdx.y): parent[j][c] = c and compmin[j][c] =
-// NONE over its ncell cells; two flat arrays cleared (counters, snapshot root
-// bits) by a grid-stride over all blocks.
+// For every group of minpts values (blockIdx.y): each cell its own parent and
+// no component minimum; two flat arrays cleared (counters, snapshot root bits)
+// by a grid-stride over all blocks.
 __global__ void k_init_parent(uint32_t *parent, uint32_t *compmin, uint32_t ncell, uint32_t *z1,
                               size_t n1, uint32_t *z2, size_t n2)
 {
     uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     if (i < ncell) {
-        parent[(size_t)blockIdx.y * ncell + i] = i;
-        compmin[(size_t)blockIdx.y * ncell + i] = kNone;
+        const size_t at = ((size_t)blockIdx.y * ncell + i) * kGroup;
+        uint4 *p = (uint4 *)(parent + at), *q = (uint4 *)(compmin + at);
+        p[0] = p[1] = make_uint4(i, i, i, i);
+        q[0] = q[1] = make_uint4(kNone, kNone, kNone, kNone);
     }
     size_t f = ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * kBlock + threadIdx.x;
     size_t stride = (size_t)gridDim.y * gridDim.x * kBlock;
@@ -1014,21 +1036,12 @@ __global__ void k_init_parent(uint32_t *parent, uint32_t *compmin, uint32_t ncel
     for (size_t t = f; t < n2; t += stride) z2[t] = 0;
 }
 
-// Append v to list[] for every lane with take set: one atomic per wave.
-__device__ __forceinline__ void wave_append(bool take, uint32_t v, uint32_t *list,
-                                            uint32_t *count)
-{
-    uint64_t m = ballot(take);
-    if (!m) return;
-    int leader = __builtin_ctzll(m);
-    uint32_t base = 0;
-    if (lane_id() == leader) base = atomicAdd(count, (uint32_t)popc64(m));
-    base = __shfl(base, leader);
-    if (take) list[base + mask_rank(m)] = v;
-}
-
 // ------------------------------------------------- per-level pair sweep
-// a cell pair with its levels: k = kmin | kfull << 8
+// A cell pair becoming eligible at a level for some of a group's minpts
+// values: k = those values (bits 0..7) | kfull << 8 | the values for which the
+// level is exact (bits 16..23). One record stands for up to 8 pairs of
+// (minpts value, level): 2M points x 64 variants take 29.4M records
+// where a record per value made 76.6M.
 struct PairRec {
     uint32_t a, b, k;
 };
@@ -1038,286 +1051,242 @@ struct LevelArgs {
     const uint32_t *cell_start, *cell_key;
     const uint32_t *cell_ds, *skbase, *sncy; // dataset of a cell, its key base and ncy
     uint32_t m;                              // strip width of the keys
-    const uint8_t *kc;
-    const uint32_t *pa, *pb;
-    const uint16_t *pk;
-    int J, j, k;
+    const uint8_t *kc;                       // JP bytes a point
+    int JP, j0, k;                           // first minpts value of the pass, level
     double T;
 };
 
-// The union-find state of every minpts value of a level pass: minpts value j
-// (blockIdx.y of the level kernels) owns its parents, carried and test lists
-// and counters at fixed strides. The pairs are sorted once for all minpts
-// values by (j, eligibility level): order holds pair indices (bit 31: exact
-// level) and bucket j*(K+1)+k of bstart is the pairs of j becoming eligible
-// at level k.
+// The union-find state of a level pass, by group of 8 minpts values
+// (blockIdx.y of the level kernels): parents, carried and test lists and
+// counters at fixed strides. The records are sorted by (group, level at which
+// they become eligible): bucket g*(K+1)+k of bstart.
 struct LevelLists {
-    uint32_t *parent;        // j: parent + j*ncell
-    const PairRec *lin;      // carried into the level: j at lin + j*lstride
+    uint32_t *parent;        // group g: parent + g*ncell*8
+    const PairRec *lin;      // carried into the level: g at lin + g*lstride
     PairRec *lout;           // carried out of it
-    PairRec *near, *far;     // test lists: j at + j*tcap
-    uint32_t *cnt;           // j at cnt + j*3*(K+1): keep[K+1], near[K+1], far[K+1]
-    const PairRec *frec;     // pair records of all minpts values, sorted by (j, level)
-    const uint32_t *bstart;  // J*(K+1)+1 bucket starts into frec
+    PairRec *near, *far;     // test lists: g at + g*tcap
+    uint32_t *cnt;           // g at cnt + g*3*(K+1): keep[K+1], near[K+1], far[K+1]
+    const PairRec *frec;     // pair records of all groups, sorted by (group, level)
+    const uint32_t *bstart;  // groups*(K+1)+1 bucket starts into frec
     size_t lstride;
     uint32_t ncell, tcap, K;
     uint32_t *ovf;
     uint32_t ppb, minb, tpb; // grid shape (BatchShape)
 };
 
-struct LevelJ {
+struct LevelG {
     uint32_t *parent;
     const PairRec *carried;
     PairRec *keep, *near, *far;
     uint32_t *nc, *nkeep, *nnear, *nfar;
-    const uint32_t *bstart; // buckets of this j: bstart[k]..bstart[k+1]
+    const uint32_t *bstart; // buckets of this group: bstart[k]..bstart[k+1]
 };
 
-__device__ __forceinline__ LevelJ level_j(const LevelLists &L, uint32_t j, int k)
+__device__ __forceinline__ LevelG level_g(const LevelLists &L, uint32_t g, int k)
 {
-    LevelJ r;
-    r.parent = L.parent + (size_t)j * L.ncell;
-    r.carried = L.lin + (size_t)j * L.lstride;
-    r.keep = L.lout + (size_t)j * L.lstride;
-    r.near = L.near + (size_t)j * L.tcap;
-    r.far = L.far + (size_t)j * L.tcap;
-    uint32_t *c = L.cnt + (size_t)j * 3u * (L.K + 1);
+    LevelG r;
+    r.parent = L.parent + (size_t)g * L.ncell * kGroup;
+    r.carried = L.lin + (size_t)g * L.lstride;
+    r.keep = L.lout + (size_t)g * L.lstride;
+    r.near = L.near + (size_t)g * L.tcap;
+    r.far = L.far + (size_t)g * L.tcap;
+    uint32_t *c = L.cnt + (size_t)g * 3u * (L.K + 1);
     r.nc = c + k;
     r.nkeep = c + k + 1;
     r.nnear = c + (L.K + 1) + k;
     r.nfar = c + 2 * (L.K + 1) + k;
-    r.bstart = L.bstart + (size_t)j * (L.K + 1);
+    r.bstart = L.bstart + (size_t)g * (L.K + 1);
     return r;
 }
 
-__device__ bool small_pair_connected(const LevelArgs &a, uint32_t A, uint32_t B)
+// the word of core levels holding minpts values j.. of a row of JP bytes,
+// value j in the lowest byte (a pass starts inside a word only when it holds
+// fewer than 8 values, all in that word)
+__device__ __forceinline__ uint64_t level_word(const uint8_t *row, int j)
 {
-    uint32_t a0 = a.cell_start[A], a1 = a.cell_start[A + 1];
-    uint32_t b0 = a.cell_start[B], b1 = a.cell_start[B + 1];
-    for (uint32_t p = a0; p < a1; p++) {
-        if (a.kc[(size_t)p * a.J + a.j] > a.k) continue;
-        double px = a.xs[p], py = a.ys[p];
-        for (uint32_t q = b0; q < b1; q++) {
-            if (a.kc[(size_t)q * a.J + a.j] > a.k) continue;
-            if (dist2_exact(px, py, a.xs[q], a.ys[q]) <= a.T) return true;
-        }
-    }
-    return false;
+    return *(const uint64_t *)(row + (j & ~7)) >> (8 * (j & 7));
 }
 
 // Eligibility level of every pair for the minpts values j0 .. j0+nj-1
-// (nj <= kEligGroup): the first level at which both cells hold a core point
-// and some pair of their boxes is within eps; K marks pairs that never
-// become eligible. For pairs of small cells (at most kSmallPairWork point
-// pairs) the level is exact instead: the first level at which some
-// core-core pair is within eps,
+// (nj <= 8): the first level at which both cells hold a core point and some
+// pair of their boxes is within eps; K marks pairs that never become eligible.
+// For pairs of small cells (at most kSmallPairWork point pairs) the level is
+// exact instead: the first level at which some core-core pair is within eps,
 //   min over (p, q) of max(level(s(p,q)), kc_j(p), kc_j(q)),
 // flagged so that the sweep unites them without a test. The point distances
 // are computed once for the whole group.
 //
-// Output: byte g of lev[i] = level | exact << 7 (levels stay below 128),
-// bytes of minpts values beyond the group K. With `hist`, the kernel also
-// counts its tile's pairs per (minpts value, level) bucket for the record
-// scatter: tile t = the kBlock consecutive pairs of block t (a pair per
-// thread: the eligibility tests are latency-bound, so every pair gets its
-// own lane), bucket (jrel0 + g)*(K+1) + level, hist[bucket * tiles + t]
-// (bucket-major, so that an exclusive scan gives every tile's first slot in
-// every bucket); the buckets of level K stay empty (those pairs get no
-// record).
-constexpr int kEligGroup = 8;
+// Output: byte g of lev[i] = level | exact << 7 (levels stay below 64), bytes
+// of minpts values beyond nj K. The kernel also counts its tile's records for
+// the scatter: tile t = the kBlock consecutive pairs of block t (a pair per
+// thread: the eligibility tests are latency-bound, so every pair gets its own
+// lane), one record per distinct level of a pair, hist[(group*(K+1) + level) *
+// tiles + t] (bucket-major, so that an exclusive scan gives every tile's first
+// slot in every bucket); the buckets of level K stay empty.
 constexpr uint32_t kEligTile = kBlock;
 // the scatter takes kPairItems eligibility tiles per block
 constexpr int kPairItems = 8;
-constexpr uint32_t kPairTile = kEligTile * kPairItems;
-constexpr int kPairBuckets = 128; // buckets of a pass for the record scatter
 
-template <int BITS>
-__global__ void __launch_bounds__(kBlock)
-    k_pair_elig(const uint32_t *pa, const uint32_t *pb, const uint16_t *pk,
-                const uint8_t *cellkc_cm, const uint32_t *cell_start, const double *xs,
-                const double *ys, const uint8_t *kc, const double *Tk, int J, int j0, int nj,
-                int K, uint32_t npairs, uint32_t jrel0, uint2 *lev, uint32_t *hist,
-                unsigned tiles)
+// the levels below K among the 8 bytes of a pair, as a bit set
+__device__ __forceinline__ uint64_t levels_present(uint2 w, int K)
 {
-    __shared__ uint32_t h[kWPB][kPairBuckets];
+    uint64_t m = 0;
+#pragma unroll
+    for (int g = 0; g < kGroup; g++) {
+        uint32_t l = ((g < 4 ? w.x : w.y) >> (8 * (g & 3))) & 0x7fu;
+        if ((int)l < K) m |= 1ull << l;
+    }
+    return m;
+}
+
+__global__ void __launch_bounds__(kBlock)
+    k_pair_elig(const uint32_t *pa, const uint32_t *pb, const uint16_t *pk, const uint8_t *cellkc,
+                const uint32_t *cell_start, const double *xs, const double *ys, const uint8_t *kc,
+                const double *Tk, int JP, int j0, int nj, int K, uint32_t npairs, uint32_t group,
+                uint2 *lev, uint32_t *hist, unsigned tiles)
+{
+    __shared__ uint32_t h[kWPB][kMaxLevels];
     __shared__ double sTk[kMaxLevels]; // level thresholds for the exact levels
-    if (hist)
-        for (int r = threadIdx.x; r < kWPB * kPairBuckets; r += kBlock) (&h[0][0])[r] = 0;
     for (int k = threadIdx.x; k < K; k += kBlock) sTk[k] = Tk[k];
     __syncthreads();
-    // with whole groups of 8 minpts values, a cell's or point's 8 levels are
-    // one aligned 8-byte word
-    const bool vec8 = (J & 7) == 0;
-    const int w = threadIdx.x / kWave;
-    {
-        uint32_t i = blockIdx.x * kEligTile + threadIdx.x;
-        bool valid = i < npairs;
-        int e[kEligGroup];
+    const int w = threadIdx.x / kWave, lane = lane_id();
+    uint32_t i = blockIdx.x * kEligTile + threadIdx.x;
+    bool valid = i < npairs;
+    int e[kGroup];
 #pragma unroll
-        for (int g = 0; g < kEligGroup; g++) e[g] = K;
-        uint32_t exact = 0; // bit g: level of j0+g computed exactly
-        if (valid) {
-            uint32_t A = pa[i], B = pb[i];
-            int e0 = pk[i] & 0xff;
-            uint32_t a0 = cell_start[A], a1 = cell_start[A + 1];
-            uint32_t b0 = cell_start[B], b1 = cell_start[B + 1];
-            bool small = (uint64_t)(a1 - a0) * (b1 - b0) <= kSmallPairWork;
-            // a cell's levels for all minpts values lie side by side
-            uint64_t wa = 0, wb = 0;
-            if (vec8) {
-                wa = *(const uint64_t *)(cellkc_cm + (size_t)A * J + j0);
-                wb = *(const uint64_t *)(cellkc_cm + (size_t)B * J + j0);
+    for (int g = 0; g < kGroup; g++) e[g] = K;
+    uint32_t exact = 0; // bit g: level of j0+g computed exactly
+    uint2 word = make_uint2(0x7f7f7f7fu, 0x7f7f7f7fu);
+    if (valid) {
+        uint32_t A = pa[i], B = pb[i];
+        int e0 = pk[i] & 0xff;
+        uint32_t a0 = cell_start[A], a1 = cell_start[A + 1];
+        uint32_t b0 = cell_start[B], b1 = cell_start[B + 1];
+        bool small = (uint64_t)(a1 - a0) * (b1 - b0) <= kSmallPairWork;
+        // a cell's levels for all minpts values lie side by side
+        uint64_t wa = level_word(cellkc + (size_t)A * JP, j0);
+        uint64_t wb = level_word(cellkc + (size_t)B * JP, j0);
+#pragma unroll
+        for (int g = 0; g < kGroup; g++) {
+            if (g < nj) {
+                int v = e0;
+                int ca = (int)((wa >> (8 * g)) & 0xffu), cb = (int)((wb >> (8 * g)) & 0xffu);
+                v = v > ca ? v : ca;
+                v = v > cb ? v : cb;
+                e[g] = v < K ? v : K;
+                if (small && v < K) exact |= 1u << g;
             }
+        }
+        if (exact) {
+            int best[kGroup];
 #pragma unroll
-            for (int g = 0; g < kEligGroup; g++) {
-                if (g < nj) {
-                    int v = e0;
-                    int ca = vec8 ? (int)((wa >> (8 * g)) & 0xffu)
-                                  : cellkc_cm[(size_t)A * J + j0 + g];
-                    int cb = vec8 ? (int)((wb >> (8 * g)) & 0xffu)
-                                  : cellkc_cm[(size_t)B * J + j0 + g];
-                    v = v > ca ? v : ca;
-                    v = v > cb ? v : cb;
-                    e[g] = v < K ? v : K;
-                    if (small && v < K) exact |= 1u << g;
-                }
-            }
-            if (exact) {
-                int best[kEligGroup];
+            for (int g = 0; g < kGroup; g++) best[g] = K;
+            for (uint32_t p = a0; p < a1; p++) {
+                double px = xs[p], py = ys[p];
+                uint64_t wp = level_word(kc + (size_t)p * JP, j0);
+                for (uint32_t q = b0; q < b1; q++) {
+                    double sq = dist2_exact(px, py, xs[q], ys[q]);
+                    uint64_t wq = level_word(kc + (size_t)q * JP, j0);
+                    int ls = 0; // first level whose eps admits the pair
+                    while (ls < K && sq > sTk[ls]) ls++;
+                    if (ls >= K) continue;
 #pragma unroll
-                for (int g = 0; g < kEligGroup; g++) best[g] = K;
-                for (uint32_t p = a0; p < a1; p++) {
-                    double px = xs[p], py = ys[p];
-                    const uint8_t *kp = kc + (size_t)p * J + j0;
-                    uint64_t wp = vec8 ? *(const uint64_t *)kp : 0;
-                    for (uint32_t q = b0; q < b1; q++) {
-                        double sq = dist2_exact(px, py, xs[q], ys[q]);
-                        int ls = 0; // first level whose eps admits the pair
-                        while (ls < K && sq > sTk[ls]) ls++;
-                        if (ls >= K) continue;
-                        const uint8_t *kq = kc + (size_t)q * J + j0;
-                        uint64_t wq = vec8 ? *(const uint64_t *)kq : 0;
-#pragma unroll
-                        for (int g = 0; g < kEligGroup; g++) {
-                            if (!((exact >> g) & 1u)) continue;
-                            int lv = ls;
-                            int x = vec8 ? (int)((wp >> (8 * g)) & 0xffu) : kp[g];
-                            int y = vec8 ? (int)((wq >> (8 * g)) & 0xffu) : kq[g];
-                            lv = lv > x ? lv : x;
-                            lv = lv > y ? lv : y;
-                            best[g] = lv < best[g] ? lv : best[g];
-                        }
+                    for (int g = 0; g < kGroup; g++) {
+                        if (!((exact >> g) & 1u)) continue;
+                        int lv = ls;
+                        int x = (int)((wp >> (8 * g)) & 0xffu), y = (int)((wq >> (8 * g)) & 0xffu);
+                        lv = lv > x ? lv : x;
+                        lv = lv > y ? lv : y;
+                        best[g] = lv < best[g] ? lv : best[g];
                     }
                 }
-#pragma unroll
-                for (int g = 0; g < kEligGroup; g++)
-                    if ((exact >> g) & 1u) e[g] = best[g];
             }
-            uint32_t lo = 0, hi = 0;
 #pragma unroll
-            for (int g = 0; g < kEligGroup; g++) {
-                uint32_t byte = (uint32_t)e[g] | (((exact >> g) & 1u) << 7);
-                if (g < 4) lo |= byte << (8 * g);
-                else hi |= byte << (8 * (g - 4));
-            }
-            lev[i] = make_uint2(lo, hi);
+            for (int g = 0; g < kGroup; g++)
+                if ((exact >> g) & 1u) e[g] = best[g];
         }
-        if (hist) {
-            // one lane per (bucket, wave) adds the wave's count to the
-            // wave's own row: no two lanes write one word
+        word = make_uint2(0u, 0u);
 #pragma unroll
-            for (int g = 0; g < kEligGroup; g++) {
-                if (g >= nj) break;
-                bool take = valid && e[g] < K;
-                uint32_t d = take ? (uint32_t)e[g] : (1u << BITS);
-                uint64_t peers = bucket_peers<BITS>(d);
-                if (take && mask_rank(peers) == 0)
-                    h[w][g * (K + 1) + e[g]] += (uint32_t)popc64(peers);
-            }
+        for (int g = 0; g < kGroup; g++) {
+            uint32_t byte = (uint32_t)e[g] | (((exact >> g) & 1u) << 7);
+            if (g < 4) word.x |= byte << (8 * g);
+            else word.y |= byte << (8 * (g - 4));
         }
+        lev[i] = word;
     }
-    if (hist) {
-        __syncthreads();
-        const int rows = nj * (K + 1);
-        for (int r = threadIdx.x; r < rows; r += kBlock) {
-            uint32_t s = 0;
+    const uint64_t present = levels_present(word, K);
+    uint32_t mine = 0; // lane l: the wave's records of level l
+    for (int l = 0; l < K; l++) {
+        uint32_t cnt = (uint32_t)popc64(ballot((present >> l) & 1ull));
+        if (lane == l) mine = cnt;
+    }
+    h[w][lane] = mine;
+    __syncthreads();
+    if ((int)threadIdx.x <= K) { // (K < kMaxLevels; level K's bucket is empty)
+        uint32_t s = 0;
 #pragma unroll
-            for (int q = 0; q < kWPB; q++) s += h[q][r];
-            hist[((size_t)jrel0 * (K + 1) + r) * tiles + blockIdx.x] = s;
-        }
+        for (int q = 0; q < kWPB; q++) s += h[q][threadIdx.x];
+        hist[((size_t)group * (K + 1) + threadIdx.x) * tiles + blockIdx.x] = s;
     }
 }
 
-// The pair records of a pass in (minpts value, level) order, stable: block
-// t takes the kPairItems eligibility tiles from tile kPairItems*t on, whose
-// records of bucket d go from offs[d*etiles + kPairItems*t] on (the
-// exclusive scan of hist over etiles tiles), in pair order. Pairs that never
-// become eligible get no record. Record: (a, b, levels | exact << 16). lev
-// holds ngroups = ceil(nj / kEligGroup) planes of npairs words.
-template <int BITS>
+// The records of group `group` in level order, stable: block t takes the
+// kPairItems eligibility tiles from tile kPairItems*t on; tile u's records of
+// bucket d go from offs[d*tiles + u] on (the exclusive scan of hist), in pair
+// order.
 __global__ void __launch_bounds__(kBlock)
     k_pair_scatter(const uint32_t *pa, const uint32_t *pb, const uint16_t *pk, const uint2 *lev,
-                   uint32_t npairs, int nj, int K, const uint32_t *offs, unsigned etiles,
+                   uint32_t npairs, int K, uint32_t group, const uint32_t *offs, unsigned tiles,
                    PairRec *out)
 {
-    __shared__ uint32_t base_d[kPairBuckets];
-    __shared__ uint32_t wcnt[kWPB][kPairBuckets];
-    const int nb = nj * (K + 1);
-    for (int d = threadIdx.x; d < nb; d += kBlock)
-        base_d[d] = offs[(size_t)d * etiles + (size_t)blockIdx.x * kPairItems];
-    for (int r = threadIdx.x; r < kWPB * kPairBuckets; r += kBlock) (&wcnt[0][0])[r] = 0;
-    __syncthreads();
-    const int w = threadIdx.x / kWave;
-    const int ngroups = (nj + kEligGroup - 1) / kEligGroup;
+    __shared__ uint32_t h[kPairItems][kWPB][kMaxLevels];
+    const int w = threadIdx.x / kWave, lane = lane_id();
+    const uint32_t t0 = blockIdx.x * (uint32_t)kPairItems;
+    uint64_t present[kPairItems];
+    uint2 word[kPairItems];
+#pragma unroll
     for (int it = 0; it < kPairItems; it++) {
-        uint32_t i = blockIdx.x * kPairTile + (uint32_t)it * kBlock + threadIdx.x;
-        bool valid = i < npairs;
-        uint32_t A = 0, B = 0, C = 0;
-        if (valid) {
+        uint32_t i = (t0 + (uint32_t)it) * kEligTile + threadIdx.x;
+        word[it] = i < npairs ? lev[i] : make_uint2(0x7f7f7f7fu, 0x7f7f7f7fu);
+        present[it] = levels_present(word[it], K);
+        uint32_t mine = 0;
+        for (int l = 0; l < K; l++) {
+            uint32_t cnt = (uint32_t)popc64(ballot((present[it] >> l) & 1ull));
+            if (lane == l) mine = cnt;
+        }
+        h[it][w][lane] = mine;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < kPairItems; it++) {
+        const uint32_t t = t0 + (uint32_t)it, i = t * kEligTile + threadIdx.x;
+        if (t >= tiles) break;
+        // lane l: the wave's first slot in level l's bucket
+        uint32_t base = 0;
+        if (lane < K) {
+            base = offs[((size_t)group * (K + 1) + lane) * tiles + t];
+            for (int u = 0; u < w; u++) base += h[it][u][lane];
+        }
+        if (!ballot(present[it] != 0)) continue;
+        uint32_t A = 0, B = 0, kf = 0;
+        if (present[it]) {
             A = pa[i];
             B = pb[i];
-            C = pk[i];
+            kf = pk[i] & 0xff00u;
         }
-        for (int q = 0; q < ngroups; q++) {
-            const int gn = nj - q * kEligGroup < kEligGroup ? nj - q * kEligGroup : kEligGroup;
-            const int r0 = q * kEligGroup * (K + 1); // first bucket of the group
-            uint2 word = valid ? lev[(size_t)q * npairs + i] : make_uint2(0u, 0u);
-            uint32_t rank[kEligGroup];
-            uint32_t bytes[kEligGroup];
+        for (int l = 0; l < K; l++) {
+            uint64_t m = ballot((present[it] >> l) & 1ull);
+            if (!m) continue;
+            uint32_t b = (uint32_t)__builtin_amdgcn_readlane((int)base, l);
+            if ((present[it] >> l) & 1ull) {
+                uint32_t vals = 0;
 #pragma unroll
-            for (int g = 0; g < kEligGroup; g++) {
-                bytes[g] = ((g < 4 ? word.x : word.y) >> (8 * (g & 3))) & 0xffu;
-                rank[g] = 0;
-                if (g >= gn) continue;
-                uint32_t l = bytes[g] & 0x7fu;
-                bool take = valid && l < (uint32_t)K;
-                uint64_t peers = bucket_peers<BITS>(take ? l : (1u << BITS));
-                rank[g] = (uint32_t)mask_rank(peers);
-                if (take && rank[g] == 0) wcnt[w][r0 + g * (K + 1) + (int)l] = (uint32_t)popc64(peers);
-            }
-            __syncthreads();
-#pragma unroll
-            for (int g = 0; g < kEligGroup; g++) {
-                if (g >= gn) continue;
-                uint32_t l = bytes[g] & 0x7fu;
-                if (!valid || l >= (uint32_t)K) continue;
-                int d = r0 + g * (K + 1) + (int)l;
-                uint32_t pos = base_d[d] + rank[g];
-                for (int u = 0; u < w; u++) pos += wcnt[u][d];
-                out[pos] = PairRec{A, B, C | ((bytes[g] >> 7) << 16)};
-            }
-            __syncthreads();
-            const int r1 = r0 + gn * (K + 1);
-            for (int d = r0 + threadIdx.x; d < r1; d += kBlock) {
-                uint32_t s = 0;
-#pragma unroll
-                for (int u = 0; u < kWPB; u++) {
-                    s += wcnt[u][d];
-                    wcnt[u][d] = 0;
+                for (int g = 0; g < kGroup; g++) {
+                    uint32_t byte = ((g < 4 ? word[it].x : word[it].y) >> (8 * (g & 3))) & 0xffu;
+                    if ((int)(byte & 0x7fu) == l) vals |= (1u | ((byte >> 7) << 16)) << g;
                 }
-                base_d[d] += s;
+                out[b + (uint32_t)mask_rank(m)] = PairRec{A, B, vals | kf};
             }
-            __syncthreads();
         }
     }
 }
@@ -1337,62 +1306,8 @@ __global__ void k_pair_bounds(const uint32_t *offs, const uint32_t *hist, unsign
     }
 }
 
-// Passes of more than kPairBuckets buckets sort by radix instead: key
-// (jrel0 + g)*(K+1) + level and value i | exact << 31 for every pair and
-// minpts value g of plane q (pairs that never become eligible sort last in
-// their minpts value's range).
-__global__ void k_level_keys(const uint2 *lev, uint32_t npairs, int nj, int K, uint32_t *key,
-                             uint32_t *val)
-{
-    uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= npairs) return;
-    const int ngroups = (nj + kEligGroup - 1) / kEligGroup;
-    for (int q = 0; q < ngroups; q++) {
-        uint2 word = lev[(size_t)q * npairs + i];
-        for (int g = 0; g < kEligGroup; g++) {
-            int j = q * kEligGroup + g;
-            if (j >= nj) break;
-            uint32_t byte = ((g < 4 ? word.x : word.y) >> (8 * (g & 3))) & 0xffu;
-            key[(size_t)j * npairs + i] = (uint32_t)j * (uint32_t)(K + 1) + (byte & 0x7fu);
-            val[(size_t)j * npairs + i] = i | ((byte >> 7) << 31);
-        }
-    }
-}
-
-// bstart[k] = first index of sorted keys with key >= k, for k = 0..K+1
-// records of the radix-sorted pair order (the bucket sort writes them itself)
-__global__ void k_pack_records(const uint32_t *order, const uint32_t *pa, const uint32_t *pb,
-                               const uint16_t *pk, uint32_t n, PairRec *rec)
-{
-    uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    uint32_t o = order[i], v = o & 0x7fffffffu;
-    rec[i] = PairRec{pa[v], pb[v], (uint32_t)pk[v] | ((o >> 31) << 16)};
-}
-
-__global__ void k_bucket_starts(const uint32_t *key, uint32_t n, int K, uint32_t *bstart)
-{
-    uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i > n) return;
-    uint32_t prev = i == 0 ? 0u : key[i - 1] + 1;
-    uint32_t cur = i == n ? (uint32_t)K + 1 : key[i];
-    if (i == 0) prev = 0;
-    for (uint32_t k = prev; k <= cur && k <= (uint32_t)K + 1; k++) bstart[k] = i;
-}
-
-__device__ __forceinline__ void wave_append_rec(bool take, const PairRec &v, PairRec *list,
-                                                uint32_t *count)
-{
-    uint64_t m = ballot(take);
-    if (!m) return;
-    int leader = __builtin_ctzll(m);
-    uint32_t base = 0;
-    if (lane_id() == leader) base = atomicAdd(count, (uint32_t)popc64(m));
-    base = __shfl(base, leader);
-    if (take) list[base + mask_rank(m)] = v;
-}
-
-// wave_append_rec into a list of cap records: records that would not fit are
+// Append v to a list of cap records for every lane with take set, one atomic
+// per wave: records that would not fit are
 // dropped and *ovf is set (the host then hands the batch to another engine).
 // The counter may pass cap; readers clamp it.
 __device__ __forceinline__ void wave_append_cap(bool take, const PairRec &v, PairRec *list,
@@ -1473,126 +1388,199 @@ __device__ __forceinline__ uint32_t level_blocks(const uint32_t *bstart, int k, 
     return want < gridDim.x ? want : gridDim.x;
 }
 
-// Grid-stride over the carried pairs (count on the device) followed by the
-// pairs that become eligible at this level, whose records (cells, levels,
-// exact-level flag in bit 16 of k) the sort has laid out contiguously per
-// (minpts value, level). Each eligible pair is settled
-// (already connected; fully inside eps; small and tested here), kept for the
-// next level, or handed to a wave test. Tests of grid-adjacent cells go to
-// `near`, the rest to `far`; the near tests run first so most far pairs are
-// already connected when theirs run.
+// Grid-stride over the carried records (count on the device) followed by the
+// records that become eligible at this level, which the scatter has laid out
+// contiguously per (group, level). Each value of a record is settled (already
+// connected; level exact or cells fully inside eps: united) or handed to a
+// wave test. Tests of grid-adjacent cells go to `near`, the rest to `far`; the
+// near tests run first so most far pairs are already connected when theirs
+// run.
+//
+// A record costs its 12 bytes and the two cells' 32 bytes of parents, and is
+// bound by those dependent loads; most values are connected by the first pair
+// of parents. The values still open walk to their roots together, all loads
+// of a step in flight.
+//
+// Most of a record's cost is the walk of a value that its first parents leave
+// open, and in list order whole stretches of the plane are walked before any
+// of it is joined. So every kSampleEvery-th new record goes first, on its own:
+// the sparse sample joins most of a level's components through short trees,
+// and the records that follow find their values connected at the first look.
+// Its tests wait until the record comes again. All levels of 2M points x 64
+// variants take 1912 us with 1 of 4 (2311 without a sample, 1759 with 1 of 8,
+// 1988 with 1 of 16), 8M skewed points 417 (662, 607, 619), 256 datasets 3126
+// (3614, 3004, 3106), 500K x 16 285 (335, 311, 320): 4 is best or near it for
+// all of them.
+constexpr uint32_t kSampleEvery = 4;
 __global__ void __launch_bounds__(kBlock) k_sweep(LevelArgs a, LevelLists L)
 {
-    a.j += (int)blockIdx.y; // global minpts index (kc); lists use the pass-relative one
-    LevelJ lj = level_j(L, blockIdx.y, a.k);
-    const PairRec *carried = lj.carried;
-    const uint32_t *ncarried = lj.nc, *bstart = lj.bstart;
-    uint32_t *parent = lj.parent;
-    PairRec *keep = lj.keep, *near = lj.near, *far = lj.far;
-    uint32_t *nkeep = lj.nkeep, *nnear = lj.nnear, *nfar = lj.nfar, *ovf = L.ovf;
-    const uint32_t tcap = L.tcap;
+    LevelG lg = level_g(L, blockIdx.y, a.k);
+    const PairRec *carried = lg.carried;
+    const uint32_t *bstart = lg.bstart;
+    uint32_t *parent = lg.parent;
     RecChunk chn, chf;
-    bool chunked = bstart[a.k + 1] - bstart[a.k] >= kChunkedFrom;
-    uint32_t nb = level_blocks(bstart, a.k, L.ppb, L.minb);
+    const uint32_t nfresh = bstart[a.k + 1] - bstart[a.k];
+    const bool chunked = nfresh >= kChunkedFrom;
+    const uint32_t nb = level_blocks(bstart, a.k, L.ppb, L.minb);
     if (blockIdx.x >= nb) return;
     const PairRec *fresh = L.frec + bstart[a.k];
-    uint32_t nfresh = bstart[a.k + 1] - bstart[a.k];
-    uint32_t nc = *ncarried;
-    uint32_t total = nc + nfresh;
+    const uint32_t nc = *lg.nc;
+    const uint32_t total = nc + nfresh;
+    const uint32_t samples = nfresh / kSampleEvery;
+    const uint32_t work = samples + total;
     auto load_rec = [&](uint32_t i) {
         PairRec r{0, 0, 0};
-        if (i < total) {
+        if (i < samples) r = fresh[(size_t)i * kSampleEvery];
+        else if (i < work) {
+            i -= samples;
             r = i < nc ? carried[i] : fresh[i - nc];
         }
         return r;
     };
     const uint32_t step = nb * kBlock;
+    const int lane = lane_id();
     // the next step's record is loaded while this one is settled: its load
     // does not wait behind this step's parent loads
     PairRec next = load_rec(blockIdx.x * kBlock + threadIdx.x);
-    for (uint32_t base = blockIdx.x * kBlock; base < total; base += step) {
-        uint32_t i = base + threadIdx.x;
-        bool valid = i < total;
-        PairRec pr = next;
-        next = load_rec(base + step < total ? i + step : total);
-        bool kp = false, tnear = false, tfar = false, uni = false;
-        uint32_t ra = 0, rb = 0;
-        if (valid) {
-            uint32_t A = pr.a, B = pr.b;
-            int kfull = (int)((pr.k >> 8) & 0xff);
-            bool exact = (pr.k >> 16) & 1u;
-            if (cf_roots(parent, A, B, ra, rb)) {
-                // connected now, hence at every later level
-            } else if (exact || kfull <= a.k) {
-                // exact pairs arrive at the level they connect
-                uni = true;
-            } else {
-                uint32_t na = a.cell_start[A + 1] - a.cell_start[A];
-                uint32_t nb = a.cell_start[B + 1] - a.cell_start[B];
-                if ((uint64_t)na * nb <= kSmallPairWork) {
-                    if (small_pair_connected(a, A, B)) cf_unite(parent, A, B);
-                    else kp = true;
-                } else {
-                    // both cells belong to one dataset
-                    uint32_t ds = a.cell_ds[A], ncy = a.sncy[ds], k0 = a.skbase[ds];
-                    uint32_t ka = a.cell_key[A] - k0, kb = a.cell_key[B] - k0;
-                    uint32_t qa = ka / a.m, qb = kb / a.m;
-                    int64_t dx = (int64_t)(qa / ncy * a.m + ka % a.m) -
-                                 (int64_t)(qb / ncy * a.m + kb % a.m);
-                    int64_t dy = (int64_t)(qa % ncy) - (int64_t)(qb % ncy);
-                    bool adj = dx >= -1 && dx <= 1 && dy >= -1 && dy <= 1;
-                    tnear = adj;
-                    tfar = !adj;
+    for (uint32_t base = blockIdx.x * kBlock; base < work; base += step) {
+        const uint32_t i = base + threadIdx.x;
+        const PairRec pr = next; // no values set beyond the last record
+        next = load_rec(base + step < work ? i + step : work);
+        const uint32_t A = pr.a, B = pr.b;
+        uint32_t ra[kGroup], rb[kGroup];
+        cf_load8(parent, A, ra);
+        cf_load8(parent, B, rb);
+        uint32_t open = 0; // values not known to be connected
+#pragma unroll
+        for (int j = 0; j < kGroup; j++)
+            if (((pr.k >> j) & 1u) && ra[j] != rb[j]) open |= 1u << j;
+        if (ballot(open != 0)) {
+            bool moving = true;
+            while (ballot(moving)) {
+                uint32_t na[kGroup], nb2[kGroup];
+#pragma unroll
+                for (int j = 0; j < kGroup; j++) {
+                    na[j] = ra[j];
+                    nb2[j] = rb[j];
+                    if (moving && ((open >> j) & 1u)) {
+                        na[j] = ld_u32(parent + cf_at(ra[j]) + j);
+                        nb2[j] = ld_u32(parent + cf_at(rb[j]) + j);
+                    }
+                }
+                moving = false;
+#pragma unroll
+                for (int j = 0; j < kGroup; j++) {
+                    moving = moving || na[j] != ra[j] || nb2[j] != rb[j];
+                    ra[j] = na[j];
+                    rb[j] = nb2[j];
                 }
             }
+#pragma unroll
+            for (int j = 0; j < kGroup; j++)
+                if ((open >> j) & 1u) {
+                    // a cell below its root is no root and stays none: its
+                    // parent may move up to any ancestor
+                    if (ra[j] != A) st_u32(parent + cf_at(A) + j, ra[j]);
+                    if (rb[j] != B) st_u32(parent + cf_at(B) + j, rb[j]);
+                    if (ra[j] == rb[j]) open &= ~(1u << j);
+                }
         }
-        // Runs of consecutive lanes uniting under one A-side root (the pairs
+        // exact levels arrive when they connect
+        const bool whole = (int)((pr.k >> 8) & 0xffu) <= a.k;
+        const uint32_t uni = whole ? open : open & (pr.k >> 16);
+        // a sampled record comes again: its tests wait until then
+        const uint32_t test = i < samples ? 0u : open & ~uni;
+        // Runs of consecutive lanes uniting under one A-side root (the records
         // of one cell come in order) hook every root of the run straight
         // under the run's smallest root, instead of racing to relink the
         // shared root one pair at a time: a segmented min over the wave, a
         // fixed number of shuffles however many runs there are. Runs of the
         // same root elsewhere in the wave hook separately; a hook that loses
         // its race falls back to a full union.
-        if (ballot(uni)) {
-            const int lane = lane_id();
-            uint32_t pra = __shfl_up(ra, 1);
-            bool puni = __shfl_up((int)uni, 1) != 0;
-            bool head = !uni || lane == 0 || !puni || pra != ra;
+#pragma unroll
+        for (int j = 0; j < kGroup; j++) {
+            const bool un = (uni >> j) & 1u;
+            if (!ballot(un)) continue;
+            const uint32_t x = ra[j], y = rb[j];
+            uint32_t px = __shfl_up(x, 1);
+            bool pun = __shfl_up((int)un, 1) != 0;
+            bool head = !un || lane == 0 || !pun || px != x;
             uint64_t H = ballot(head); // run starts (lanes outside runs too)
             uint64_t upto = lane == kWave - 1 ? ~0ull : (2ull << lane) - 1ull;
             int hpos = 63 - __builtin_clzll(H & upto);
             uint64_t above = H & ~upto;
             int last = above ? __builtin_ctzll(above) - 1 : kWave - 1;
-            uint32_t m = uni ? (rb < ra ? rb : ra) : kNone;
+            uint32_t m = un ? (y < x ? y : x) : kNone;
 #pragma unroll
             for (int d = 1; d < kWave; d <<= 1) {
                 uint32_t t = __shfl_up(m, d);
                 if (lane - d >= hpos) m = t < m ? t : m;
             }
             m = __shfl(m, last); // the run's minimum, held by its last lane
-            if (uni && rb != m) cf_hook(parent, rb, m);
-            if (uni && head && ra != m) cf_hook(parent, ra, m);
+            if (un && y != m) cf_hook(parent + j, y, m);
+            if (un && head && x != m) cf_hook(parent + j, x, m);
         }
-        wave_append_rec(kp, pr, keep, nkeep);
+        bool near = false, far = false;
+        if (test) {
+            // both cells belong to one dataset
+            uint32_t ds = a.cell_ds[A], ncy = a.sncy[ds], k0 = a.skbase[ds];
+            uint32_t ka = a.cell_key[A] - k0, kb = a.cell_key[B] - k0;
+            uint32_t qa = ka / a.m, qb = kb / a.m;
+            int64_t dx = (int64_t)(qa / ncy * a.m + ka % a.m) -
+                         (int64_t)(qb / ncy * a.m + kb % a.m);
+            int64_t dy = (int64_t)(qa % ncy) - (int64_t)(qb % ncy);
+            near = dx >= -1 && dx <= 1 && dy >= -1 && dy <= 1;
+            far = !near;
+        }
+        const PairRec tr{A, B, (pr.k & 0xff00u) | test};
         if (chunked) {
-            chunk_append(tnear, pr, near, nnear, tcap, ovf, chn);
-            chunk_append(tfar, pr, far, nfar, tcap, ovf, chf);
+            chunk_append(near, tr, lg.near, lg.nnear, L.tcap, L.ovf, chn);
+            chunk_append(far, tr, lg.far, lg.nfar, L.tcap, L.ovf, chf);
         } else {
-            wave_append_cap(tnear, pr, near, nnear, tcap, ovf);
-            wave_append_cap(tfar, pr, far, nfar, tcap, ovf);
+            wave_append_cap(near, tr, lg.near, lg.nnear, L.tcap, L.ovf);
+            wave_append_cap(far, tr, lg.far, lg.nfar, L.tcap, L.ovf);
         }
     }
-    chunk_close(chn, near);
-    chunk_close(chf, far);
+    chunk_close(chn, lg.near);
+    chunk_close(chf, lg.far);
 }
 
-// Wave per test pair: any core-core pair within eps_k connects the two cells.
-// The smaller cell A is screened 64 points at a time (core at level k and
-// within eps of B's box); only the survivors are tested, one after another,
-// against B. B's points are held in registers when B fits one wave. The
-// loads go out in two rounds: both cells' point ranges with both parents,
-// then B's box with the first 64 points of each cell (indices clamped into
-// the cell, so no load waits behind a branch).
+// The values of a test record that are still to be connected.
+__device__ __forceinline__ uint32_t test_open(const PairRec &pr, uint32_t *parent)
+{
+    uint32_t pa[kGroup], pb[kGroup], open = 0;
+    cf_load8(parent, pr.a, pa);
+    cf_load8(parent, pr.b, pb);
+#pragma unroll
+    for (int j = 0; j < kGroup; j++)
+        if (((pr.k >> j) & 1u) && pa[j] != pb[j] &&
+            cf_find(parent + j, pa[j]) != cf_find(parent + j, pb[j]))
+            open |= 1u << j;
+    return open;
+}
+
+// Lanes l < 8 unite the pair for the values found connected; lane 0 keeps the
+// record for the next level with those that were not.
+__device__ __forceinline__ void test_end(const PairRec &pr, uint32_t l, uint32_t found,
+                                         uint32_t left, uint32_t *parent, PairRec *list_out,
+                                         uint32_t *nout)
+{
+    if (l < kGroup && ((found >> l) & 1u)) cf_unite(parent + l, pr.a, pr.b);
+    if (l == 0 && left)
+        list_out[atomicAdd(nout, 1u)] = PairRec{pr.a, pr.b, (pr.k & 0xff00u) | left};
+}
+
+// core values of a point at the pass's level, as bits of the group
+__device__ __forceinline__ uint32_t core_bits(const LevelArgs &a, uint32_t p)
+{
+    return levels_reached(level_word(a.kc + (size_t)p * a.JP, a.j0), a.k);
+}
+
+// Wave per test record: for each of its values, any pair of points core for
+// it within eps_k connects the two cells. The smaller cell A is screened 64
+// points at a time (core for an open value and within eps of B's box); only
+// the survivors are tested, one after another, against B. B's points are held
+// in registers when B fits one wave.
 __device__ void test_pair(const LevelArgs &a, const PairRec &pr, uint32_t *parent,
                           PairRec *list_out, uint32_t *nout)
 {
@@ -1600,7 +1588,6 @@ __device__ void test_pair(const LevelArgs &a, const PairRec &pr, uint32_t *paren
     uint32_t A = pr.a, B = pr.b;
     uint32_t a0 = a.cell_start[A], a1 = a.cell_start[A + 1];
     uint32_t b0 = a.cell_start[B], b1 = a.cell_start[B + 1];
-    uint32_t pa = ld_u32(parent + A), pb = ld_u32(parent + B);
     if (a1 - a0 > b1 - b0) { // lanes sweep the larger cell
         uint32_t t = A;
         A = B;
@@ -1612,56 +1599,56 @@ __device__ void test_pair(const LevelArgs &a, const PairRec &pr, uint32_t *paren
         a1 = b1;
         b1 = t;
     }
-    bool found = pa == pb || cf_find(parent, pa) == cf_find(parent, pb);
-    if (found) return;
+    uint32_t open = test_open(pr, parent);
+    if (!open) return;
     const int lane = lane_id();
     const uint32_t na = a1 - a0, nb = b1 - b0; // both >= 1
     const double *bB = a.box + 4 * (size_t)B;
     double bx0 = bB[0], bx1 = bB[1], by0 = bB[2], by1 = bB[3];
     uint32_t qi = b0 + min((uint32_t)lane, nb - 1);
-    int kq = a.kc[(size_t)qi * a.J + a.j];
     double qx = a.xs[qi], qy = a.ys[qi];
+    uint32_t qm = (uint32_t)lane < nb ? core_bits(a, qi) : 0u;
     uint32_t pi = a0 + min((uint32_t)lane, na - 1);
-    int kp = a.kc[(size_t)pi * a.J + a.j];
     double px = a.xs[pi], py = a.ys[pi];
-    // B in one wave: lane q holds point b0+q (NaN when absent or not core)
+    uint32_t pm = core_bits(a, pi);
     const bool bsmall = nb <= (uint32_t)kWave;
-    if (!((uint32_t)lane < nb && kq <= a.k)) qx = qy = __longlong_as_double(0x7ff8000000000000ll);
-    for (uint32_t p0 = a0; p0 < a1 && !found; p0 += kWave) {
+    uint32_t found = 0;
+    for (uint32_t p0 = a0; p0 < a1 && open; p0 += kWave) {
         uint32_t p = p0 + lane;
         if (p0 != a0) { // later chunks of a cell larger than a wave
             uint32_t pc = min(p, a1 - 1);
-            kp = a.kc[(size_t)pc * a.J + a.j];
             px = a.xs[pc];
             py = a.ys[pc];
+            pm = core_bits(a, pc);
         }
         // a core point of A from which some point of B can be within eps
-        bool cand = p < a1 && kp <= a.k && box_dist2_min(px, py, bx0, bx1, by0, by1) <= a.T;
+        bool cand =
+            p < a1 && (pm & open) && box_dist2_min(px, py, bx0, bx1, by0, by1) <= a.T;
         uint64_t cm = ballot(cand);
-        while (cm && !found) {
+        while (cm && open) {
             int bit = __builtin_ctzll(cm);
             cm &= cm - 1;
             double cx = __shfl(px, bit), cy = __shfl(py, bit);
-            if (bsmall) {
-                // NaN coordinates never pass the test
-                found = ballot(dist2_exact(cx, cy, qx, qy) <= a.T) != 0;
-                continue;
-            }
+            const uint32_t cv = (uint32_t)__builtin_amdgcn_readlane((int)pm, bit) & open;
+            if (!cv) continue;
             for (uint32_t q0 = b0; q0 < b1; q0 += kWave) {
-                uint32_t q = q0 + lane;
-                bool hit = q < b1 && a.kc[(size_t)q * a.J + a.j] <= a.k &&
-                           dist2_exact(cx, cy, a.xs[q], a.ys[q]) <= a.T;
-                if (ballot(hit)) {
-                    found = true;
-                    break;
+                uint32_t hit = 0;
+                if (bsmall) {
+                    if (dist2_exact(cx, cy, qx, qy) <= a.T) hit = qm & cv;
+                } else {
+                    uint32_t q = q0 + lane;
+                    if (q < b1 && dist2_exact(cx, cy, a.xs[q], a.ys[q]) <= a.T)
+                        hit = core_bits(a, q) & cv;
                 }
+                if (!ballot(hit != 0)) continue;
+                for (int o = kWave / 2; o > 0; o >>= 1) hit |= __shfl_xor(hit, o);
+                found |= hit;
+                open &= ~hit;
+                if (!(cv & open)) break;
             }
         }
     }
-    if (lane == 0) {
-        if (found) cf_unite(parent, A, B);
-        else list_out[atomicAdd(nout, 1u)] = pr;
-    }
+    test_end(pr, (uint32_t)lane, found, open, parent, list_out, nout);
 }
 
 // Two tests in one wave, one per 32-lane half (lanes 32h..32h+31 take r_h),
@@ -1687,9 +1674,8 @@ __device__ uint32_t test_pair_halves(const LevelArgs &a, const PairRec &r0, cons
     if ((lm & 0xffffffffull) && !(fm & 0xffffffffull)) back |= 1u;
     if ((lm >> 32) && !(fm >> 32)) back |= 2u;
     if (fits) {
-        uint32_t pa = ld_u32(parent + A), pb = ld_u32(parent + B);
-        bool found = pa == pb || cf_find(parent, pa) == cf_find(parent, pb);
-        if (!found) {
+        uint32_t open = test_open(pr, parent);
+        if (open) {
             if (a1 - a0 > b1 - b0) { // lanes hold the larger cell
                 uint32_t t = A;
                 A = B;
@@ -1705,25 +1691,26 @@ __device__ uint32_t test_pair_halves(const LevelArgs &a, const PairRec &r0, cons
             const double *bB = a.box + 4 * (size_t)B;
             double bx0 = bB[0], bx1 = bB[1], by0 = bB[2], by1 = bB[3];
             uint32_t qi = b0 + min(l, nb - 1);
-            int kq = a.kc[(size_t)qi * a.J + a.j];
             double qx = a.xs[qi], qy = a.ys[qi];
+            const uint32_t qm = l < nb ? core_bits(a, qi) : 0u;
             uint32_t pi = a0 + min(l, na - 1);
-            int kp = a.kc[(size_t)pi * a.J + a.j];
             double px = a.xs[pi], py = a.ys[pi];
-            // lane l holds point b0+l of B (NaN when absent or not core)
-            if (!(l < nb && kq <= a.k)) qx = qy = __longlong_as_double(0x7ff8000000000000ll);
-            bool cand = l < na && kp <= a.k && box_dist2_min(px, py, bx0, bx1, by0, by1) <= a.T;
-            uint32_t cm = (uint32_t)(ballot(cand) >> (32 * h));
-            while (cm && !found) {
+            const uint32_t pm = core_bits(a, pi);
+            bool cand =
+                l < na && (pm & open) && box_dist2_min(px, py, bx0, bx1, by0, by1) <= a.T;
+            uint32_t cm = (uint32_t)(ballot(cand) >> (32 * h)), found = 0;
+            while (cm && open) {
                 int bit = __builtin_ctz(cm);
                 cm &= cm - 1;
                 double cx = __shfl(px, 32 * h + bit), cy = __shfl(py, 32 * h + bit);
-                found = (uint32_t)(ballot(dist2_exact(cx, cy, qx, qy) <= a.T) >> (32 * h)) != 0u;
+                const uint32_t cv = (uint32_t)__shfl((int)pm, 32 * h + bit) & open;
+                uint32_t hit = dist2_exact(cx, cy, qx, qy) <= a.T ? qm & cv : 0u;
+                if (!(uint32_t)(ballot(hit != 0) >> (32 * h))) continue;
+                for (int o = 16; o > 0; o >>= 1) hit |= __shfl_xor(hit, o);
+                found |= hit;
+                open &= ~hit;
             }
-            if (l == 0) {
-                if (found) cf_unite(parent, A, B);
-                else list_out[atomicAdd(nout, 1u)] = pr;
-            }
+            test_end(pr, l, found, open, parent, list_out, nout);
         }
     }
     return back;
@@ -1733,18 +1720,18 @@ __device__ uint32_t test_pair_halves(const LevelArgs &a, const PairRec &r0, cons
 // them in order, so most far tests start after the near ones)
 __global__ void __launch_bounds__(kBlock) k_test(LevelArgs a, LevelLists L)
 {
-    a.j += (int)blockIdx.y; // global minpts index (kc); lists use the pass-relative one
-    LevelJ lj = level_j(L, blockIdx.y, a.k);
-    const uint32_t *bstart = lj.bstart, *nnear = lj.nnear, *nfar = lj.nfar, *ovf = L.ovf;
-    const PairRec *near = lj.near, *far = lj.far;
-    uint32_t *parent = lj.parent, *nout = lj.nkeep;
-    PairRec *list_out = lj.keep;
+    a.j0 += kGroup * (int)blockIdx.y; // first minpts value of the group
+    LevelG lg = level_g(L, blockIdx.y, a.k);
+    const uint32_t *bstart = lg.bstart;
+    const PairRec *near = lg.near, *far = lg.far;
+    uint32_t *parent = lg.parent, *nout = lg.nkeep;
+    PairRec *list_out = lg.keep;
     const uint32_t tcap = L.tcap;
     // a test list that ran out of room (reported to the host) is not read
-    if (*ovf) return;
-    // tests are latency-bound waves: one block per kTestsPerBlock tests,
-    // up to the launched grid
-    uint32_t nn = *nnear, nf = *nfar;
+    if (*L.ovf) return;
+    // tests are latency-bound waves: one block per tpb tests, up to the
+    // launched grid
+    uint32_t nn = *lg.nnear, nf = *lg.nfar;
     nn = nn < tcap ? nn : tcap;
     nf = nf < tcap ? nf : tcap;
     uint32_t nt = nn + nf;
@@ -1791,18 +1778,10 @@ __global__ void __launch_bounds__(kBlock) k_test(LevelArgs a, LevelLists L)
 }
 
 // ---------------------------------------------------------- snapshots
-// Flattens the forest (every cell with a core point at level k points at its
-// root) and sets
-// compmin[root] = smallest core rank of the component (compmin holds NONE on
-// entry: k_init_parent and k_cell_labels clear it). Lanes of a wave that
-// share a root (the common case inside a large cluster) reduce first, so a
-// giant component takes one atomic per wave rather than one per cell; after
-// the two most common roots of the wave the remaining lanes, spread over
-// small components, update theirs one atomic each.
-// Snapshots of one level k for every minpts value j in jmask (blockIdx.y = j):
-// j's parents, compmin and per-cell tables sit at j*ncell, its core ranks at
-// cmr + (j*K + k)*ncell, and its snapshot takes slot sbase + (number of
-// minpts values of jmask below j).
+// Snapshots of one level k for every minpts value j in jmask, a group of 8 at
+// a time (blockIdx.y), a thread per cell: parents and compmin of a group side
+// by side per cell, core ranks at cmr + (j*K + k)*ncell, and value j's
+// snapshot in slot sbase + (number of values of jmask below j).
 struct SnapArgs {
     uint32_t *parent, *compmin;
     const uint32_t *cmr;
@@ -1810,76 +1789,120 @@ struct SnapArgs {
     uint32_t *root, *lab, *bits, *pre; // slot s: root/lab + s*ncell, bits/pre + s*nw
     uint64_t jmask;
     uint32_t sbase, ncell, nw, K;
-    int k;
+    int k, JP, j0;
 };
 
-__device__ __forceinline__ bool snap_slot(const SnapArgs &S, uint32_t j, uint32_t *slot)
+__device__ __forceinline__ uint32_t snap_slot(const SnapArgs &S, uint32_t j)
 {
-    if (!((S.jmask >> j) & 1ull)) return false;
-    *slot = S.sbase + (uint32_t)__popcll(S.jmask & ((1ull << j) - 1ull));
-    return true;
+    return S.sbase + (uint32_t)__popcll(S.jmask & ((1ull << j) - 1ull));
+}
+// the group's requested values, and those of them core in cell c
+__device__ __forceinline__ uint32_t snap_wanted(const SnapArgs &S, uint32_t g)
+{
+    return (uint32_t)(S.jmask >> (kGroup * g)) & 0xffu;
+}
+__device__ __forceinline__ uint32_t snap_core(const SnapArgs &S, uint32_t g, uint32_t c)
+{
+    return levels_reached(level_word(S.cellkc + (size_t)c * S.JP, S.j0 + (int)(kGroup * g)), S.k);
+}
+__device__ __forceinline__ void load8(const uint32_t *p, uint32_t (&v)[kGroup])
+{
+    const uint4 *q = (const uint4 *)p;
+    uint4 x = q[0], y = q[1];
+    v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
+    v[4] = y.x; v[5] = y.y; v[6] = y.z; v[7] = y.w;
+}
+__device__ __forceinline__ void store8(uint32_t *p, const uint32_t (&v)[kGroup])
+{
+    uint4 *q = (uint4 *)p;
+    q[0] = make_uint4(v[0], v[1], v[2], v[3]);
+    q[1] = make_uint4(v[4], v[5], v[6], v[7]);
 }
 
-__global__ void k_roots_min(SnapArgs S)
+// Flattens the forest (every cell with a core point at level k points at its
+// root) and sets compmin[root] = smallest core rank of the component (compmin
+// holds NONE on entry: k_init_parent and k_cell_labels clear it). Lanes of a
+// wave that share a root (the common case inside a large cluster) reduce
+// first, so a giant component takes one atomic per wave rather than one per
+// cell; after the two most common roots of the wave the remaining lanes,
+// spread over small components, update theirs one atomic each.
+__global__ void __launch_bounds__(kBlock) k_roots_min(SnapArgs S)
 {
-    uint32_t j = blockIdx.y, slot;
-    if (!snap_slot(S, j, &slot)) return;
-    uint32_t *parent = S.parent + (size_t)j * S.ncell, *compmin = S.compmin + (size_t)j * S.ncell;
-    const uint32_t *cmrjk = S.cmr + ((size_t)j * S.K + S.k) * S.ncell;
-    const uint8_t *ckj = S.cellkc + (size_t)j * S.ncell;
-    const uint32_t ncell = S.ncell;
-    const int k = S.k;
-    uint32_t c = blockIdx.x * kBlock + threadIdx.x;
-    uint32_t root = kNone;
+    const uint32_t g = blockIdx.y, want = snap_wanted(S, g);
+    if (!want) return;
+    uint32_t *parent = S.parent + (size_t)g * S.ncell * kGroup;
+    uint32_t *compmin = S.compmin + (size_t)g * S.ncell * kGroup;
+    const uint32_t c = blockIdx.x * kBlock + threadIdx.x;
     // a cell without a core point at level k is in no eligible pair yet, so
-    // nothing points at it and it points at itself: nothing to flatten (its
-    // parent is loaded anyway, beside its level, to keep the chain short)
-    uint32_t p = c < ncell ? ld_u32(parent + c) : 0u;
-    bool valid = c < ncell && ckj[c] <= k;
-    if (valid) {
-        uint32_t x = c;
-        while (p != x) { // read-only walk; only true roots are stored
-            x = p;
-            p = ld_u32(parent + x);
-        }
-        st_u32(parent + c, x);
-        root = x;
+    // nothing points at it and it points at itself: nothing to flatten
+    uint32_t core = 0, x[kGroup];
+    if (c < S.ncell) {
+        core = snap_core(S, g, c) & want;
+        load8(parent + cf_at(c), x);
     }
-    uint32_t v = valid ? cmrjk[c] : kNone;
-    uint64_t todo = ballot(valid);
-    for (int it = 0; it < 2 && todo; it++) {
-        int leader = __builtin_ctzll(todo);
-        uint32_t r = __shfl(root, leader);
-        bool same = valid && root == r;
-        todo &= ~ballot(same);
-        uint32_t m = same ? v : kNone;
-        for (int o = kWave / 2; o > 0; o >>= 1) {
-            uint32_t t = __shfl_xor(m, o);
-            m = t < m ? t : m;
+    // read-only walks, all values at once; only true roots are stored
+    bool moving = core != 0;
+    while (ballot(moving)) {
+        uint32_t nx[kGroup];
+#pragma unroll
+        for (int j = 0; j < kGroup; j++) {
+            nx[j] = x[j];
+            if (moving && ((core >> j) & 1u)) nx[j] = ld_u32(parent + cf_at(x[j]) + j);
         }
-        if (lane_id() == leader && m < ld_u32(compmin + r)) atomicMin(compmin + r, m);
+        bool more = false;
+#pragma unroll
+        for (int j = 0; j < kGroup; j++)
+            if ((core >> j) & 1u) {
+                more = more || nx[j] != x[j];
+                x[j] = nx[j];
+            }
+        moving = moving && more;
     }
-    if (((todo >> lane_id()) & 1ull) && v < ld_u32(compmin + root)) atomicMin(compmin + root, v);
+    if (core) store8(parent + cf_at(c), x);
+#pragma unroll
+    for (int j = 0; j < kGroup; j++) {
+        const bool valid = (core >> j) & 1u;
+        uint64_t todo = ballot(valid);
+        if (!todo) continue;
+        const uint32_t root = valid ? x[j] : kNone;
+        const uint32_t v =
+            valid ? S.cmr[((size_t)(kGroup * g + j) * S.K + S.k) * S.ncell + c] : kNone;
+        for (int it = 0; it < 2 && todo; it++) {
+            int leader = __builtin_ctzll(todo);
+            uint32_t r = __shfl(root, leader);
+            bool same = valid && root == r;
+            todo &= ~ballot(same);
+            uint32_t m = wave_min(same ? v : kNone);
+            uint32_t *at = compmin + cf_at(r) + j;
+            if (lane_id() == leader && m < ld_u32(at)) atomicMin(at, m);
+        }
+        if ((todo >> lane_id()) & 1ull) {
+            uint32_t *at = compmin + cf_at(root) + j;
+            if (v < ld_u32(at)) atomicMin(at, v);
+        }
+    }
 }
 
 // Snapshot of level k: root rank of every cell (NONE if the cell holds no
 // core point), and bit r of bits set for every root rank r.
-__global__ void k_snapshot(SnapArgs S)
+__global__ void __launch_bounds__(kBlock) k_snapshot(SnapArgs S)
 {
-    uint32_t j = blockIdx.y, slot;
-    if (!snap_slot(S, j, &slot)) return;
-    const uint32_t *parent = S.parent + (size_t)j * S.ncell;
-    const uint32_t *compmin = S.compmin + (size_t)j * S.ncell;
-    const uint8_t *ckj = S.cellkc + (size_t)j * S.ncell;
-    uint32_t *rootrank = S.root + (size_t)slot * S.ncell, *bits = S.bits + (size_t)slot * S.nw;
-    const int k = S.k;
-    uint32_t c = blockIdx.x * kBlock + threadIdx.x;
-    if (c >= S.ncell) return;
-    bool core = ckj[c] <= k;
-    uint32_t r = core ? parent[c] : c;
-    uint32_t m = core ? compmin[r] : kNone;
-    rootrank[c] = m;
-    if (core && r == c) atomicOr(bits + (m >> 5), 1u << (m & 31));
+    const uint32_t g = blockIdx.y, want = snap_wanted(S, g);
+    const uint32_t c = blockIdx.x * kBlock + threadIdx.x;
+    if (!want || c >= S.ncell) return;
+    const uint32_t *compmin = S.compmin + (size_t)g * S.ncell * kGroup;
+    const uint32_t core = snap_core(S, g, c);
+    uint32_t r[kGroup];
+    load8(S.parent + ((size_t)g * S.ncell + c) * kGroup, r);
+#pragma unroll
+    for (int j = 0; j < kGroup; j++) {
+        if (!((want >> j) & 1u)) continue;
+        const uint32_t slot = snap_slot(S, kGroup * g + j);
+        uint32_t m = (core >> j) & 1u ? compmin[cf_at(r[j]) + j] : kNone;
+        S.root[(size_t)slot * S.ncell + c] = m;
+        if (m != kNone && r[j] == c)
+            atomicOr(S.bits + (size_t)slot * S.nw + (m >> 5), 1u << (m & 31));
+    }
 }
 
 // Labels of up to kLabelSlots variants sharing minpts j, from their level
@@ -1915,22 +1938,24 @@ __device__ __forceinline__ uint32_t roots_below(const uint32_t *bits, const uint
 // root, counted from the first root of the cell's dataset (base 1: the
 // reference's numbering; 0: the standard rule's)
 // (also clears compmin for the next snapshot: it is no longer read)
-__global__ void k_cell_labels(SnapArgs S, const uint32_t *cell_ds, const uint32_t *seg,
-                              uint32_t base)
+__global__ void __launch_bounds__(kBlock)
+    k_cell_labels(SnapArgs S, const uint32_t *cell_ds, const uint32_t *seg, uint32_t base)
 {
-    uint32_t j = blockIdx.y, slot;
-    if (!snap_slot(S, j, &slot)) return;
-    const uint32_t *rootrank = S.root + (size_t)slot * S.ncell;
-    const uint32_t *bits = S.bits + (size_t)slot * S.nw, *pre = S.pre + (size_t)slot * S.nw;
-    uint32_t *celllab = S.lab + (size_t)slot * S.ncell;
-    uint32_t *compmin = S.compmin + (size_t)j * S.ncell;
-    uint32_t c = blockIdx.x * kBlock + threadIdx.x;
-    if (c >= S.ncell) return;
-    compmin[c] = kNone;
-    uint32_t rr = rootrank[c];
-    celllab[c] = rr == kNone ? 0u
-                             : roots_below(bits, pre, rr) -
-                                   roots_below(bits, pre, seg[cell_ds[c]]) + base;
+    const uint32_t g = blockIdx.y, want = snap_wanted(S, g);
+    const uint32_t c = blockIdx.x * kBlock + threadIdx.x;
+    if (!want || c >= S.ncell) return;
+    const uint32_t none[kGroup] = {kNone, kNone, kNone, kNone, kNone, kNone, kNone, kNone};
+    store8(S.compmin + ((size_t)g * S.ncell + c) * kGroup, none);
+    const uint32_t first = seg[cell_ds[c]];
+#pragma unroll
+    for (int j = 0; j < kGroup; j++) {
+        if (!((want >> j) & 1u)) continue;
+        const uint32_t slot = snap_slot(S, kGroup * g + j);
+        const uint32_t *bits = S.bits + (size_t)slot * S.nw, *pre = S.pre + (size_t)slot * S.nw;
+        uint32_t rr = S.root[(size_t)slot * S.ncell + c];
+        S.lab[(size_t)slot * S.ncell + c] =
+            rr == kNone ? 0u : roots_below(bits, pre, rr) - roots_below(bits, pre, first) + base;
+    }
 }
 
 // does a point of cell C have a neighbour list?
@@ -1946,7 +1971,7 @@ __device__ __forceinline__ bool has_list(const uint32_t *cell_start, uint32_t C,
 template <bool STD>
 __global__ void __launch_bounds__(kBlock)
     k_labels_j(LabelSlots S, const uint32_t *cell_start, const uint32_t *cell_of_pos,
-               const uint32_t *cell_ds, const uint32_t *pos_rank, const uint8_t *kc, int J, int j,
+               const uint32_t *cell_ds, const uint32_t *pos_rank, const uint8_t *kc, int JP, int j,
                const uint32_t *lst_idx, const uint8_t *lst_lev, const uint32_t *lst_id,
                const uint32_t *lst_n, int L, uint32_t n)
 {
@@ -1954,7 +1979,7 @@ __global__ void __launch_bounds__(kBlock)
     if (p >= n) return;
     uint32_t r = pos_rank[p];
     uint32_t C = cell_of_pos[p];
-    int kcp = kc[(size_t)p * J + j];
+    int kcp = kc[(size_t)p * JP + j];
     uint32_t best[kLabelSlots];
     bool any_border = false;
     int kmax = -1; // largest level of a border slot
@@ -1992,7 +2017,7 @@ __global__ void __launch_bounds__(kBlock)
 #pragma unroll
                 for (int u = 0; u < kU; u++) {
                     bool ok = se[u] <= kmax;
-                    kq[u] = ok ? (int)kc[(size_t)q[u] * J + j] : kMaxLevels;
+                    kq[u] = ok ? (int)kc[(size_t)q[u] * JP + j] : kMaxLevels;
                     cq[u] = ok ? cell_of_pos[q[u]] : 0u;
                 }
 #pragma unroll
@@ -2464,9 +2489,9 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
     // pinned read-back area of the call, written by k_report_*: [0, 8) pair
     // count, [8, 16) clique check, [32, ...) the final overflow flag, list count
     // and worklist counters
-    const size_t ncnt_all = (size_t)J * 3 * ((size_t)K + 1);
     char *hs = nullptr;
-    VDB_TRY(c.host_scratch(32 + 4 * (4 + ncnt_all + (size_t)J * (K + 1) + 1), (void **)&hs));
+    const size_t hgroups = ((size_t)J + kGroup - 1) / kGroup;
+    VDB_TRY(c.host_scratch(32 + 4 * (4 + hgroups * 4 * ((size_t)K + 1) + 1), (void **)&hs));
 
     // ---- truncated neighbour table: a list per position, so that nothing
     // counts or numbers the listed points, unless that takes more than 8 GB:
@@ -2522,15 +2547,16 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
     VDB_TRY(c.get("b.lst_id", lsz, &lst_id));
     VDB_TRY(c.get("b.lst_n", nlist_cap ? nlist_cap : 1, &lst_n));
     uint8_t *kc, *cellkc;
+    const int JP = (J + kGroup - 1) / kGroup * kGroup; // whole words of levels
     uint32_t *cmr;
-    VDB_TRY(c.get("b.kc", (size_t)n * J, &kc));
+    VDB_TRY(c.get("b.kc", (size_t)n * JP, &kc));
     // packed levels for the one-sweep label pass (J <= kAllJ, K <= kAllK)
     uint32_t *kc4 = nullptr;
     if (J <= kAllJ && K <= kAllK) VDB_TRY(c.get("b.kc4", n, &kc4));
     uint32_t *mid, *crowd;
     VDB_TRY(c.get("b.mid", n, &mid));
     VDB_TRY(c.get("b.crowd", n, &crowd));
-    const NearOut no{lst_idx, lst_id, lst_lev, lst_n, kc, kc4, (int)L, K, J, dmj};
+    const NearOut no{lst_idx, lst_id, lst_lev, lst_n, kc, kc4, (int)L, K, J, JP, dmj};
     const FG fg = fview(G);
     const unsigned gl = std::min(ceil_div(n, kWPB), kListBlocks);
     VDB_TRY(c.kt_begin("k_knn"));
@@ -2554,9 +2580,7 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
     VDB_TRY(c.kt_end("k_knn"));
     VDB_HIP(hipGetLastError());
     VDB_TRY(c.get("b.cmr", (size_t)G.ncell * J * K, &cmr));
-    VDB_TRY(c.get("b.cellkc", (size_t)G.ncell * J, &cellkc));
-    uint8_t *cellkc_cm;
-    VDB_TRY(c.get("b.cellkc_cm", (size_t)G.ncell * J, &cellkc_cm));
+    VDB_TRY(c.get("b.cellkc", (size_t)G.ncell * JP, &cellkc));
     unsigned gc0 = ceil_div(G.ncell, kBlock);
     // caller index of every position: the standard rule's key, and the label
     // pass's scatter order
@@ -2569,15 +2593,14 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
     if (std_rule) {
         uint32_t *big;
         VDB_TRY(c.get("b.bigcore", G.ncell, &big));
-        k_cell_core_std<<<gc0, kBlock, 0, c.stream()>>>(G.cell_start, G.ncell, kc, J, K,
-                                                        caller_of_pos, cmr, cellkc, cellkc_cm, big,
-                                                        bad + 4);
+        k_cell_core_std<<<gc0, kBlock, 0, c.stream()>>>(
+            G.cell_start, G.ncell, kc, J, JP, K, caller_of_pos, cmr, cellkc, big, bad + 4);
         VDB_HIP(hipGetLastError());
         k_cell_core_std_big<<<std::min(ceil_div(G.ncell, kWPB), 2048u), kBlock, 0, c.stream()>>>(
-            G.cell_start, G.ncell, kc, J, K, L, caller_of_pos, cmr, cellkc, cellkc_cm, big, bad + 4);
+            G.cell_start, G.ncell, kc, J, JP, K, L, caller_of_pos, cmr, cellkc, big, bad + 4);
     } else {
-        k_cell_core<<<gc0, kBlock, 0, c.stream()>>>(G.cell_start, G.ncell, kc, J, K, G.pos_rank,
-                                                    cmr, cellkc, cellkc_cm);
+        k_cell_core<<<gc0, kBlock, 0, c.stream()>>>(G.cell_start, G.ncell, kc, J, JP, K,
+                                                    G.pos_rank, cmr, cellkc);
     }
     VDB_HIP(hipGetLastError());
     tknn.stop();
@@ -2604,20 +2627,6 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
     VDB_TRY(c.get("b.pa", psz, &pa));
     VDB_TRY(c.get("b.pb", psz, &pb));
     VDB_TRY(c.get("b.pk", psz, &pk));
-    // test lists are filled in chunks (see kRecChunk): room for the records
-    // plus the chunks' unused slots
-    size_t tcap64 = psz + psz / 2 + (size_t)kMaxPersistent * kWPB * kRecChunk + kRecChunk;
-    if (tcap64 > 0x7fffffffull) { // the two lists' counts add up in 32 bits
-        set_error("too many cell pairs");
-        return kErrUnsupported;
-    }
-    uint32_t tcap = (uint32_t)tcap64;
-    // VDB_BATCH_TEST_CAP (records, testing only) shrinks the test lists so
-    // that the overflow fallback can be exercised on small inputs
-    if (const char *ev = getenv("VDB_BATCH_TEST_CAP")) {
-        unsigned long long v = strtoull(ev, nullptr, 10);
-        if (v > 0 && v < tcap) tcap = (uint32_t)v;
-    }
     // the cell pairs stored on the second stream too, beside the lists; the
     // main stream waits for them before the level passes
     {
@@ -2641,17 +2650,44 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
         want[{k, j}].push_back(v);
     }
     // Minpts values run side by side: every level kernel takes all minpts
-    // values of a pass at once (blockIdx.y), each with its own union-find,
-    // worklists and snapshots. A pass holds as many as the memory bound and
-    // the 32-bit sort size allow (all of them on the benchmark workloads).
+    // values of a pass at once, 8 to a group (blockIdx.y), each group with its
+    // own union-finds, worklists and snapshots. A pass holds as many as the
+    // memory bound and 32-bit list sizes allow (all of them on the benchmark
+    // workloads); passes of fewer than 8 start inside a word of core levels
+    // but never run past it.
     const uint32_t nw = (n + 31) / 32;
     const uint32_t ncnt = 3 * ((uint32_t)K + 1);
-    const size_t per_j = 8 * (size_t)G.ncell + 2 * sizeof(PairRec) * (psz + (size_t)tcap) +
-                         (16 + sizeof(PairRec)) * psz + 4 * (size_t)ncnt;
     const size_t kPassBytes = (size_t)64 << 30;
+    // test lists are filled in chunks (see kRecChunk): room for the records
+    // plus the chunks' unused slots
+    auto test_cap = [&](int j) { // records of a group's test list, j values a pass
+        return (uint64_t)std::min(j, kGroup) * (psz + psz / 2) +
+               (uint64_t)kMaxPersistent * kWPB * kRecChunk + kRecChunk;
+    };
+    auto fits = [&](int j) {
+        const uint64_t per_j =
+            8 * (uint64_t)G.ncell + 5 * sizeof(PairRec) * (uint64_t)psz + (1 + sizeof(PairRec)) * psz;
+        return test_cap(j) <= 0x7fffffffull && (uint64_t)j * psz <= 0x7fffffffull &&
+               (uint64_t)j * per_j <= kPassBytes;
+    };
     int jc = J;
-    while (jc > 1 && ((uint64_t)jc * psz > 0x7fffffffull || (size_t)jc * per_j > kPassBytes))
-        jc = (jc + 1) / 2;
+    while (jc > 1 && !fits(jc)) {
+        int half = ((jc + 1) / 2 + kGroup - 1) / kGroup * kGroup;
+        jc = jc > kGroup ? (half < jc ? half : kGroup) : jc > 4 ? 4 : jc > 2 ? 2 : 1;
+    }
+    if (test_cap(jc) > 0x7fffffffull) { // the two lists' counts add up in 32 bits
+        set_error("too many cell pairs");
+        return kErrUnsupported;
+    }
+    const int ngroups = (jc + kGroup - 1) / kGroup;
+    const size_t gcap = (size_t)std::min(jc, kGroup) * psz; // records of a group, at most
+    uint32_t tcap = (uint32_t)test_cap(jc);
+    // VDB_BATCH_TEST_CAP (records, testing only) shrinks the test lists so
+    // that the overflow fallback can be exercised on small inputs
+    if (const char *ev = getenv("VDB_BATCH_TEST_CAP")) {
+        unsigned long long v = strtoull(ev, nullptr, 10);
+        if (v > 0 && v < tcap) tcap = (uint32_t)v;
+    }
     // snapshot slots: at most one per requested (k, j) of a pass
     size_t max_slots = 1;
     for (int j0 = 0; j0 < J; j0 += jc) {
@@ -2660,36 +2696,24 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
             if (w.first.second >= j0 && w.first.second < j0 + jc) ns++;
         max_slots = std::max(max_slots, ns);
     }
-    uint32_t *parent, *compmin, *ekey, *eval, *stk, *stv, *bstart;
-    VDB_TRY(c.get("b.parent", (size_t)jc * G.ncell, &parent));
-    VDB_TRY(c.get("b.compmin", (size_t)jc * G.ncell, &compmin));
-    VDB_TRY(c.get("b.la", (size_t)jc * psz, &la));
-    VDB_TRY(c.get("b.lb", (size_t)jc * psz, &lb));
-    VDB_TRY(c.get("b.tests", (size_t)jc * tcap, &tests));
-    VDB_TRY(c.get("b.tests2", (size_t)jc * tcap, &tests2));
-    VDB_TRY(c.get("b.cnts", (size_t)jc * ncnt, &cnts));
+    uint32_t *parent, *compmin, *bstart;
+    VDB_TRY(c.get("b.parent", (size_t)ngroups * G.ncell * kGroup, &parent));
+    VDB_TRY(c.get("b.compmin", (size_t)ngroups * G.ncell * kGroup, &compmin));
+    VDB_TRY(c.get("b.la", ngroups * gcap, &la));
+    VDB_TRY(c.get("b.lb", ngroups * gcap, &lb));
+    VDB_TRY(c.get("b.tests", (size_t)ngroups * tcap, &tests));
+    VDB_TRY(c.get("b.tests2", (size_t)ngroups * tcap, &tests2));
+    VDB_TRY(c.get("b.cnts", (size_t)ngroups * ncnt, &cnts));
     // eligibility levels: a byte per (pair, minpts value), planes of 8
-    const size_t nplanes = ((size_t)jc + kEligGroup - 1) / kEligGroup;
     uint2 *plev;
-    VDB_TRY(c.get("b.lev", nplanes * psz * 2, (uint32_t **)&plev));
-    // passes of up to kPairBuckets (minpts, level) buckets scatter the
-    // records by tile counts; larger ones radix-sort keys and values
-    const bool pair_scatter = (size_t)jc * (K + 1) <= (size_t)kPairBuckets;
+    VDB_TRY(c.get("b.lev", (size_t)ngroups * psz * 2, (uint32_t **)&plev));
     const unsigned ptiles = ceil_div(std::max<size_t>(psz, 1), kEligTile);
     uint32_t *phist = nullptr, *poffs = nullptr;
-    ekey = eval = stk = stv = nullptr;
-    if (pair_scatter) {
-        VDB_TRY(c.get("b.phist", (size_t)jc * (K + 1) * ptiles, &phist));
-        VDB_TRY(c.get("b.poffs", (size_t)jc * (K + 1) * ptiles, &poffs));
-    } else {
-        VDB_TRY(c.get("b.ekey", (size_t)jc * psz, &ekey));
-        VDB_TRY(c.get("b.eval", (size_t)jc * psz, &eval));
-        VDB_TRY(c.get("b.stk", (size_t)jc * psz, &stk));
-        VDB_TRY(c.get("b.stv", (size_t)jc * psz, &stv));
-    }
-    PairRec *frec; // pair records sorted by (minpts value, level)
-    VDB_TRY(c.get("b.frec", (size_t)jc * psz, &frec));
-    VDB_TRY(c.get("b.bstart", (size_t)jc * (K + 1) + 2, &bstart));
+    VDB_TRY(c.get("b.phist", (size_t)ngroups * (K + 1) * ptiles, &phist));
+    VDB_TRY(c.get("b.poffs", (size_t)ngroups * (K + 1) * ptiles, &poffs));
+    PairRec *frec; // pair records sorted by (group, level)
+    VDB_TRY(c.get("b.frec", ngroups * gcap, &frec));
+    VDB_TRY(c.get("b.bstart", (size_t)ngroups * (K + 1) + 2, &bstart));
     // per-slot snapshots: cell root ranks, cell labels, the root ranks as a
     // bitset over ranks with its per-word prefix counts (cluster ids)
     uint32_t *snap_root, *snap_lab, *snap_bits, *snap_pre;
@@ -2774,62 +2798,39 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
             std::vector<uint32_t> sbase(K + 1, 0);
             for (int k = 0; k < K; k++) sbase[k + 1] = sbase[k] + (uint32_t)__builtin_popcountll(jmask[k]);
             size_t nslot = sbase[K];
-            k_init_parent<<<dim3(gc, nj), kBlock, 0, c.stream()>>>(
-                parent, compmin, G.ncell, cnts, (size_t)nj * ncnt, snap_bits, nslot * nw);
+            const int ng = (nj + kGroup - 1) / kGroup;
+            k_init_parent<<<dim3(gc, ng), kBlock, 0, c.stream()>>>(
+                parent, compmin, G.ncell, cnts, (size_t)ng * ncnt, snap_bits, nslot * nw);
             VDB_HIP(hipGetLastError());
-            // pairs bucketed by (minpts value, level at which they become
-            // eligible): bucket j*(K+1)+k of bstart
-            const uint32_t nb = (uint32_t)nj * (uint32_t)(K + 1);
+            // records bucketed by (group, level at which they become
+            // eligible): bucket g*(K+1)+k of bstart
+            const uint32_t nb = (uint32_t)ng * (uint32_t)(K + 1);
 
             if (npairs) {
                 // eligibility tiles of this pass (npairs <= psz)
                 const unsigned tiles = ceil_div(npairs, kEligTile);
-                uint32_t *hist = pair_scatter ? phist : nullptr;
-                for (int g0 = 0; g0 < nj; g0 += kEligGroup) {
-                    int gn = std::min(kEligGroup, nj - g0);
-                    uint2 *plane = plev + (size_t)(g0 / kEligGroup) * npairs;
+                for (int g = 0; g < ng; g++) {
                     VDB_TRY(c.kt_begin("k_pair_elig"));
-                    if (K <= 16)
-                        k_pair_elig<4><<<tiles, kBlock, 0, c.stream()>>>(
-                            pa, pb, pk, cellkc_cm, G.cell_start, G.xs, G.ys, kc, dTk, J, j0 + g0,
-                            gn, K, npairs, (uint32_t)g0, plane, hist, tiles);
-                    else
-                        k_pair_elig<7><<<tiles, kBlock, 0, c.stream()>>>(
-                            pa, pb, pk, cellkc_cm, G.cell_start, G.xs, G.ys, kc, dTk, J, j0 + g0,
-                            gn, K, npairs, (uint32_t)g0, plane, hist, tiles);
+                    k_pair_elig<<<tiles, kBlock, 0, c.stream()>>>(
+                        pa, pb, pk, cellkc, G.cell_start, G.xs, G.ys, kc, dTk, JP, j0 + g * kGroup,
+                        std::min(kGroup, nj - g * kGroup), K, npairs, (uint32_t)g,
+                        plev + (size_t)g * npairs, phist, tiles);
                     VDB_TRY(c.kt_end("k_pair_elig"));
                     VDB_HIP(hipGetLastError());
                 }
-                if (pair_scatter) {
-                    // tile counts -> every tile's first slot in every bucket,
-                    // then the records in (minpts value, level) order
-                    VDB_TRY(scan_exclusive_u32(c, phist, poffs, (size_t)nb * tiles, nullptr));
+                // tile counts -> every tile's first slot in every bucket, then
+                // the records in (group, level) order
+                VDB_TRY(scan_exclusive_u32(c, phist, poffs, (size_t)nb * tiles, nullptr));
+                for (int g = 0; g < ng; g++) {
                     VDB_TRY(c.kt_begin("k_pair_scatter"));
-                    if (K <= 16)
-                        k_pair_scatter<4><<<ceil_div(npairs, kPairTile), kBlock, 0, c.stream()>>>(
-                            pa, pb, pk, plev, npairs, nj, K, poffs, tiles, frec);
-                    else
-                        k_pair_scatter<7><<<ceil_div(npairs, kPairTile), kBlock, 0, c.stream()>>>(
-                            pa, pb, pk, plev, npairs, nj, K, poffs, tiles, frec);
+                    k_pair_scatter<<<ceil_div(tiles, kPairItems), kBlock, 0, c.stream()>>>(
+                        pa, pb, pk, plev + (size_t)g * npairs, npairs, K, (uint32_t)g, poffs, tiles,
+                        frec);
                     VDB_TRY(c.kt_end("k_pair_scatter"));
                     VDB_HIP(hipGetLastError());
-                    k_pair_bounds<<<1, kBlock, 0, c.stream()>>>(poffs, phist, tiles, (int)nb,
-                                                                 bstart);
-                    VDB_HIP(hipGetLastError());
-                } else {
-                    uint32_t nkeys = (uint32_t)nj * npairs;
-                    k_level_keys<<<ceil_div(npairs, kBlock), kBlock, 0, c.stream()>>>(
-                        plev, npairs, nj, K, ekey, eval);
-                    VDB_HIP(hipGetLastError());
-                    uint32_t *sk, *sv;
-                    VDB_TRY(radix_sort_pairs(c, ekey, eval, stk, stv, nkeys, bits_for(nb), &sk, &sv));
-                    k_bucket_starts<<<ceil_div((size_t)nkeys + 1, kBlock), kBlock, 0, c.stream()>>>(
-                        sk, nkeys, (int)nb - 1, bstart);
-                    VDB_HIP(hipGetLastError());
-                    k_pack_records<<<ceil_div(nkeys, kBlock), kBlock, 0, c.stream()>>>(
-                        sv, pa, pb, pk, nkeys, frec);
-                    VDB_HIP(hipGetLastError());
                 }
+                k_pair_bounds<<<1, kBlock, 0, c.stream()>>>(poffs, phist, tiles, (int)nb, bstart);
+                VDB_HIP(hipGetLastError());
             } else {
                 k_fill_u32<<<ceil_div((size_t)nb + 1, kBlock), kBlock, 0, c.stream()>>>(bstart, 0u,
                                                                                        nb + 1);
@@ -2838,55 +2839,55 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
             PairRec *lin = la, *lout = lb;
             for (int k = 0; k <= kmax; k++) {
                 LevelArgs a{G.xs, G.ys, G.cell_box, G.cell_start, G.cell_key, G.cell_ds, G.skbase,
-                            G.sncy, (uint32_t)G.m, kc, pa, pb, pk, J, j0, k, Th[k]};
+                            G.sncy, (uint32_t)G.m, kc, JP, j0, k, Th[k]};
                 LevelLists LL{parent, lin, lout, tests, tests2, cnts, frec, bstart,
-                              psz, G.ncell, tcap, (uint32_t)K, tovf, shape.ppb, shape.minb,
+                              gcap, G.ncell, tcap, (uint32_t)K, tovf, shape.ppb, shape.minb,
                               shape.tpb};
                 // worklist sizes stay on the device: bounded grids stride over them
                 VDB_TRY(c.kt_begin("k_sweep"));
-                k_sweep<<<dim3(shape.maxb, nj), kBlock, 0, c.stream()>>>(a, LL);
+                k_sweep<<<dim3(shape.maxb, ng), kBlock, 0, c.stream()>>>(a, LL);
                 VDB_TRY(c.kt_end("k_sweep"));
                 VDB_HIP(hipGetLastError());
                 VDB_TRY(c.kt_begin("k_test"));
-                k_test<<<dim3(shape.maxtb, nj), kBlock, 0, c.stream()>>>(a, LL);
+                k_test<<<dim3(shape.maxtb, ng), kBlock, 0, c.stream()>>>(a, LL);
                 VDB_TRY(c.kt_end("k_test"));
                 VDB_HIP(hipGetLastError());
                 if (verbose) {
                     // worklist sizes of this level (a sync per level: verbose only)
-                    std::vector<uint32_t> hc((size_t)nj * ncnt), hb(nb + 1);
+                    std::vector<uint32_t> hc((size_t)ng * ncnt), hb(nb + 1);
                     VDB_HIP(hipMemcpyAsync(hc.data(), cnts, sizeof(uint32_t) * hc.size(),
                                            hipMemcpyDeviceToHost, c.stream()));
                     VDB_HIP(hipMemcpyAsync(hb.data(), bstart, sizeof(uint32_t) * hb.size(),
                                            hipMemcpyDeviceToHost, c.stream()));
                     VDB_HIP(hipStreamSynchronize(c.stream()));
-                    for (int jr = 0; jr < nj; jr++) {
-                        const uint32_t *h = hc.data() + (size_t)jr * ncnt;
-                        uint32_t b0 = (uint32_t)jr * (K + 1) + k;
-                        printf("\n[vdbscan] batch j=%d k=%d: %u fresh, %u near + %u far tests, "
-                               "%u carried on",
-                               j0 + jr, k, hb[b0 + 1] - hb[b0], h[K + 1 + k], h[2 * (K + 1) + k],
-                               h[k + 1]);
+                    for (int g = 0; g < ng; g++) {
+                        const uint32_t *h = hc.data() + (size_t)g * ncnt;
+                        uint32_t b0 = (uint32_t)g * (K + 1) + k;
+                        printf("\n[vdbscan] batch group of minpts %d.. k=%d: %u fresh, %u near + %u "
+                               "far tests, %u carried on",
+                               j0 + g * kGroup, k, hb[b0 + 1] - hb[b0], h[K + 1 + k],
+                               h[2 * (K + 1) + k], h[k + 1]);
                     }
                 }
                 std::swap(lin, lout);
                 if (!jmask[k]) continue;
                 // snapshots of level k: component roots, their smallest core
                 // rank, cluster ids in ascending root rank
-                SnapArgs S{parent, compmin, cmr + (size_t)j0 * K * G.ncell, cellkc + (size_t)j0 * G.ncell,
+                SnapArgs S{parent, compmin, cmr + (size_t)j0 * K * G.ncell, cellkc,
                            snap_root, snap_lab, snap_bits, snap_pre, jmask[k], sbase[k], G.ncell, nw,
-                           (uint32_t)K, k};
+                           (uint32_t)K, k, JP, j0};
                 VDB_TRY(c.kt_begin("k_roots_min"));
-                k_roots_min<<<dim3(gc, nj), kBlock, 0, c.stream()>>>(S);
+                k_roots_min<<<dim3(gc, ng), kBlock, 0, c.stream()>>>(S);
                 VDB_TRY(c.kt_end("k_roots_min"));
                 VDB_HIP(hipGetLastError());
-                k_snapshot<<<dim3(gc, nj), kBlock, 0, c.stream()>>>(S);
+                k_snapshot<<<dim3(gc, ng), kBlock, 0, c.stream()>>>(S);
                 VDB_HIP(hipGetLastError());
                 // one scan over the level's slots: a slot's counts start at the
                 // slots before it, an offset the label passes subtract away
                 size_t ns_k = sbase[k + 1] - sbase[k];
                 VDB_TRY(scan_popc_u32(c, snap_bits + (size_t)sbase[k] * nw,
                                       snap_pre + (size_t)sbase[k] * nw, ns_k * nw));
-                k_cell_labels<<<dim3(gc, nj), kBlock, 0, c.stream()>>>(S, G.cell_ds, P.seg,
+                k_cell_labels<<<dim3(gc, ng), kBlock, 0, c.stream()>>>(S, G.cell_ds, P.seg,
                                                                        std_rule ? 0u : 1u);
                 VDB_HIP(hipGetLastError());
             }
@@ -2971,13 +2972,13 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
                     if (std_rule) {
                         VDB_TRY(c.kt_begin("k_labels_j"));
                         k_labels_j<true><<<gn, kBlock, 0, c.stream()>>>(
-                            S, G.cell_start, G.cell_of_pos, G.cell_ds, G.pos_rank, kc, J, j, lst_idx,
+                            S, G.cell_start, G.cell_of_pos, G.cell_ds, G.pos_rank, kc, JP, j, lst_idx,
                             lst_lev, lst_id, lst_n, (int)L, n);
                         VDB_TRY(c.kt_end("k_labels_j"));
                     } else {
                         VDB_TRY(c.kt_begin("k_labels_j"));
                         k_labels_j<false><<<gn, kBlock, 0, c.stream()>>>(
-                            S, G.cell_start, G.cell_of_pos, G.cell_ds, G.pos_rank, kc, J, j, lst_idx,
+                            S, G.cell_start, G.cell_of_pos, G.cell_ds, G.pos_rank, kc, JP, j, lst_idx,
                             lst_lev, lst_id, lst_n, (int)L, n);
                         VDB_TRY(c.kt_end("k_labels_j"));
                     }
@@ -3000,7 +3001,7 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
     // runs the sequence once per grid shape of kBatchShapes and keeps the
     // fastest; the choice persists in the tuning cache.
     char tkey[160];
-    snprintf(tkey, sizeof tkey, "batch:%u:%u:%d:%d:%u:%d:%d", n, P.nsets, K, J, L,
+    snprintf(tkey, sizeof tkey, "batch:g8:%u:%u:%d:%d:%u:%d:%d", n, P.nsets, K, J, L,
              bits_for((uint64_t)G.ncell + 1), bits_for((uint64_t)npairs + 1));
     int shape_id = 0;
     bool tuned_now = false;
@@ -3021,7 +3022,7 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
             c.tuned_put(tkey, shape_id);
         }
     }
-    const BatchShape &shape = kBatchShapes[shape_id];
+    BatchShape shape = kBatchShapes[shape_id];
     if (res) res->shape = shape_id;
     Ev tuf(c.stream(), st != nullptr);
     double ms_labels = 0;
@@ -3051,11 +3052,12 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
     // all minpts values ran in one pass, whose counters are still in place)
     // the worklist counters, for the byte model of the level kernels
     const bool counters = jc == J && npairs;
+    const uint32_t ncnt_all = (uint32_t)ngroups * ncnt, nbst = (uint32_t)ngroups * (K + 1) + 1;
     uint32_t *hc = (uint32_t *)(hs + 32 + 8);
     uint32_t *hb = hc + ncnt_all;
     k_report_final<<<1, kBlock, 0, c.stream()>>>(bad, tovf, cnts,
-                                                 counters ? (uint32_t)ncnt_all : 0u, bstart,
-                                                 counters ? (uint32_t)(J * (K + 1) + 1) : 0u,
+                                                 counters ? ncnt_all : 0u, bstart,
+                                                 counters ? nbst : 0u,
                                                  (uint32_t *)(hs + 32));
     VDB_HIP(hipGetLastError());
     VDB_TRY(c.wait(c.stream()));
@@ -3084,10 +3086,10 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
     if (counters) {
         int kmax = -1;
         for (auto &w : want) kmax = std::max(kmax, w.first.first);
-        for (int j = 0; j < J; j++) {
-            const uint32_t *h = hc + (size_t)j * ncnt;
+        for (int g = 0; g < ngroups; g++) {
+            const uint32_t *h = hc + (size_t)g * ncnt;
             for (int k = 0; k <= kmax; k++) {
-                size_t b0 = (size_t)j * (K + 1) + k;
+                size_t b0 = (size_t)g * (K + 1) + k;
                 nfresh_all += hb[b0 + 1] - hb[b0];
                 ncarried_all += h[k];
                 ntests_all += (uint64_t)h[K + 1 + k] + h[2 * (K + 1) + k];

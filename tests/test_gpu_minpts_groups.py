@@ -1,7 +1,8 @@
 """Batched engine around its groups of 8 minpts values: one, a full group, one
 beyond it and two groups and one, with values that make every point core (1)
 and none (above the point count), on points whose levels leave pairs open from
-one level to the next. Labels are the oracle's."""
+one level to the next; and cell pairs of few points around the sizes at which
+they are looked at one by one. Labels are the oracle's."""
 import numpy as np
 import pytest
 
@@ -33,6 +34,27 @@ def test_minpts_groups(points, nmp, levels):
     eps = np.repeat(E, nmp)
     mp = np.tile(np.array(MINPTS[:nmp], dtype=np.uint32), levels)
     print("12k points, %d minpts values x %d levels" % (nmp, levels), flush=True)
+    got = vd.cluster(x, y, eps, mp, path=vd.PATH_BATCH)
+    want = oracle.libvdbscan(x, y, eps, mp)
+    for v in range(len(eps)):
+        assert (got[v] == want[v]).all(), (eps[v], mp[v])
+
+
+@pytest.mark.parametrize("m", [1, 2, 3, 4, 5, 9])
+def test_cells_of_few_points(m):
+    # tight knots of 1..m points on a jittered lattice of about eps spacing:
+    # pairs of 1 x 1 up to m x m points, near the thresholds of every level
+    r = np.random.default_rng(70 + m)
+    gx, gy = np.meshgrid(np.arange(40) * 0.5, np.arange(37) * 0.5)
+    cx = gx.ravel() + r.uniform(-0.06, 0.06, gx.size)
+    cy = gy.ravel() + r.uniform(-0.06, 0.06, gy.size)
+    rep = r.integers(1, m + 1, cx.size)
+    x, y = np.repeat(cx, rep), np.repeat(cy, rep)
+    x = x + r.uniform(-0.05, 0.05, x.size)
+    y = y + r.uniform(-0.05, 0.05, y.size)
+    eps = np.repeat([0.45, 0.5, 0.52, 0.6], 3)
+    mp = np.tile(np.array([2, m + 2, 2 * m + 3], dtype=np.uint32), 4)
+    print("knots of 1..%d points" % m, flush=True)
     got = vd.cluster(x, y, eps, mp, path=vd.PATH_BATCH)
     want = oracle.libvdbscan(x, y, eps, mp)
     for v in range(len(eps)):

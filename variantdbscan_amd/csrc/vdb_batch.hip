@@ -42,7 +42,7 @@ constexpr uint32_t kNone = 0xffffffffu;
 constexpr int kMaxList = 64;
 constexpr int kMaxLevels = 64;
 constexpr int kMaxMinpts = 64;
-// pairs whose cells hold at most this many point pairs are tested by one thread
+// pairs whose cells hold at most this many point pairs get exact levels
 constexpr uint32_t kSmallPairWork = 16;
 // Grids of the worklist kernels, whose sizes live on the device (one grid
 // row per minpts value): the sweep takes one block per `ppb` pairs becoming
@@ -930,91 +930,58 @@ __device__ __forceinline__ void pair_levels(const double *A, const double *B, co
     *kfull = b;
 }
 
-// Pairs (A, B > A) that some eps level may connect, counted per cell A with
-// a thread per cell (the same acceptance test as k_pairs below, which stores
-// them).
-__global__ void k_pair_count(const double *box, const uint32_t *row_lo, const uint32_t *row_hi,
-                             int W, uint32_t ncell, const double *Tk, int K, uint32_t *cnt)
+// Cell pairs (A, B > A) that some eps level may connect: f(B, kmin, kfull) for
+// each, in row order, B ascending within a row.
+struct CellPair {
+    uint32_t a, b, k; // k = kmin | kfull << 8
+};
+template <typename F>
+__device__ __forceinline__ void walk_pairs(const double *box, const uint32_t *row_lo,
+                                           const uint32_t *row_hi, int W, uint32_t A,
+                                           const double *Tk, int K, F f)
 {
-    uint32_t A = blockIdx.x * kBlock + threadIdx.x;
-    if (A >= ncell) return;
-    const double *bA = box + 4 * (size_t)A;
-    uint32_t k = 0;
+    double bA[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) bA[i] = box[4 * (size_t)A + i];
     for (int r = 0; r < W; r++) {
         uint32_t lo = row_lo[(size_t)A * W + r], hi = row_hi[(size_t)A * W + r];
         if (lo <= A) lo = A + 1;
         for (uint32_t B = lo; B < hi; B++) {
             int kmin, kfull;
             pair_levels(bA, box + 4 * (size_t)B, Tk, K, &kmin, &kfull);
-            k += kmin < K ? 1u : 0u;
+            if (kmin < K) f(B, kmin, kfull);
         }
     }
+}
+
+__global__ void __launch_bounds__(kBlock)
+    k_pair_count(const double *box, const uint32_t *row_lo, const uint32_t *row_hi, int W,
+                 uint32_t ncell, const double *Tk, int K, uint32_t *cnt)
+{
+    const uint32_t A = blockIdx.x * kBlock + threadIdx.x;
+    if (A >= ncell) return;
+    uint32_t k = 0;
+    walk_pairs(box, row_lo, row_hi, W, A, Tk, K, [&](uint32_t, int, int) { k++; });
     cnt[A] = k;
 }
 
-// Cell pairs (A, B > A) that some eps level may connect: a wave per cell A.
-// Lane r < W holds window row r's run of cells after A; a scan of the run
-// lengths flattens the window, and each step the lanes take the next 64
-// candidates in row order (a lane finds its row by binary search over the
-// scanned run ends). Accepted pairs of A are stored in row order, B
-// ascending within a row, by one ballot-compacted store per step (a thread
-// per cell, storing its own run, made 64 scattered stores per instruction).
-// A's share of the output starts at off[A] (k_pair_count, scanned). Needs
-// W <= 64.
+// A's pairs are stored from off[A] on (k_pair_count, scanned), a thread per
+// cell as in the count, 12 bytes to a store. Cells of a wave lie side by side,
+// so their stores fill the same lines in L2 soon after one another. 75M pairs
+// of 256 datasets take 1.97 ms beside the neighbour search, 1.4M of one
+// variant 45 us. (A wave per cell over its flattened window: 6.96 ms and 217
+// us. Stores compacted over the wave's 64 cells: 0.97 ms and 28 us, but the
+// sweep wants a cell's pairs together: 4.1 ms for 3.1.)
 __global__ void __launch_bounds__(kBlock)
     k_pairs(const double *box, const uint32_t *row_lo, const uint32_t *row_hi, int W,
-            uint32_t ncell, const double *Tk, int K, const uint64_t *off, uint32_t *pa,
-            uint32_t *pb, uint16_t *pk)
+            uint32_t ncell, const double *Tk, int K, const uint64_t *off, CellPair *out)
 {
-    uint32_t A = blockIdx.x * kWPB + wave_id_in_block();
-    if (A >= ncell) return; // wave-uniform
-    int lane = lane_id();
-    uint32_t lo = 0, len = 0;
-    if (lane < W) {
-        uint32_t l = row_lo[(size_t)A * W + lane], h = row_hi[(size_t)A * W + lane];
-        if (l <= A) l = A + 1;
-        lo = l;
-        len = h > l ? h - l : 0u;
-    }
-    uint32_t incl = len;
-    for (int o = 1; o < kWave; o <<= 1) {
-        uint32_t t = __shfl_up(incl, o);
-        if (lane >= o) incl += t;
-    }
-    uint32_t excl = incl - len;
-    uint32_t total = __shfl(incl, kWave - 1);
-    const double *bA = box + 4 * (size_t)A;
-    uint64_t o = off[A];
-    uint32_t k = 0;
-    for (uint32_t t0 = 0; t0 < total; t0 += kWave) {
-        uint32_t t = t0 + (uint32_t)lane;
-        // row of t: the first row whose run ends after t (6 halvings cover
-        // 64 rows; every lane shuffles, finished or not)
-        int rlo = 0, rhi = W - 1;
-#pragma unroll
-        for (int step = 0; step < 6; step++) {
-            int mid = (rlo + rhi) >> 1;
-            uint32_t im = __shfl(incl, mid);
-            if (rlo < rhi) {
-                if (im > t) rhi = mid;
-                else rlo = mid + 1;
-            }
-        }
-        uint32_t rs = __shfl(excl, rlo), rl = __shfl(lo, rlo);
-        bool v = t < total;
-        uint32_t B = rl + (t - rs);
-        int kmin = K, kfull = K;
-        if (v) pair_levels(bA, box + 4 * (size_t)B, Tk, K, &kmin, &kfull);
-        bool acc = v && kmin < K;
-        uint64_t m = ballot(acc);
-        if (acc) {
-            uint64_t d = o + k + (uint32_t)mask_rank(m);
-            pa[d] = A;
-            pb[d] = B;
-            pk[d] = (uint16_t)(kmin | (kfull << 8));
-        }
-        k += (uint32_t)popc64(m);
-    }
+    const uint32_t A = blockIdx.x * kBlock + threadIdx.x;
+    if (A >= ncell) return;
+    out += off[A];
+    walk_pairs(box, row_lo, row_hi, W, A, Tk, K, [&](uint32_t B, int kmin, int kfull) {
+        *out++ = CellPair{A, B, (uint32_t)(kmin | (kfull << 8))};
+    });
 }
 
 // For every group of minpts values (blockIdx.y): each cell its own parent and
@@ -1113,17 +1080,29 @@ __device__ __forceinline__ uint64_t level_word(const uint8_t *row, int j)
 // For pairs of small cells (at most kSmallPairWork point pairs) the level is
 // exact instead: the first level at which some core-core pair is within eps,
 //   min over (p, q) of max(level(s(p,q)), kc_j(p), kc_j(q)),
-// flagged so that the sweep unites them without a test. The point distances
-// are computed once for the whole group.
+// flagged so that the sweep unites them without a test. From kfull on every
+// point pair is within eps and the first formula is exact already, so only
+// values below kfull look at points, and their levels lie in [kmin, kfull].
+//
+// A block takes kEligTiles tiles of kBlock pairs. Its first pass gives every
+// pair its box level and queues those that must look at points, the light
+// ones (at most kLightPairWork point pairs) from the front and the others from
+// the back; the second takes the queue, so that a wave's lanes all have such a
+// pair and of like size. What bounds it are the gathers of the second pass.
+// 75M pairs of 256 datasets: 1.87 ms (3.29 with every pair on its own lane and
+// no bound at kfull), 11.6M pairs of 2M points x 64 variants 236 us (396);
+// one tile to a block 2.52 and 298, four 1.74 and 223 but 32 us for 22 where
+// blocks are few (50,000 points x 16). With kSmallPairWork 32 the test kernel
+// of the 256 datasets saves 0.7 ms and this one costs 1.1 more.
 //
 // Output: byte g of lev[i] = level | exact << 7 (levels stay below 64), bytes
-// of minpts values beyond nj K. The kernel also counts its tile's records for
-// the scatter: tile t = the kBlock consecutive pairs of block t (a pair per
-// thread: the eligibility tests are latency-bound, so every pair gets its own
-// lane), one record per distinct level of a pair, hist[(group*(K+1) + level) *
-// tiles + t] (bucket-major, so that an exclusive scan gives every tile's first
-// slot in every bucket); the buckets of level K stay empty.
+// of minpts values beyond nj K. The kernel also counts each tile's records for
+// the scatter: one record per distinct level of a pair, hist[(group*(K+1) +
+// level) * tiles + t] (bucket-major, so that an exclusive scan gives every
+// tile's first slot in every bucket); the buckets of level K stay empty.
 constexpr uint32_t kEligTile = kBlock;
+constexpr int kEligTiles = 2; // tiles a block of the eligibility kernel takes
+constexpr uint32_t kLightPairWork = 4;
 // the scatter takes kPairItems eligibility tiles per block
 constexpr int kPairItems = 8;
 
@@ -1139,94 +1118,174 @@ __device__ __forceinline__ uint64_t levels_present(uint2 w, int K)
     return m;
 }
 
-__global__ void __launch_bounds__(kBlock)
-    k_pair_elig(const uint32_t *pa, const uint32_t *pb, const uint16_t *pk, const uint8_t *cellkc,
-                const uint32_t *cell_start, const double *xs, const double *ys, const uint8_t *kc,
-                const double *Tk, int JP, int j0, int nj, int K, uint32_t npairs, uint32_t group,
-                uint2 *lev, uint32_t *hist, unsigned tiles)
+// 8 levels as packed 16-bit values
+typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+struct Lev8 {
+    us2 v[4];
+};
+__device__ __forceinline__ Lev8 lev8(uint64_t w)
 {
+    Lev8 r;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        uint32_t h = (uint32_t)(i < 2 ? w : w >> 32);
+        uint32_t u = __builtin_amdgcn_perm(0u, h, i & 1 ? 0x0c030c02u : 0x0c010c00u);
+        r.v[i] = __builtin_bit_cast(us2, u);
+    }
+    return r;
+}
+__device__ __forceinline__ Lev8 lev8_all(uint32_t l)
+{
+    us2 x = {(unsigned short)l, (unsigned short)l};
+    return Lev8{{x, x, x, x}};
+}
+__device__ __forceinline__ Lev8 lev8_max(Lev8 a, const Lev8 &b, uint32_t l)
+{
+    const us2 x = {(unsigned short)l, (unsigned short)l};
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        a.v[i] = __builtin_elementwise_max(__builtin_elementwise_max(a.v[i], b.v[i]), x);
+    return a;
+}
+__device__ __forceinline__ Lev8 lev8_min(Lev8 a, const Lev8 &b)
+{
+#pragma unroll
+    for (int i = 0; i < 4; i++) a.v[i] = __builtin_elementwise_min(a.v[i], b.v[i]);
+    return a;
+}
+__device__ __forceinline__ bool lev8_same(const Lev8 &a, const Lev8 &b)
+{
+    uint32_t d = 0;
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        d |= __builtin_bit_cast(uint32_t, a.v[i]) ^ __builtin_bit_cast(uint32_t, b.v[i]);
+    return d == 0;
+}
+
+__global__ void __launch_bounds__(kBlock)
+    k_pair_elig(const CellPair *pairs, const uint8_t *cellkc, const uint32_t *cell_start,
+                const double *xs, const double *ys, const uint8_t *kc, const double *Tk, int JP,
+                int j0, int nj, int K, uint32_t npairs, uint32_t group, uint2 *lev, uint32_t *hist,
+                unsigned tiles)
+{
+    constexpr uint32_t kSpan = kEligTiles * kEligTile;
+    __shared__ uint2 words[kSpan];
+    __shared__ uint16_t queue[kSpan]; // light pairs from the front, others from the back
+    __shared__ uint32_t nq[2];
     __shared__ uint32_t h[kWPB][kMaxLevels];
     __shared__ double sTk[kMaxLevels]; // level thresholds for the exact levels
     for (int k = threadIdx.x; k < K; k += kBlock) sTk[k] = Tk[k];
+    if (threadIdx.x < 2) nq[threadIdx.x] = 0;
     __syncthreads();
     const int w = threadIdx.x / kWave, lane = lane_id();
-    uint32_t i = blockIdx.x * kEligTile + threadIdx.x;
-    bool valid = i < npairs;
-    int e[kGroup];
+    const uint32_t t0 = blockIdx.x * kSpan;
+    const uint32_t K4 = (uint32_t)K * 0x01010101u;
+    // bytes of minpts values beyond nj become K
+    const uint64_t beyond = nj < kGroup ? ~0ull << (8 * nj) : 0ull;
+    auto bytes = [&](const Lev8 &e, bool exact) {
+        uint32_t q[2];
 #pragma unroll
-    for (int g = 0; g < kGroup; g++) e[g] = K;
-    uint32_t exact = 0; // bit g: level of j0+g computed exactly
-    uint2 word = make_uint2(0x7f7f7f7fu, 0x7f7f7f7fu);
-    if (valid) {
-        uint32_t A = pa[i], B = pb[i];
-        int e0 = pk[i] & 0xff;
-        uint32_t a0 = cell_start[A], a1 = cell_start[A + 1];
-        uint32_t b0 = cell_start[B], b1 = cell_start[B + 1];
-        bool small = (uint64_t)(a1 - a0) * (b1 - b0) <= kSmallPairWork;
+        for (int u = 0; u < 2; u++) {
+            uint32_t lo = __builtin_bit_cast(uint32_t, e.v[2 * u]);
+            uint32_t hi = __builtin_bit_cast(uint32_t, e.v[2 * u + 1]);
+            q[u] = __builtin_amdgcn_perm(hi, lo, 0x06040200u);
+            uint32_t m = (uint32_t)(beyond >> (32 * u));
+            q[u] = (q[u] & ~m) | (K4 & m);
+            if (exact) {
+                // levels are at most K < 128: a byte below K borrows nothing
+                // from its 0x80 + K and keeps the top bit
+                uint32_t below = ((K4 | 0x80808080u) - 0x01010101u - q[u]) & 0x80808080u;
+                q[u] |= below;
+            }
+        }
+        return make_uint2(q[0], q[1]);
+    };
+    auto first_of = [&](const CellPair &pr) {
         // a cell's levels for all minpts values lie side by side
-        uint64_t wa = level_word(cellkc + (size_t)A * JP, j0);
-        uint64_t wb = level_word(cellkc + (size_t)B * JP, j0);
+        Lev8 f = lev8_max(lev8(level_word(cellkc + (size_t)pr.a * JP, j0)),
+                          lev8(level_word(cellkc + (size_t)pr.b * JP, j0)), pr.k & 0xffu);
+        return lev8_min(f, lev8_all(K));
+    };
 #pragma unroll
-        for (int g = 0; g < kGroup; g++) {
-            if (g < nj) {
-                int v = e0;
-                int ca = (int)((wa >> (8 * g)) & 0xffu), cb = (int)((wb >> (8 * g)) & 0xffu);
-                v = v > ca ? v : ca;
-                v = v > cb ? v : cb;
-                e[g] = v < K ? v : K;
-                if (small && v < K) exact |= 1u << g;
-            }
+    for (int it = 0; it < kEligTiles; it++) {
+        const uint32_t s = (uint32_t)it * kEligTile + threadIdx.x, i = t0 + s;
+        uint2 word = make_uint2(0x7f7f7f7fu, 0x7f7f7f7fu);
+        uint32_t work = 0; // point pairs to look at
+        if (i < npairs) {
+            const CellPair pr = pairs[i];
+            const uint32_t np = cell_start[pr.a + 1] - cell_start[pr.a];
+            const uint32_t nq2 = cell_start[pr.b + 1] - cell_start[pr.b];
+            const Lev8 f = first_of(pr);
+            const bool small = (uint64_t)np * nq2 <= kSmallPairWork;
+            const uint32_t kfull = pr.k >> 8;
+            bool open = false;
+#pragma unroll
+            for (int g = 0; g < kGroup; g++) open = open || (g < nj && f.v[g / 2][g & 1] < kfull);
+            if (small && open) work = np * nq2;
+            word = bytes(f, small);
         }
-        if (exact) {
-            int best[kGroup];
-#pragma unroll
-            for (int g = 0; g < kGroup; g++) best[g] = K;
-            for (uint32_t p = a0; p < a1; p++) {
-                double px = xs[p], py = ys[p];
-                uint64_t wp = level_word(kc + (size_t)p * JP, j0);
-                for (uint32_t q = b0; q < b1; q++) {
-                    double sq = dist2_exact(px, py, xs[q], ys[q]);
-                    uint64_t wq = level_word(kc + (size_t)q * JP, j0);
-                    int ls = 0; // first level whose eps admits the pair
-                    while (ls < K && sq > sTk[ls]) ls++;
-                    if (ls >= K) continue;
-#pragma unroll
-                    for (int g = 0; g < kGroup; g++) {
-                        if (!((exact >> g) & 1u)) continue;
-                        int lv = ls;
-                        int x = (int)((wp >> (8 * g)) & 0xffu), y = (int)((wq >> (8 * g)) & 0xffu);
-                        lv = lv > x ? lv : x;
-                        lv = lv > y ? lv : y;
-                        best[g] = lv < best[g] ? lv : best[g];
-                    }
-                }
-            }
-#pragma unroll
-            for (int g = 0; g < kGroup; g++)
-                if ((exact >> g) & 1u) e[g] = best[g];
+        words[s] = word;
+        const uint64_t ml = ballot(work > 0 && work <= kLightPairWork);
+        const uint64_t mh = ballot(work > kLightPairWork);
+        uint32_t at[2] = {0, 0};
+        if (lane == 0) {
+            if (ml) at[0] = atomicAdd(&nq[0], (uint32_t)popc64(ml));
+            if (mh) at[1] = atomicAdd(&nq[1], (uint32_t)popc64(mh));
         }
-        word = make_uint2(0u, 0u);
-#pragma unroll
-        for (int g = 0; g < kGroup; g++) {
-            uint32_t byte = (uint32_t)e[g] | (((exact >> g) & 1u) << 7);
-            if (g < 4) word.x |= byte << (8 * g);
-            else word.y |= byte << (8 * (g - 4));
-        }
-        lev[i] = word;
+        const uint32_t al = (uint32_t)__builtin_amdgcn_readfirstlane((int)at[0]);
+        const uint32_t ah = (uint32_t)__builtin_amdgcn_readfirstlane((int)at[1]);
+        if (work > kLightPairWork) queue[kSpan - 1 - ah - (uint32_t)mask_rank(mh)] = (uint16_t)s;
+        else if (work) queue[al + (uint32_t)mask_rank(ml)] = (uint16_t)s;
     }
-    const uint64_t present = levels_present(word, K);
-    uint32_t mine = 0; // lane l: the wave's records of level l
-    for (int l = 0; l < K; l++) {
-        uint32_t cnt = (uint32_t)popc64(ballot((present >> l) & 1ull));
-        if (lane == l) mine = cnt;
-    }
-    h[w][lane] = mine;
     __syncthreads();
-    if ((int)threadIdx.x <= K) { // (K < kMaxLevels; level K's bucket is empty)
-        uint32_t s = 0;
+    const uint32_t nlight = nq[0], nall = nlight + nq[1];
+    for (uint32_t u = threadIdx.x; u < nall; u += kBlock) {
+        const uint32_t s = queue[u < nlight ? u : kSpan - 1 - (u - nlight)];
+        const CellPair pr = pairs[t0 + s];
+        const uint32_t a0 = cell_start[pr.a], a1 = cell_start[pr.a + 1];
+        const uint32_t b0 = cell_start[pr.b], b1 = cell_start[pr.b + 1];
+        const uint32_t kmin = pr.k & 0xffu, kfull = pr.k >> 8;
+        // a level from kfull on is exact as it is; the others are looked for
+        const Lev8 f = first_of(pr);
+        Lev8 e = f;
 #pragma unroll
-        for (int q = 0; q < kWPB; q++) s += h[q][threadIdx.x];
-        hist[((size_t)group * (K + 1) + threadIdx.x) * tiles + blockIdx.x] = s;
+        for (int g = 0; g < kGroup; g++)
+            if (g < nj && f.v[g / 2][g & 1] < kfull) e.v[g / 2][g & 1] = (unsigned short)K;
+        for (uint32_t p = a0; p < a1; p++) {
+            const double px = xs[p], py = ys[p];
+            const Lev8 wp = lev8(level_word(kc + (size_t)p * JP, j0));
+            for (uint32_t q = b0; q < b1; q++) {
+                double sq = dist2_exact(px, py, xs[q], ys[q]);
+                uint32_t ls = kmin; // first level whose eps admits the pair
+                while (ls < kfull && sq > sTk[ls]) ls++;
+                e = lev8_min(e, lev8_max(wp, lev8(level_word(kc + (size_t)q * JP, j0)), ls));
+            }
+            if (lev8_same(e, f)) break;
+        }
+        words[s] = bytes(e, true);
+    }
+    __syncthreads();
+    for (int it = 0; it < kEligTiles; it++) {
+        const uint32_t s = (uint32_t)it * kEligTile + threadIdx.x, i = t0 + s;
+        const uint32_t t = blockIdx.x * kEligTiles + (uint32_t)it;
+        if (t >= tiles) break; // block-uniform
+        const uint2 word = words[s];
+        if (i < npairs) lev[i] = word;
+        const uint64_t present = levels_present(word, K);
+        uint32_t mine = 0; // lane l: the wave's records of level l
+        for (int l = 0; l < K; l++) {
+            uint32_t cnt = (uint32_t)popc64(ballot((present >> l) & 1ull));
+            if (lane == l) mine = cnt;
+        }
+        h[w][lane] = mine;
+        __syncthreads();
+        if ((int)threadIdx.x <= K) { // (K < kMaxLevels; level K's bucket is empty)
+            uint32_t sum = 0;
+#pragma unroll
+            for (int q = 0; q < kWPB; q++) sum += h[q][threadIdx.x];
+            hist[((size_t)group * (K + 1) + threadIdx.x) * tiles + t] = sum;
+        }
+        __syncthreads();
     }
 }
 
@@ -1235,7 +1294,7 @@ __global__ void __launch_bounds__(kBlock)
 // bucket d go from offs[d*tiles + u] on (the exclusive scan of hist), in pair
 // order.
 __global__ void __launch_bounds__(kBlock)
-    k_pair_scatter(const uint32_t *pa, const uint32_t *pb, const uint16_t *pk, const uint2 *lev,
+    k_pair_scatter(const CellPair *pairs, const uint2 *lev,
                    uint32_t npairs, int K, uint32_t group, const uint32_t *offs, unsigned tiles,
                    PairRec *out)
 {
@@ -1268,12 +1327,8 @@ __global__ void __launch_bounds__(kBlock)
             for (int u = 0; u < w; u++) base += h[it][u][lane];
         }
         if (!ballot(present[it] != 0)) continue;
-        uint32_t A = 0, B = 0, kf = 0;
-        if (present[it]) {
-            A = pa[i];
-            B = pb[i];
-            kf = pk[i] & 0xff00u;
-        }
+        CellPair pr{0, 0, 0};
+        if (present[it]) pr = pairs[i];
         for (int l = 0; l < K; l++) {
             uint64_t m = ballot((present[it] >> l) & 1ull);
             if (!m) continue;
@@ -1285,7 +1340,7 @@ __global__ void __launch_bounds__(kBlock)
                     uint32_t byte = ((g < 4 ? word[it].x : word[it].y) >> (8 * (g & 3))) & 0xffu;
                     if ((int)(byte & 0x7fu) == l) vals |= (1u | ((byte >> 7) << 16)) << g;
                 }
-                out[b + (uint32_t)mask_rank(m)] = PairRec{A, B, vals | kf};
+                out[b + (uint32_t)mask_rank(m)] = PairRec{pr.a, pr.b, vals | (pr.k & 0xff00u)};
             }
         }
     }
@@ -2525,7 +2580,6 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
     VDB_TRY(c.get("b.pcnt", G.ncell, &pcnt));
     VDB_TRY(c.get("b.poff", (size_t)G.ncell + 1, &poff));
     unsigned gc = ceil_div(G.ncell, kBlock);
-    unsigned gcw = ceil_div(G.ncell, kWPB); // a wave per cell
     int W = 2 * G.RS + 1;
     {
         StreamScope on(c, ps);
@@ -2620,20 +2674,18 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
         return kErrUnsupported;
     }
     uint32_t npairs = (uint32_t)npairs64;
-    uint32_t *pa, *pb, *cnts;
-    uint16_t *pk;
+    CellPair *pairs;
+    uint32_t *cnts;
     PairRec *la, *lb, *tests, *tests2;
     size_t psz = npairs ? npairs : 1;
-    VDB_TRY(c.get("b.pa", psz, &pa));
-    VDB_TRY(c.get("b.pb", psz, &pb));
-    VDB_TRY(c.get("b.pk", psz, &pk));
+    VDB_TRY(c.get("b.pairs", psz, &pairs));
     // the cell pairs stored on the second stream too, beside the lists; the
     // main stream waits for them before the level passes
     {
         StreamScope on(c, ps);
         VDB_TRY(c.kt_begin("k_pairs"));
-        k_pairs<<<gcw, kBlock, 0, c.stream()>>>(G.cell_box, G.row_lo, G.row_hi, W, G.ncell, dTk, K,
-                                                poff, pa, pb, pk);
+        k_pairs<<<gc, kBlock, 0, c.stream()>>>(G.cell_box, G.row_lo, G.row_hi, W, G.ncell, dTk, K,
+                                               poff, pairs);
         VDB_TRY(c.kt_end("k_pairs"));
         VDB_HIP(hipGetLastError());
         VDB_HIP(hipEventRecord(c.aux_event(2), ps));
@@ -2811,8 +2863,8 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
                 const unsigned tiles = ceil_div(npairs, kEligTile);
                 for (int g = 0; g < ng; g++) {
                     VDB_TRY(c.kt_begin("k_pair_elig"));
-                    k_pair_elig<<<tiles, kBlock, 0, c.stream()>>>(
-                        pa, pb, pk, cellkc, G.cell_start, G.xs, G.ys, kc, dTk, JP, j0 + g * kGroup,
+                    k_pair_elig<<<ceil_div(tiles, kEligTiles), kBlock, 0, c.stream()>>>(
+                        pairs, cellkc, G.cell_start, G.xs, G.ys, kc, dTk, JP, j0 + g * kGroup,
                         std::min(kGroup, nj - g * kGroup), K, npairs, (uint32_t)g,
                         plev + (size_t)g * npairs, phist, tiles);
                     VDB_TRY(c.kt_end("k_pair_elig"));
@@ -2824,7 +2876,7 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
                 for (int g = 0; g < ng; g++) {
                     VDB_TRY(c.kt_begin("k_pair_scatter"));
                     k_pair_scatter<<<ceil_div(tiles, kPairItems), kBlock, 0, c.stream()>>>(
-                        pa, pb, pk, plev + (size_t)g * npairs, npairs, K, (uint32_t)g, poffs, tiles,
+                        pairs, plev + (size_t)g * npairs, npairs, K, (uint32_t)g, poffs, tiles,
                         frec);
                     VDB_TRY(c.kt_end("k_pair_scatter"));
                     VDB_HIP(hipGetLastError());

@@ -59,3 +59,27 @@ def test_cells_of_few_points(m):
     want = oracle.libvdbscan(x, y, eps, mp)
     for v in range(len(eps)):
         assert (got[v] == want[v]).all(), (eps[v], mp[v])
+
+
+@pytest.mark.parametrize("border", [vd.BORDER_REFERENCE, vd.BORDER_STANDARD], ids=["ref", "std"])
+@pytest.mark.parametrize("levels,nmp", [(1, 1), (1, 3), (1, 8), (2, 1), (4, 5), (7, 1), (15, 1),
+                                        (15, 8), (16, 2)])
+def test_label_shapes(points, levels, nmp, border):
+    # level and minpts counts on both sides of every shape of the label pass
+    x, y = points[0][::4], points[1][::4]
+    E = np.round(np.linspace(0.3, 1.1, levels), 4)
+    M = np.array([4, 6, 9, 12, 3, 20, 7, 2], dtype=np.uint32)[:nmp]
+    eps, mp = np.repeat(E, nmp), np.tile(M, levels)
+    keep = np.arange(len(eps)) % 5 != 3  # some (level, value) pairs not asked for
+    eps, mp = eps[keep], mp[keep]
+    print("%d levels x %d minpts values" % (levels, nmp), flush=True)
+    got = vd.cluster(x, y, eps, mp, path=vd.PATH_BATCH, border=border)
+    if border == vd.BORDER_REFERENCE:
+        want = oracle.libvdbscan(x, y, eps, mp)
+    else:
+        from sklearn.cluster import DBSCAN
+        X = np.column_stack([x, y])
+        want = [DBSCAN(eps=e, min_samples=int(m), algorithm="kd_tree").fit(X).labels_
+                for e, m in zip(eps, mp)]
+    for v in range(len(eps)):
+        assert (got[v] == want[v]).all(), (eps[v], mp[v])

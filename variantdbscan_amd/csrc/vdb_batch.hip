@@ -149,13 +149,10 @@ __device__ __forceinline__ void cf_hook(uint32_t *parent, uint32_t x, uint32_t m
 // a cell's 8 parents as other waves left them
 __device__ __forceinline__ void cf_load8(const uint32_t *parent, uint32_t x, uint32_t (&p)[kGroup])
 {
-    const uint64_t *q = (const uint64_t *)(parent + cf_at(x));
-#pragma unroll
-    for (int i = 0; i < kGroup / 2; i++) {
-        uint64_t v = __hip_atomic_load(q + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        p[2 * i] = (uint32_t)v;
-        p[2 * i + 1] = (uint32_t)(v >> 32);
-    }
+    const uint4 *q = (const uint4 *)(parent + cf_at(x));
+    const uint4 u = q[0], v = q[1];
+    p[0] = u.x; p[1] = u.y; p[2] = u.z; p[3] = u.w;
+    p[4] = v.x; p[5] = v.y; p[6] = v.z; p[7] = v.w;
 }
 
 // Core levels of a point or cell for the 8 minpts values of a word, a byte
@@ -987,15 +984,15 @@ __global__ void __launch_bounds__(kBlock)
 // For every group of minpts values (blockIdx.y): each cell its own parent and
 // no component minimum; two flat arrays cleared (counters, snapshot root bits)
 // by a grid-stride over all blocks.
-__global__ void k_init_parent(uint32_t *parent, uint32_t *compmin, uint32_t ncell, uint32_t *z1,
+__global__ void k_init_parent(uint32_t *parent, uint32_t *compmin, uint32_t *spare, uint32_t ncell, uint32_t *z1,
                               size_t n1, uint32_t *z2, size_t n2)
 {
     uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     if (i < ncell) {
         const size_t at = ((size_t)blockIdx.y * ncell + i) * kGroup;
-        uint4 *p = (uint4 *)(parent + at), *q = (uint4 *)(compmin + at);
+        uint4 *p = (uint4 *)(parent + at), *q = (uint4 *)(compmin + at), *q2 = (uint4 *)(spare + at);
         p[0] = p[1] = make_uint4(i, i, i, i);
-        q[0] = q[1] = make_uint4(kNone, kNone, kNone, kNone);
+        q[0] = q[1] = q2[0] = q2[1] = make_uint4(kNone, kNone, kNone, kNone);
     }
     size_t f = ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * kBlock + threadIdx.x;
     size_t stride = (size_t)gridDim.y * gridDim.x * kBlock;
@@ -1838,12 +1835,13 @@ __global__ void __launch_bounds__(kBlock) k_test(LevelArgs a, LevelLists L)
 // by side per cell, core ranks at cmr + (j*K + k)*ncell, and value j's
 // snapshot in slot sbase + (number of values of jmask below j).
 struct SnapArgs {
-    uint32_t *parent, *compmin;
+    uint32_t *parent, *compmin, *spare; // spare: the other compmin
     const uint32_t *cmr;
     const uint8_t *cellkc;
-    uint32_t *root, *lab, *bits, *pre; // slot s: root/lab + s*ncell, bits/pre + s*nw
+    uint2 *snap; // the level's snapshot: (root rank, label) of cell c for its i-th value at [c*ns + i]
+    uint32_t *bits, *pre; // slot s at + s*nw
     uint64_t jmask;
-    uint32_t sbase, ncell, nw, K;
+    uint32_t sbase, ns, ncell, nw, K;
     int k, JP, j0;
 };
 
@@ -1876,88 +1874,128 @@ __device__ __forceinline__ void store8(uint32_t *p, const uint32_t (&v)[kGroup])
 
 // Flattens the forest (every cell with a core point at level k points at its
 // root) and sets compmin[root] = smallest core rank of the component (compmin
-// holds NONE on entry: k_init_parent and k_cell_labels clear it). Lanes of a
-// wave that share a root (the common case inside a large cluster) reduce
-// first, so a giant component takes one atomic per wave rather than one per
-// cell; after the two most common roots of the wave the remaining lanes,
-// spread over small components, update theirs one atomic each.
+// holds NONE on entry: the snapshots use two in turn, and k_cell_labels clears
+// the one not in use). The minima of a giant component all go to one address,
+// which takes them one after another, so waves keep the minimum of the root
+// they meet most: a wave takes a stretch of cells, every lane holding its own
+// minimum for the wave's current root, and a block hands in one value per root
+// at the end. Cells of other roots reduce within the wave where lanes share a
+// root, the rest update theirs one atomic each. 2M points x
+// 64 variants, 8 levels: 317 us (695 with one value per 64 cells).
+constexpr unsigned kRootBlocks = 1024; // from there on four stretches to a wave
+__device__ __forceinline__ void root_min(uint32_t *at, uint32_t m)
+{
+    if (m < ld_u32(at)) atomicMin(at, m);
+}
 __global__ void __launch_bounds__(kBlock) k_roots_min(SnapArgs S)
 {
+    __shared__ uint32_t hroot[kWPB][kGroup], hmin[kWPB][kGroup];
     const uint32_t g = blockIdx.y, want = snap_wanted(S, g);
     if (!want) return;
     uint32_t *parent = S.parent + (size_t)g * S.ncell * kGroup;
     uint32_t *compmin = S.compmin + (size_t)g * S.ncell * kGroup;
-    const uint32_t c = blockIdx.x * kBlock + threadIdx.x;
-    // a cell without a core point at level k is in no eligible pair yet, so
-    // nothing points at it and it points at itself: nothing to flatten
-    uint32_t core = 0, x[kGroup];
-    if (c < S.ncell) {
-        core = snap_core(S, g, c) & want;
-        load8(parent + cf_at(c), x);
-    }
-    // read-only walks, all values at once; only true roots are stored
-    bool moving = core != 0;
-    while (ballot(moving)) {
-        uint32_t nx[kGroup];
+    const int lane = lane_id(), w = threadIdx.x / kWave;
+    const uint32_t chunks = (S.ncell + kWave - 1) / kWave, waves = gridDim.x * kWPB;
+    const uint32_t per = (chunks + waves - 1) / waves, c0 = (blockIdx.x * kWPB + w) * per;
+    const uint32_t c1 = c0 + per < chunks ? c0 + per : chunks;
+    uint32_t held[kGroup], low[kGroup]; // the wave's root, the lane's minimum for it
+#pragma unroll
+    for (int j = 0; j < kGroup; j++) held[j] = low[j] = kNone;
+    for (uint32_t chunk = c0; chunk < c1; chunk++) {
+        const uint32_t c = chunk * kWave + (uint32_t)lane;
+        // a cell without a core point at level k is in no eligible pair yet,
+        // so nothing points at it and it points at itself: nothing to flatten
+        uint32_t core = 0, x[kGroup];
+        if (c < S.ncell) {
+            core = snap_core(S, g, c) & want;
+            load8(parent + cf_at(c), x);
+        }
+        // read-only walks, all values at once; only true roots are stored, so
+        // a parent read before another wave's store is still an ancestor
+        bool moving = core != 0;
+        while (ballot(moving)) {
+            uint32_t nx[kGroup];
+#pragma unroll
+            for (int j = 0; j < kGroup; j++) {
+                nx[j] = x[j];
+                if (moving && ((core >> j) & 1u)) nx[j] = parent[cf_at(x[j]) + j];
+            }
+            bool more = false;
+#pragma unroll
+            for (int j = 0; j < kGroup; j++)
+                if ((core >> j) & 1u) {
+                    more = more || nx[j] != x[j];
+                    x[j] = nx[j];
+                }
+            moving = moving && more;
+        }
+        if (core) store8(parent + cf_at(c), x);
 #pragma unroll
         for (int j = 0; j < kGroup; j++) {
-            nx[j] = x[j];
-            if (moving && ((core >> j) & 1u)) nx[j] = ld_u32(parent + cf_at(x[j]) + j);
-        }
-        bool more = false;
-#pragma unroll
-        for (int j = 0; j < kGroup; j++)
-            if ((core >> j) & 1u) {
-                more = more || nx[j] != x[j];
-                x[j] = nx[j];
+            const bool valid = (core >> j) & 1u;
+            uint64_t todo = ballot(valid);
+            if (!todo) continue;
+            const uint32_t root = valid ? x[j] : kNone;
+            const uint32_t v =
+                valid ? S.cmr[((size_t)(kGroup * g + j) * S.K + S.k) * S.ncell + c] : kNone;
+            if (!ballot(valid && root == held[j])) { // the wave has left its root
+                const uint32_t m = wave_min(low[j]);
+                if (lane == 0 && m != kNone) root_min(compmin + cf_at(held[j]) + j, m);
+                held[j] = (uint32_t)__builtin_amdgcn_readlane((int)root, __builtin_ctzll(todo));
+                low[j] = kNone;
             }
-        moving = moving && more;
+            bool same = valid && root == held[j];
+            if (same) low[j] = v < low[j] ? v : low[j];
+            todo &= ~ballot(same);
+            if (todo) {
+                const int leader = __builtin_ctzll(todo);
+                const uint32_t r = (uint32_t)__builtin_amdgcn_readlane((int)root, leader);
+                same = valid && root == r;
+                todo &= ~ballot(same);
+                const uint32_t m = wave_min(same ? v : kNone);
+                if (lane == leader) root_min(compmin + cf_at(r) + j, m);
+            }
+            if ((todo >> lane) & 1ull) root_min(compmin + cf_at(root) + j, v);
+        }
     }
-    if (core) store8(parent + cf_at(c), x);
 #pragma unroll
     for (int j = 0; j < kGroup; j++) {
-        const bool valid = (core >> j) & 1u;
-        uint64_t todo = ballot(valid);
-        if (!todo) continue;
-        const uint32_t root = valid ? x[j] : kNone;
-        const uint32_t v =
-            valid ? S.cmr[((size_t)(kGroup * g + j) * S.K + S.k) * S.ncell + c] : kNone;
-        for (int it = 0; it < 2 && todo; it++) {
-            int leader = __builtin_ctzll(todo);
-            uint32_t r = __shfl(root, leader);
-            bool same = valid && root == r;
-            todo &= ~ballot(same);
-            uint32_t m = wave_min(same ? v : kNone);
-            uint32_t *at = compmin + cf_at(r) + j;
-            if (lane_id() == leader && m < ld_u32(at)) atomicMin(at, m);
+        if (!((want >> j) & 1u)) continue;
+        const uint32_t m = wave_min(low[j]);
+        if (lane == j) {
+            hroot[w][j] = m == kNone ? kNone : held[j];
+            hmin[w][j] = m;
         }
-        if ((todo >> lane_id()) & 1ull) {
-            uint32_t *at = compmin + cf_at(root) + j;
-            if (v < ld_u32(at)) atomicMin(at, v);
-        }
+    }
+    __syncthreads();
+    if (w == 0 && lane < kWPB * kGroup && ((want >> (lane % kGroup)) & 1u)) {
+        const int u = lane / kGroup, j = lane % kGroup;
+        const uint32_t r = hroot[u][j];
+        uint32_t m = hmin[u][j];
+        bool first = r != kNone;
+        for (int q = 0; q < kWPB; q++)
+            if (q != u && hroot[q][j] == r) {
+                if (q < u) first = false;
+                m = hmin[q][j] < m ? hmin[q][j] : m;
+            }
+        if (first) root_min(compmin + cf_at(r) + j, m);
     }
 }
 
-// Snapshot of level k: root rank of every cell (NONE if the cell holds no
-// core point), and bit r of bits set for every root rank r.
-__global__ void __launch_bounds__(kBlock) k_snapshot(SnapArgs S)
+// Bit r of bits is set for every root rank r of level k: the cells whose
+// compmin k_roots_min has set are the roots.
+__global__ void __launch_bounds__(kBlock) k_root_bits(SnapArgs S)
 {
     const uint32_t g = blockIdx.y, want = snap_wanted(S, g);
     const uint32_t c = blockIdx.x * kBlock + threadIdx.x;
     if (!want || c >= S.ncell) return;
-    const uint32_t *compmin = S.compmin + (size_t)g * S.ncell * kGroup;
-    const uint32_t core = snap_core(S, g, c);
-    uint32_t r[kGroup];
-    load8(S.parent + ((size_t)g * S.ncell + c) * kGroup, r);
+    uint32_t m[kGroup];
+    load8(S.compmin + ((size_t)g * S.ncell + c) * kGroup, m);
 #pragma unroll
-    for (int j = 0; j < kGroup; j++) {
-        if (!((want >> j) & 1u)) continue;
-        const uint32_t slot = snap_slot(S, kGroup * g + j);
-        uint32_t m = (core >> j) & 1u ? compmin[cf_at(r[j]) + j] : kNone;
-        S.root[(size_t)slot * S.ncell + c] = m;
-        if (m != kNone && r[j] == c)
-            atomicOr(S.bits + (size_t)slot * S.nw + (m >> 5), 1u << (m & 31));
-    }
+    for (int j = 0; j < kGroup; j++)
+        if (((want >> j) & 1u) && m[j] != kNone)
+            atomicOr(S.bits + (size_t)snap_slot(S, kGroup * g + j) * S.nw + (m[j] >> 5),
+                     1u << (m[j] & 31));
 }
 
 // Labels of up to kLabelSlots variants sharing minpts j, from their level
@@ -1969,10 +2007,8 @@ static_assert(kLabelSlots == 8, "staged labels move as two 16-byte vectors per p
 struct LabelSlots {
     int n;
     int k[kLabelSlots];
-    const uint32_t *rootrank[kLabelSlots]; // per cell
-    const uint32_t *cbits[kLabelSlots];    // root ranks as a bitset over ranks
-    const uint32_t *cpre[kLabelSlots];     // per 32-rank word: roots before it
-    const uint32_t *celllab[kLabelSlots];  // per cell: label of its core points
+    const uint2 *snap[kLabelSlots]; // cell c of the variant's snapshot at + c*ns
+    uint32_t ns[kLabelSlots];
     uint32_t row[kLabelSlots];
     uint32_t *out;
     uint32_t nrows;
@@ -1989,34 +2025,66 @@ __device__ __forceinline__ uint32_t roots_below(const uint32_t *bits, const uint
     return pre[w] + (uint32_t)__popc(bits[w] & ((1u << (r & 31)) - 1u));
 }
 
-// label of a cell's core points at a snapshot: base + cluster id of its
-// root, counted from the first root of the cell's dataset (base 1: the
-// reference's numbering; 0: the standard rule's)
-// (also clears compmin for the next snapshot: it is no longer read)
+// Snapshot of level k: every cell's root rank and the label of its core points
+// (NONE, 0: it holds none), base + cluster id of the root, counted from the
+// first root of the cell's dataset (base 1: the reference's numbering; 0: the
+// standard rule's). A cell's minpts values lie side by side: the lanes of a
+// point read one stretch. (Its levels too would leave each level's pass 64 of
+// every 512 bytes to write: 547 us for 8 levels x 8 values of 733,000 cells;
+// so it takes 224, or 430 with a lane to a cell for all its values.)
+// Labels ascend with the root ranks, so the smallest rank brings its label.
 __global__ void __launch_bounds__(kBlock)
     k_cell_labels(SnapArgs S, const uint32_t *cell_ds, const uint32_t *seg, uint32_t base)
 {
     const uint32_t g = blockIdx.y, want = snap_wanted(S, g);
-    const uint32_t c = blockIdx.x * kBlock + threadIdx.x;
-    if (!want || c >= S.ncell) return;
-    const uint32_t none[kGroup] = {kNone, kNone, kNone, kNone, kNone, kNone, kNone, kNone};
-    store8(S.compmin + ((size_t)g * S.ncell + c) * kGroup, none);
-    const uint32_t first = seg[cell_ds[c]];
-#pragma unroll
-    for (int j = 0; j < kGroup; j++) {
-        if (!((want >> j) & 1u)) continue;
-        const uint32_t slot = snap_slot(S, kGroup * g + j);
-        const uint32_t *bits = S.bits + (size_t)slot * S.nw, *pre = S.pre + (size_t)slot * S.nw;
-        uint32_t rr = S.root[(size_t)slot * S.ncell + c];
-        S.lab[(size_t)slot * S.ncell + c] =
-            rr == kNone ? 0u : roots_below(bits, pre, rr) - roots_below(bits, pre, first) + base;
+    // two requested values to a lane
+    const uint32_t lanes = ((uint32_t)__popc(want) + 1) / 2;
+    const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
+    // (a group without requested values still clears its cells)
+    const uint32_t c = lanes > 1 ? t / lanes : t, i = lanes > 1 ? t % lanes : 0u;
+    if (c >= S.ncell) return;
+    if (i == 0) {
+        const uint32_t none[kGroup] = {kNone, kNone, kNone, kNone, kNone, kNone, kNone, kNone};
+        store8(S.spare + ((size_t)g * S.ncell + c) * kGroup, none);
     }
+    if (!want) return;
+    uint32_t left = want; // the values from the lane's first on
+    for (uint32_t u = 2 * i; u; u--) left &= left - 1;
+    const uint32_t core = snap_core(S, g, c), s0 = seg[cell_ds[c]];
+    const size_t first_cell = (size_t)g * S.ncell;
+    const uint32_t *parent = S.parent + (first_cell + c) * kGroup;
+    uint32_t slot = snap_slot(S, kGroup * g + (uint32_t)__builtin_ctz(left));
+    uint2 *at = S.snap + (size_t)c * S.ns + (slot - S.sbase);
+    uint2 v[2];
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        v[u] = make_uint2(kNone, 0u);
+        const uint32_t j = left ? (uint32_t)__builtin_ctz(left) : 0u;
+        if (left && ((core >> j) & 1u)) {
+            const uint32_t *bits = S.bits + (size_t)(slot + u) * S.nw;
+            const uint32_t *pre = S.pre + (size_t)(slot + u) * S.nw;
+            v[u].x = S.compmin[(first_cell + parent[j]) * kGroup + j];
+            v[u].y = roots_below(bits, pre, v[u].x) - roots_below(bits, pre, s0) + base;
+        }
+        if (u == 0) left &= left - 1;
+    }
+    at[0] = v[0];
+    if (left) at[1] = v[1];
 }
 
 // does a point of cell C have a neighbour list?
 __device__ __forceinline__ bool has_list(const uint32_t *cell_start, uint32_t C, int L)
 {
     return cell_start[C + 1] - cell_start[C] < (uint32_t)L;
+}
+
+// label of a point that is not core, of rank r, whose smallest neighbouring
+// root is b
+template <bool STD>
+__device__ __forceinline__ uint32_t border_label(uint2 b, uint32_t r)
+{
+    if (STD) return b.x != kNone ? b.y : kNone;
+    return b.x < r ? b.y : 0u;
 }
 
 // Thread per cell-order position: the point's data are read in sequence, the
@@ -2026,8 +2094,7 @@ __device__ __forceinline__ bool has_list(const uint32_t *cell_start, uint32_t C,
 template <bool STD>
 __global__ void __launch_bounds__(kBlock)
     k_labels_j(LabelSlots S, const uint32_t *cell_start, const uint32_t *cell_of_pos,
-               const uint32_t *cell_ds, const uint32_t *pos_rank, const uint8_t *kc, int JP, int j,
-               const uint32_t *lst_idx, const uint8_t *lst_lev, const uint32_t *lst_id,
+               const uint32_t *pos_rank, const uint8_t *kc, int JP, int j, const uint32_t *lst_idx, const uint8_t *lst_lev, const uint32_t *lst_id,
                const uint32_t *lst_n, int L, uint32_t n)
 {
     uint32_t p = blockIdx.x * kBlock + threadIdx.x;
@@ -2035,12 +2102,12 @@ __global__ void __launch_bounds__(kBlock)
     uint32_t r = pos_rank[p];
     uint32_t C = cell_of_pos[p];
     int kcp = kc[(size_t)p * JP + j];
-    uint32_t best[kLabelSlots];
+    uint2 best[kLabelSlots];
     bool any_border = false;
     int kmax = -1; // largest level of a border slot
 #pragma unroll
     for (int t = 0; t < kLabelSlots; t++) {
-        best[t] = kNone;
+        best[t] = make_uint2(kNone, 0u);
         if (t < S.n && kcp > S.k[t]) {
             any_border = true;
             kmax = S.k[t] > kmax ? S.k[t] : kmax;
@@ -2080,34 +2147,21 @@ __global__ void __launch_bounds__(kBlock)
 #pragma unroll
                     for (int t = 0; t < kLabelSlots; t++) {
                         if (t < S.n && kcp > S.k[t] && se[u] <= S.k[t] && kq[u] <= S.k[t]) {
-                            uint32_t rr = S.rootrank[t][cq[u]];
-                            best[t] = rr < best[t] ? rr : best[t];
+                            uint2 v = S.snap[t][(size_t)cq[u] * S.ns[t]];
+                            if (v.x < best[t].x) best[t] = v;
                         }
                     }
                 }
             }
         }
     }
-    uint32_t ds = cell_ds[C];
-    uint32_t s0 = S.seg[ds];
     uint32_t lbl[kLabelSlots];
 #pragma unroll
     for (int t = 0; t < kLabelSlots; t++) {
         lbl[t] = 0u;
         if (t >= S.n) continue;
-        if (kcp <= S.k[t]) {
-            lbl[t] = S.celllab[t][C];
-        } else if (STD) {
-            uint32_t b = best[t];
-            lbl[t] = b != kNone ? roots_below(S.cbits[t], S.cpre[t], b) -
-                                      roots_below(S.cbits[t], S.cpre[t], s0)
-                                : kNone;
-        } else {
-            uint32_t b = best[t];
-            lbl[t] = (b != kNone && b < r) ? roots_below(S.cbits[t], S.cpre[t], b) -
-                                                 roots_below(S.cbits[t], S.cpre[t], s0) + 1
-                                           : 0u;
-        }
+        if (kcp <= S.k[t]) lbl[t] = S.snap[t][(size_t)C * S.ns[t]].y;
+        else lbl[t] = border_label<STD>(best[t], r);
     }
     // position order, the point's labels side by side: k_rows_from_pos moves
     // them to caller order with one 32-byte read per point
@@ -2139,161 +2193,158 @@ __global__ void k_rows_from_pos(LabelSlots S, const uint32_t *pos_of_caller, uin
 }
 
 // Labels of every variant of a pass in one kernel, for passes of at most
-// kAllJ minpts values and kAllK levels. The minpts values are taken JG at a
-// time (a group); for each group a point's list is walked once, an entry
-// (neighbour q at s = d^2) updating, for every minpts value j of the group,
-// the border slots at levels max(level of s, kc_j(q)) .. kc_j(p)-1: the
-// levels at which q is a core point within eps and p is not core. The
-// running minima sit in registers, one per (j of the group, level < KB),
-// unrolled, so the snapshot loads of an entry are all in flight together.
-// Staging: per position, word j*KB + k holds the label of (j, k) (zero when
-// not requested), JG*KB words per group, written in 16-byte stores.
+// kAllJ minpts values and kAllK levels. JG >= J lanes to a point, a minpts
+// value each: they walk the point's list together, a read of an entry serving
+// all of them, and every lane keeps the smallest root of its border levels. An
+// entry (neighbour q at s = d^2) concerns lane j at the levels
+// max(level of s, kc_j(q)) .. kc_j(p)-1: those at which q is a core point
+// within eps and p is not core. The next entries' points are loaded while an
+// entry's cells are read.
+// Staging: per position JG*KB words, word j*KB + k the label of (j, k), KB >= K
+// (nothing reads the words of pairs that are not requested).
+// An entry concerns few levels, and rarely more than the entry before it when
+// both lie in one cell. Up to 4 levels the minima are registers and their
+// loads are predicated; from 8 on they are LDS columns and the lane loops over
+// its levels (2M points x 8 levels x 8 values: 1.03 ms, unrolled 1.21).
+// Bound by the gathers' latency and the lanes that lists of other lengths
+// leave idle: 2M points x 64 variants 1.03 ms (1.44 with a lane per point and
+// 32 minima in its registers), 256 datasets x 16 variants 2.35 (4.0), 8M
+// points x 1 variant 0.085 (0.505).
 constexpr int kAllJ = 8, kAllK = 15, kAllRows = 256, kAllStage = 128;
 struct AllSlots {
-    int J, K;
-    uint32_t stride;              // staged words per position
-    int8_t slot[kAllJ][16];       // (j, k) -> snapshot; -1: not requested
-    uint16_t jreq[kAllJ];         // bit k: (j, k) requested
-    const uint32_t *root, *lab, *bits, *pre; // snapshot t at + t*ncell (root, lab), + t*nw
-    uint32_t ncell, nw;
-    const uint32_t *seg;
+    int J;
+    uint16_t jreq[kAllJ];   // bit k: (j, k) requested
+    uint16_t kreq[16];      // bit j: (j, k) requested
+    const uint2 *snap[16];  // level k's snapshot, kreq[k] values a cell
     uint32_t *tmp;
 };
 
 template <bool STD, int KB, int JG>
 __global__ void __launch_bounds__(kBlock)
-    k_labels_all(AllSlots S, const uint32_t *cell_of_pos, const uint32_t *cell_ds,
-                 const uint32_t *pos_rank, const uint32_t *kc4, const uint32_t *cell_start,
-                 const uint32_t *lst_idx, const uint8_t *lst_lev, const uint32_t *lst_id,
-                 const uint32_t *lst_n, int L, uint32_t n)
+    k_labels_all(AllSlots S, const uint32_t *cell_of_pos, const uint32_t *pos_rank,
+                 const uint32_t *kc4, const uint32_t *cell_start, const uint32_t *lst_idx,
+                 const uint8_t *lst_lev, const uint32_t *lst_id, const uint32_t *lst_n, int L,
+                 uint32_t n)
 {
-    static_assert((JG * KB) % 4 == 0 && KB <= 16 && JG <= kAllJ, "whole 16-byte groups");
-    // the call's slot table and requests in LDS: the walk reads them at
-    // run-time indices without scalar memory round trips
-    __shared__ int8_t sslot[kAllJ][16];
-    __shared__ uint16_t sjreq[kAllJ];
-    if (threadIdx.x < kAllJ * 16) (&sslot[0][0])[threadIdx.x] = (&S.slot[0][0])[threadIdx.x];
-    if (threadIdx.x < kAllJ) sjreq[threadIdx.x] = S.jreq[threadIdx.x];
-    __syncthreads();
-    uint32_t p = blockIdx.x * kBlock + threadIdx.x;
-    if (p >= n) return;
-    const uint32_t r = pos_rank[p];
+    static_assert(KB <= 16 && JG <= kAllJ && KB * JG <= kAllStage, "");
+    constexpr bool kLds = KB >= 8;
+    __shared__ uint2 lbest[kLds ? KB : 1][kBlock]; // a lane's own column
+    const uint32_t p = blockIdx.x * (kBlock / JG) + threadIdx.x / JG;
+    const int j = threadIdx.x % JG;
+    if (p >= n || j >= S.J) return;
+    const uint32_t req = S.jreq[j];
+    // the lane's place in cell c's values at level k
+    auto at_level = [&](int k, uint32_t c) {
+        return S.snap[k] + (size_t)c * (uint32_t)__popc(S.kreq[k]) +
+               (uint32_t)__popc(S.kreq[k] & ((1u << j) - 1u));
+    };
     const uint32_t C = cell_of_pos[p];
-    const uint32_t kp4 = kc4[p];
-    const uint32_t li = lst_idx ? lst_idx[p] : p;
-    const bool listed = has_list(cell_start, C, L);
-    const uint32_t s0 = S.seg[cell_ds[C]];
-    const int K = S.K;
-    for (int j0 = 0; j0 < S.J; j0 += JG) {
-        // per minpts value of the group: p's core level, and the walk bound
-        // (one past the largest requested level at which p is not core)
-        int kp[JG];
-        int kend = 0;
+    const int kp = (int)((kc4[p] >> (4 * j)) & 15u);
+    // the requested levels at which p is not core
+    const uint32_t border = req & ((1u << kp) - 1u);
+    uint2 best[kLds ? 1 : KB];
 #pragma unroll
-        for (int jj = 0; jj < JG; jj++) {
-            int j = j0 + jj;
-            kp[jj] = j < S.J ? (int)((kp4 >> (4 * j)) & 15u) : 0;
-            uint32_t below = sjreq[j < S.J ? j : 0] & ((1u << kp[jj]) - 1u);
-            if (j < S.J && below) {
-                int t = 32 - __builtin_clz(below);
-                kend = t > kend ? t : kend;
+    for (int k = 0; k < KB; k++) (kLds ? lbest[k][threadIdx.x] : best[kLds ? 0 : k]) = make_uint2(kNone, 0u);
+    uint32_t m = 0, li = 0;
+    if (border && has_list(cell_start, C, L)) {
+        // non-core at level k: count_k(p) < m_j <= L, so its list holds
+        // every eps_k neighbour (the entries of levels <= k)
+        li = lst_idx ? lst_idx[p] : p;
+        m = lst_n[li];
+    }
+    if (m) {
+        const uint8_t *sv = lst_lev + lst_at(li, 0, L); // entry e at sv[64 e]
+        const uint32_t *iv = lst_id + lst_at(li, 0, L);
+        constexpr int kU = 4;
+        int se[kU];
+        uint32_t q[kU], kq[kU], cq[kU];
+        auto entries = [&](uint32_t e0) {
+#pragma unroll
+            for (int u = 0; u < kU; u++) {
+                const uint32_t e = e0 + u < m ? e0 + u : m - 1; // (the last again)
+                se[u] = (int)sv[(size_t)e * 64u];
+                q[u] = iv[(size_t)e * 64u];
             }
-        }
-        uint32_t best[JG][KB];
+        };
+        auto points = [&]() {
 #pragma unroll
-        for (int jj = 0; jj < JG; jj++)
+            for (int u = 0; u < kU; u++) {
+                // an entry beyond the border levels is not looked at
+                const bool ok = (border >> se[u]) != 0;
+                kq[u] = ok ? kc4[q[u]] : 0xffffffffu;
+                cq[u] = ok ? cell_of_pos[q[u]] : 0u;
+            }
+        };
+        uint32_t pcell = kNone, seen = 0;
+        entries(0);
+        points();
+        for (uint32_t e0 = 0; e0 < m; e0 += kU) {
+            uint32_t at[kU], cell[kU];
 #pragma unroll
-            for (int k = 0; k < KB; k++) best[jj][k] = kNone;
-        if (kend > 0 && listed) {
-            // non-core at level k: count_k(p) < m_j <= L, so its list holds
-            // every eps_k neighbour (the entries of levels <= k)
-            uint32_t m = lst_n[li];
-            const uint8_t *sv = lst_lev + lst_at(li, 0, L); // entry e at sv[64 e]
-            const uint32_t *iv = lst_id + lst_at(li, 0, L);
-            constexpr int kU = 2;
-            for (uint32_t e0 = 0; e0 < m; e0 += kU) {
-                int se[kU];
-                uint32_t q[kU];
+            for (int u = 0; u < kU; u++) {
+                const int kqj = (int)((kq[u] >> (4 * j)) & 15u);
+                const int lo = kqj > se[u] ? kqj : se[u];
+                at[u] = border >> lo << lo;
+                cell[u] = cq[u];
+                // levels seen with the entry before it, of the same cell
+                if (cell[u] != pcell) seen = 0;
+                pcell = cell[u];
+                at[u] &= ~seen;
+                seen |= at[u];
+            }
+            if (e0 + kU < m) {
+                entries(e0 + kU);
+                points();
+            }
 #pragma unroll
-                for (int u = 0; u < kU; u++) {
-                    bool ok = e0 + u < m;
-                    se[u] = ok ? (int)sv[(size_t)(e0 + u) * 64u] : kMaxLevels;
-                    q[u] = ok ? iv[(size_t)(e0 + u) * 64u] : 0u;
-                }
-                uint32_t kq[kU], cq[kU];
+            for (int u = 0; u < kU; u++) {
+                if constexpr (kLds) {
+                    while (at[u]) {
+                        const int k = __builtin_ctz(at[u]);
+                        at[u] &= at[u] - 1;
+                        const uint2 v = *at_level(k, cell[u]);
+                        if (v.x < lbest[k][threadIdx.x].x) lbest[k][threadIdx.x] = v;
+                    }
+                } else {
+                    if (!at[u]) continue;
+                    uint2 v[KB];
 #pragma unroll
-                for (int u = 0; u < kU; u++) {
-                    bool ok = se[u] < kend;
-                    kq[u] = ok ? kc4[q[u]] : 0xffffffffu;
-                    cq[u] = ok ? cell_of_pos[q[u]] : 0u;
-                }
-#pragma unroll
-                for (int u = 0; u < kU; u++) {
-                    const int ke = se[u];
-                    if (ke >= kend) continue;
-                    uint32_t v[JG][KB];
-#pragma unroll
-                    for (int jj = 0; jj < JG; jj++) {
-                        int j = j0 + jj;
-                        int kqj = (int)((kq[u] >> (4 * (j & 7))) & 15u);
-                        int lo = kqj > ke ? kqj : ke;
-                        int hi = kp[jj] < K ? kp[jj] : K;
-#pragma unroll
-                        for (int k = 0; k < KB; k++) {
-                            v[jj][k] = kNone;
-                            int t = sslot[j & 7][k];
-                            if (j < S.J && t >= 0 && k >= lo && k < hi)
-                                v[jj][k] = S.root[(size_t)t * S.ncell + cq[u]];
-                        }
+                    for (int k = 0; k < KB; k++) {
+                        v[k] = make_uint2(kNone, 0u);
+                        if ((at[u] >> k) & 1u) v[k] = *at_level(k, cell[u]);
                     }
 #pragma unroll
-                    for (int jj = 0; jj < JG; jj++)
-#pragma unroll
-                        for (int k = 0; k < KB; k++)
-                            best[jj][k] = v[jj][k] < best[jj][k] ? v[jj][k] : best[jj][k];
+                    for (int k = 0; k < KB; k++)
+                        if (v[k].x < best[k].x) best[k] = v[k];
                 }
             }
         }
-        uint32_t lbl[JG * KB];
+    }
+    const uint32_t r = STD ? 0u : pos_rank[p];
+    uint32_t lbl[KB];
 #pragma unroll
-        for (int jj = 0; jj < JG; jj++) {
-            int j = j0 + jj;
+    for (int k = 0; k < KB; k++) {
+        lbl[k] = 0u;
+        if ((req >> k) & 1u)
+            lbl[k] = kp <= k ? at_level(k, C)->y
+                             : border_label<STD>(kLds ? lbest[k][threadIdx.x] : best[kLds ? 0 : k], r);
+    }
+    uint32_t *dst = S.tmp + ((size_t)p * JG + j) * KB;
+    if constexpr (KB >= 4) {
 #pragma unroll
-            for (int k = 0; k < KB; k++) {
-                uint32_t x = 0u;
-                int t = sslot[j & 7][k];
-                if (j < S.J && t >= 0) {
-                    if (kp[jj] <= k) {
-                        x = S.lab[(size_t)t * S.ncell + C];
-                    } else {
-                        const uint32_t *bits = S.bits + (size_t)t * S.nw;
-                        const uint32_t *pre = S.pre + (size_t)t * S.nw;
-                        uint32_t b = best[jj][k];
-                        if (STD)
-                            x = b != kNone ? roots_below(bits, pre, b) - roots_below(bits, pre, s0)
-                                           : kNone;
-                        else
-                            x = (b != kNone && b < r)
-                                    ? roots_below(bits, pre, b) - roots_below(bits, pre, s0) + 1
-                                    : 0u;
-                    }
-                }
-                lbl[jj * KB + k] = x;
-            }
-        }
-        uint4 *dst = (uint4 *)(S.tmp + (size_t)p * S.stride + (size_t)j0 * KB);
+        for (int w = 0; w < KB; w += 4)
+            ((uint4 *)dst)[w / 4] = make_uint4(lbl[w], lbl[w + 1], lbl[w + 2], lbl[w + 3]);
+    } else {
 #pragma unroll
-        for (int w = 0; w < JG * KB; w += 4)
-            dst[w / 4] = make_uint4(lbl[w], lbl[w + 1], lbl[w + 2], lbl[w + 3]);
+        for (int w = 0; w < KB; w++) dst[w] = lbl[w];
     }
 }
 
 // Rows from the staged labels, thread per caller index (every row is written
-// contiguously). A point's WMAX staged words are loaded at once (read while
+// contiguously). A point's W staged words are loaded at once (read while
 // their cache lines are in cache), then up to kAllRows rows are written, the
 // rows first[w] .. first[w+1]-1 taking staged word w.
 struct AllRows {
-    uint32_t stride;
     uint16_t first[kAllStage + 1];
     uint32_t row[kAllRows];
     uint32_t *out;
@@ -2302,30 +2353,33 @@ struct AllRows {
     const uint32_t *tmp;
 };
 
-template <int WMAX>
+template <int W>
 __global__ void __launch_bounds__(kBlock)
     k_rows_all(AllRows R, const uint32_t *pos_of_caller, uint32_t nsets, uint32_t n)
 {
-    static_assert(WMAX % 4 == 0 && WMAX <= kAllStage, "whole 16-byte groups");
+    static_assert((W == 1 || W % 4 == 0) && W <= kAllStage, "a word or whole 16-byte groups");
     uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
     uint32_t p = pos_of_caller[i];
     uint32_t ds = seg_of(R.seg, nsets, i);
     uint32_t s0 = R.seg[ds], nd = R.seg[ds + 1] - s0;
     uint32_t *base = R.out + (size_t)s0 * R.nrows + (i - s0);
-    const uint4 *src = (const uint4 *)(R.tmp + (size_t)p * R.stride);
-    uint32_t v[WMAX];
+    uint32_t v[W];
+    if constexpr (W == 1) {
+        v[0] = R.tmp[p];
+    } else {
+        const uint4 *src = (const uint4 *)(R.tmp + (size_t)p * W);
 #pragma unroll
-    for (int g = 0; g < WMAX / 4; g++) {
-        uint4 x = make_uint4(0u, 0u, 0u, 0u);
-        if (4u * g < R.stride) x = src[g];
-        v[4 * g] = x.x;
-        v[4 * g + 1] = x.y;
-        v[4 * g + 2] = x.z;
-        v[4 * g + 3] = x.w;
+        for (int g = 0; g < W / 4; g++) {
+            uint4 x = src[g];
+            v[4 * g] = x.x;
+            v[4 * g + 1] = x.y;
+            v[4 * g + 2] = x.z;
+            v[4 * g + 3] = x.w;
+        }
     }
 #pragma unroll
-    for (int w = 0; w < WMAX; w++)
+    for (int w = 0; w < W; w++)
         for (int e = R.first[w]; e < R.first[w + 1]; e++) base[(size_t)R.row[e] * nd] = v[w];
 }
 
@@ -2748,9 +2802,10 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
             if (w.first.second >= j0 && w.first.second < j0 + jc) ns++;
         max_slots = std::max(max_slots, ns);
     }
-    uint32_t *parent, *compmin, *bstart;
+    uint32_t *parent, *compmin, *spare, *bstart;
     VDB_TRY(c.get("b.parent", (size_t)ngroups * G.ncell * kGroup, &parent));
     VDB_TRY(c.get("b.compmin", (size_t)ngroups * G.ncell * kGroup, &compmin));
+    VDB_TRY(c.get("b.compmin2", (size_t)ngroups * G.ncell * kGroup, &spare));
     VDB_TRY(c.get("b.la", ngroups * gcap, &la));
     VDB_TRY(c.get("b.lb", ngroups * gcap, &lb));
     VDB_TRY(c.get("b.tests", (size_t)ngroups * tcap, &tests));
@@ -2766,11 +2821,11 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
     PairRec *frec; // pair records sorted by (group, level)
     VDB_TRY(c.get("b.frec", ngroups * gcap, &frec));
     VDB_TRY(c.get("b.bstart", (size_t)ngroups * (K + 1) + 2, &bstart));
-    // per-slot snapshots: cell root ranks, cell labels, the root ranks as a
+    // snapshots: every cell's root ranks and labels, a slot's root ranks as a
     // bitset over ranks with its per-word prefix counts (cluster ids)
-    uint32_t *snap_root, *snap_lab, *snap_bits, *snap_pre;
-    VDB_TRY(c.get("b.snap_root", max_slots * G.ncell, &snap_root));
-    VDB_TRY(c.get("b.snap_lab", max_slots * G.ncell, &snap_lab));
+    uint32_t *snap_bits, *snap_pre;
+    uint2 *snap;
+    VDB_TRY(c.get("b.snap", 2 * max_slots * G.ncell, (uint32_t **)&snap));
     VDB_TRY(c.get("b.snap_bits", max_slots * nw, &snap_bits));
     VDB_TRY(c.get("b.snap_pre", max_slots * nw, &snap_pre));
     // one label kernel for the whole call when every minpts value runs in
@@ -2779,26 +2834,22 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
     const bool one_sweep = kc4 && jc == J;
     AllSlots A;
     std::vector<AllRows> all_rows;
-    int all_kb = 0, all_jg = 0, all_wmax = 0;
+    int all_kb = 0, all_jg = 0;
     if (one_sweep) {
         memset(&A, 0, sizeof A);
-        memset(A.slot, -1, sizeof A.slot);
         A.J = J;
-        A.K = K;
-        // snapshot of (k, j): level-major over the requested pairs, as the
-        // level passes number them
-        int nsnap = 0;
-        for (int k = 0; k < K; k++)
+        size_t nsnap = 0; // snapshots are level-major, as the level passes number them
+        for (int k = 0; k < K; k++) {
+            A.snap[k] = snap + nsnap * G.ncell;
             for (int j = 0; j < J; j++)
                 if (want.count({k, j})) {
-                    A.slot[j][k] = (int8_t)nsnap++;
+                    nsnap++;
+                    A.kreq[k] |= (uint16_t)(1u << j);
                     A.jreq[j] |= (uint16_t)(1u << k);
                 }
-        // register tiles of 32 minima: 4 minpts values x 8 levels, or 2 x 16
-        all_kb = K <= 8 ? 8 : 16;
-        all_jg = all_kb == 8 ? 4 : 2;
-        A.stride = (uint32_t)(((J + all_jg - 1) / all_jg) * all_jg * all_kb);
-        all_wmax = A.stride <= 16 ? 16 : A.stride <= 32 ? 32 : A.stride <= 64 ? 64 : 128;
+        }
+        all_kb = K == 1 ? 1 : K <= 4 ? 4 : K <= 8 ? 8 : 16;
+        all_jg = J == 1 ? 1 : J <= 4 ? 4 : 8;
         std::vector<std::pair<uint32_t, uint32_t>> word_row; // (staged word, output row)
         for (auto &w : want)
             for (uint32_t v : w.second)
@@ -2808,7 +2859,6 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
             AllRows R;
             memset(&R, 0, sizeof R);
             size_t r1 = std::min(word_row.size(), r0 + kAllRows);
-            R.stride = A.stride;
             size_t e = r0;
             for (int t = 0; t <= kAllStage; t++) {
                 while (e < r1 && word_row[e].first < (uint32_t)t) e++;
@@ -2819,7 +2869,7 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
         }
     }
     uint32_t *labtmp;
-    VDB_TRY(c.get("b.labtmp", (size_t)(one_sweep ? A.stride : kLabelSlots) * n, &labtmp));
+    VDB_TRY(c.get("b.labtmp", (size_t)(one_sweep ? all_kb * all_jg : kLabelSlots) * n, &labtmp));
     // label-pass events, read once the batch is done (reading them inside
     // the loop would make the host wait once per pass)
     struct EventList {
@@ -2852,7 +2902,7 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
             size_t nslot = sbase[K];
             const int ng = (nj + kGroup - 1) / kGroup;
             k_init_parent<<<dim3(gc, ng), kBlock, 0, c.stream()>>>(
-                parent, compmin, G.ncell, cnts, (size_t)ng * ncnt, snap_bits, nslot * nw);
+                parent, compmin, spare, G.ncell, cnts, (size_t)ng * ncnt, snap_bits, nslot * nw);
             VDB_HIP(hipGetLastError());
             // records bucketed by (group, level at which they become
             // eligible): bucket g*(K+1)+k of bstart
@@ -2889,6 +2939,7 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
                 VDB_HIP(hipGetLastError());
             }
             PairRec *lin = la, *lout = lb;
+            uint32_t *cm = compmin, *cm2 = spare;
             for (int k = 0; k <= kmax; k++) {
                 LevelArgs a{G.xs, G.ys, G.cell_box, G.cell_start, G.cell_key, G.cell_ds, G.skbase,
                             G.sncy, (uint32_t)G.m, kc, JP, j0, k, Th[k]};
@@ -2925,22 +2976,26 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
                 if (!jmask[k]) continue;
                 // snapshots of level k: component roots, their smallest core
                 // rank, cluster ids in ascending root rank
-                SnapArgs S{parent, compmin, cmr + (size_t)j0 * K * G.ncell, cellkc,
-                           snap_root, snap_lab, snap_bits, snap_pre, jmask[k], sbase[k], G.ncell, nw,
-                           (uint32_t)K, k, JP, j0};
+                SnapArgs S{parent, cm, cm2, cmr + (size_t)j0 * K * G.ncell, cellkc,
+                           snap + (size_t)sbase[k] * G.ncell, snap_bits, snap_pre, jmask[k],
+                           sbase[k], sbase[k + 1] - sbase[k], G.ncell, nw, (uint32_t)K, k, JP, j0};
+                std::swap(cm, cm2);
                 VDB_TRY(c.kt_begin("k_roots_min"));
-                k_roots_min<<<dim3(gc, ng), kBlock, 0, c.stream()>>>(S);
+                k_roots_min<<<dim3(std::max(std::min(gc, kRootBlocks), gc / 4), ng), kBlock, 0, c.stream()>>>(S);
                 VDB_TRY(c.kt_end("k_roots_min"));
                 VDB_HIP(hipGetLastError());
-                k_snapshot<<<dim3(gc, ng), kBlock, 0, c.stream()>>>(S);
+                k_root_bits<<<dim3(gc, ng), kBlock, 0, c.stream()>>>(S);
                 VDB_HIP(hipGetLastError());
                 // one scan over the level's slots: a slot's counts start at the
                 // slots before it, an offset the label passes subtract away
                 size_t ns_k = sbase[k + 1] - sbase[k];
                 VDB_TRY(scan_popc_u32(c, snap_bits + (size_t)sbase[k] * nw,
                                       snap_pre + (size_t)sbase[k] * nw, ns_k * nw));
-                k_cell_labels<<<dim3(gc, ng), kBlock, 0, c.stream()>>>(S, G.cell_ds, P.seg,
-                                                                       std_rule ? 0u : 1u);
+                int lanes = 1; // two values to a lane, of the group with the most
+                for (int g = 0; g < ng; g++)
+                    lanes = std::max(lanes, (__builtin_popcountll((jmask[k] >> (kGroup * g)) & 0xffu) + 1) / 2);
+                k_cell_labels<<<dim3(ceil_div((uint64_t)G.ncell * lanes, kBlock), ng), kBlock, 0,
+                                c.stream()>>>(S, G.cell_ds, P.seg, std_rule ? 0u : 1u);
                 VDB_HIP(hipGetLastError());
             }
             // labels of every requested variant of the pass
@@ -2953,27 +3008,28 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
                 VDB_HIP(hipEventRecord(le0, c.stream()));
             }
             if (one_sweep) {
-                A.root = snap_root;
-                A.lab = snap_lab;
-                A.bits = snap_bits;
-                A.pre = snap_pre;
-                A.ncell = G.ncell;
-                A.nw = nw;
-                A.seg = P.seg;
                 A.tmp = labtmp;
                 VDB_TRY(c.kt_begin("k_labels_all"));
-#define VDB_LABELS_ALL(STD, KB, JG)                                                              \
-    k_labels_all<STD, KB, JG><<<gn, kBlock, 0, c.stream()>>>(A, G.cell_of_pos, G.cell_ds,        \
-                                                             G.pos_rank, kc4, G.cell_start,       \
-                                                             lst_idx, lst_lev, lst_id, lst_n,     \
-                                                             (int)L, n)
-                if (all_kb == 8) {
-                    if (std_rule) VDB_LABELS_ALL(true, 8, 4);
-                    else VDB_LABELS_ALL(false, 8, 4);
-                } else {
-                    if (std_rule) VDB_LABELS_ALL(true, 16, 2);
-                    else VDB_LABELS_ALL(false, 16, 2);
-                }
+                auto labels = [&](auto kernel) {
+                    kernel<<<ceil_div(n, kBlock / all_jg), kBlock, 0, c.stream()>>>(
+                        A, G.cell_of_pos, G.pos_rank, kc4, G.cell_start, lst_idx, lst_lev, lst_id,
+                        lst_n, (int)L, n);
+                };
+#define VDB_LABELS_ALL(KB, JG)                                                                   \
+    if (all_kb == KB && all_jg == JG)                                                            \
+        std_rule ? labels(k_labels_all<true, KB, JG>) : labels(k_labels_all<false, KB, JG>)
+                VDB_LABELS_ALL(1, 1);
+                VDB_LABELS_ALL(1, 4);
+                VDB_LABELS_ALL(1, 8);
+                VDB_LABELS_ALL(4, 1);
+                VDB_LABELS_ALL(4, 4);
+                VDB_LABELS_ALL(4, 8);
+                VDB_LABELS_ALL(8, 1);
+                VDB_LABELS_ALL(8, 4);
+                VDB_LABELS_ALL(8, 8);
+                VDB_LABELS_ALL(16, 1);
+                VDB_LABELS_ALL(16, 4);
+                VDB_LABELS_ALL(16, 8);
 #undef VDB_LABELS_ALL
                 VDB_TRY(c.kt_end("k_labels_all"));
                 VDB_HIP(hipGetLastError());
@@ -2983,14 +3039,18 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
                     R.seg = P.seg;
                     R.tmp = labtmp;
                     VDB_TRY(c.kt_begin("k_rows_all"));
-                    if (all_wmax == 16)
-                        k_rows_all<16><<<gn, kBlock, 0, c.stream()>>>(R, pos_of_caller, P.nsets, n);
-                    else if (all_wmax == 32)
-                        k_rows_all<32><<<gn, kBlock, 0, c.stream()>>>(R, pos_of_caller, P.nsets, n);
-                    else if (all_wmax == 64)
-                        k_rows_all<64><<<gn, kBlock, 0, c.stream()>>>(R, pos_of_caller, P.nsets, n);
-                    else
-                        k_rows_all<128><<<gn, kBlock, 0, c.stream()>>>(R, pos_of_caller, P.nsets, n);
+                    auto rows_of = [&](auto kernel) {
+                        kernel<<<gn, kBlock, 0, c.stream()>>>(R, pos_of_caller, P.nsets, n);
+                    };
+                    switch (all_kb * all_jg) {
+                    case 1: rows_of(k_rows_all<1>); break;
+                    case 4: rows_of(k_rows_all<4>); break;
+                    case 8: rows_of(k_rows_all<8>); break;
+                    case 16: rows_of(k_rows_all<16>); break;
+                    case 32: rows_of(k_rows_all<32>); break;
+                    case 64: rows_of(k_rows_all<64>); break;
+                    default: rows_of(k_rows_all<128>); break;
+                    }
                     VDB_TRY(c.kt_end("k_rows_all"));
                     VDB_HIP(hipGetLastError());
                 }
@@ -3008,13 +3068,10 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
                     S.n = (int)std::min<size_t>(kLabelSlots, rows_j.size() - r0);
                     for (int t = 0; t < S.n; t++) {
                         int k = rows_j[r0 + t].first;
-                        size_t sl = sbase[k] + (uint32_t)__builtin_popcountll(
-                                                   jmask[k] & ((1ull << jr) - 1ull));
                         S.k[t] = k;
-                        S.rootrank[t] = snap_root + sl * G.ncell;
-                        S.cbits[t] = snap_bits + sl * nw;
-                        S.cpre[t] = snap_pre + sl * nw;
-                        S.celllab[t] = snap_lab + sl * G.ncell;
+                        S.ns[t] = sbase[k + 1] - sbase[k];
+                        S.snap[t] = snap + (size_t)sbase[k] * G.ncell +
+                                    (uint32_t)__builtin_popcountll(jmask[k] & ((1ull << jr) - 1ull));
                         S.row[t] = rows[rows_j[r0 + t].second];
                     }
                     S.out = out;
@@ -3024,13 +3081,13 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
                     if (std_rule) {
                         VDB_TRY(c.kt_begin("k_labels_j"));
                         k_labels_j<true><<<gn, kBlock, 0, c.stream()>>>(
-                            S, G.cell_start, G.cell_of_pos, G.cell_ds, G.pos_rank, kc, JP, j, lst_idx,
+                            S, G.cell_start, G.cell_of_pos, G.pos_rank, kc, JP, j, lst_idx,
                             lst_lev, lst_id, lst_n, (int)L, n);
                         VDB_TRY(c.kt_end("k_labels_j"));
                     } else {
                         VDB_TRY(c.kt_begin("k_labels_j"));
                         k_labels_j<false><<<gn, kBlock, 0, c.stream()>>>(
-                            S, G.cell_start, G.cell_of_pos, G.cell_ds, G.pos_rank, kc, JP, j, lst_idx,
+                            S, G.cell_start, G.cell_of_pos, G.pos_rank, kc, JP, j, lst_idx,
                             lst_lev, lst_id, lst_n, (int)L, n);
                         VDB_TRY(c.kt_end("k_labels_j"));
                     }

@@ -132,7 +132,7 @@ int run_per_variant(Context &c, Points &P, const double *eps, const uint32_t *mi
         // float32 screening reports its rechecks over all of them
         const bool core_only = mode == 0 && precision == VDB_PREC_FP64;
         int k = cells ? cells : kFusedCellsPerEps;
-        if (!core_only) VDB_TRY(tune_cells_per_eps(c, P, e, precision, cells, &k));
+        if (!core_only) VDB_TRY(tune_cells_per_eps(c, P, e, precision, cells, true, &k));
         VDB_TRY(build_eps_grid(c, P, e, k, "g1", G));
         if (!core_only) VDB_TRY(build_items(c, G, "g1", I));
         if (st) st->ms_prepare += t0.ms();
@@ -525,7 +525,7 @@ int vdb_neighbor_counts(const double *x, const double *y, uint32_t n, double eps
     Grid G;
     Items I;
     int k = 0;
-    VDB_TRY(tune_cells_per_eps(c, P, eps, precision, 0, &k));
+    VDB_TRY(tune_cells_per_eps(c, P, eps, precision, 0, false, &k));
     VDB_TRY(build_eps_grid(c, P, eps, k, "g1", G));
     VDB_TRY(build_items(c, G, "g1", I));
     uint32_t *cpos, *ccal;
@@ -579,7 +579,7 @@ int vdb_neighbor_table(const double *x, const double *y, uint32_t n, double eps,
     Grid G;
     Items I;
     int k = 0;
-    VDB_TRY(tune_cells_per_eps(c, P, eps, precision, 0, &k));
+    VDB_TRY(tune_cells_per_eps(c, P, eps, precision, 0, false, &k));
     VDB_TRY(build_eps_grid(c, P, eps, k, "g1", G));
     VDB_TRY(build_items(c, G, "g1", I));
     if (st) st->ms_prepare = tprep.ms();
@@ -646,7 +646,7 @@ int vdb_neighbor_table_digest(const double *x, const double *y, uint32_t n, doub
     Grid G;
     Items I;
     int k = 0;
-    VDB_TRY(tune_cells_per_eps(c, P, eps, precision, 0, &k));
+    VDB_TRY(tune_cells_per_eps(c, P, eps, precision, 0, false, &k));
     VDB_TRY(build_eps_grid(c, P, eps, k, "g1", G));
     VDB_TRY(build_items(c, G, "g1", I));
     return table_digest(c, P, G, I, eps, precision, digest, pairs, rechecked);

@@ -23,15 +23,18 @@ struct PhaseTimes {
 };
 
 // Work items: (cell, first origin) groups of kOrigins origins of one cell.
+// Cells of small windows have none unless all are asked for: their points are
+// taken by a thread each, and cnt (null: all cells have items) is 0 for them.
 struct Items {
     uint32_t n = 0;
     uint32_t *cell = nullptr;
     uint32_t *o0 = nullptr;
+    const uint32_t *cnt = nullptr;
 };
 
 constexpr int kOrigins = 8;
 
-int build_items(Context &c, const Grid &G, const char *tag, Items &I);
+int build_items(Context &c, const Grid &G, const char *tag, Items &I, bool all = false);
 
 // Grid of the per-variant kernels at eps: cells of side eps*(1+2^-24)/k and a
 // window of k cells each way (any pair accepted at eps is at most
@@ -49,12 +52,13 @@ constexpr int kMaxCellsPerEps = 8;
 constexpr int kFusedCellsPerEps = 2;
 int cells_per_eps(const vdb_options *opt);
 
-// Autotuner: the first time a workload (point count, eps, extent, precision)
-// is seen, times grid build + count pass at every resolution 1..4 and keeps
-// the fastest; later calls reuse the choice. Small inputs skip the timing.
-// Uses the "g1" grid slots. requested > 0 is returned unchanged.
+// Autotuner: the first time a workload (point count, extent in eps, precision)
+// is seen, times grid build + count pass (and the components, from resolution
+// 2 on, when they follow) at rising resolutions and keeps the coarsest near the
+// best; later calls reuse the choice. Small inputs skip the timing. Uses the
+// "g1" grid slots. requested > 0 is returned unchanged.
 int tune_cells_per_eps(Context &c, const Points &P, double eps, int precision, int requested,
-                       int *k_out);
+                       bool components, int *k_out);
 
 // counts[p] = |N_eps(p)| for every position p of G (self included).
 // precision 0 = FP64 exact, 1 = FP32 with an FP64 recheck inside the error band.

@@ -60,6 +60,19 @@ __device__ __forceinline__ RowSeg row_seg(const GridView &g, uint32_t c, int r)
     return s;
 }
 
+// the rows of cell c's window, row r in lane r (W <= 2 kMaxCellsPerEps + 1)
+__device__ __forceinline__ RowSeg lane_rows(const GridView &g, uint32_t c)
+{
+    RowSeg s{0, 0, 0, 0};
+    if (lane_id() < g.W) s = row_seg(g, c, lane_id());
+    return s;
+}
+__device__ __forceinline__ RowSeg row_at(const RowSeg &rows, int r)
+{
+    auto at = [&](uint32_t v) { return (uint32_t)__builtin_amdgcn_readlane((int)v, r); };
+    return RowSeg{at(rows.a), at(rows.f0), at(rows.f1), at(rows.e)};
+}
+
 // 64-candidate blocks of positions [a, e): lane l holds a + 64*i + l; lanes
 // past e see NaN coordinates (never accepted).
 template <class F>
@@ -166,20 +179,50 @@ __device__ __forceinline__ uint32_t sgpr_u32(uint32_t v)
 }
 
 // ----------------------------------------------------------------- items
-__global__ void k_item_counts(const uint32_t *cell_start, uint32_t ncell, uint32_t *cnt)
+// The blocks of a launch from `from` on take the points of cells without items
+// (cnt 0): the two share the chip instead of waiting for each other's tails.
+struct FewPoints {
+    const uint32_t *cell_of_pos, *cnt;
+    uint32_t from;
+};
+// Points whose window holds at most this many points are taken by a thread
+// each: a wave for a handful of candidates is mostly idle lanes and padded
+// origins. Counts, float32
+// screening, 1M points, eps 0.4: 2.83 ms to 1.97; the table of 504,000 points
+// at eps 0.215 with its clusters 4.48 to 2.1.
+constexpr uint32_t kFewCands = 192;
+constexpr int kFewUnroll = 4;
+
+// points of cell c's window
+__device__ __forceinline__ uint32_t window_points(const GridView &g, uint32_t c)
+{
+    uint32_t w = 0;
+    for (int r = 0; r < g.W; r++) {
+        size_t t = (size_t)c * g.W + r;
+        uint32_t lo = g.row_lo[t], hi = g.row_hi[t];
+        if (lo < hi) w += g.cell_start[hi] - g.cell_start[lo];
+    }
+    return w;
+}
+
+// items of a cell; none for the cells whose points take a thread each (windows
+// of at most `few` points)
+__global__ void k_item_counts(GridView g, uint32_t ncell, uint32_t few, uint32_t *cnt)
 {
     uint32_t c = blockIdx.x * kBlock + threadIdx.x;
     if (c >= ncell) return;
-    uint32_t n = cell_start[c + 1] - cell_start[c];
+    uint32_t n = g.cell_start[c + 1] - g.cell_start[c];
+    if (few && window_points(g, c) <= few) n = 0;
     cnt[c] = (n + kOrigins - 1) / kOrigins;
 }
 
-__global__ void k_item_fill(const uint32_t *cell_start, const uint32_t *excl, uint32_t ncell,
+__global__ void k_item_fill(const uint32_t *cell_start, const uint32_t *cnt, const uint32_t *excl, uint32_t ncell,
                             uint32_t *item_cell, uint32_t *item_o0)
 {
     uint32_t c = blockIdx.x * kBlock + threadIdx.x;
     if (c >= ncell) return;
     uint32_t a = cell_start[c], e = cell_start[c + 1], k = excl[c];
+    if (!cnt[c]) return;
     for (uint32_t o = a; o < e; o += kOrigins, k++) {
         item_cell[k] = c;
         item_o0[k] = o;
@@ -187,55 +230,125 @@ __global__ void k_item_fill(const uint32_t *cell_start, const uint32_t *excl, ui
 }
 
 // ------------------------------------------------------------- counting
+// Points of cells without items, a thread each.
+template <int PREC>
+__device__ __forceinline__ void count_near(const GridView &g, const FewPoints &few, uint32_t block,
+                                           double T, const Band &band, uint32_t *counts,
+                                           unsigned long long *recheck)
+{
+    const uint32_t p = block * kBlock + threadIdx.x;
+    uint32_t c = 0, nre = 0;
+    const bool mine = p < g.n && few.cnt[c = few.cell_of_pos[p]] == 0;
+    if (mine) {
+        const double px = g.xs[p], py = g.ys[p];
+        uint32_t cnt = 0;
+        for (int r = 0; r < g.W; r++) {
+            size_t t = (size_t)c * g.W + r;
+            uint32_t lo = g.row_lo[t], hi = g.row_hi[t];
+            if (lo >= hi) continue;
+            uint32_t e = g.cell_start[hi];
+            for (uint32_t a = g.cell_start[lo]; a < e; a += kFewUnroll) {
+#pragma unroll
+                for (int i = 0; i < kFewUnroll; i++) {
+                    uint32_t q = a + i < e ? a + i : e - 1;
+                    double qx = g.xs[q], qy = g.ys[q];
+                    bool in;
+                    if (PREC == 0) {
+                        in = dist2_exact(px, py, qx, qy) <= T;
+                    } else {
+                        float s = dist2_f32(0.0f, 0.0f, (float)__dsub_rn(qx, px),
+                                            (float)__dsub_rn(qy, py));
+                        in = s <= band.lo;
+                        if (!in && s <= band.hi && a + i < e) {
+                            in = dist2_exact(px, py, qx, qy) <= T;
+                            nre++;
+                        }
+                    }
+                    cnt += in && a + i < e ? 1u : 0u;
+                }
+            }
+        }
+        counts[p] = cnt;
+    }
+    if (PREC == 1 && ballot(nre != 0)) {
+        for (int o = kWave / 2; o > 0; o >>= 1) nre += __shfl_xor(nre, o);
+        if (lane_id() == 0) atomicAdd(recheck, (unsigned long long)nre);
+    }
+}
+
+// The other cells, a wave per item. The window's rows are looked up by a lane
+// each, all at once.
 template <int PREC>
 __global__ void __launch_bounds__(kBlock)
     k_count(GridView g, const uint32_t *__restrict__ item_cell,
-            const uint32_t *__restrict__ item_o0, uint32_t nitems, double T, Band band,
-            uint32_t *__restrict__ counts, unsigned long long *recheck)
+            const uint32_t *__restrict__ item_o0, uint32_t nitems, FewPoints few, double T,
+            Band band, uint32_t *__restrict__ counts, unsigned long long *recheck)
 {
+    if (blockIdx.x >= few.from) {
+        count_near<PREC>(g, few, blockIdx.x - few.from, T, band, counts, recheck);
+        return;
+    }
     uint32_t it = blockIdx.x * kWavesPerBlock + wave_id_in_block();
     if (it >= nitems) return;
     uint32_t c = sgpr_u32(item_cell[it]), o0 = sgpr_u32(item_o0[it]);
     uint32_t nb = sgpr_u32(g.cell_start[c + 1]) - o0;
     nb = nb < kOrigins ? nb : kOrigins;
     const double qnan = __longlong_as_double(0x7ff8000000000000ll);
-    double ox[kOrigins], oy[kOrigins];
-    float fx[kOrigins], fy[kOrigins];
+    // binary64 origins in scalar registers; of the float32 screening's only
+    // the differences to the first (the few pairs it leaves open read the rest)
+    double ox[PREC == 0 ? kOrigins : 1], oy[PREC == 0 ? kOrigins : 1];
+    float fx[PREC == 0 ? 1 : kOrigins], fy[PREC == 0 ? 1 : kOrigins];
     uint32_t cnt[kOrigins];
-    double rx = sgpr_d(g.xs[o0]), ry = sgpr_d(g.ys[o0]);
+    const double rx = sgpr_d(g.xs[o0]), ry = sgpr_d(g.ys[o0]);
 #pragma unroll
     for (int b = 0; b < kOrigins; b++) {
         uint32_t ob = o0 + (b < (int)nb ? b : 0);
         // padded origins are NaN: they accept nothing
-        ox[b] = b < (int)nb ? sgpr_d(g.xs[ob]) : qnan;
-        oy[b] = sgpr_d(g.ys[ob]);
-        fx[b] = (float)__dsub_rn(ox[b], rx);
-        fy[b] = (float)__dsub_rn(oy[b], ry);
+        double x = b < (int)nb ? sgpr_d(g.xs[ob]) : qnan, y = sgpr_d(g.ys[ob]);
+        if constexpr (PREC == 0) {
+            ox[b] = x;
+            oy[b] = y;
+        } else {
+            fx[b] = (float)__dsub_rn(x, rx);
+            fy[b] = (float)__dsub_rn(y, ry);
+        }
         cnt[b] = 0;
     }
     uint32_t nre = 0, full = 0;
-    auto test = [&](uint32_t q, bool v, double qx, double qy) {
-        if (PREC == 0) {
-#pragma unroll
-            for (int b = 0; b < kOrigins; b++)
-                cnt[b] += popc64(ballot(dist2_exact(ox[b], oy[b], qx, qy) <= T));
-        } else {
-            float gx = (float)__dsub_rn(qx, rx), gy = (float)__dsub_rn(qy, ry);
+    auto test = [&](uint32_t, bool, double qx, double qy) {
+        if constexpr (PREC == 0) {
 #pragma unroll
             for (int b = 0; b < kOrigins; b++) {
-                float s = dist2_f32(fx[b], fy[b], gx, gy);
-                bool acc = s <= band.lo;
-                uint64_t amb = ballot(!acc && s <= band.hi);
-                if (amb) {
-                    if ((amb >> lane_id()) & 1ull) acc = dist2_exact(ox[b], oy[b], qx, qy) <= T;
-                    nre += popc64(amb);
+                if (b % 2 == 0 && b >= (int)nb) break;
+                cnt[b] += popc64(ballot(dist2_exact(ox[b], oy[b], qx, qy) <= T));
+            }
+        } else {
+            const float gx = (float)__dsub_rn(qx, rx), gy = (float)__dsub_rn(qy, ry);
+            uint64_t open = 0; // lanes with a pair the screening leaves open
+#pragma unroll
+            for (int b = 0; b < kOrigins; b++) {
+                if (b % 2 == 0 && b >= (int)nb) break;
+                const float s = dist2_f32(fx[b], fy[b], gx, gy);
+                const uint64_t in = ballot(s <= band.lo);
+                open |= ballot(s <= band.hi) & ~in;
+                cnt[b] += popc64(in);
+            }
+            if (open) {
+#pragma unroll
+                for (int b = 0; b < kOrigins; b++) {
+                    if (b >= (int)nb) break;
+                    const float s = dist2_f32(fx[b], fy[b], gx, gy);
+                    const bool amb = s <= band.hi && !(s <= band.lo);
+                    nre += popc64(ballot(amb));
+                    cnt[b] += popc64(
+                        ballot(amb && dist2_exact(g.xs[o0 + b], g.ys[o0 + b], qx, qy) <= T));
                 }
-                cnt[b] += popc64(ballot(acc));
             }
         }
     };
+    const RowSeg rows = lane_rows(g, c);
     for (int r = 0; r < g.W; r++) {
-        RowSeg sg = row_seg(g, c, r);
+        RowSeg sg = row_at(rows, r);
         run_blocks(g, sg.a, sg.f0, test);
         full += sg.f1 - sg.f0;
         run_blocks(g, sg.f1, sg.e, test);
@@ -255,20 +368,6 @@ __global__ void __launch_bounds__(kBlock)
 // origins of a cell at a time, to a wave each, which first adds up the cells
 // accepted whole: where those hold `need` points nothing is tested. At 1M
 // points, eps 0.4, need 100: the exact count (6 to 8 cells per eps) 1.66 ms, this 0.26.
-constexpr uint32_t kFewCands = 192;
-constexpr int kFewUnroll = 4;
-
-// points of cell c's window
-__device__ __forceinline__ uint32_t window_points(const GridView &g, uint32_t c)
-{
-    uint32_t w = 0;
-    for (int r = 0; r < g.W; r++) {
-        size_t t = (size_t)c * g.W + r;
-        uint32_t lo = g.row_lo[t], hi = g.row_hi[t];
-        if (lo < hi) w += g.cell_start[hi] - g.cell_start[lo];
-    }
-    return w;
-}
 
 // append v to list for every lane with take set, one atomic per wave
 __device__ __forceinline__ void list_append(bool take, uint32_t v, uint32_t *list, uint32_t *count)
@@ -393,6 +492,69 @@ __device__ __forceinline__ uint64_t pair_mix(uint64_t row, uint64_t id)
     return z ^ (z >> 31);
 }
 
+// The rows of points of cells without items, a thread each: the same entries
+// in the same order (window rows in turn, positions ascending).
+template <bool D2, bool DIGEST>
+__device__ __forceinline__ void fill_near(const GridView &g, const FewPoints &few, uint32_t block,
+                                          double T, const uint64_t *offsets,
+                                          const uint32_t *rowmap, const uint32_t *idmap,
+                                          uint32_t *ids, float *d2, uint64_t cap,
+                                          uint32_t *overflow)
+{
+    const uint32_t p = block * kBlock + threadIdx.x;
+    uint32_t c = 0;
+    const bool mine = p < g.n && few.cnt[c = few.cell_of_pos[p]] == 0;
+    bool over = false;
+    uint64_t dig = 0;
+    if (mine) {
+        const double px = g.xs[p], py = g.ys[p];
+        const uint32_t row = rowmap ? rowmap[p] : p;
+        uint64_t run = 0, lim = 0;
+        if (!DIGEST) {
+            run = offsets[row];
+            lim = offsets[row + 1];
+        }
+        for (int r = 0; r < g.W; r++) {
+            size_t t = (size_t)c * g.W + r;
+            uint32_t lo = g.row_lo[t], hi = g.row_hi[t];
+            if (lo >= hi) continue;
+            uint32_t e = g.cell_start[hi];
+            for (uint32_t a = g.cell_start[lo]; a < e; a += kFewUnroll) {
+                double s[kFewUnroll];
+#pragma unroll
+                for (int i = 0; i < kFewUnroll; i++) {
+                    uint32_t q = a + i < e ? a + i : e - 1;
+                    s[i] = dist2_exact(px, py, g.xs[q], g.ys[q]);
+                }
+#pragma unroll
+                for (int i = 0; i < kFewUnroll; i++) {
+                    if (a + i >= e || !(s[i] <= T)) continue;
+                    const uint32_t id = idmap ? idmap[a + i] : a + i;
+                    if (DIGEST) {
+                        dig += pair_mix(row, id);
+                        continue;
+                    }
+                    // the count pass sized every row; never write past it
+                    const bool w = run < lim && run < cap;
+                    over |= !w;
+                    if (w) {
+                        ids[run] = id;
+                        if (D2) d2[run] = (float)s[i];
+                    }
+                    run++;
+                }
+            }
+        }
+    }
+    if (DIGEST) {
+        if (!ballot(mine)) return;
+        for (int o = kWave / 2; o > 0; o >>= 1) dig += __shfl_xor(dig, o);
+        if (lane_id() == 0) atomicAdd((unsigned long long *)ids, (unsigned long long)dig);
+        return;
+    }
+    if (ballot(over) && lane_id() == 0) atomicOr(overflow, 1u);
+}
+
 template <int PREC, bool D2, bool DIGEST = false>
 __global__ void __launch_bounds__(kBlock)
     k_fill(GridView g, const uint32_t *__restrict__ item_cell,
@@ -400,8 +562,13 @@ __global__ void __launch_bounds__(kBlock)
            Band band, const uint64_t *__restrict__ offsets, uint64_t off_base,
            const uint32_t *__restrict__ rowmap, const uint32_t *__restrict__ idmap,
            uint32_t *__restrict__ ids, float *__restrict__ d2, uint64_t cap,
-           uint32_t *overflow)
+           uint32_t *overflow, FewPoints few)
 {
+    if (blockIdx.x >= few.from) {
+        fill_near<D2, DIGEST>(g, few, blockIdx.x - few.from, T, offsets, rowmap, idmap, ids, d2,
+                              cap, overflow);
+        return;
+    }
     // block-uniform: do the block's 4 items exist and share one cell?
     uint32_t ib = it0 + blockIdx.x * kWavesPerBlock;
     bool shared = ib + kWavesPerBlock <= it1 &&
@@ -445,6 +612,7 @@ __global__ void __launch_bounds__(kBlock)
             lim[b] = sgpr_u64(offsets[row + 1] - off_base);
         }
     }
+    const RowSeg rows = lane_rows(g, c);
     bool over = false;
     uint64_t dig = 0;
     // Row staging (ids only: no D2, no digest). Accepted ids are appended to
@@ -651,7 +819,7 @@ __global__ void __launch_bounds__(kBlock)
             }
         };
         for (int r = 0; r < g.W; r++) {
-            RowSeg sg = row_seg(g, c, r);
+            RowSeg sg = row_at(rows, r);
             if (D2) sg.f0 = sg.f1 = sg.e;
             staged(sg.a, sg.f0);
             full(sg.f0, sg.f1);
@@ -670,7 +838,7 @@ __global__ void __launch_bounds__(kBlock)
             chunk(q0, nblk, qx, qy, qid);
         };
         for (int r = 0; r < g.W; r++) {
-            RowSeg sg = row_seg(g, c, r);
+            RowSeg sg = row_at(rows, r);
             if (D2) sg.f0 = sg.f1 = sg.e;
             run_chunks(g, sg.a, sg.f0, tested);
             full(sg.f0, sg.f1);
@@ -1359,21 +1527,22 @@ struct EvTimer {
 
 } // namespace
 
-int build_items(Context &c, const Grid &G, const char *tag, Items &I)
+int build_items(Context &c, const Grid &G, const char *tag, Items &I, bool all)
 {
     uint32_t *cnt, *excl;
     std::string t(tag);
     VDB_TRY(c.get((t + ".icnt").c_str(), G.ncell, &cnt));
     VDB_TRY(c.get((t + ".iexcl").c_str(), G.ncell, &excl));
-    k_item_counts<<<ceil_div(G.ncell, kBlock), kBlock, 0, c.stream()>>>(G.cell_start, G.ncell,
-                                                                        cnt);
+    k_item_counts<<<ceil_div(G.ncell, kBlock), kBlock, 0, c.stream()>>>(
+        view(G, G.npts), G.ncell, all ? 0u : kFewCands, cnt);
     VDB_HIP(hipGetLastError());
     uint32_t total = 0;
     VDB_TRY(compact_count(c, cnt, excl, G.ncell, &total));
     I.n = total;
-    VDB_TRY(c.get((t + ".icell").c_str(), total, &I.cell));
-    VDB_TRY(c.get((t + ".io0").c_str(), total, &I.o0));
-    k_item_fill<<<ceil_div(G.ncell, kBlock), kBlock, 0, c.stream()>>>(G.cell_start, excl,
+    I.cnt = all ? nullptr : cnt;
+    VDB_TRY(c.get((t + ".icell").c_str(), std::max(total, 1u), &I.cell));
+    VDB_TRY(c.get((t + ".io0").c_str(), std::max(total, 1u), &I.o0));
+    k_item_fill<<<ceil_div(G.ncell, kBlock), kBlock, 0, c.stream()>>>(G.cell_start, cnt, excl,
                                                                       G.ncell, I.cell, I.o0);
     VDB_HIP(hipGetLastError());
     return kOk;
@@ -1395,8 +1564,11 @@ int cells_per_eps(const vdb_options *opt)
     return 0;
 }
 
+static int core_components(Context &c, const Grid &G, double T, const uint8_t *core,
+                           uint32_t *parent);
+
 int tune_cells_per_eps(Context &c, const Points &P, double eps, int precision, int requested,
-                       int *k_out)
+                       bool components, int *k_out)
 {
     if (requested >= 1 && requested <= kMaxCellsPerEps) {
         *k_out = requested;
@@ -1409,17 +1581,19 @@ int tune_cells_per_eps(Context &c, const Points &P, double eps, int precision, i
         *k_out = kDefaultCellsPerEps;
         return kOk;
     }
-    auto bits = [](double v) {
-        uint64_t u;
-        memcpy(&u, &v, sizeof u);
-        return (unsigned long long)u;
+    // Components run over cells, which have to be cliques: from 2 cells per
+    // eps on. (490,000 points, eps 0.107: the count 0.15 ms at 1 and at 2, the
+    // components 0.98 and 0.20.)
+    const int k0 = components ? 2 : 1;
+    // the key names the tuned range and the workload's shape: the point count
+    // and the extent in eps, to a twelfth
+    auto spans = [&](double a, double b) {
+        const double w = (b - a) / eps;
+        return (int)std::floor(8.0 * std::log2(w > 1.0 ? w : 1.0));
     };
-    // the key names the tuned range (1..kMaxCellsPerEps): a choice cached
-    // over a narrower range is tuned again
     char key[160];
-    snprintf(key, sizeof key, "cells%d:%u:%d:%llx:%llx:%llx:%llx:%llx", kMaxCellsPerEps, P.n,
-             precision, bits(eps),
-             bits(P.ext[0]), bits(P.ext[1]), bits(P.ext[2]), bits(P.ext[3]));
+    snprintf(key, sizeof key, "few:cells%d-%d:%u:%d:%d:%d", k0, kMaxCellsPerEps, P.n, precision,
+             spans(P.ext[0], P.ext[1]), spans(P.ext[2], P.ext[3]));
     int cached = 0;
     if (c.tuned_get(key, &cached) && cached >= 1 && cached <= kMaxCellsPerEps) {
         *k_out = cached;
@@ -1429,26 +1603,48 @@ int tune_cells_per_eps(Context &c, const Points &P, double eps, int precision, i
     unsigned long long *rc;
     VDB_TRY(c.get("tune.counts", P.n, &counts));
     VDB_TRY(c.get("tune.recheck", 1, &rc));
+    constexpr uint32_t kTuneMinpts = 8; // the core points of the components timed
+    uint8_t *core = nullptr;
+    uint32_t *parent = nullptr, *best_of = nullptr;
+    if (components) {
+        VDB_TRY(c.get("cv.core", P.n, &core));
+        VDB_TRY(c.get("cv.parent", P.n, &parent));
+        VDB_TRY(c.get("cv.best", P.n, &best_of));
+    }
     // Finer cells test fewer candidates (more of the window is accepted whole)
-    // but add rows per window; past the point where the count stops gaining,
-    // the fill and the core pass run a little slower on the finer grid. The
-    // choice is the coarsest k whose count is within kTuneSlack of the best.
-    constexpr float kTuneSlack = 1.05f;
+    // but add rows per window and cells to unite; past the point where the
+    // count stops gaining, the fill runs a little slower on the finer grid. The
+    // choice is the coarsest k whose passes are within kTuneSlack of the best,
+    // of two runs each (the first also grows the buffers); the search ends
+    // where two resolutions in a row are well past the best.
+    constexpr float kTuneSlack = 1.05f, kTuneStop = 1.25f;
     float ms_k[kMaxCellsPerEps + 1] = {};
     float best_ms = 0;
-    for (int k = 1; k <= kMaxCellsPerEps; k++) {
-        Grid G;
-        Items I;
-        EvTimer tm(c.stream());
-        tm.start();
-        VDB_TRY(build_eps_grid(c, P, eps, k, "g1", G));
-        VDB_TRY(build_items(c, G, "g1", I));
-        VDB_TRY(count_neighbors(c, G, I, eps, precision, counts, (uint64_t *)rc));
-        ms_k[k] = tm.stop();
-        if (k == 1 || ms_k[k] < best_ms) best_ms = ms_k[k];
+    int last = kMaxCellsPerEps;
+    for (int k = k0; k <= last; k++) {
+        for (int run = 0; run < 2; run++) {
+            Grid G;
+            Items I;
+            EvTimer tm(c.stream());
+            tm.start();
+            VDB_TRY(build_eps_grid(c, P, eps, k, "g1", G));
+            VDB_TRY(build_items(c, G, "g1", I));
+            VDB_TRY(count_neighbors(c, G, I, eps, precision, counts, (uint64_t *)rc));
+            if (components) {
+                k_core_init<<<ceil_div(P.n, kBlock), kBlock, 0, c.stream()>>>(
+                    counts, P.n, kTuneMinpts, core, parent, best_of, G.words + 3);
+                VDB_HIP(hipGetLastError());
+                VDB_TRY(core_components(c, G, threshold_for_eps(eps), core, parent));
+            }
+            const float ms = tm.stop();
+            if (run == 0 || ms < ms_k[k]) ms_k[k] = ms;
+        }
+        if (k == k0 || ms_k[k] < best_ms) best_ms = ms_k[k];
+        if (k > k0 + 1 && ms_k[k] > best_ms * kTuneStop && ms_k[k - 1] > best_ms * kTuneStop)
+            last = k;
     }
-    int best = kMaxCellsPerEps;
-    for (int k = 1; k <= kMaxCellsPerEps; k++)
+    int best = last;
+    for (int k = k0; k <= last; k++)
         if (ms_k[k] <= best_ms * kTuneSlack) {
             best = k;
             break;
@@ -1458,24 +1654,32 @@ int tune_cells_per_eps(Context &c, const Points &P, double eps, int precision, i
     return kOk;
 }
 
+// the blocks of a launch over all points: those of the items, then those of
+// the points without
+static FewPoints few_points(const Grid &G, const Items &I, unsigned *blocks)
+{
+    const unsigned items = ceil_div(I.n, kWavesPerBlock);
+    *blocks = items + (I.cnt ? ceil_div(G.npts, kBlock) : 0u);
+    return FewPoints{G.cell_of_pos, I.cnt, items};
+}
+
 int count_neighbors(Context &c, const Grid &G, const Items &I, double eps, int precision,
                     uint32_t *counts, uint64_t *recheck_dev)
 {
     double T = threshold_for_eps(eps);
-    if (I.n == 0) return kOk;
-    unsigned blocks = ceil_div(I.n, kWavesPerBlock);
-    if (precision == 0) {
-        VDB_TRY(c.kt_begin("k_count"));
-        k_count<0><<<blocks, kBlock, 0, c.stream()>>>(view(G, G.npts), I.cell, I.o0, I.n, T, Band{},
-                                                      counts, nullptr);
-        VDB_TRY(c.kt_end("k_count"));
-    } else {
-        VDB_TRY(c.kt_begin("k_count"));
-        k_count<1><<<blocks, kBlock, 0, c.stream()>>>(view(G, G.npts), I.cell, I.o0, I.n, T,
-                                                      band_for(G, T), counts,
+    if (G.npts == 0) return kOk;
+    const Band band = precision ? band_for(G, T) : Band{};
+    unsigned blocks = 0;
+    const FewPoints few = few_points(G, I, &blocks);
+    VDB_TRY(c.kt_begin("k_count"));
+    if (precision == 0)
+        k_count<0><<<blocks, kBlock, 0, c.stream()>>>(view(G, G.npts), I.cell, I.o0, I.n, few, T,
+                                                      band, counts, nullptr);
+    else
+        k_count<1><<<blocks, kBlock, 0, c.stream()>>>(view(G, G.npts), I.cell, I.o0, I.n, few, T,
+                                                      band, counts,
                                                       (unsigned long long *)recheck_dev);
-        VDB_TRY(c.kt_end("k_count"));
-    }
+    VDB_TRY(c.kt_end("k_count"));
     VDB_HIP(hipGetLastError());
     return kOk;
 }
@@ -1622,16 +1826,12 @@ int cluster_variant(Context &c, const Points &P, const Grid &G, const Items &I, 
         if (pt) tm.start();
         VDB_TRY(scan_exclusive_u32_u64(c, counts, offsets, n, offsets + n));
         if (pt) pt->scan += tm.stop();
-        std::vector<uint64_t> hoff(n + 1);
-        std::vector<uint32_t> hstart(G.ncell + 1), hio0(I.n);
-        VDB_HIP(hipMemcpyAsync(hoff.data(), offsets, sizeof(uint64_t) * (n + 1),
-                               hipMemcpyDeviceToHost, c.stream()));
-        VDB_HIP(hipMemcpyAsync(hstart.data(), G.cell_start, sizeof(uint32_t) * (G.ncell + 1),
-                               hipMemcpyDeviceToHost, c.stream()));
-        VDB_HIP(hipMemcpyAsync(hio0.data(), I.o0, sizeof(uint32_t) * I.n,
-                               hipMemcpyDeviceToHost, c.stream()));
-        VDB_HIP(hipStreamSynchronize(c.stream()));
-        uint64_t P_total = hoff[n];
+        void *hs = nullptr;
+        VDB_TRY(c.host_scratch(sizeof(uint64_t), &hs));
+        VDB_HIP(hipMemcpyAsync(hs, offsets + n, sizeof(uint64_t), hipMemcpyDeviceToHost,
+                               c.stream()));
+        VDB_TRY(c.wait(c.stream()));
+        uint64_t P_total = *(uint64_t *)hs;
         if (pt) pt->pairs = P_total;
         uint64_t cap = table_budget / sizeof(uint32_t);
         // largest single cell must fit
@@ -1654,39 +1854,68 @@ int cluster_variant(Context &c, const Points &P, const Grid &G, const Items &I, 
         VDB_TRY(core_components(c, G, T, core, parent));
         VDB_TRY(root_keys());
         if (pt) pt->uf += tm.stop();
-        // The table, tile by tile (tiles are runs of items: items are ordered
-        // by cell, origins ascending), each tile filled once and its border
-        // rows (fewer than minpts entries each) read back for the border pass.
         uint32_t ntiles = 0;
-        uint32_t i0 = 0;
-        while (i0 < I.n) {
-            uint32_t i1 = i0;
-            uint64_t base = hoff[hio0[i0]];
-            while (i1 < I.n) {
-                uint32_t oend = (i1 + 1 < I.n) ? hio0[i1 + 1] : n;
-                if (hoff[oend] - base > cap && i1 > i0) break;
-                i1++;
-            }
-            uint32_t pend = i1 < I.n ? hio0[i1] : n;
-            uint32_t p0 = hio0[i0];
-            if (hoff[pend] - base > cap) {
-                set_error("neighbour table tile does not fit the table budget");
-                return kErrNoMemory;
-            }
+        if (P_total <= cap) {
+            // the whole table at once
             if (pt) tm.start();
             VDB_TRY(c.kt_begin("k_fill"));
-            k_fill<0, false><<<ceil_div(i1 - i0, kWavesPerBlock), kBlock, 0, c.stream()>>>(
-                view(G, G.npts), I.cell, I.o0, i0, i1, T, Band{}, offsets, base, nullptr, nullptr,
-                ids, nullptr, cap, ovf);
+            unsigned blocks = 0;
+            const FewPoints few = few_points(G, I, &blocks);
+            k_fill<0, false><<<blocks, kBlock, 0, c.stream()>>>(
+                view(G, n), I.cell, I.o0, 0, I.n, T, Band{}, offsets, 0, nullptr, nullptr, ids,
+                nullptr, cap, ovf, few);
             VDB_TRY(c.kt_end("k_fill"));
             VDB_HIP(hipGetLastError());
             if (pt) pt->fill += tm.stop(), tm.start();
-            k_border_table<<<ceil_div(pend - p0, kWavesPerBlock), kBlock, 0, c.stream()>>>(
-                offsets, base, ids, p0, pend, core, bkey, parent, best);
+            k_border_table<<<ceil_div(n, kWavesPerBlock), kBlock, 0, c.stream()>>>(
+                offsets, 0, ids, 0, n, core, bkey, parent, best);
             VDB_HIP(hipGetLastError());
             if (pt) pt->border += tm.stop();
-            ntiles++;
-            i0 = i1;
+            ntiles = 1;
+        } else {
+            // The table, tile by tile (tiles are runs of items, here of all
+            // cells: items are ordered by cell, origins ascending), each tile
+            // filled once and its border rows (fewer than minpts entries each)
+            // read back for the border pass.
+            Items A;
+            VDB_TRY(build_items(c, G, "g1all", A, true));
+            std::vector<uint64_t> hoff(n + 1);
+            std::vector<uint32_t> hio0(A.n);
+            VDB_HIP(hipMemcpyAsync(hoff.data(), offsets, sizeof(uint64_t) * (n + 1),
+                                   hipMemcpyDeviceToHost, c.stream()));
+            VDB_HIP(hipMemcpyAsync(hio0.data(), A.o0, sizeof(uint32_t) * A.n,
+                                   hipMemcpyDeviceToHost, c.stream()));
+            VDB_HIP(hipStreamSynchronize(c.stream()));
+            uint32_t i0 = 0;
+            while (i0 < A.n) {
+                uint32_t i1 = i0;
+                uint64_t base = hoff[hio0[i0]];
+                while (i1 < A.n) {
+                    uint32_t oend = (i1 + 1 < A.n) ? hio0[i1 + 1] : n;
+                    if (hoff[oend] - base > cap && i1 > i0) break;
+                    i1++;
+                }
+                uint32_t pend = i1 < A.n ? hio0[i1] : n;
+                uint32_t p0 = hio0[i0];
+                if (hoff[pend] - base > cap) {
+                    set_error("neighbour table tile does not fit the table budget");
+                    return kErrNoMemory;
+                }
+                if (pt) tm.start();
+                VDB_TRY(c.kt_begin("k_fill"));
+                k_fill<0, false><<<ceil_div(i1 - i0, kWavesPerBlock), kBlock, 0, c.stream()>>>(
+                    view(G, G.npts), A.cell, A.o0, i0, i1, T, Band{}, offsets, base, nullptr,
+                    nullptr, ids, nullptr, cap, ovf, FewPoints{nullptr, nullptr, kNone});
+                VDB_TRY(c.kt_end("k_fill"));
+                VDB_HIP(hipGetLastError());
+                if (pt) pt->fill += tm.stop(), tm.start();
+                k_border_table<<<ceil_div(pend - p0, kWavesPerBlock), kBlock, 0, c.stream()>>>(
+                    offsets, base, ids, p0, pend, core, bkey, parent, best);
+                VDB_HIP(hipGetLastError());
+                if (pt) pt->border += tm.stop();
+                ntiles++;
+                i0 = i1;
+            }
         }
         if (pt) pt->tiles += ntiles;
         uint32_t hov = 0;
@@ -1780,24 +2009,18 @@ int table_digest(Context &c, const Points &P, const Grid &G, const Items &I, dou
     uint64_t *offs;
     VDB_TRY(c.get("nt.off", (size_t)n + 1, &offs));
     VDB_TRY(scan_exclusive_u32_u64(c, dummy, offs, n, tot));
-    if (I.n) {
-        unsigned blocks = ceil_div(I.n, kWavesPerBlock);
-        Band bd = precision ? band_for(G, T) : Band{};
-        if (precision == 0) {
-            VDB_TRY(c.kt_begin("k_fill"));
-            k_fill<0, false, true><<<blocks, kBlock, 0, c.stream()>>>(
-                view(G, G.npts), I.cell, I.o0, 0, I.n, T, bd, nullptr, 0, caller_of_pos, caller_of_pos,
-                (uint32_t *)acc, nullptr, 0, nullptr);
-            VDB_TRY(c.kt_end("k_fill"));
-        } else {
-            VDB_TRY(c.kt_begin("k_fill"));
-            k_fill<1, false, true><<<blocks, kBlock, 0, c.stream()>>>(
-                view(G, G.npts), I.cell, I.o0, 0, I.n, T, bd, nullptr, 0, caller_of_pos, caller_of_pos,
-                (uint32_t *)acc, nullptr, 0, nullptr);
-            VDB_TRY(c.kt_end("k_fill"));
-        }
-        VDB_HIP(hipGetLastError());
-    }
+    unsigned blocks = 0;
+    const FewPoints few = few_points(G, I, &blocks);
+    const Band bd = precision ? band_for(G, T) : Band{};
+    VDB_TRY(c.kt_begin("k_fill"));
+    auto fill = [&](auto kernel) {
+        kernel<<<blocks, kBlock, 0, c.stream()>>>(view(G, G.npts), I.cell, I.o0, 0, I.n, T, bd,
+                                                  nullptr, 0, caller_of_pos, caller_of_pos,
+                                                  (uint32_t *)acc, nullptr, 0, nullptr, few);
+    };
+    precision == 0 ? fill(k_fill<0, false, true>) : fill(k_fill<1, false, true>);
+    VDB_TRY(c.kt_end("k_fill"));
+    VDB_HIP(hipGetLastError());
     unsigned long long h[2];
     VDB_HIP(hipMemcpyAsync(h, acc, sizeof h, hipMemcpyDeviceToHost, c.stream()));
     uint64_t t = 0;
@@ -1845,40 +2068,23 @@ int neighbor_table(Context &c, const Points &P, const Grid &G, const Items &I, d
         pt->recheck = r;
     }
     if (tot > capacity) return kOk; // caller sizes its buffers from *total
-    if (I.n == 0) return kOk;
+    if (n == 0) return kOk;
     if (pt) tm.start();
     uint32_t *ovf = nullptr;
     VDB_TRY(c.get("nt.ovf", 1, &ovf));
     VDB_HIP(hipMemsetAsync(ovf, 0, sizeof(uint32_t), c.stream()));
-    unsigned blocks = ceil_div(I.n, kWavesPerBlock);
+    unsigned blocks = 0;
+    const FewPoints few = few_points(G, I, &blocks);
     Band bd = precision ? band_for(G, T) : Band{};
-    if (precision == 0 && !d2) {
-        VDB_TRY(c.kt_begin("k_fill"));
-        k_fill<0, false><<<blocks, kBlock, 0, c.stream()>>>(
-            view(G, G.npts), I.cell, I.o0, 0, I.n, T, bd, offsets, 0, caller_of_pos, caller_of_pos, ids,
-            d2, capacity, ovf);
-        VDB_TRY(c.kt_end("k_fill"));
-    }
-    else if (precision == 0) {
-        VDB_TRY(c.kt_begin("k_fill"));
-        k_fill<0, true><<<blocks, kBlock, 0, c.stream()>>>(
-            view(G, G.npts), I.cell, I.o0, 0, I.n, T, bd, offsets, 0, caller_of_pos, caller_of_pos, ids,
-            d2, capacity, ovf);
-        VDB_TRY(c.kt_end("k_fill"));
-    }
-    else if (!d2) {
-        VDB_TRY(c.kt_begin("k_fill"));
-        k_fill<1, false><<<blocks, kBlock, 0, c.stream()>>>(
-            view(G, G.npts), I.cell, I.o0, 0, I.n, T, bd, offsets, 0, caller_of_pos, caller_of_pos, ids,
-            d2, capacity, ovf);
-        VDB_TRY(c.kt_end("k_fill"));
-    } else {
-        VDB_TRY(c.kt_begin("k_fill"));
-        k_fill<1, true><<<blocks, kBlock, 0, c.stream()>>>(
-            view(G, G.npts), I.cell, I.o0, 0, I.n, T, bd, offsets, 0, caller_of_pos, caller_of_pos, ids,
-            d2, capacity, ovf);
-        VDB_TRY(c.kt_end("k_fill"));
-    }
+    VDB_TRY(c.kt_begin("k_fill"));
+    auto fill = [&](auto kernel) {
+        kernel<<<blocks, kBlock, 0, c.stream()>>>(view(G, G.npts), I.cell, I.o0, 0, I.n, T, bd,
+                                                  offsets, 0, caller_of_pos, caller_of_pos, ids,
+                                                  d2, capacity, ovf, few);
+    };
+    if (precision == 0) d2 ? fill(k_fill<0, true>) : fill(k_fill<0, false>);
+    else d2 ? fill(k_fill<1, true>) : fill(k_fill<1, false>);
+    VDB_TRY(c.kt_end("k_fill"));
     VDB_HIP(hipGetLastError());
     if (pt) pt->fill += tm.stop();
     uint32_t hov = 0;

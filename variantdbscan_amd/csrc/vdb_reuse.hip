@@ -343,9 +343,9 @@ int reuse_grid(Context &c, const Points &P, double eps, int precision, int cells
     VDB_TRY(c.get("ru.recheck", 1, &recheck));
     VDB_HIP(hipMemsetAsync(recheck, 0, sizeof(unsigned long long), c.stream()));
     int k = 0;
-    VDB_TRY(tune_cells_per_eps(c, P, eps, precision, cells, &k));
+    VDB_TRY(tune_cells_per_eps(c, P, eps, precision, cells, true, &k));
     VDB_TRY(build_eps_grid(c, P, eps, k, "g1", G));
-    VDB_TRY(build_items(c, G, "g1", I));
+    VDB_TRY(build_items(c, G, "g1", I, true)); // border_pairs takes every cell by items
     VDB_TRY(count_neighbors(c, G, I, eps, precision, counts, (uint64_t *)recheck));
     return kOk;
 }

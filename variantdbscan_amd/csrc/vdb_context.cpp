@@ -40,6 +40,8 @@ Context::~Context()
     if (stage_) hipHostFree(stage_);
     for (hipEvent_t e : aux_ev_)
         if (e) hipEventDestroy(e);
+    for (hipEvent_t e : stage_ev_)
+        if (e) hipEventDestroy(e);
     if (wait_ev_) hipEventDestroy(wait_ev_);
     if (aux_) hipStreamDestroy(aux_);
     if (own_stream_) hipStreamDestroy(own_stream_);
@@ -190,6 +192,14 @@ int Context::host_stage(size_t bytes, void **out)
         stage_bytes_ = want;
     }
     *out = stage_;
+    return kOk;
+}
+
+int Context::stage_event(size_t chunk, hipEvent_t *out)
+{
+    hipEvent_t &e = stage_ev_[chunk];
+    if (!e) VDB_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    *out = e;
     return kOk;
 }
 

@@ -50,10 +50,12 @@ public:
     // Pinned host staging for small device->host reads.
     int host_scratch(size_t bytes, void **out);
 
-    // A second pinned area, for the arrays of small host calls (grow-only, so
-    // at most kStageBytes; device kernels may read and write it).
-    static constexpr size_t kStageBytes = (size_t)1 << 20;
+    // A second pinned area, for the arrays of host calls (grow-only, at most
+    // kStageBytes; device kernels may read and write it), and an event for
+    // each kStageChunk of it.
+    static constexpr size_t kStageBytes = (size_t)8 << 20, kStageChunk = (size_t)1 << 19;
     int host_stage(size_t bytes, void **out);
+    int stage_event(size_t chunk, hipEvent_t *out);
 
     // A second stream of the library (default priority, created on first
     // use) for work that may run beside the current stream's, with events
@@ -127,6 +129,7 @@ private:
     hipStream_t own_stream_ = nullptr;
     hipStream_t stream_ = nullptr;
     hipStream_t aux_ = nullptr;
+    hipEvent_t stage_ev_[kStageBytes / kStageChunk] = {};
     hipEvent_t aux_ev_[kAuxEvents] = {};
     hipEvent_t wait_ev_ = nullptr;
     std::unordered_map<std::string, Buffer> pool_;

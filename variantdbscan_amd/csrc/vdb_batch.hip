@@ -241,10 +241,12 @@ __global__ void k_list_flags(const uint32_t *cell_start, const uint32_t *cell_of
 //   more              a wave per point, cells pruned by their box
 // Times of the three kernels together against the wave per point for all
 // (which kept the L nearest sorted), MI355X: 256 sets of 17.8M points x 4 eps
-// 11.3 ms against 26.9; 8M skewed points, 1 eps: 1.2 ms against 3.3; 2M points
-// x 8 eps 1.4 ms against 2.1. One thread for windows up to 512 points took
+// 9.3 ms against 26.9; 8M skewed points, 1 eps: 0.91 ms against 3.3; 2M points
+// x 8 eps 1.1 ms against 2.1. One thread for windows up to 512 points took
 // 1.5 ms instead of 0.4 on the last (waves wait for their longest walk), 16
-// lanes for windows up to 1024 points 1.1 ms more on the first.
+// lanes for windows up to 1024 points 0.4 ms more on the first. A wave's and a
+// group's next candidates are loaded before the current ones are taken: 4.1 to
+// 3.5 and 2.6 to 2.3 ms of the first, 0.74 to 0.50 and 0.21 to 0.18 of the last.
 constexpr uint32_t kNearMid = 128;
 constexpr uint32_t kNearCrowded = 512;
 constexpr int kNearGroup = 16;
@@ -463,6 +465,17 @@ __device__ __forceinline__ bool near_point(const FG &g, const NearOut &O, const 
             }
             len += h;
         };
+        double cx[U], cy[U]; // candidates
+        bool ahead = false;  // loaded for the next step already
+        auto load = [&](uint32_t from, uint32_t to) {
+#pragma unroll
+            for (int i = 0; i < U; i++) {
+                uint32_t tc = from + (uint32_t)(i * G + gl);
+                tc = tc < to ? tc : to - 1;
+                cx[i] = g.xs[tc];
+                cy[i] = g.ys[tc];
+            }
+        };
         uint32_t q = 0, e = 0, q2 = 0, e2 = 0; // the span walked, one waiting
         int u = 0;                             // rows started
         bool first = inner && window > kNearDense;
@@ -507,15 +520,22 @@ __device__ __forceinline__ bool near_point(const FG &g, const NearOut &O, const 
                 }
             }
             if (q < e) {
-                // U candidates a lane, their loads issued together
+                // U candidates a lane, their loads issued together, and the
+                // span's next ones loaded while these are taken
                 double s[U];
                 uint32_t t[U];
+                if (!ahead) load(q, e);
 #pragma unroll
                 for (int i = 0; i < U; i++) {
                     t[i] = q + (uint32_t)(i * G + gl);
-                    uint32_t tc = t[i] < e ? t[i] : e - 1;
-                    s[i] = dist2_exact(px, py, g.xs[tc], g.ys[tc]);
+                    s[i] = dist2_exact(px, py, cx[i], cy[i]);
                     if (t[i] >= e) s[i] = INFINITY;
+                }
+                // (a thread by itself has its windows' lines in L1 and loses
+                // more by the registers)
+                if constexpr (G > 1) {
+                    ahead = q + U * G < e;
+                    if (ahead) load(q + U * G, e);
                 }
 #pragma unroll
                 for (int i = 0; i < U; i++) take(s[i], t[i]);
@@ -594,7 +614,7 @@ __global__ void __launch_bounds__(kBlock)
         uint32_t window = 0;
         const uint2 *rows = g.row_pts + (size_t)c * g.W;
         for (int d = 0; d < g.W; d++) window += rows[d].y;
-        near_point<KL, kNearGroup, 1>(g, O, sT, p, c, window);
+        near_point<KL, kNearGroup, 2>(g, O, sT, p, c, window);
     }
 }
 
@@ -648,11 +668,19 @@ __global__ void __launch_bounds__(kBlock)
         double thr = sT[K - 1];
         // candidates [a, e), 64 per step, until L are found at level 0
         auto sweep = [&](uint32_t a, uint32_t e) {
+            // the next step's candidates are loaded while this one's are kept
+            double nx = 0.0, ny = 0.0;
+            auto load = [&](uint32_t q) {
+                uint32_t qc = q < e ? q : e - 1;
+                nx = g.xs[qc];
+                ny = g.ys[qc];
+            };
+            if (a < e) load(a + (uint32_t)lane);
             for (uint32_t q0 = a; q0 < e && cut; q0 += kWave) {
                 uint32_t q = q0 + (uint32_t)lane;
-                uint32_t qc = q < e ? q : e - 1;
-                double s = dist2_exact(px, py, g.xs[qc], g.ys[qc]);
+                double s = dist2_exact(px, py, nx, ny);
                 if (q >= e) s = INFINITY;
+                if (q0 + kWave < e) load(q + kWave);
                 bool hit = s <= thr;
                 uint64_t hm = ballot(hit);
                 if (!hm) continue;

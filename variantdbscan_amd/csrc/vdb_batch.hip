@@ -1064,6 +1064,7 @@ struct LevelLists {
     uint32_t ncell, tcap, K;
     uint32_t *ovf;
     uint32_t ppb, minb, tpb; // grid shape (BatchShape)
+    uint32_t take;           // records of a short test list a wave takes at once
 };
 
 struct LevelG {
@@ -1536,6 +1537,7 @@ __global__ void __launch_bounds__(kBlock) k_sweep(LevelArgs a, LevelLists L)
             if (((pr.k >> j) & 1u) && ra[j] != rb[j]) open |= 1u << j;
         if (ballot(open != 0)) {
             bool moving = true;
+            uint32_t ma = 0, mb = 0; // values whose walk left the first parent
             while (ballot(moving)) {
                 uint32_t na[kGroup], nb2[kGroup];
 #pragma unroll
@@ -1551,6 +1553,8 @@ __global__ void __launch_bounds__(kBlock) k_sweep(LevelArgs a, LevelLists L)
 #pragma unroll
                 for (int j = 0; j < kGroup; j++) {
                     moving = moving || na[j] != ra[j] || nb2[j] != rb[j];
+                    ma |= na[j] != ra[j] ? 1u << j : 0u;
+                    mb |= nb2[j] != rb[j] ? 1u << j : 0u;
                     ra[j] = na[j];
                     rb[j] = nb2[j];
                 }
@@ -1560,8 +1564,8 @@ __global__ void __launch_bounds__(kBlock) k_sweep(LevelArgs a, LevelLists L)
                 if ((open >> j) & 1u) {
                     // a cell below its root is no root and stays none: its
                     // parent may move up to any ancestor
-                    if (ra[j] != A) st_u32(parent + cf_at(A) + j, ra[j]);
-                    if (rb[j] != B) st_u32(parent + cf_at(B) + j, rb[j]);
+                    if (((ma >> j) & 1u) && ra[j] != A) st_u32(parent + cf_at(A) + j, ra[j]);
+                    if (((mb >> j) & 1u) && rb[j] != B) st_u32(parent + cf_at(B) + j, rb[j]);
                     if (ra[j] == rb[j]) open &= ~(1u << j);
                 }
         }
@@ -1664,7 +1668,6 @@ __device__ __forceinline__ uint32_t core_bits(const LevelArgs &a, uint32_t p)
 __device__ void test_pair(const LevelArgs &a, const PairRec &pr, uint32_t *parent,
                           PairRec *list_out, uint32_t *nout)
 {
-    if (pr.a == kNone) return; // unused slot of a test chunk
     uint32_t A = pr.a, B = pr.b;
     uint32_t a0 = a.cell_start[A], a1 = a.cell_start[A + 1];
     uint32_t b0 = a.cell_start[B], b1 = a.cell_start[B + 1];
@@ -1734,26 +1737,18 @@ __device__ void test_pair(const LevelArgs &a, const PairRec &pr, uint32_t *paren
 // Two tests in one wave, one per 32-lane half (lanes 32h..32h+31 take r_h),
 // for pairs whose cells both hold at most 32 points: each half holds its B
 // cell in registers and screens its A cell in one step, so two dependent
-// load chains are in flight per wave. A half whose pair has a larger cell
-// tests nothing; its bit (1 for r0, 2 for r1) in the wave-uniform result
-// asks the caller for a whole-wave test. Absent records have a == NONE.
-__device__ uint32_t test_pair_halves(const LevelArgs &a, const PairRec &r0, const PairRec &r1,
-                                     uint32_t *parent, PairRec *list_out, uint32_t *nout)
+// load chains are in flight per wave. An absent second record has a == NONE.
+__device__ void test_pair_halves(const LevelArgs &a, const PairRec &r0, const PairRec &r1,
+                                 uint32_t *parent, PairRec *list_out, uint32_t *nout)
 {
     const int lane = lane_id();
     const int h = lane >> 5;
     const uint32_t l = (uint32_t)lane & 31u;
     const PairRec pr = h ? r1 : r0;
-    const bool live = pr.a != kNone;
-    uint32_t A = live ? pr.a : 0u, B = live ? pr.b : 0u;
-    uint32_t a0 = a.cell_start[A], a1 = a.cell_start[A + 1];
-    uint32_t b0 = a.cell_start[B], b1 = a.cell_start[B + 1];
-    const bool fits = live && a1 - a0 <= 32u && b1 - b0 <= 32u;
-    const uint64_t lm = ballot(live), fm = ballot(fits);
-    uint32_t back = 0;
-    if ((lm & 0xffffffffull) && !(fm & 0xffffffffull)) back |= 1u;
-    if ((lm >> 32) && !(fm >> 32)) back |= 2u;
-    if (fits) {
+    if (pr.a != kNone) {
+        uint32_t A = pr.a, B = pr.b;
+        uint32_t a0 = a.cell_start[A], a1 = a.cell_start[A + 1];
+        uint32_t b0 = a.cell_start[B], b1 = a.cell_start[B + 1];
         uint32_t open = test_open(pr, parent);
         if (open) {
             if (a1 - a0 > b1 - b0) { // lanes hold the larger cell
@@ -1793,7 +1788,6 @@ __device__ uint32_t test_pair_halves(const LevelArgs &a, const PairRec &r0, cons
             test_end(pr, l, found, open, parent, list_out, nout);
         }
     }
-    return back;
 }
 
 // the near tests, then the far ones, in one grid-stride pass (waves take
@@ -1819,40 +1813,52 @@ __global__ void __launch_bounds__(kBlock) k_test(LevelArgs a, LevelLists L)
     nb = nb > L.minb ? nb : L.minb;
     nb = nb < gridDim.x ? nb : gridDim.x;
     if (blockIdx.x >= nb) return;
-    if (bstart[a.k + 1] - bstart[a.k] < kChunkedFrom) {
-        // exact lists: a record per wave
+    const bool chunked = bstart[a.k + 1] - bstart[a.k] >= kChunkedFrom;
+    if (!chunked && L.take == 1) {
+        // a short list of one minpts value: nearly every record has to be
+        // tested and a look beforehand is only in the way (2M points 0.107 ms,
+        // 0.13 to 0.17 with it)
         for (uint32_t w = blockIdx.x * kWPB + wave_id_in_block(); w < nt; w += nb * kWPB)
             test_pair(a, w < nn ? near[w] : far[w - nn], parent, list_out, nout);
         return;
     }
-    // chunked lists: a wave takes 64 consecutive records at a time (one load
-    // each), skips the unused chunk slots with one ballot and tests the rest
-    // in turn
-    uint32_t ng = (nt + kWave - 1) / kWave;
+    // A wave takes 64 consecutive records at a time (short lists: 4, to spread
+    // wider), one load each, skips the unused chunk slots and the pairs
+    // connected by now all at once, and tests the rest in turn. Most far pairs
+    // are connected by the near tests: 256 datasets 2.82 -> 1.03 ms, 8M skewed
+    // points 0.36 -> 0.22 (each one looked at in its turn before); short lists
+    // of 2M points x 64 variants 0.35 -> 0.20, 500K x 16 0.115 -> 0.072 (2 at a
+    // time 0.27, 0.085; 8 0.18, 0.092).
+    const uint32_t take = chunked ? kWave : L.take;
+    uint32_t ng = (nt + take - 1) / take;
     for (uint32_t gi = blockIdx.x * kWPB + wave_id_in_block(); gi < ng; gi += nb * kWPB) {
-        uint32_t w = gi * kWave + lane_id();
+        uint32_t w = gi * take + lane_id();
         PairRec r{kNone, kNone, 0};
-        if (w < nt) r = w < nn ? near[w] : far[w - nn];
-        uint64_t real = ballot(r.a != kNone);
-        // two records at a time, a half-wave each when their cells are small
+        if (w < nt && (uint32_t)lane_id() < take) r = w < nn ? near[w] : far[w - nn];
+        const bool real = r.a != kNone && test_open(r, parent) != 0;
+        const bool small = real && a.cell_start[r.a + 1] - a.cell_start[r.a] <= 32u &&
+                           a.cell_start[r.b + 1] - a.cell_start[r.b] <= 32u;
+        uint64_t halves = ballot(small), waves = ballot(real && !small);
+        auto rec = [&](uint64_t &m) {
+            if (!m) return PairRec{kNone, kNone, 0};
+            int bit = __builtin_ctzll(m);
+            m &= m - 1;
+            return PairRec{(uint32_t)__builtin_amdgcn_readlane((int)r.a, bit),
+                           (uint32_t)__builtin_amdgcn_readlane((int)r.b, bit),
+                           (uint32_t)__builtin_amdgcn_readlane((int)r.k, bit)};
+        };
+        // in list order, those of small cells two at a time, a half-wave each
         // (a record of a later pair in the same wave may then be tested
         // although an earlier one connected its cells: redundant work only,
         // since pairs kept for the next level are settled there)
-        while (real) {
-            int bit0 = __builtin_ctzll(real);
-            real &= real - 1;
-            PairRec p0{(uint32_t)__shfl((int)r.a, bit0), (uint32_t)__shfl((int)r.b, bit0),
-                       (uint32_t)__shfl((int)r.k, bit0)};
-            PairRec p1{kNone, kNone, 0};
-            if (real) {
-                int bit1 = __builtin_ctzll(real);
-                real &= real - 1;
-                p1 = PairRec{(uint32_t)__shfl((int)r.a, bit1), (uint32_t)__shfl((int)r.b, bit1),
-                             (uint32_t)__shfl((int)r.k, bit1)};
+        while (waves | halves) {
+            const uint64_t all = waves | halves;
+            if ((waves & -waves) == (all & -all)) {
+                test_pair(a, rec(waves), parent, list_out, nout);
+            } else {
+                const PairRec p0 = rec(halves), p1 = rec(halves);
+                test_pair_halves(a, p0, p1, parent, list_out, nout);
             }
-            uint32_t back = test_pair_halves(a, p0, p1, parent, list_out, nout);
-            if (back & 1u) test_pair(a, p0, parent, list_out, nout);
-            if (back & 2u) test_pair(a, p1, parent, list_out, nout);
         }
     }
 }
@@ -2973,7 +2979,7 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
                             G.sncy, (uint32_t)G.m, kc, JP, j0, k, Th[k]};
                 LevelLists LL{parent, lin, lout, tests, tests2, cnts, frec, bstart,
                               gcap, G.ncell, tcap, (uint32_t)K, tovf, shape.ppb, shape.minb,
-                              shape.tpb};
+                              shape.tpb, nj > 1 ? 4u : 1u};
                 // worklist sizes stay on the device: bounded grids stride over them
                 VDB_TRY(c.kt_begin("k_sweep"));
                 k_sweep<<<dim3(shape.maxb, ng), kBlock, 0, c.stream()>>>(a, LL);

@@ -934,15 +934,20 @@ __global__ void __launch_bounds__(kBlock)
 }
 
 // ------------------------------------------------------------ cell pairs
-__device__ __forceinline__ void pair_levels(const double *A, const double *B, const double *Tk,
-                                            int K, int *kmin, int *kfull)
+// no two points of boxes A and B (x0, x1, y0, y1) have a smaller d^2
+__device__ __forceinline__ double pair_min2(const double *A, const double *B)
 {
     double gx = 0.0, gy = 0.0;
     if (B[0] > A[1]) gx = __dsub_rn(B[0], A[1]);
     else if (A[0] > B[1]) gx = __dsub_rn(A[0], B[1]);
     if (B[2] > A[3]) gy = __dsub_rn(B[2], A[3]);
     else if (A[2] > B[3]) gy = __dsub_rn(A[2], B[3]);
-    double smin = __dadd_rn(__dmul_rn(gx, gx), __dmul_rn(gy, gy));
+    return __dadd_rn(__dmul_rn(gx, gx), __dmul_rn(gy, gy));
+}
+__device__ __forceinline__ void pair_levels(const double *A, const double *B, const double *Tk,
+                                            int K, int *kmin, int *kfull)
+{
+    const double smin = pair_min2(A, B);
     double hx = fmax(__dsub_rn(A[1], B[0]), __dsub_rn(B[1], A[0]));
     double hy = fmax(__dsub_rn(A[3], B[2]), __dsub_rn(B[3], A[2]));
     double smax = __dadd_rn(__dmul_rn(hx, hx), __dmul_rn(hy, hy));
@@ -960,22 +965,40 @@ __device__ __forceinline__ void pair_levels(const double *A, const double *B, co
 struct CellPair {
     uint32_t a, b, k; // k = kmin | kfull << 8
 };
+// A thread's walk is a serial chain of loads from L2, so the boxes of the next
+// kPairAhead cells of a row are loaded together, and a row's bounds while the
+// row before it is walked: count and store 2.09 + 1.31 -> 1.35 + 0.68 ms on
+// 256 datasets, 0.46 + 0.28 -> 0.29 + 0.17 on 2M points x 64 variants (both
+// beside the neighbour search), 15 + 11 -> 10 + 6 us on 1,000 points.
+constexpr int kPairAhead = 4;
 template <typename F>
-__device__ __forceinline__ void walk_pairs(const double *box, const uint32_t *row_lo,
-                                           const uint32_t *row_hi, int W, uint32_t A,
-                                           const double *Tk, int K, F f)
+__device__ __forceinline__ void walk_pairs(const double *__restrict__ box,
+                                           const uint32_t *__restrict__ row_lo,
+                                           const uint32_t *__restrict__ row_hi, int W, uint32_t A,
+                                           F f)
 {
     double bA[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) bA[i] = box[4 * (size_t)A + i];
+    const size_t at = (size_t)A * W;
+    uint32_t lo = row_lo[at], hi = row_hi[at];
     for (int r = 0; r < W; r++) {
-        uint32_t lo = row_lo[(size_t)A * W + r], hi = row_hi[(size_t)A * W + r];
-        if (lo <= A) lo = A + 1;
-        for (uint32_t B = lo; B < hi; B++) {
-            int kmin, kfull;
-            pair_levels(bA, box + 4 * (size_t)B, Tk, K, &kmin, &kfull);
-            if (kmin < K) f(B, kmin, kfull);
+        const size_t next = at + (r + 1 < W ? r + 1 : r);
+        const uint32_t nlo = row_lo[next], nhi = row_hi[next];
+        for (uint32_t B = lo <= A ? A + 1 : lo; B < hi; B += kPairAhead) {
+            double bB[kPairAhead][4];
+#pragma unroll
+            for (int i = 0; i < kPairAhead; i++) {
+                const size_t c = B + i < hi ? B + i : hi - 1; // in the row
+#pragma unroll
+                for (int q = 0; q < 4; q++) bB[i][q] = box[4 * c + q];
+            }
+#pragma unroll
+            for (int i = 0; i < kPairAhead; i++)
+                if (B + i < hi) f(B + i, bA, bB[i]);
         }
+        lo = nlo;
+        hi = nhi;
     }
 }
 
@@ -985,17 +1008,20 @@ __global__ void __launch_bounds__(kBlock)
 {
     const uint32_t A = blockIdx.x * kBlock + threadIdx.x;
     if (A >= ncell) return;
+    const double T = Tk[K - 1]; // thresholds ascend
     uint32_t k = 0;
-    walk_pairs(box, row_lo, row_hi, W, A, Tk, K, [&](uint32_t, int, int) { k++; });
+    walk_pairs(box, row_lo, row_hi, W, A, [&](uint32_t, const double *bA, const double *bB) {
+        k += pair_min2(bA, bB) <= T ? 1u : 0u;
+    });
     cnt[A] = k;
 }
 
 // A's pairs are stored from off[A] on (k_pair_count, scanned), a thread per
 // cell as in the count, 12 bytes to a store. Cells of a wave lie side by side,
-// so their stores fill the same lines in L2 soon after one another. 75M pairs
-// of 256 datasets take 1.97 ms beside the neighbour search, 1.4M of one
-// variant 45 us. (A wave per cell over its flattened window: 6.96 ms and 217
-// us. Stores compacted over the wave's 64 cells: 0.97 ms and 28 us, but the
+// so their stores fill the same lines in L2 soon after one another. (With one
+// box loaded at a time the 75M pairs of 256 datasets took 1.97 ms, 1.4M of one
+// variant 45 us; a wave per cell over its flattened window 6.96 ms and 217 us.
+// Stores compacted over the wave's 64 cells: 0.97 ms and 28 us, but the
 // sweep wants a cell's pairs together: 4.1 ms for 3.1.)
 __global__ void __launch_bounds__(kBlock)
     k_pairs(const double *box, const uint32_t *row_lo, const uint32_t *row_hi, int W,
@@ -1004,8 +1030,10 @@ __global__ void __launch_bounds__(kBlock)
     const uint32_t A = blockIdx.x * kBlock + threadIdx.x;
     if (A >= ncell) return;
     out += off[A];
-    walk_pairs(box, row_lo, row_hi, W, A, Tk, K, [&](uint32_t B, int kmin, int kfull) {
-        *out++ = CellPair{A, B, (uint32_t)(kmin | (kfull << 8))};
+    walk_pairs(box, row_lo, row_hi, W, A, [&](uint32_t B, const double *bA, const double *bB) {
+        int kmin, kfull;
+        pair_levels(bA, bB, Tk, K, &kmin, &kfull);
+        if (kmin < K) *out++ = CellPair{A, B, (uint32_t)(kmin | (kfull << 8))};
     });
 }
 

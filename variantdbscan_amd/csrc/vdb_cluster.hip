@@ -1209,7 +1209,13 @@ __global__ void k_cf_points(CellForest F, const uint8_t *core, const uint32_t *c
 // (rank is the binned rank, or any per-root key the caller orders roots by).
 // A thread per point for windows up to kFewCands points, a wave for others;
 // minima stay in the lanes until the end (8 origins a wave with a reduction
-// across lanes per block: 0.57 ms at 1M points, eps 0.4 to 0.6; now 0.25).
+// across lanes per block: 0.57 ms at 1M points, eps 0.4 to 0.6; now 0.12).
+// A walk is a chain of loads (flags and coordinates, then parents, then ranks):
+// a thread takes kBorderNear candidates of each link together, a wave
+// kBorderFar times 64 (1M points, eps 0.4 and 0.6, minpts 100: 160 -> 105 us and
+// 38 -> 16; the thread's count of neighbours, with no such chain, gains nothing
+// from more than 4).
+constexpr int kBorderNear = 8, kBorderFar = 4;
 __global__ void __launch_bounds__(kBlock)
     k_border_near(GridView g, const uint32_t *__restrict__ cell_of_pos, double T,
                   const uint8_t *__restrict__ core, const uint32_t *__restrict__ rank,
@@ -1232,19 +1238,22 @@ __global__ void __launch_bounds__(kBlock)
         uint32_t lo = g.row_lo[t], hi = g.row_hi[t];
         if (lo >= hi) continue;
         uint32_t a = g.cell_start[lo], e = g.cell_start[hi];
-        for (; a < e; a += kFewUnroll) {
-            bool hit[kFewUnroll];
+        for (; a < e; a += kBorderNear) {
+            bool hit[kBorderNear];
 #pragma unroll
-            for (int i = 0; i < kFewUnroll; i++) {
+            for (int i = 0; i < kBorderNear; i++) {
                 uint32_t q = a + i < e ? a + i : e - 1;
-                hit[i] = core[q] && dist2_exact(px, py, g.xs[q], g.ys[q]) <= T;
+                hit[i] = (core[q] != 0) & (dist2_exact(px, py, g.xs[q], g.ys[q]) <= T);
             }
+            uint32_t root[kBorderNear];
 #pragma unroll
-            for (int i = 0; i < kFewUnroll; i++)
-                if (hit[i]) {
-                    uint32_t v = rank[parent[a + i < e ? a + i : e - 1]];
-                    m = v < m ? v : m;
-                }
+            for (int i = 0; i < kBorderNear; i++)
+                root[i] = hit[i] ? parent[a + i < e ? a + i : e - 1] : 0u;
+#pragma unroll
+            for (int i = 0; i < kBorderNear; i++) {
+                uint32_t v = hit[i] ? rank[root[i]] : kNone;
+                m = v < m ? v : m;
+            }
         }
     }
     best[p] = m;
@@ -1264,13 +1273,22 @@ __global__ void __launch_bounds__(kBlock)
         uint32_t m = kNone;
         for (int r = 0; r < g.W; r++) {
             RowSeg sg = row_seg(g, c, r);
-            for (uint32_t q0 = sg.a; q0 < sg.e; q0 += kWave) {
-                uint32_t q = q0 + (uint32_t)lane_id();
-                uint32_t qc = q < sg.e ? q : sg.e - 1;
-                bool hit = q < sg.e && core[qc] &&
-                           dist2_exact(px, py, g.xs[qc], g.ys[qc]) <= T;
-                if (hit) {
-                    uint32_t v = rank[parent[qc]];
+            for (uint32_t q0 = sg.a; q0 < sg.e; q0 += kBorderFar * kWave) {
+                uint32_t qc[kBorderFar];
+                bool hit[kBorderFar];
+#pragma unroll
+                for (int i = 0; i < kBorderFar; i++) {
+                    uint32_t q = q0 + (uint32_t)(i * kWave + lane_id());
+                    qc[i] = q < sg.e ? q : sg.e - 1; // seen twice: the same minimum
+                    hit[i] = (core[qc[i]] != 0) &
+                             (dist2_exact(px, py, g.xs[qc[i]], g.ys[qc[i]]) <= T);
+                }
+                uint32_t root[kBorderFar];
+#pragma unroll
+                for (int i = 0; i < kBorderFar; i++) root[i] = hit[i] ? parent[qc[i]] : 0u;
+#pragma unroll
+                for (int i = 0; i < kBorderFar; i++) {
+                    uint32_t v = hit[i] ? rank[root[i]] : kNone;
                     m = v < m ? v : m;
                 }
             }

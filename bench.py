@@ -70,18 +70,15 @@ BATCH_KERNELS = ("k_knn", "k_sweep", "k_test", "k_labels_all", "k_rows_all", "k_
 
 def batch_kernel_bytes(name, info, W):
     """Algorithmic bytes per step of a batched-engine kernel (summed over its
-    launches; None for k_test and k_roots_min, whose traffic follows the
-    data). info: vdb_batch_info; W: fine-grid window width (2R+1).
-      k_sweep       per record read (a pair entering at its level or carried
-                    from an earlier one) 12; per record the two cells'
-                    parents (8); per record written (carried on or a test
-                    slot) 12
-      k_knn         points read once (16 N), per listed point its position (4),
-                    its L sorted (s, id) entries (12 L) and count (4) written,
-                    per cell its start, key, dataset (12), box (32) and W
-                    window rows (8 W)
-      k_labels_all  per point: rank, cell, packed core levels, list index (16),
-                    per variant its cell label in and staged label out (8 V);
+    launches; None for k_knn, k_test and k_roots_min, whose traffic follows
+    the data). info: vdb_batch_info; W: fine-grid window width (2R+1), an
+    upper bound of the window's rows (strips of columns).
+      k_sweep       per record read (a pair entering at its level, for up to 8
+                    minpts values, or carried from an earlier one) 12; per
+                    record the two cells' parents (8 per minpts value); per
+                    record written (carried on or a test slot) 12
+      k_labels_all  per point: rank, cell, packed core levels (12), per
+                    variant its cell label in and staged label out (8 V);
                     the list walk of non-core points is not counted
       k_rows_all    per point: its position (4), dataset bounds (8), its V
                     staged labels in and V output labels out (8 V)
@@ -89,30 +86,29 @@ def batch_kernel_bytes(name, info, W):
                     the 8 slots' cell labels (32) and its 8 staged labels (32)
       k_rows_from_pos per point: its position (4), dataset bounds (8), its
                     8 staged labels (32) and 8 output labels (32)
-      k_pair_elig   per cell pair: cells and levels (10), both cells' core
-                    levels for each minpts value (2 J), a level byte per
-                    minpts value out (8 per plane of 8 values)
-      k_pair_scatter per cell pair: cells and levels (10) and its level
-                    bytes (8 per plane); per record written (a pair entering
-                    at its level) 12
+      k_pair_elig   per cell pair: its record (12), both cells' core levels
+                    for each minpts value (2 J), a level byte per minpts value
+                    out (8 per plane of 8 values)
+      k_pair_scatter per cell pair: its record (12) and its level bytes (8 per
+                    plane); per record written (a pair entering at its
+                    level) 12
       k_pairs       per cell: its window rows (8 W) and box (32); per stored
-                    pair 10 bytes
+                    pair 12 bytes
       k_pair_count  per cell: window rows (8 W), box (32), count (4)"""
-    n, J, L = info["points"], info["minpts_values"], info["list_len"]
-    nl, nc, npairs = info["listed_points"], info["cells"], info["cell_pairs"]
+    n, J = info["points"], info["minpts_values"]
+    nc, npairs = info["cells"], info["cell_pairs"]
     planes = -(-J // 8)
     V = info.get("snapshots") or info["levels"] * J  # one per requested (level, minpts)
     fr, ca, te = info.get("fresh_pairs", 0), info.get("carried_pairs", 0), info.get("test_records", 0)
     return {
-        "k_sweep": (12 * (fr + ca) + 8 * (fr + ca) + 12 * (ca + te)) if fr + ca else None,
-        "k_labels_all": (16 + 8 * V) * n,
+        "k_sweep": ((12 + 8 * min(J, 8)) * (fr + ca) + 12 * (ca + te)) if fr + ca else None,
+        "k_labels_all": (12 + 8 * V) * n,
         "k_rows_all": (12 + 8 * V) * n,
-        "k_knn": 16 * n + nl * (8 + 12 * L) + nc * (44 + 8 * W),
         "k_labels_j": 77 * n * -(-V // 8),
         "k_rows_from_pos": 76 * n * -(-V // 8),
-        "k_pair_elig": npairs * (10 + 2 * J + 8 * planes),
-        "k_pair_scatter": (npairs * (10 + 8 * planes) + 12 * fr) if fr else None,
-        "k_pairs": nc * (8 * W + 32) + npairs * 10,
+        "k_pair_elig": npairs * (12 + 2 * J + 8 * planes),
+        "k_pair_scatter": (npairs * (12 + 8 * planes) + 12 * fr) if fr else None,
+        "k_pairs": nc * (8 * W + 32) + npairs * 12,
         "k_pair_count": nc * (8 * W + 36),
     }.get(name)
 

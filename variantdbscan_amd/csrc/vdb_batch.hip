@@ -3205,7 +3205,11 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
                            (uint64_t)(uintptr_t)out, (uint64_t)G.ncell, (uint64_t)nlist_cap,
                            (uint64_t)npairs, (uint64_t)tcap, (uint64_t)P.nsets, (uint64_t)L,
                            (uint64_t)K, (uint64_t)J, (uint64_t)jc, (uint64_t)R,
-                           (uint64_t)shape_id})
+                           (uint64_t)shape_id,
+                           // where the data put them: the order's ranks lie in the
+                           // buffer of the sort's last pass, the dataset bounds in
+                           // that of the call's own points
+                           (uint64_t)(uintptr_t)G.pos_rank, (uint64_t)(uintptr_t)P.seg})
             mix(v);
         for (uint32_t v = 0; v < nvar; v++) {
             uint64_t eb;

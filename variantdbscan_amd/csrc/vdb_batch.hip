@@ -146,7 +146,11 @@ __device__ __forceinline__ void cf_hook(uint32_t *parent, uint32_t x, uint32_t m
     if (ret != x && ret != m) cf_unite(parent, ret, m);
 }
 
-// a cell's 8 parents as other waves left them
+// A cell's 8 parents by ordinary loads, which may miss other waves' latest
+// stores: a parent read late is still an ancestor, so equal ones prove the
+// cells connected, and whatever follows from different ones goes through the
+// atomic reads of cf_find or the compare of cf_hook. Lanes that read one cell
+// need not see the same.
 __device__ __forceinline__ void cf_load8(const uint32_t *parent, uint32_t x, uint32_t (&p)[kGroup])
 {
     const uint4 *q = (const uint4 *)(parent + cf_at(x));
@@ -1657,7 +1661,10 @@ __global__ void __launch_bounds__(kBlock) k_sweep(LevelArgs a, LevelLists L)
     chunk_close(chf, lg.far);
 }
 
-// The values of a test record that are still to be connected.
+// The values of a test record that are still to be connected, as this lane
+// sees them: other waves unite cells meanwhile, so lanes given one record may
+// differ, and those that go on with it together take one lane's answer (a lane
+// leaving their loops early would be read as zeros by the others' shuffles).
 __device__ __forceinline__ uint32_t test_open(const PairRec &pr, uint32_t *parent)
 {
     uint32_t pa[kGroup], pb[kGroup], open = 0;
@@ -1710,7 +1717,8 @@ __device__ void test_pair(const LevelArgs &a, const PairRec &pr, uint32_t *paren
         a1 = b1;
         b1 = t;
     }
-    uint32_t open = test_open(pr, parent);
+    uint32_t open =
+        (uint32_t)__builtin_amdgcn_readfirstlane((int)test_open(pr, parent));
     if (!open) return;
     const int lane = lane_id();
     const uint32_t na = a1 - a0, nb = b1 - b0; // both >= 1
@@ -1777,7 +1785,7 @@ __device__ void test_pair_halves(const LevelArgs &a, const PairRec &r0, const Pa
         uint32_t A = pr.a, B = pr.b;
         uint32_t a0 = a.cell_start[A], a1 = a.cell_start[A + 1];
         uint32_t b0 = a.cell_start[B], b1 = a.cell_start[B + 1];
-        uint32_t open = test_open(pr, parent);
+        uint32_t open = __shfl(test_open(pr, parent), 32 * h); // its first lane's
         if (open) {
             if (a1 - a0 > b1 - b0) { // lanes hold the larger cell
                 uint32_t t = A;

@@ -147,7 +147,7 @@ int run_per_variant(Context &c, Points &P, const double *eps, const uint32_t *mi
         Items I;
         Timer t0(c.stream(), st != nullptr);
         // the fused engine in binary64 only asks which points reach the
-        // largest minpts of this eps; the table needs every count, and the
+        // minpts values of this eps; the table needs every count, and the
         // float32 screening reports its rechecks over all of them
         const bool core_only = mode == 0 && precision == VDB_PREC_FP64;
         int k = cells ? cells : kFusedCellsPerEps;
@@ -157,10 +157,9 @@ int run_per_variant(Context &c, Points &P, const double *eps, const uint32_t *mi
         if (st) st->ms_prepare += t0.ms();
         Timer t1(c.stream(), st != nullptr);
         if (core_only) {
-            uint32_t need = 0; // minpts above INT_MAX is never reached
-            for (uint32_t v : kv.second)
-                if (minpts[v] <= 0x7fffffffu) need = std::max(need, minpts[v]);
-            VDB_TRY(count_core(c, G, e, need, counts));
+            std::vector<uint32_t> mp;
+            for (uint32_t v : kv.second) mp.push_back(minpts[v]);
+            VDB_TRY(count_core(c, G, e, mp, counts));
         } else {
             VDB_TRY(count_neighbors(c, G, I, e, precision, counts, (uint64_t *)rc));
         }

@@ -65,8 +65,10 @@ int tune_cells_per_eps(Context &c, const Points &P, double eps, int precision, i
 int count_neighbors(Context &c, const Grid &G, const Items &I, double eps, int precision,
                     uint32_t *counts, uint64_t *recheck_dev);
 
-// counts[p] is >= need exactly when |N_eps(p)| is, and exact below (binary64).
-int count_core(Context &c, const Grid &G, double eps, uint32_t need, uint32_t *counts);
+// counts[p] >= m exactly when |N_eps(p)| >= m, for each of the minpts values m
+// up to INT_MAX (binary64).
+int count_core(Context &c, const Grid &G, double eps, std::vector<uint32_t> minpts,
+               uint32_t *counts);
 
 // Full per-variant clustering; labels written in caller order to out (device).
 // mode 0 = fused (no table), 1 = CSR table (count/scan/fill, union-find over

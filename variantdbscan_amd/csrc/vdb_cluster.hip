@@ -10,6 +10,7 @@
 #include "vdb_cluster.h"
 #include "vdb_prims.h"
 
+#include <algorithm>
 #include <cfloat>
 #include <cmath>
 #include <cstdio>
@@ -369,12 +370,29 @@ __global__ void __launch_bounds__(kBlock)
 }
 
 // ------------------------------------------------------------ core test
-// Counts that only have to tell whether a point has `need` neighbours: they
-// stop there. Windows up to kFewCands points take a thread per point (about
-// 15 vector instructions for 64 candidates of 64 points); the others go, 8
-// origins of a cell at a time, to a wave each, which first adds up the cells
-// accepted whole: where those hold `need` points nothing is tested. At 1M
-// points, eps 0.4, need 100: the exact count (6 to 8 cells per eps) 1.66 ms, this 0.26.
+// Counts that only have to tell which of the call's minpts values a point
+// reaches: they stop at the largest, and where the candidates left cannot bring
+// a point to its next value. Windows up to kFewCands points take a thread per
+// point (about 15 vector instructions for 64 candidates of 64 points); the
+// others go, 8 origins of a cell at a time, to a wave each, which first adds up
+// the cells accepted whole. At 1M points, eps 0.4, minpts 100: the exact count
+// (6 to 8 cells per eps) 1.66 ms, this 0.26; eps 0.9, minpts 100,000: 5.5 ms
+// without the second stop, 4.0 with it.
+constexpr int kNeeds = 8;
+struct Needs {
+    uint32_t m[kNeeds]; // the values ascending, NONE beyond; with more than
+    bool range;         // kNeeds of them any count from low to top may be one
+    uint32_t low, top;
+    // the first value above a count, NONE without one
+    __device__ __forceinline__ uint32_t above(uint32_t cnt) const
+    {
+        if (range) return cnt < low ? low : (cnt < top ? cnt + 1 : kNone);
+        int i = 0;
+#pragma unroll 1
+        while (i < kNeeds && m[i] <= cnt) i++; // (NONE ends it)
+        return i < kNeeds ? m[i] : kNone;
+    }
+};
 
 // append v to list for every lane with take set, one atomic per wave
 __device__ __forceinline__ void list_append(bool take, uint32_t v, uint32_t *list, uint32_t *count)
@@ -389,19 +407,23 @@ __device__ __forceinline__ void list_append(bool take, uint32_t v, uint32_t *lis
 }
 
 __global__ void __launch_bounds__(kBlock)
-    k_core_near(GridView g, const uint32_t *__restrict__ cell_of_pos, double T, uint32_t need,
+    k_core_near(GridView g, const uint32_t *__restrict__ cell_of_pos, double T, uint32_t low,
+                uint32_t top,
                 uint32_t *__restrict__ counts, uint32_t *__restrict__ list,
                 uint32_t *__restrict__ nlist)
 {
     uint32_t p = blockIdx.x * kBlock + threadIdx.x;
     bool valid = p < g.n, far = false;
-    uint32_t c = 0;
+    uint32_t c = 0, window = 0;
     if (valid) {
         c = cell_of_pos[p];
-        far = window_points(g, c) > kFewCands;
+        window = window_points(g, c);
+        far = window > kFewCands;
     }
     list_append(far && (p - g.cell_start[c]) % kOrigins == 0, p, list, nlist);
     if (!valid || far) return;
+    // (a window short of the smallest value counts as none)
+    const uint32_t need = window < low ? 0u : top;
     const double px = g.xs[p], py = g.ys[p];
     uint32_t cnt = 0;
     const int R = g.W / 2;
@@ -424,7 +446,7 @@ __global__ void __launch_bounds__(kBlock)
 }
 
 __global__ void __launch_bounds__(kBlock)
-    k_core_far(GridView g, const uint32_t *__restrict__ cell_of_pos, double T, uint32_t need,
+    k_core_far(GridView g, const uint32_t *__restrict__ cell_of_pos, double T, Needs N,
                uint32_t *__restrict__ counts, const uint32_t *__restrict__ list,
                const uint32_t *__restrict__ nlist)
 {
@@ -436,17 +458,22 @@ __global__ void __launch_bounds__(kBlock)
         const uint32_t o0 = sgpr_u32(list[i]), c = sgpr_u32(cell_of_pos[o0]);
         uint32_t nb = sgpr_u32(g.cell_start[c + 1]) - o0;
         nb = nb < kOrigins ? nb : kOrigins;
-        uint32_t full = 0;
-        for (int r = lane; r < g.W; r += kWave) {
-            RowSeg sg = row_seg(g, c, r);
-            full += sg.f1 - sg.f0;
+        const RowSeg rows = lane_rows(g, c);
+        // points accepted whole, and those to be tested
+        uint32_t full = rows.f1 - rows.f0, left = (rows.f0 - rows.a) + (rows.e - rows.f1);
+        for (int o = kWave / 2; o > 0; o >>= 1) {
+            full += __shfl_xor(full, o);
+            left += __shfl_xor(left, o);
         }
-        for (int o = kWave / 2; o > 0; o >>= 1) full += __shfl_xor(full, o);
         full = sgpr_u32(full);
+        left = sgpr_u32(left);
         uint32_t cnt[kOrigins];
 #pragma unroll
         for (int b = 0; b < kOrigins; b++) cnt[b] = full;
-        if (full < need) {
+        // the first value that not all the origins have reached
+        uint32_t next = N.above(full);
+        bool done = next > full + left;
+        if (!done) {
             double ox[kOrigins], oy[kOrigins];
 #pragma unroll
             for (int b = 0; b < kOrigins; b++) {
@@ -454,25 +481,28 @@ __global__ void __launch_bounds__(kBlock)
                 ox[b] = b < (int)nb ? sgpr_d(g.xs[ob]) : qnan;
                 oy[b] = sgpr_d(g.ys[ob]);
             }
-            bool done = false;
             auto test = [&](uint32_t a, uint32_t e) {
                 for (uint32_t q0 = a; q0 < e && !done; q0 += kWave) {
                     uint32_t q = q0 + (uint32_t)lane;
                     uint32_t qc = q < e ? q : e - 1;
                     double qx = g.xs[qc], qy = g.ys[qc];
                     if (q >= e) qx = qnan;
-                    done = true;
+                    left -= e - q0 < (uint32_t)kWave ? e - q0 : (uint32_t)kWave;
+                    uint32_t least = kNone, most = 0;
 #pragma unroll
                     for (int b = 0; b < kOrigins; b++) {
                         if (b >= (int)nb) break;
                         cnt[b] += (uint32_t)popc64(ballot(dist2_exact(ox[b], oy[b], qx, qy) <= T));
-                        done = done && cnt[b] >= need;
+                        least = cnt[b] < least ? cnt[b] : least;
+                        most = cnt[b] > most ? cnt[b] : most;
                     }
+                    if (least >= next) next = N.above(least);
+                    done = next > most + left;
                 }
             };
             for (int u = 0; u < g.W && !done; u++) {
                 int d = (u & 1) ? -((u + 1) >> 1) : (u >> 1); // centre out
-                RowSeg sg = row_seg(g, c, d + R);
+                RowSeg sg = row_at(rows, d + R);
                 test(sg.a, sg.f0);
                 test(sg.f1, sg.e);
             }
@@ -1785,18 +1815,30 @@ int count_neighbors(Context &c, const Grid &G, const Items &I, double eps, int p
     return kOk;
 }
 
-int count_core(Context &c, const Grid &G, double eps, uint32_t need, uint32_t *counts)
+int count_core(Context &c, const Grid &G, double eps, std::vector<uint32_t> minpts,
+               uint32_t *counts)
 {
     uint32_t n = G.npts;
     uint32_t *list; // a buffer of the label pass, unused until then
     VDB_TRY(c.get("lab.flag", n, &list));
     const double T = threshold_for_eps(eps);
+    // values above INT_MAX are never reached
+    std::sort(minpts.begin(), minpts.end());
+    minpts.erase(std::unique(minpts.begin(), minpts.end()), minpts.end());
+    while (!minpts.empty() && minpts.back() > 0x7fffffffu) minpts.pop_back();
+    Needs N{};
+    N.range = minpts.size() > kNeeds;
+    for (int i = 0; i < kNeeds; i++) N.m[i] = (size_t)i < minpts.size() ? minpts[i] : kNone;
+    if (!minpts.empty()) {
+        N.low = minpts.front();
+        N.top = minpts.back();
+    }
     VDB_TRY(c.kt_begin("k_count"));
     k_core_near<<<ceil_div(n, kBlock), kBlock, 0, c.stream()>>>(
-        view(G, n), G.cell_of_pos, T, need, counts, list, G.words + 2);
+        view(G, n), G.cell_of_pos, T, N.low, N.top, counts, list, G.words + 2);
     VDB_HIP(hipGetLastError());
     k_core_far<<<std::min(ceil_div(n, kWavesPerBlock * kOrigins), kListBlocks), kBlock, 0,
-                 c.stream()>>>(view(G, n), G.cell_of_pos, T, need, counts, list, G.words + 2);
+                 c.stream()>>>(view(G, n), G.cell_of_pos, T, N, counts, list, G.words + 2);
     VDB_TRY(c.kt_end("k_count"));
     VDB_HIP(hipGetLastError());
     return kOk;

@@ -94,10 +94,9 @@ int noalloc_impl(Context &c, const double *x, const double *y, uint32_t n, const
         Items I;
         VDB_TRY(build_eps_grid(c, P, e, k, "g1", G));
         if (precision == VDB_PREC_FP64) {
-            uint32_t need = 0; // minpts above INT_MAX is never reached
-            for (uint32_t v : kv.second)
-                if (minpts[v] <= 0x7fffffffu) need = minpts[v] > need ? minpts[v] : need;
-            VDB_TRY(count_core(c, G, e, need, counts));
+            std::vector<uint32_t> mp;
+            for (uint32_t v : kv.second) mp.push_back(minpts[v]);
+            VDB_TRY(count_core(c, G, e, mp, counts));
         } else {
             VDB_TRY(build_items(c, G, "g1", I));
             VDB_TRY(count_neighbors(c, G, I, e, precision, counts, (uint64_t *)rc));

@@ -3178,9 +3178,11 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
     // per-kernel timing needs host work between launches.
     // Autotuner: the first call of a workload (sizes, levels, minpts values)
     // runs the sequence once per grid shape of kBatchShapes and keeps the
-    // fastest; the choice persists in the tuning cache.
+    // fastest; the choice persists in the tuning cache. Point counts are told
+    // apart to a twelfth, cells and pairs to a factor of two.
     char tkey[160];
-    snprintf(tkey, sizeof tkey, "batch:g8:%u:%u:%d:%d:%u:%d:%d", n, P.nsets, K, J, L,
+    snprintf(tkey, sizeof tkey, "batch:g8:n8:%d:%u:%d:%d:%u:%d:%d",
+             (int)std::floor(8.0 * std::log2((double)n)), P.nsets, K, J, L,
              bits_for((uint64_t)G.ncell + 1), bits_for((uint64_t)npairs + 1));
     int shape_id = 0;
     bool tuned_now = false;

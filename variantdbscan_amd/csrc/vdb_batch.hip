@@ -59,7 +59,13 @@ constexpr BatchShape kBatchShapes[] = {
     {320, 128, 4096, 32, 1024},
 };
 constexpr int kNumBatchShapes = sizeof(kBatchShapes) / sizeof(kBatchShapes[0]);
-constexpr unsigned kMaxPersistent = 4096; // at least any maxb or maxtb of kBatchShapes
+constexpr unsigned max_sweep()
+{
+    unsigned m = 0;
+    for (const BatchShape &s : kBatchShapes) m = s.maxb > m ? s.maxb : m;
+    return m;
+}
+constexpr unsigned kMaxSweep = max_sweep();
 
 struct FG {
     const double *xs, *ys, *box;
@@ -2834,11 +2840,14 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
     const uint32_t nw = (n + 31) / 32;
     const uint32_t ncnt = 3 * ((uint32_t)K + 1);
     const size_t kPassBytes = (size_t)64 << 30;
-    // test lists are filled in chunks (see kRecChunk): room for the records
-    // plus the chunks' unused slots
-    auto test_cap = [&](int j) { // records of a group's test list, j values a pass
-        return (uint64_t)std::min(j, kGroup) * (psz + psz / 2) +
-               (uint64_t)kMaxPersistent * kWPB * kRecChunk + kRecChunk;
+    // room for the records of a group's test list, j values a pass: a record
+    // holds at least one value of a pair; where a level may fill the lists in
+    // chunks (see kRecChunk), the chunks' unused slots too, which for every
+    // call would be 63 MB
+    auto test_cap = [&](int j) {
+        const uint64_t recs = (uint64_t)std::min(j, kGroup) * psz;
+        if (psz < kChunkedFrom) return recs;
+        return recs + recs / 2 + (uint64_t)kMaxSweep * kWPB * kRecChunk + kRecChunk;
     };
     auto fits = [&](int j) {
         const uint64_t per_j =

@@ -2685,7 +2685,12 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
     unsigned gn = ceil_div(n, kBlock);
     uint32_t *lst_idx = nullptr;
     uint32_t nlist_cap = n;
-    if ((size_t)n * L * 5 > ((size_t)8 << 30)) {
+    size_t lists_most = (size_t)8 << 30; // (VDB_BATCH_LIST_BYTES: testing only)
+    if (const char *ev = getenv("VDB_BATCH_LIST_BYTES")) {
+        unsigned long long v = strtoull(ev, nullptr, 10);
+        if (v > 0 && v < lists_most) lists_most = (size_t)v;
+    }
+    if ((size_t)n * L * 5 > lists_most) {
         uint32_t *flag;
         VDB_TRY(c.get("b.flag", n, &flag));
         VDB_TRY(c.get("b.lst_idx", n, &lst_idx));
@@ -2855,8 +2860,15 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
         return test_cap(j) <= 0x7fffffffull && (uint64_t)j * psz <= 0x7fffffffull &&
                (uint64_t)j * per_j <= kPassBytes;
     };
+    // (VDB_BATCH_PASS_VALUES, testing only, bounds the values of a pass, so that
+    // calls of several passes can be exercised on small inputs)
+    unsigned long long most = (unsigned long long)J;
+    if (const char *ev = getenv("VDB_BATCH_PASS_VALUES")) {
+        unsigned long long v = strtoull(ev, nullptr, 10);
+        if (v > 0) most = v;
+    }
     int jc = J;
-    while (jc > 1 && !fits(jc)) {
+    while (jc > 1 && (!fits(jc) || (unsigned long long)jc > most)) {
         int half = ((jc + 1) / 2 + kGroup - 1) / kGroup * kGroup;
         jc = jc > kGroup ? (half < jc ? half : kGroup) : jc > 4 ? 4 : jc > 2 ? 2 : 1;
     }

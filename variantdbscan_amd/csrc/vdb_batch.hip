@@ -324,7 +324,8 @@ struct NearOut {
     uint8_t *lst_lev;
     uint32_t *lst_n;
     uint8_t *kc;
-    uint32_t *kc4;
+    uint32_t *kc4; // by group of 8 minpts values, then position; or null
+    uint32_t n;
     int L, K, J, JP; // JP: J rounded up to whole words of 8 levels
     const uint32_t *mj;
 };
@@ -356,13 +357,14 @@ __device__ __forceinline__ void near_levels(const NearOut &O, uint32_t p, const 
             }
         if (need > 0x7fffffffu) lev = O.K;
         O.kc[(size_t)p * O.JP + j] = (uint8_t)lev;
-        packed |= (uint32_t)(lev & 15) << (4 * (j & 7));
-    }
-    // with J <= 8 and K <= 15 also packed, 4 bits per minpts value, for the
-    // label pass that takes all variants of a call at once
-    if (O.kc4) {
-        packed = group_or<G>(packed);
-        if (gl == 0) O.kc4[p] = packed;
+        // with K <= 15 also packed, 4 bits per minpts value of a group, for the
+        // label pass that takes all levels of a group at once
+        if (O.kc4) {
+            packed |= (uint32_t)lev << (4 * (j & 7));
+            if constexpr (G > 1) packed = group_or<8>(packed);
+            if ((j & 7) == (G > 1 ? 0 : 7)) O.kc4[(size_t)(j >> 3) * O.n + p] = packed;
+            if (G > 1 || (j & 7) == 7) packed = 0;
+        }
     }
 }
 
@@ -795,9 +797,8 @@ __global__ void __launch_bounds__(kBlock)
         if (need > 0x7fffffffu) lj = K;
         if (lane < J) O.kc[(size_t)p * J + lane] = (uint8_t)lj;
         if (O.kc4) {
-            uint32_t w = lane < J ? (uint32_t)(lj & 15) << (4 * (lane & 7)) : 0u;
-            w = group_or<8>(w);
-            if (lane == 0) O.kc4[p] = w;
+            uint32_t w = group_or<8>((uint32_t)(lj & 15) << (4 * (lane & 7)));
+            if (lane < J && (lane & 7) == 0) O.kc4[(size_t)(lane >> 3) * O.n + p] = w;
         }
         const size_t li = O.lst_idx ? O.lst_idx[p] : p;
         if (cut && (uint32_t)lane < cnt) {
@@ -2268,8 +2269,8 @@ __global__ void k_rows_from_pos(LabelSlots S, const uint32_t *pos_of_caller, uin
     }
 }
 
-// Labels of every variant of a pass in one kernel, for passes of at most
-// kAllJ minpts values and kAllK levels. JG >= J lanes to a point, a minpts
+// Labels of all variants of a group of 8 minpts values in one kernel, for at
+// most kAllK levels. JG >= J lanes to a point, a minpts
 // value each: they walk the point's list together, a read of an entry serving
 // all of them, and every lane keeps the smallest root of its border levels. An
 // entry (neighbour q at s = d^2) concerns lane j at the levels
@@ -2288,10 +2289,12 @@ __global__ void k_rows_from_pos(LabelSlots S, const uint32_t *pos_of_caller, uin
 // points x 1 variant 0.085 (0.505).
 constexpr int kAllJ = 8, kAllK = 15, kAllRows = 256, kAllStage = 128;
 struct AllSlots {
-    int J;
-    uint16_t jreq[kAllJ];   // bit k: (j, k) requested
-    uint16_t kreq[16];      // bit j: (j, k) requested
-    const uint2 *snap[16];  // level k's snapshot, kreq[k] values a cell
+    int J, joff;          // values, and those before them in the group's word
+    uint16_t jreq[kAllJ]; // bit k: (j, k) requested
+    struct {              // (one 16-byte load of a lane)
+        const uint2 *snap; // level k's snapshot, the group's first value
+        uint32_t req, ns;  // bit j: (j, k) requested; values of a cell in it
+    } lv[16];
     uint32_t *tmp;
 };
 
@@ -2311,11 +2314,12 @@ __global__ void __launch_bounds__(kBlock)
     const uint32_t req = S.jreq[j];
     // the lane's place in cell c's values at level k
     auto at_level = [&](int k, uint32_t c) {
-        return S.snap[k] + (size_t)c * (uint32_t)__popc(S.kreq[k]) +
-               (uint32_t)__popc(S.kreq[k] & ((1u << j) - 1u));
+        const auto &v = S.lv[k];
+        return v.snap + (size_t)c * v.ns + (uint32_t)__popc(v.req & ((1u << j) - 1u));
     };
     const uint32_t C = cell_of_pos[p];
-    const int kp = (int)((kc4[p] >> (4 * j)) & 15u);
+    const int nibble = 4 * (S.joff + j);
+    const int kp = (int)((kc4[p] >> nibble) & 15u);
     // the requested levels at which p is not core
     const uint32_t border = req & ((1u << kp) - 1u);
     uint2 best[kLds ? 1 : KB];
@@ -2358,7 +2362,7 @@ __global__ void __launch_bounds__(kBlock)
             uint32_t at[kU], cell[kU];
 #pragma unroll
             for (int u = 0; u < kU; u++) {
-                const int kqj = (int)((kq[u] >> (4 * j)) & 15u);
+                const int kqj = (int)((kq[u] >> nibble) & 15u);
                 const int lo = kqj > se[u] ? kqj : se[u];
                 at[u] = border >> lo << lo;
                 cell[u] = cq[u];
@@ -2739,13 +2743,13 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
     const int JP = (J + kGroup - 1) / kGroup * kGroup; // whole words of levels
     uint32_t *cmr;
     VDB_TRY(c.get("b.kc", (size_t)n * JP, &kc));
-    // packed levels for the one-sweep label pass (J <= kAllJ, K <= kAllK)
+    // packed levels for the label pass of whole groups
     uint32_t *kc4 = nullptr;
-    if (J <= kAllJ && K <= kAllK) VDB_TRY(c.get("b.kc4", n, &kc4));
+    if (K <= kAllK) VDB_TRY(c.get("b.kc4", (size_t)n * (JP / kGroup), &kc4));
     uint32_t *mid, *crowd;
     VDB_TRY(c.get("b.mid", n, &mid));
     VDB_TRY(c.get("b.crowd", n, &crowd));
-    const NearOut no{lst_idx, lst_id, lst_lev, lst_n, kc, kc4, (int)L, K, J, JP, dmj};
+    const NearOut no{lst_idx, lst_id, lst_lev, lst_n, kc, kc4, n, (int)L, K, J, JP, dmj};
     const FG fg = fview(G);
     const unsigned gl = std::min(ceil_div(n, kWPB), kListBlocks);
     VDB_TRY(c.kt_begin("k_knn"));
@@ -2916,35 +2920,46 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
     // bitset over ranks with its per-word prefix counts (cluster ids)
     uint32_t *snap_bits, *snap_pre;
     uint2 *snap;
+    uint32_t *labtmp;
     VDB_TRY(c.get("b.snap", 2 * max_slots * G.ncell, (uint32_t **)&snap));
     VDB_TRY(c.get("b.snap_bits", max_slots * nw, &snap_bits));
     VDB_TRY(c.get("b.snap_pre", max_slots * nw, &snap_pre));
-    // one label kernel for the whole call when every minpts value runs in
-    // one pass and the core levels are packed; else a kernel per minpts
-    // value, kLabelSlots snapshots at a time
-    const bool one_sweep = kc4 && jc == J;
-    AllSlots A;
-    std::vector<AllRows> all_rows;
-    int all_kb = 0, all_jg = 0;
-    if (one_sweep) {
+    // a label kernel per group of a pass where the core levels are packed; else
+    // one per minpts value, kLabelSlots snapshots at a time
+    struct LabelGroup {
+        AllSlots A;
+        std::vector<AllRows> rows;
+        int jg;
+    };
+    const int all_kb = K == 1 ? 1 : K <= 4 ? 4 : K <= 8 ? 8 : 16;
+    int most_words = kLabelSlots; // staged words of a point
+    if (kc4) most_words = all_kb * (jc == 1 ? 1 : jc <= 4 ? 4 : 8);
+    VDB_TRY(c.get("b.labtmp", (size_t)most_words * n, &labtmp));
+    // the variants of group g of the pass from j0 on (at most nj values in all),
+    // requested values and slots by level
+    auto label_group = [&](int j0, int nj, int g, const std::vector<uint64_t> &jmask,
+                           const std::vector<uint32_t> &sbase) {
+        LabelGroup G8;
+        AllSlots &A = G8.A;
         memset(&A, 0, sizeof A);
-        A.J = J;
-        size_t nsnap = 0; // snapshots are level-major, as the level passes number them
+        const int jf = j0 + kGroup * g; // first value
+        A.J = std::min(kGroup, nj - kGroup * g);
+        A.joff = jf % kGroup;
+        G8.jg = A.J == 1 ? 1 : A.J <= 4 ? 4 : 8;
+        std::vector<std::pair<uint32_t, uint32_t>> word_row; // (staged word, output row)
         for (int k = 0; k < K; k++) {
-            A.snap[k] = snap + nsnap * G.ncell;
-            for (int j = 0; j < J; j++)
-                if (want.count({k, j})) {
-                    nsnap++;
-                    A.kreq[k] |= (uint16_t)(1u << j);
+            A.lv[k].req = (uint32_t)(jmask[k] >> (kGroup * g)) & 0xffu;
+            A.lv[k].ns = sbase[k + 1] - sbase[k];
+            A.lv[k].snap = snap + (size_t)sbase[k] * G.ncell +
+                           __builtin_popcountll(jmask[k] & ((1ull << (kGroup * g)) - 1ull));
+            for (int j = 0; j < A.J; j++)
+                if ((A.lv[k].req >> j) & 1u) {
                     A.jreq[j] |= (uint16_t)(1u << k);
+                    for (uint32_t v : want[{k, jf + j}])
+                        word_row.push_back({(uint32_t)(j * all_kb + k), rows[v]});
                 }
         }
-        all_kb = K == 1 ? 1 : K <= 4 ? 4 : K <= 8 ? 8 : 16;
-        all_jg = J == 1 ? 1 : J <= 4 ? 4 : 8;
-        std::vector<std::pair<uint32_t, uint32_t>> word_row; // (staged word, output row)
-        for (auto &w : want)
-            for (uint32_t v : w.second)
-                word_row.push_back({(uint32_t)(w.first.second * all_kb + w.first.first), rows[v]});
+        A.tmp = labtmp;
         std::sort(word_row.begin(), word_row.end());
         for (size_t r0 = 0; r0 < word_row.size(); r0 += kAllRows) {
             AllRows R;
@@ -2956,11 +2971,14 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
                 R.first[t] = (uint16_t)(e - r0);
             }
             for (size_t q = r0; q < r1; q++) R.row[q - r0] = word_row[q].second;
-            all_rows.push_back(R);
+            R.out = out;
+            R.nrows = nrows;
+            R.seg = P.seg;
+            R.tmp = labtmp;
+            G8.rows.push_back(R);
         }
-    }
-    uint32_t *labtmp;
-    VDB_TRY(c.get("b.labtmp", (size_t)(one_sweep ? all_kb * all_jg : kLabelSlots) * n, &labtmp));
+        return G8;
+    };
     // label-pass events, read once the batch is done (reading them inside
     // the loop would make the host wait once per pass)
     struct EventList {
@@ -3098,16 +3116,18 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
                 lab_ev.push_back(le1);
                 VDB_HIP(hipEventRecord(le0, c.stream()));
             }
-            if (one_sweep) {
-                A.tmp = labtmp;
+            for (int g = 0; g < ng && kc4; g++) {
+                const LabelGroup G8 = label_group(j0, nj, g, jmask, sbase);
+                if (G8.rows.empty()) continue;
                 VDB_TRY(c.kt_begin("k_labels_all"));
                 auto labels = [&](auto kernel) {
-                    kernel<<<ceil_div(n, kBlock / all_jg), kBlock, 0, c.stream()>>>(
-                        A, G.cell_of_pos, G.pos_rank, kc4, G.cell_start, lst_idx, lst_lev, lst_id,
-                        lst_n, (int)L, n);
+                    kernel<<<ceil_div(n, kBlock / G8.jg), kBlock, 0, c.stream()>>>(
+                        G8.A, G.cell_of_pos, G.pos_rank,
+                        kc4 + (size_t)((j0 + kGroup * g) / kGroup) * n, G.cell_start, lst_idx,
+                        lst_lev, lst_id, lst_n, (int)L, n);
                 };
 #define VDB_LABELS_ALL(KB, JG)                                                                   \
-    if (all_kb == KB && all_jg == JG)                                                            \
+    if (all_kb == KB && G8.jg == JG)                                                             \
         std_rule ? labels(k_labels_all<true, KB, JG>) : labels(k_labels_all<false, KB, JG>)
                 VDB_LABELS_ALL(1, 1);
                 VDB_LABELS_ALL(1, 4);
@@ -3124,16 +3144,12 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
 #undef VDB_LABELS_ALL
                 VDB_TRY(c.kt_end("k_labels_all"));
                 VDB_HIP(hipGetLastError());
-                for (AllRows R : all_rows) {
-                    R.out = out;
-                    R.nrows = nrows;
-                    R.seg = P.seg;
-                    R.tmp = labtmp;
+                for (const AllRows &R : G8.rows) {
                     VDB_TRY(c.kt_begin("k_rows_all"));
                     auto rows_of = [&](auto kernel) {
                         kernel<<<gn, kBlock, 0, c.stream()>>>(R, pos_of_caller, P.nsets, n);
                     };
-                    switch (all_kb * all_jg) {
+                    switch (all_kb * G8.jg) {
                     case 1: rows_of(k_rows_all<1>); break;
                     case 4: rows_of(k_rows_all<4>); break;
                     case 8: rows_of(k_rows_all<8>); break;
@@ -3146,7 +3162,7 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
                     VDB_HIP(hipGetLastError());
                 }
             }
-            for (int jr = 0; jr < nj && !one_sweep; jr++) {
+            for (int jr = 0; jr < nj && !kc4; jr++) {
                 int j = j0 + jr;
                 std::vector<std::pair<int, uint32_t>> rows_j; // (level, variant)
                 for (int k = 0; k < K; k++) {

@@ -1670,8 +1670,9 @@ __global__ void __launch_bounds__(kBlock) k_sweep(LevelArgs a, LevelLists L)
 
 // The values of a test record that are still to be connected, as this lane
 // sees them: other waves unite cells meanwhile, so lanes given one record may
-// differ, and those that go on with it together take one lane's answer (a lane
-// leaving their loops early would be read as zeros by the others' shuffles).
+// differ. Those that go on with it together leave its loops together (a lane
+// that left early would be read as zeros by the others' shuffles); a value that
+// only some of them see open is tested by those, at worst in vain.
 __device__ __forceinline__ uint32_t test_open(const PairRec &pr, uint32_t *parent)
 {
     uint32_t pa[kGroup], pb[kGroup], open = 0;
@@ -1724,9 +1725,8 @@ __device__ void test_pair(const LevelArgs &a, const PairRec &pr, uint32_t *paren
         a1 = b1;
         b1 = t;
     }
-    uint32_t open =
-        (uint32_t)__builtin_amdgcn_readfirstlane((int)test_open(pr, parent));
-    if (!open) return;
+    uint32_t open = test_open(pr, parent);
+    if (!ballot(open != 0)) return;
     const int lane = lane_id();
     const uint32_t na = a1 - a0, nb = b1 - b0; // both >= 1
     const double *bB = a.box + 4 * (size_t)B;
@@ -1739,7 +1739,7 @@ __device__ void test_pair(const LevelArgs &a, const PairRec &pr, uint32_t *paren
     uint32_t pm = core_bits(a, pi);
     const bool bsmall = nb <= (uint32_t)kWave;
     uint32_t found = 0;
-    for (uint32_t p0 = a0; p0 < a1 && open; p0 += kWave) {
+    for (uint32_t p0 = a0; p0 < a1 && ballot(open != 0); p0 += kWave) {
         uint32_t p = p0 + lane;
         if (p0 != a0) { // later chunks of a cell larger than a wave
             uint32_t pc = min(p, a1 - 1);
@@ -1751,12 +1751,12 @@ __device__ void test_pair(const LevelArgs &a, const PairRec &pr, uint32_t *paren
         bool cand =
             p < a1 && (pm & open) && box_dist2_min(px, py, bx0, bx1, by0, by1) <= a.T;
         uint64_t cm = ballot(cand);
-        while (cm && open) {
+        while (cm && ballot(open != 0)) {
             int bit = __builtin_ctzll(cm);
             cm &= cm - 1;
             double cx = __shfl(px, bit), cy = __shfl(py, bit);
             const uint32_t cv = (uint32_t)__builtin_amdgcn_readlane((int)pm, bit) & open;
-            if (!cv) continue;
+            if (!ballot(cv != 0)) continue;
             for (uint32_t q0 = b0; q0 < b1; q0 += kWave) {
                 uint32_t hit = 0;
                 if (bsmall) {
@@ -1770,7 +1770,7 @@ __device__ void test_pair(const LevelArgs &a, const PairRec &pr, uint32_t *paren
                 for (int o = kWave / 2; o > 0; o >>= 1) hit |= __shfl_xor(hit, o);
                 found |= hit;
                 open &= ~hit;
-                if (!(cv & open)) break;
+                if (!ballot((cv & open) != 0)) break;
             }
         }
     }
@@ -1792,8 +1792,9 @@ __device__ void test_pair_halves(const LevelArgs &a, const PairRec &r0, const Pa
         uint32_t A = pr.a, B = pr.b;
         uint32_t a0 = a.cell_start[A], a1 = a.cell_start[A + 1];
         uint32_t b0 = a.cell_start[B], b1 = a.cell_start[B + 1];
-        uint32_t open = __shfl(test_open(pr, parent), 32 * h); // its first lane's
-        if (open) {
+        uint32_t open = test_open(pr, parent);
+        auto any = [&](bool v) { return (uint32_t)(ballot(v) >> (32 * h)) != 0; }; // of the half
+        if (any(open != 0)) {
             if (a1 - a0 > b1 - b0) { // lanes hold the larger cell
                 uint32_t t = A;
                 A = B;
@@ -1817,7 +1818,7 @@ __device__ void test_pair_halves(const LevelArgs &a, const PairRec &r0, const Pa
             bool cand =
                 l < na && (pm & open) && box_dist2_min(px, py, bx0, bx1, by0, by1) <= a.T;
             uint32_t cm = (uint32_t)(ballot(cand) >> (32 * h)), found = 0;
-            while (cm && open) {
+            while (cm && any(open != 0)) {
                 int bit = __builtin_ctz(cm);
                 cm &= cm - 1;
                 double cx = __shfl(px, 32 * h + bit), cy = __shfl(py, 32 * h + bit);

@@ -945,23 +945,11 @@ __global__ void __launch_bounds__(kBlock)
 }
 
 // ------------------------------------------------------------ cell pairs
-// no two points of boxes A and B (x0, x1, y0, y1) have a smaller d^2
-__device__ __forceinline__ double pair_min2(const double *A, const double *B)
-{
-    double gx = 0.0, gy = 0.0;
-    if (B[0] > A[1]) gx = __dsub_rn(B[0], A[1]);
-    else if (A[0] > B[1]) gx = __dsub_rn(A[0], B[1]);
-    if (B[2] > A[3]) gy = __dsub_rn(B[2], A[3]);
-    else if (A[2] > B[3]) gy = __dsub_rn(A[2], B[3]);
-    return __dadd_rn(__dmul_rn(gx, gx), __dmul_rn(gy, gy));
-}
 __device__ __forceinline__ void pair_levels(const double *A, const double *B, const double *Tk,
                                             int K, int *kmin, int *kfull)
 {
-    const double smin = pair_min2(A, B);
-    double hx = fmax(__dsub_rn(A[1], B[0]), __dsub_rn(B[1], A[0]));
-    double hy = fmax(__dsub_rn(A[3], B[2]), __dsub_rn(B[3], A[2]));
-    double smax = __dadd_rn(__dmul_rn(hx, hx), __dmul_rn(hy, hy));
+    const double smin = boxes_dist2_min(A, B);
+    const double smax = boxes_dist2_max(A, B);
     int a = K, b = K;
     for (int k = K - 1; k >= 0; k--) {
         if (smin <= Tk[k]) a = k;
@@ -1022,7 +1010,7 @@ __global__ void __launch_bounds__(kBlock)
     const double T = Tk[K - 1]; // thresholds ascend
     uint32_t k = 0;
     walk_pairs(box, row_lo, row_hi, W, A, [&](uint32_t, const double *bA, const double *bB) {
-        k += pair_min2(bA, bB) <= T ? 1u : 0u;
+        k += boxes_dist2_min(bA, bB) <= T ? 1u : 0u;
     });
     cnt[A] = k;
 }
@@ -2567,16 +2555,6 @@ uint64_t splitmix(uint64_t z)
     z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;
     z = (z ^ (z >> 27)) * 0x94d049bb133111ebull;
     return z ^ (z >> 31);
-}
-
-int read_u32(Context &c, const uint32_t *d, uint32_t *h)
-{
-    void *hs;
-    VDB_TRY(c.host_scratch(sizeof(uint32_t), &hs));
-    VDB_HIP(hipMemcpyAsync(hs, d, sizeof(uint32_t), hipMemcpyDeviceToHost, c.stream()));
-    VDB_HIP(hipStreamSynchronize(c.stream()));
-    *h = *(uint32_t *)hs;
-    return kOk;
 }
 
 } // namespace

@@ -90,31 +90,13 @@ __device__ __forceinline__ void run_blocks(const GridView &g, uint32_t a, uint32
     }
 }
 
-// Visit the window of cell c in 64-candidate blocks. With `half`, only rows
-// below the centre row and the centre row up to (excluding) qmax are visited:
-// every unordered pair inside the window is then seen from one side.
+// Visit the window of cell c in 64-candidate blocks.
 template <class F>
-__device__ __forceinline__ void window_blocks(const GridView &g, uint32_t c, bool half,
-                                              uint32_t qmax, F &&f)
+__device__ __forceinline__ void window_blocks(const GridView &g, uint32_t c, F &&f)
 {
-    int R = g.W / 2;
     for (int r = 0; r < g.W; r++) {
-        int d = r - R;
-        if (half && d > 0) break;
         uint32_t lo = g.row_lo[(size_t)c * g.W + r], hi = g.row_hi[(size_t)c * g.W + r];
-        if (lo >= hi) continue;
-        uint32_t a = g.cell_start[lo], e = g.cell_start[hi];
-        if (half && d == 0 && qmax < e) e = qmax;
-        for (uint32_t q0 = a; q0 < e; q0 += kWave) {
-            uint32_t q = q0 + lane_id();
-            bool v = q < e;
-            // clamp instead of branching; lanes past the run see NaN (never accepted)
-            uint32_t qc = v ? q : e - 1;
-            double qx = g.xs[qc], qy = g.ys[qc];
-            qx = v ? qx : __longlong_as_double(0x7ff8000000000000ll);
-            qy = v ? qy : __longlong_as_double(0x7ff8000000000000ll);
-            f(q, v, qx, qy);
-        }
+        if (lo < hi) run_blocks(g, g.cell_start[lo], g.cell_start[hi], f);
     }
 }
 
@@ -1455,7 +1437,7 @@ __global__ void __launch_bounds__(kBlock)
         any |= cb;
     }
     if (!any) return;
-    window_blocks(g, c, false, 0, [&](uint32_t q, bool v, double qx, double qy) {
+    window_blocks(g, c, [&](uint32_t q, bool v, double qx, double qy) {
         bool qc = v && core[q];
         if (!ballot(qc)) return;
         uint32_t rr = qc ? parent[q] : kNone;

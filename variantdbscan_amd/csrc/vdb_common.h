@@ -56,7 +56,7 @@ __device__ __forceinline__ double dist2_exact(double px, double py, double qx,
     return __dadd_rn(__dmul_rn(dx, dx), __dmul_rn(dy, dy));
 }
 
-// Exact lower / upper bounds of dist2_exact(p, q) over every q inside a box
+// Exact lower bound of dist2_exact(p, q) over every q inside a box
 // [bx0,bx1]x[by0,by1] (bounds taken from actual point coordinates). Rounding
 // is monotone in each operand, so evaluating the formula at the extreme
 // coordinate differences bounds every pair inside the box.
@@ -68,14 +68,6 @@ __device__ __forceinline__ double box_dist2_min(double px, double py, double bx0
     else if (px > bx1) gx = __dsub_rn(px, bx1);
     if (py < by0) gy = __dsub_rn(by0, py);
     else if (py > by1) gy = __dsub_rn(py, by1);
-    return __dadd_rn(__dmul_rn(gx, gx), __dmul_rn(gy, gy));
-}
-
-__device__ __forceinline__ double box_dist2_max(double px, double py, double bx0,
-                                                double bx1, double by0, double by1)
-{
-    double gx = fmax(__dsub_rn(px, bx0), __dsub_rn(bx1, px));
-    double gy = fmax(__dsub_rn(py, by0), __dsub_rn(by1, py));
     return __dadd_rn(__dmul_rn(gx, gx), __dmul_rn(gy, gy));
 }
 
@@ -115,12 +107,6 @@ __device__ __forceinline__ int mask_rank(uint64_t m)
 
 __device__ __forceinline__ int wave_id_in_block() { return threadIdx.x / kWave; }
 
-template <typename T> __device__ __forceinline__ T uniform(T v)
-{
-    // value of lane 0 (caller guarantees the value is wave-uniform)
-    return __shfl(v, 0);
-}
-
 // v of lane (lane ^ J), J a constant power of two below 16, without the LDS
 // permute: DPP moves inside rows of 16 lanes (J = 1, 2: quad permutes; 4:
 // quad reversal then row half-mirror; 8: row rotate by 8).
@@ -137,20 +123,6 @@ template <int J> __device__ __forceinline__ uint32_t lane_xor(uint32_t v)
     } else {
         return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xf, 0xf, false);
     }
-}
-
-// lanes of the wave holding the same key d < 2^BITS (d == 2^BITS: no key, a
-// lane that matches no key lane), from BITS + 1 ballots
-template <int BITS> __device__ __forceinline__ uint64_t bucket_peers(uint32_t d)
-{
-    uint64_t peers = ~0ull;
-#pragma unroll
-    for (int b = 0; b <= BITS; b++) {
-        bool bit = (d >> b) & 1u;
-        uint64_t bal = ballot(bit);
-        peers &= bit ? bal : ~bal;
-    }
-    return peers;
 }
 
 inline unsigned ceil_div(uint64_t a, uint64_t b) { return (unsigned)((a + b - 1) / b); }

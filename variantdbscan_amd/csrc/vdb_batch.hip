@@ -3195,11 +3195,10 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
     // per-kernel timing needs host work between launches.
     // Autotuner: the first call of a workload (sizes, levels, minpts values)
     // runs the sequence once per grid shape of kBatchShapes and keeps the
-    // fastest, after a run that is not timed where the call's buffers are new
-    // (the first to touch them takes longer: with it timed, the first shape was
-    // now and then passed over for one 4% slower); the choice persists in the
-    // tuning cache. Point counts are told apart to a twelfth, cells and pairs
-    // to a factor of two.
+    // fastest; the choice persists in the tuning cache. The first run also
+    // touches the call's new buffers: where it lost, it gets a second one (the
+    // first shape was now and then passed over for one 4% slower). Point counts
+    // are told apart to a twelfth, cells and pairs to a factor of two.
     char tkey[160];
     snprintf(tkey, sizeof tkey, "batch:g8w:n8:%d:%u:%d:%d:%u:%d:%d",
              (int)std::floor(8.0 * std::log2((double)n)), P.nsets, K, J, L,
@@ -3210,16 +3209,18 @@ int cluster_batch(Context &c, const Points &P, const double *eps, const uint32_t
         shape_id = 0;
         if (n >= (1u << 17) && !verbose && !c.kt_active()) {
             float best_ms = 0;
-            if (c.pool_epoch() != epoch0) VDB_TRY(sequence(false, kBatchShapes[0]));
-            for (int t = 0; t < kNumBatchShapes; t++) {
+            auto time_shape = [&](int t) -> int {
                 Ev tt(c.stream(), true);
                 VDB_TRY(sequence(false, kBatchShapes[t]));
                 float ms = (float)tt.ms();
-                if (t == 0 || ms < best_ms) {
+                if (best_ms == 0 || ms < best_ms) {
                     best_ms = ms;
                     shape_id = t;
                 }
-            }
+                return kOk;
+            };
+            for (int t = 0; t < kNumBatchShapes; t++) VDB_TRY(time_shape(t));
+            if (shape_id != 0 && c.pool_epoch() != epoch0) VDB_TRY(time_shape(0));
             tuned_now = true; // the last run's labels are in place
             c.tuned_put(tkey, shape_id);
         }

@@ -514,8 +514,8 @@ def main():
             L.vdb_release()
             torch.cuda.empty_cache()
         out["plain_fp64"] = {"variants_per_s": res["fused"]["variants_per_s"],
-                             "engine": "fused per-variant (grid, count, union-find over the "
-                                       "grid window, labels)",
+                             "engine": "fused per-variant (grid, core test, components over "
+                                       "cells, borders, labels)",
                              "ms_per_eps_level": res["fused"]["ms_per_eps_level"],
                              "table_engine": res["table"],
                              "sample": "minpts 8 at each of the 8 eps levels"}

@@ -60,7 +60,7 @@ int libVDBSCAN(double *inputx, double *inputy, unsigned int datasetSize,
 #define VDB_PATH_AUTO 0    /* batched engine when applicable, else fused */
 #define VDB_PATH_FUSED 1   /* per variant: count, union-find, border; no table */
 #define VDB_PATH_TABLE 2   /* per variant: count/scan/fill CSR table, union-find over it */
-#define VDB_PATH_BATCH 3   /* all variants from one distance-sorted truncated table */
+#define VDB_PATH_BATCH 3   /* all variants from one truncated table with eps levels */
 
 #define VDB_PREC_FP64 0      /* every distance test in binary64 */
 #define VDB_PREC_FP32_RECHECK 1 /* float32 screening, binary64 inside the error band */

@@ -1,7 +1,12 @@
 // Batched variants: all (eps, minpts) pairs of one call from a single fine
-// grid whose cells are verified cliques at the smallest eps, a distance-sorted
-// neighbour list per point truncated at the largest minpts, and union-find over
-// cell pairs, carried across eps levels for each minpts.
+// grid whose cells are verified cliques at the smallest eps, a neighbour list
+// per point with the eps level of each entry, and union-find over cell pairs,
+// carried across eps levels for each minpts.
+//
+// A list is unsorted, and complete only below its point's cutoff, the first
+// level with as many neighbours as the largest minpts (from there on the point
+// is core whatever the minpts); entries at or above the cutoff may be left in
+// it, so readers go by each entry's level.
 #pragma once
 
 #include "vdbscan.h"

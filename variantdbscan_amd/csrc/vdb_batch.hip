@@ -20,7 +20,8 @@
 //     only merge as eps grows); a pair leaves the worklist once connected.
 //     After each level the component roots give the labels of variant (k,j):
 //     core points by the smallest rank of their component, border points by
-//     the smallest such root among the core entries of their list prefix.
+//     the smallest such root among the core entries of their list at levels
+//     up to k (lists are unsorted).
 #include "vdb_batch.h"
 #include "vdb_prims.h"
 
@@ -1445,7 +1446,9 @@ __device__ __forceinline__ void wave_append_cap(bool take, const PairRec &v, Pai
 // A * kRecChunk / (kRecChunk - 63) + kRecChunk per wave.
 constexpr uint32_t kRecChunk = 256;
 // levels with fewer pairs becoming eligible append exactly (one atomic per
-// wave and step; few steps per wave, and the test lists stay dense)
+// wave and step; few steps per wave, and the test lists stay dense): from 2^20
+// on the same times, from 2^24 on the atomics tell, 256 datasets 28.0 ms for
+// 24.2, 8M skewed points 4.85 for 3.48
 constexpr uint32_t kChunkedFrom = 1u << 22;
 struct RecChunk {
     uint32_t at = 0, left = 0; // next free record, records left (wave-uniform)
@@ -2064,8 +2067,8 @@ __global__ void __launch_bounds__(kBlock) k_root_bits(SnapArgs S)
                      1u << (m[j] & 31));
 }
 
-// Labels of up to kLabelSlots variants sharing minpts j, from their level
-// snapshots. Output layout: dataset d (caller indices seg[d] .. seg[d+1]-1)
+// Beyond kAllK levels: labels of up to kLabelSlots variants sharing minpts j,
+// from their level snapshots. Output layout: dataset d (caller indices seg[d] .. seg[d+1]-1)
 // owns the block out + seg[d]*nrows, holding nrows rows of its n_d labels;
 // variant t writes row row[t] of it.
 constexpr int kLabelSlots = 8;

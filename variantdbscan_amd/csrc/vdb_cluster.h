@@ -47,15 +47,21 @@ int build_eps_grid(Context &c, const Points &P, double eps, int k, const char *t
 // (1..kMaxCellsPerEps), else 0 (let tune_cells_per_eps choose).
 constexpr int kMaxCellsPerEps = 8;
 // The fused engine in binary64 (whose counts stop at minpts and whose
-// components run over cells) gains little from finer cells: 1M points, eps 0.4
-// and 0.6, minpts 100, kernel time 2.05, 2.12, 2.26, 2.47 ms at 2, 3, 4, 5.
+// components run over cells) gains little from finer cells up to minpts of about
+// a thousand: calls of 1M points, eps 0.6, at 2, 3, 4 and 8 cells per eps take
+// 1.04, 1.23, 1.49, 2.35 ms for minpts 8, 0.83, 0.82, 0.92, 1.44 for 100 and
+// 0.99, 0.91, 0.96, 1.40 for 1,000; 500,000 skewed points, eps 1, minpts 1,000
+// 0.61, 0.61, 0.65, 0.82. Where few points reach a larger minpts finer cells
+// would pay (minpts 20,000: 3.52, 2.33, 2.12, 2.35), where none do they cost
+// (eps 0.3, minpts 100,000: 0.99, 1.05, 1.11, 1.58), which no call knows
+// beforehand.
 constexpr int kFusedCellsPerEps = 2;
 int cells_per_eps(const vdb_options *opt);
 
-// Autotuner: the first time a workload (point count, extent in eps, precision)
-// is seen, times grid build + count pass (and the components, from resolution
-// 2 on, when they follow) at rising resolutions and keeps the coarsest near the
-// best; later calls reuse the choice. Small inputs skip the timing. Uses the
+// Autotuner: the first time a workload (point count and extent in eps to a
+// twelfth, precision) is seen, times grid build + count pass (and the
+// components, from resolution 2 on, when they follow) at rising resolutions and
+// keeps the coarsest near the best; later calls reuse the choice. Small inputs skip the timing. Uses the
 // "g1" grid slots. requested > 0 is returned unchanged.
 int tune_cells_per_eps(Context &c, const Points &P, double eps, int precision, int requested,
                        bool components, int *k_out);

@@ -367,7 +367,7 @@ __global__ void __launch_bounds__(kBlock)
 // point (about 15 vector instructions for 64 candidates of 64 points); the
 // others go, 8 origins of a cell at a time, to a wave each, which first adds up
 // the cells accepted whole. At 1M points, eps 0.4, minpts 100: the exact count
-// (6 to 8 cells per eps) 1.66 ms, this 0.26; eps 0.9, minpts 100,000: 5.5 ms
+// (6 to 8 cells per eps) 1.66 ms, this 0.17; eps 0.9, minpts 100,000: 5.5 ms
 // without the second stop, 4.0 with it.
 constexpr int kNeeds = 8;
 struct Needs {
